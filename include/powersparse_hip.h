@@ -549,6 +549,13 @@ int ps_pre_gather_workset(int group_size, const uint32_t* perm, int groups,
                           const uint32_t* ranked_vals, const int* col_ind,
                           const float* sp_data, int* out_col, float* out_val,
                           int* out_csr_pos, ps_stream_t stream);
+/* The same for a matrix of `cols` columns (every column id below it): with
+ * fewer column bits, more of the small groups are sorted together. */
+int ps_pre_gather_workset_cols(int group_size, int cols, const uint32_t* perm, int groups,
+                               const int* group_start, const int* residue_offset,
+                               const uint32_t* ranked_vals, const int* col_ind,
+                               const float* sp_data, int* out_col, float* out_val,
+                               int* out_csr_pos, ps_stream_t stream);
 
 #ifdef __cplusplus
 }

@@ -248,6 +248,9 @@ HIP_API = [
     ("ps_pre_gather_workset", ctypes.c_int,
      [ctypes.c_int, c_void_p, ctypes.c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
       c_void_p, c_void_p, c_void_p, c_void_p]),
+    ("ps_pre_gather_workset_cols", ctypes.c_int,
+     [ctypes.c_int, ctypes.c_int, c_void_p, ctypes.c_int, c_void_p, c_void_p, c_void_p, c_void_p,
+      c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
 ]
 
 BENCH_API = [

@@ -10,6 +10,7 @@
 // in fine mode (S == 1) the row is cut into chunks of `fine` nonzeros.
 #include <vector>
 
+#include "ps_block_sort.hpp"
 #include "ps_common.hpp"
 
 namespace ps {
@@ -1003,57 +1004,49 @@ __global__ void gather_small_kernel(int gs, const uint32_t* __restrict__ perm, i
   }
 }
 
-// Blocks of 64 .. 8192 nonzeros: bitonic sort of (column << 32 | ranked index)
-// in LDS, `tile / gs` groups per workgroup.
-__global__ __launch_bounds__(kThreads) void gather_bitonic_kernel(
-    int gs, int tile, const uint32_t* __restrict__ perm, int groups,
+// Blocks of 64 .. 8192 nonzeros: `per_block` groups per workgroup, sorted
+// together in LDS by (group, column), ties in ranked order (the sort is
+// stable and the tile is read in ranked order). A tile is the smallest of
+// 2048, 4096 and 8192 elements that holds a group, so that the short groups'
+// workgroups are small and many run per CU. Against an LDS bitonic sort in one
+// 256-thread workgroup per tile: 50.0 -> 8.4 ms over the 264 M-nonzero C3 build
+// (138 M of them in groups of 8192: 3.1 ms for two passes over them), 2.12 ->
+// 1.32 ms on C1. 64 VGPRs (a few spilled) keep 8 waves per SIMD, i.e. two of
+// the largest tiles per CU.
+template <int NT>
+__global__ __launch_bounds__(NT, 8) void gather_tile_kernel(
+    int gs_log2, int per_block, int col_bits, const uint32_t* __restrict__ perm, int groups,
     const int* __restrict__ group_start, const uint32_t* __restrict__ ranked_vals,
     const int* __restrict__ col_ind, const float* __restrict__ sp_data, int* __restrict__ out_col,
     float* __restrict__ out_val, int* __restrict__ out_pos) {
-  extern __shared__ uint64_t smem[];
-  uint64_t* keys = smem;
-  uint32_t* pos = reinterpret_cast<uint32_t*>(smem + tile);
-  const int per_block = tile / gs;
-  const int first = blockIdx.x * per_block;
-  for (int e = threadIdx.x; e < tile; e += blockDim.x) {
-    const int k = first + e / gs;
-    const int t = e % gs;
-    if (k < groups) {
-      const uint32_t p = ranked_vals[group_start[perm[k]] + t];
-      keys[e] = (uint64_t(uint32_t(col_ind[p])) << 32) | uint32_t(t);
-      pos[e] = p;
-    } else {
-      keys[e] = ~0ull;
-      pos[e] = 0;
-    }
+  using Sort = BlockSort<NT, true>;
+  __shared__ typename Sort::Lds lds;
+  const int first = int(blockIdx.x) * per_block;
+  const int here = groups - first < per_block ? groups - first : per_block;
+  const int valid = here << gs_log2;
+  uint32_t key[kSortItems], p[kSortItems];
+#pragma unroll
+  for (int r = 0; r < kSortItems; ++r) {
+    const int e = Sort::at(r) < valid ? Sort::at(r) : valid - 1;
+    const int k = e >> gs_log2;
+    p[r] = ranked_vals[group_start[perm[first + k]] + (e - (k << gs_log2))];
   }
-  __syncthreads();
-  for (int k2 = 2; k2 <= gs; k2 <<= 1) {
-    for (int j = k2 >> 1; j > 0; j >>= 1) {
-      for (int e = threadIdx.x; e < tile / 2; e += blockDim.x) {
-        const int i = (e / j) * 2 * j + (e % j);
-        const int l = i + j;
-        const bool asc = (k2 == gs) || ((i & k2) == 0);
-        const uint64_t a = keys[i], b = keys[l];
-        if ((a > b) == asc) {
-          keys[i] = b;
-          keys[l] = a;
-          const uint32_t tp = pos[i];
-          pos[i] = pos[l];
-          pos[l] = tp;
-        }
-      }
-      __syncthreads();
-    }
+#pragma unroll
+  for (int r = 0; r < kSortItems; ++r) {
+    const uint32_t k = uint32_t(Sort::at(r)) >> gs_log2;
+    const uint32_t c = uint32_t(col_ind[p[r]]);
+    key[r] = Sort::at(r) < valid ? (per_block > 1 ? k << col_bits : 0u) | c : Sort::kPad;
   }
-  for (int e = threadIdx.x; e < tile; e += blockDim.x) {
-    const int k = first + e / gs;
-    if (k < groups) {
-      const size_t dst = size_t(k) * gs + (e % gs);
-      out_col[dst] = int(keys[e] >> 32);
-      out_val[dst] = sp_data[pos[e]];
-      if (out_pos) out_pos[dst] = int(pos[e]);
-    }
+  Sort::sort(lds, key, p, valid);
+  const uint32_t col_mask = per_block > 1 ? (1u << col_bits) - 1u : ~0u;
+  const size_t dst = size_t(first) << gs_log2;
+#pragma unroll
+  for (int r = 0; r < kSortItems; ++r) {
+    const int e = Sort::at(r);
+    if (e >= valid) continue;
+    out_col[dst + e] = int(key[r] & col_mask);
+    out_val[dst + e] = sp_data[p[r]];
+    if (out_pos) out_pos[dst + e] = int(p[r]);
   }
 }
 
@@ -1138,6 +1131,28 @@ __global__ void window_distinct_kernel(SeqTable seq, uint64_t stride, uint32_t w
   }
   for (int d = 1; d < kWave; d <<= 1) added += __shfl_xor(added, d, kWave);
   if (lane_id() == 0 && added) atomicAdd(&distinct[0], (unsigned long long)added);
+}
+
+// Largest group sorted in LDS: one 1024-thread tile.
+constexpr int kGatherTileMax = 1024 * kSortItems;
+
+// As many groups per tile as fit both the tile and the bits that the columns
+// leave free in a 32-bit key (128 groups of 64 in a tile: columns below 2^27
+// lose nothing).
+template <int NT>
+int gather_tile(int group_size, int cols, const uint32_t* perm, int groups, const int* group_start,
+                const uint32_t* ranked_vals, const int* col_ind, const float* sp_data,
+                int* out_col, float* out_val, int* out_pos, hipStream_t st) {
+  int col_bits = 1;
+  while (col_bits < 31 && (uint32_t(cols) - 1u) >> col_bits) ++col_bits;
+  int per_block = BlockSort<NT, true>::kTile / group_size;
+  while (per_block > 1 && uint64_t(per_block) << col_bits > uint64_t(1) << 32) per_block /= 2;
+  const unsigned grid = unsigned((groups + per_block - 1) / per_block);
+  gather_tile_kernel<NT><<<grid, NT, 0, st>>>(__builtin_ctz(unsigned(group_size)), per_block,
+                                              col_bits, perm, groups, group_start, ranked_vals,
+                                              col_ind, sp_data, out_col, out_val, out_pos);
+  PS_LAUNCHED();
+  return PS_OK;
 }
 
 unsigned grid_for(size_t n) {
@@ -1457,8 +1472,18 @@ int ps_pre_gather_workset(int group_size, const uint32_t* perm, int groups,
                           const int* group_start, const int* residue_offset,
                           const uint32_t* ranked_vals, const int* col_ind, const float* sp_data,
                           int* out_col, float* out_val, int* out_csr_pos, ps_stream_t stream) {
+  return ps_pre_gather_workset_cols(group_size, INT32_MAX, perm, groups, group_start,
+                                    residue_offset, ranked_vals, col_ind, sp_data, out_col, out_val,
+                                    out_csr_pos, stream);
+}
+
+int ps_pre_gather_workset_cols(int group_size, int cols, const uint32_t* perm, int groups,
+                               const int* group_start, const int* residue_offset,
+                               const uint32_t* ranked_vals, const int* col_ind,
+                               const float* sp_data, int* out_col, float* out_val,
+                               int* out_csr_pos, ps_stream_t stream) {
   PS_CHECK_ARG(perm && group_start && ranked_vals && col_ind && sp_data && out_col && out_val &&
-                   groups > 0,
+                   groups > 0 && cols > 0,
                "ps_pre_gather_workset: bad argument");
   PS_CHECK_ARG(group_size == 0 || (group_size >= 32 && (group_size & (group_size - 1)) == 0),
                "ps_pre_gather_workset: group size must be 0 (residue) or a power of two >= 32");
@@ -1473,19 +1498,15 @@ int ps_pre_gather_workset(int group_size, const uint32_t* perm, int groups,
     PS_LAUNCHED();
     return PS_OK;
   }
-  constexpr int kMaxTile = 8192;
-  if (group_size <= kMaxTile) {
-    const int tile = group_size > 1024 ? group_size : 1024;
-    const size_t lds = size_t(tile) * (sizeof(uint64_t) + sizeof(uint32_t));
-    PS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&ps::gather_bitonic_kernel),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-    const int per_block = tile / group_size;
-    const unsigned grid = unsigned((groups + per_block - 1) / per_block);
-    ps::gather_bitonic_kernel<<<grid, ps::kThreads, lds, st>>>(
-        group_size, tile, perm, groups, group_start, ranked_vals, col_ind, sp_data, out_col,
-        out_val, out_csr_pos);
-    PS_LAUNCHED();
-    return PS_OK;
+  if (group_size <= ps::kGatherTileMax) {
+    switch (group_size) {
+      case 8192: return ps::gather_tile<1024>(group_size, cols, perm, groups, group_start, ranked_vals,
+                                              col_ind, sp_data, out_col, out_val, out_csr_pos, st);
+      case 4096: return ps::gather_tile<512>(group_size, cols, perm, groups, group_start, ranked_vals,
+                                             col_ind, sp_data, out_col, out_val, out_csr_pos, st);
+      default: return ps::gather_tile<256>(group_size, cols, perm, groups, group_start, ranked_vals,
+                                           col_ind, sp_data, out_col, out_val, out_csr_pos, st);
+    }
   }
   // Large groups: radix sort on (sorted group index, column).
   const size_t total = size_t(groups) * group_size;

@@ -479,7 +479,7 @@ void PowerSparseMatrixGPU::Build(const int* row_ptr, Prepared& in, bool last_par
       ThrowOnError(ps_malloc(reinterpret_cast<void**>(&_exec_sp_data[s]), sizeof(float) * size));
       if (_keep_csr_pos)
         ThrowOnError(ps_malloc(reinterpret_cast<void**>(&_exec_csr_pos[s]), sizeof(int) * size));
-      ThrowOnError(ps_pre_gather_workset(s == 0 ? 0 : GROUP_SIZE(s), iota.data(), G,
+      ThrowOnError(ps_pre_gather_workset_cols(s == 0 ? 0 : GROUP_SIZE(s), _matrix_col, iota.data(), G,
                                          start[size_t(s)].data(),
                                          s == 0 ? _exec_residue_offset : nullptr, vals.data(),
                                          d_ci.data(), d_sv.data(), _exec_col_ind[s],
@@ -594,7 +594,7 @@ void PowerSparseMatrixGPU::Build(const int* row_ptr, Prepared& in, bool last_par
     ThrowOnError(ps_malloc(reinterpret_cast<void**>(&_workset_sp_data[s]), sizeof(float) * size));
     if (_keep_csr_pos)
       ThrowOnError(ps_malloc(reinterpret_cast<void**>(&_workset_csr_pos[s]), sizeof(int) * size));
-    ThrowOnError(ps_pre_gather_workset(s == 0 ? 0 : GROUP_SIZE(s), perm[size_t(s)].data(), G,
+    ThrowOnError(ps_pre_gather_workset_cols(s == 0 ? 0 : GROUP_SIZE(s), _matrix_col, perm[size_t(s)].data(), G,
                                        start[size_t(s)].data(), s == 0 ? _residue_offset : nullptr,
                                        vals.data(), d_ci.data(), d_sv.data(), _workset_col_ind[s],
                                        _workset_sp_data[s],
