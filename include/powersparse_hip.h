@@ -443,11 +443,17 @@ int ps_pre_rank_keys(const int* row_ptr, int rows, const int* col_ind, int nnz,
  * col_nnz[col], CSR position), sorting only inside rows (rows arrive in
  * order): one wave per row up to 256 nonzeros, an LDS bitonic sort per row up
  * to 8192, a radix sort over the elements of longer rows. count_bits <= 32.
- * Synchronises the stream.
+ * keys may be NULL: only vals is written. Synchronises the stream.
  * Replaces: thrust::sort of NNZPoint (matrix_utils.cu:518-524). */
 int ps_pre_rank_sort(const int* row_ptr, int rows, const int* col_ind, int nnz,
                      const int* col_nnz, int max_count, int count_bits, uint64_t* keys,
                      uint32_t* vals, ps_stream_t stream);
+
+/* keys[i] = row of ranked position i << count_bits: the row half of
+ * ps_pre_rank_sort's keys, all that ps_pre_signatures and
+ * ps_pre_signature_lists read of them. No reference counterpart. */
+int ps_pre_row_keys(const int* row_ptr, int rows, int count_bits, uint64_t* keys,
+                    ps_stream_t stream);
 
 /* Per-row group counts: counts[s * rows + r] = groups of row r in workset s
  * (s = 0 residue). Replaces: GetGroupNumArray (matrix_utils.cu:132-156). */
@@ -516,6 +522,18 @@ int ps_pre_signature_lists(const int* row_ptr, int rows, int group_type_num, int
                            const int* group_num, uint32_t* lists, uint32_t* list_begin,
                            ps_stream_t stream);
 
+/* The same lists group by group, without a sort over all of them: group g of
+ * workset s (its members start at ranked position group_start[s][g], as
+ * ps_pre_group_meta gives them, residue_len[g] of them in workset 0, 32 <<
+ * (s - 1) in workset s) gets lists[list_at[q] .. list_end[q]), q its global
+ * number, inside its members' own nnz-sized range. Worksets of groups of more
+ * than 8192 nonzeros must be empty; ps_pre_signature_lists takes those.
+ * Replaces: GetResidueSignature / GetBlockSignature (matrix_utils.cu:261-327). */
+int ps_pre_group_lists(int group_type_num, const int* group_num, const int* const* group_start,
+                       const int* residue_len, const uint32_t* ranked_vals, const int* col_ind,
+                       const int* sigbit, int signature_len, uint32_t* lists, uint32_t* list_at,
+                       uint32_t* list_end, ps_stream_t stream);
+
 /* perm[s][k] = the group of workset s at position k of the stable descending
  * signature order, from the lists of ps_pre_signature_lists: the same order as
  * the per-word stable sorts. Ties are refined in rounds: each class of tied
@@ -528,6 +546,11 @@ int ps_pre_signature_lists(const int* row_ptr, int rows, int group_type_num, int
 int ps_pre_signature_order(const uint32_t* lists, const uint32_t* list_begin,
                            int group_type_num, const int* group_num, int signature_len,
                            uint32_t* const* perm, ps_stream_t stream);
+/* The same with group q's list at lists[list_begin[q] .. list_end[q]). */
+int ps_pre_signature_order_spans(const uint32_t* lists, const uint32_t* list_begin,
+                                 const uint32_t* list_end, int group_type_num,
+                                 const int* group_num, int signature_len, uint32_t* const* perm,
+                                 ps_stream_t stream);
 
 /* Final metadata in sorted order: des[k] = src_des[perm[k]]; for the residue
  * workset also len[k] = src_len[perm[k]] and atomic[k] = src_atomic[perm[k]].

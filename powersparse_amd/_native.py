@@ -242,6 +242,14 @@ HIP_API = [
     ("ps_pre_signature_order", ctypes.c_int,
      [c_void_p, c_void_p, ctypes.c_int, c_int_p, ctypes.c_int, ctypes.POINTER(c_void_p),
       c_void_p]),
+    ("ps_pre_group_lists", ctypes.c_int,
+     [ctypes.c_int, c_int_p, ctypes.POINTER(c_void_p), c_void_p, c_void_p, c_void_p, c_void_p,
+      ctypes.c_int, c_void_p, c_void_p, c_void_p, c_void_p]),
+    ("ps_pre_signature_order_spans", ctypes.c_int,
+     [c_void_p, c_void_p, c_void_p, ctypes.c_int, c_int_p, ctypes.c_int, ctypes.POINTER(c_void_p),
+      c_void_p]),
+    ("ps_pre_row_keys", ctypes.c_int,
+     [c_void_p, ctypes.c_int, ctypes.c_int, c_void_p, c_void_p]),
     ("ps_pre_permute_meta", ctypes.c_int,
      [c_void_p, ctypes.c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
       c_void_p]),

@@ -108,8 +108,8 @@ __global__ void rank_keys_kernel(const int* __restrict__ row_ptr, int rows,
 // counted against the others. 257 .. 8192: one workgroup per row, bitonic sort of
 // (count key, index) pairs in LDS. Longer rows: their elements are compacted
 // and radix-sorted (stable) with the row's list index in the high bits.
-// Output as the stable sort of (row, count key): keys = row << count_bits |
-// count key, vals = CSR position.
+// Output as the stable sort of (row, count key): keys (when asked for) = row <<
+// count_bits | count key, vals = CSR position.
 constexpr int kRankTileSmall = 1024, kRankTileLarge = 8192;
 
 __device__ __forceinline__ uint32_t count_key(const int* __restrict__ col_ind,
@@ -159,7 +159,7 @@ __global__ void rank_small_kernel(const int* __restrict__ row_ptr, int rows,
   for (int q = 0; q < kRankWavePer; ++q) {
     const int j = q * kWave + lane;
     if (j < d) {
-      keys[b + rank[q]] = (uint64_t(r) << count_bits) | ck[q];
+      if (keys) keys[b + rank[q]] = (uint64_t(r) << count_bits) | ck[q];
       vals[b + rank[q]] = uint32_t(b + j);
     }
   }
@@ -197,7 +197,7 @@ __global__ __launch_bounds__(kThreads) void rank_tile_kernel(
   }
   for (int e = threadIdx.x; e < d; e += blockDim.x) {
     const uint64_t v = pairs[e];
-    keys[b + e] = (uint64_t(r) << count_bits) | (v >> 32);
+    if (keys) keys[b + e] = (uint64_t(r) << count_bits) | (v >> 32);
     vals[b + e] = uint32_t(b) + uint32_t(v & 0xFFFFFFFFu);
   }
 }
@@ -270,9 +270,18 @@ __global__ void rank_long_write_kernel(size_t total, const uint64_t* __restrict_
     const uint32_t i = uint32_t(ck[j] >> count_bits);
     const int r = int(list[i]);
     const size_t out = size_t(row_ptr[r]) + (j - seg_start[i]);
-    keys[out] = (uint64_t(r) << count_bits) | (ck[j] & mask);
+    if (keys) keys[out] = (uint64_t(r) << count_bits) | (ck[j] & mask);
     vals[out] = cv[j];
   }
+}
+
+// keys[i] = row of ranked position i << count_bits, one wave per row.
+__global__ void row_keys_kernel(const int* __restrict__ row_ptr, int rows, int count_bits,
+                                uint64_t* __restrict__ keys) {
+  const int waves = blockDim.x / kWave;
+  for (int r = blockIdx.x * waves + threadIdx.x / kWave; r < rows; r += gridDim.x * waves)
+    for (int p = row_ptr[r] + lane_id(); p < row_ptr[r + 1]; p += kWave)
+      keys[p] = uint64_t(r) << count_bits;
 }
 
 // counts[s * (rows + 1) + r]; the extra entry per workset stays 0 so that the
@@ -453,6 +462,122 @@ __global__ void entry_lists_kernel(const uint64_t* __restrict__ e, uint32_t n, i
   }
 }
 
+// Lists straight from the groups: a group's members are consecutive ranked
+// positions, so its list is sorted and stripped of repeats by the wave or the
+// workgroup that reads them, and written where its members start: lists
+// [at[g], end[g]), with gaps. Ranked members come in nearly bit order already
+// (the bits follow the column counts; only ties mix them), and a signature of
+// a few thousand bits takes two digits, so a tile sorts in 0 to 2 passes.
+__device__ __forceinline__ uint32_t member_bit(uint32_t p, const int* __restrict__ col_ind,
+                                               const int* __restrict__ sigbit) {
+  return uint32_t(sigbit[col_ind[p]]);
+}
+
+// Groups of at most 32 members (len null: all 32), one 32-lane half wave per
+// group: members ranked against each other, then the repeats dropped.
+__global__ __launch_bounds__(kThreads) void group_lists_small_kernel(
+    int groups, const int* __restrict__ start, const int* __restrict__ len,
+    const uint32_t* __restrict__ ranked_vals, const int* __restrict__ col_ind,
+    const int* __restrict__ sigbit, uint32_t* __restrict__ lists, uint32_t* __restrict__ at,
+    uint32_t* __restrict__ end) {
+  __shared__ uint32_t sorted[kThreads];
+  const int k = int(blockIdx.x) * (kThreads / 32) + int(threadIdx.x) / 32;
+  const int t = threadIdx.x & 31, half = lane_id() & 32;
+  uint32_t* const mine = sorted + (threadIdx.x & ~31u);
+  const int n = k < groups ? (len ? len[k] : 32) : 0;
+  const int b = k < groups ? start[k] : 0;
+  const uint32_t bit = t < n ? member_bit(ranked_vals[b + t], col_ind, sigbit) : 0xFFFFFFFFu;
+  int rank = 0;
+#pragma unroll 8
+  for (int u = 0; u < 32; ++u) {
+    const uint32_t other = uint32_t(__shfl(int(bit), half + u, kWave));
+    rank += other < bit || (other == bit && u < t);
+  }
+  mine[rank] = bit;
+  wave_lds_sync();
+  const uint32_t v = mine[t];
+  const bool first = t < n && (t == 0 || v != mine[t - 1]);
+  const uint32_t firsts = uint32_t(__ballot(first) >> half);
+  if (first) lists[b + __popc(firsts & ((1u << t) - 1u))] = v;
+  if (t == 0 && k < groups) {
+    at[k] = uint32_t(b);
+    end[k] = uint32_t(b + __popc(firsts));
+  }
+}
+
+// Groups of 64 .. 8192 members, `per_block` of them sorted in one LDS tile.
+template <int NT>
+__global__ __launch_bounds__(NT, 8) void group_lists_tile_kernel(
+    int gs_log2, int per_block, int bit_bits, int groups, const int* __restrict__ start,
+    const uint32_t* __restrict__ ranked_vals, const int* __restrict__ col_ind,
+    const int* __restrict__ sigbit, uint32_t* __restrict__ lists, uint32_t* __restrict__ at,
+    uint32_t* __restrict__ end) {
+  using Sort = BlockSort<NT, false>;
+  __shared__ typename Sort::Lds lds;
+  constexpr int kRows = Sort::kTile / kWave;  // rows of 64 elements
+  __shared__ uint32_t before[kRows + 1];      // first-of-their-value elements before a row
+  const int first_group = int(blockIdx.x) * per_block;
+  const int here = groups - first_group < per_block ? groups - first_group : per_block;
+  const int valid = here << gs_log2;
+  uint32_t key[kSortItems], unused[kSortItems];
+#pragma unroll
+  for (int r = 0; r < kSortItems; ++r) {
+    const int e = Sort::at(r) < valid ? Sort::at(r) : valid - 1;
+    const int k = e >> gs_log2;
+    key[r] = ranked_vals[start[first_group + k] + (e - (k << gs_log2))];
+    unused[r] = 0;
+  }
+#pragma unroll
+  for (int r = 0; r < kSortItems; ++r) {
+    const uint32_t k = uint32_t(Sort::at(r)) >> gs_log2;
+    const uint32_t bit = member_bit(key[r], col_ind, sigbit);
+    key[r] = Sort::at(r) < valid ? (per_block > 1 ? k << bit_bits : 0u) | bit : Sort::kPad;
+  }
+  Sort::sort(lds, key, unused, valid);
+  const int w = int(threadIdx.x) / kWave, lane = lane_id();
+  uint64_t firsts[kSortItems];
+#pragma unroll
+  for (int r = 0; r < kSortItems; ++r) {
+    const int e = Sort::at(r);
+    firsts[r] = __ballot(e < valid && (e == 0 || lds.key[e] != lds.key[e - 1]));
+    if (lane == 0) before[w * kSortItems + r] = uint32_t(__popcll(firsts[r]));
+  }
+  __syncthreads();
+  if (threadIdx.x < kWave) {  // exclusive scan of the rows' counts
+    uint32_t run = 0;
+    for (int q = 0; q < kRows; q += kWave) {
+      uint32_t incl = q + lane < kRows ? before[q + lane] : 0u;
+      const uint32_t own = incl;
+      for (int d = 1; d < kWave; d <<= 1) {
+        const uint32_t t = uint32_t(__shfl_up(int(incl), d, kWave));
+        if (lane >= d) incl += t;
+      }
+      if (q + lane < kRows) before[q + lane] = run + incl - own;
+      run += uint32_t(__shfl(int(incl), kWave - 1, kWave));
+    }
+    if (lane == 0) before[kRows] = run;
+  }
+  __syncthreads();
+  const uint32_t bit_mask = per_block > 1 ? (1u << bit_bits) - 1u : ~0u;
+#pragma unroll
+  for (int r = 0; r < kSortItems; ++r) {
+    const int e = Sort::at(r);
+    if (e >= valid) continue;
+    const int k = e >> gs_log2, e0 = k << gs_log2;  // the group and its first element
+    if ((firsts[r] >> lane) & 1u) {
+      const uint32_t rank = before[e / kWave] +
+                            uint32_t(__popcll(firsts[r] & ((uint64_t(1) << lane) - 1u))) -
+                            before[e0 / kWave];
+      lists[uint32_t(start[first_group + k]) + rank] = lds.key[e] & bit_mask;
+    }
+    if (e == e0) {
+      const uint32_t b = uint32_t(start[first_group + k]);
+      at[first_group + k] = b;
+      end[first_group + k] = b + before[(e0 + (1 << gs_log2)) / kWave] - before[e0 / kWave];
+    }
+  }
+}
+
 // Refinement. The active groups (still tied with another group of their
 // class) are kept in class order, each with its class base (final position
 // of the class's first member) and class depth (all members have equal lists
@@ -483,12 +608,13 @@ __global__ void order_init_kernel(uint32_t n, GroupBase gb, uint32_t* __restrict
 }
 
 // Longest list (bounds the divergence depth).
-__global__ void max_list_kernel(const uint32_t* __restrict__ list_begin, uint32_t groups,
+__global__ void max_list_kernel(const uint32_t* __restrict__ list_begin,
+                                const uint32_t* __restrict__ list_end, uint32_t groups,
                                 uint32_t* __restrict__ out) {
   uint32_t m = 0;
   for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < groups;
        g += gridDim.x * blockDim.x)
-    m = max(m, list_begin[g + 1] - list_begin[g]);
+    m = max(m, list_end[g] - list_begin[g]);
   for (int d = 1; d < kWave; d <<= 1) m = max(m, uint32_t(__shfl_xor(int(m), d, kWave)));
   if (lane_id() == 0) atomicMax(out, m);
 }
@@ -515,6 +641,7 @@ __global__ void order_diverge_kernel(const uint32_t* __restrict__ act_group,
                                      const uint32_t* __restrict__ act_depth, uint32_t n,
                                      const uint32_t* __restrict__ lists,
                                      const uint32_t* __restrict__ list_begin,
+                                     const uint32_t* __restrict__ list_end,
                                      const uint32_t* __restrict__ head,
                                      const uint32_t* __restrict__ rank,
                                      const uint32_t* __restrict__ head_at, uint32_t end,
@@ -527,8 +654,8 @@ __global__ void order_diverge_kernel(const uint32_t* __restrict__ act_group,
     const uint32_t r = act_group[head_at[c]];
     const uint32_t* m = lists + list_begin[g];
     const uint32_t* q = lists + list_begin[r];
-    const uint32_t nm = list_begin[g + 1] - list_begin[g];
-    const uint32_t nq = list_begin[r + 1] - list_begin[r];
+    const uint32_t nm = list_end[g] - list_begin[g];
+    const uint32_t nq = list_end[r] - list_begin[r];
     uint32_t d = act_depth[i];
     if (g != r)
       while (d < nm && d < nq && m[d] == q[d]) ++d;
@@ -621,8 +748,8 @@ __device__ void block_scan(uint32_t* v, uint32_t* wsum) {
 __global__ __launch_bounds__(kFinishThreads) void order_finish_kernel(
     uint32_t n0, const uint32_t* __restrict__ act_group, const uint32_t* __restrict__ act_base,
     const uint32_t* __restrict__ act_depth, const uint32_t* __restrict__ lists,
-    const uint32_t* __restrict__ list_begin, uint32_t end, uint32_t max_len, int lo_bits,
-    GroupBase gb, SigTable perm, uint32_t* __restrict__ status) {
+    const uint32_t* __restrict__ list_begin, const uint32_t* __restrict__ list_end, uint32_t end,
+    uint32_t max_len, int lo_bits, GroupBase gb, SigTable perm, uint32_t* __restrict__ status) {
   extern __shared__ __attribute__((aligned(16))) uint64_t finish_lds[];
   constexpr int P = kFinishMax;
   uint64_t* key = finish_lds;                            // [P]
@@ -678,8 +805,8 @@ __global__ __launch_bounds__(kFinishThreads) void order_finish_kernel(
       const uint32_t r = grp[t1[c]];
       const uint32_t* m = lists + list_begin[g];
       const uint32_t* rq = lists + list_begin[r];
-      const uint32_t nm = list_begin[g + 1] - list_begin[g];
-      const uint32_t nq = list_begin[r + 1] - list_begin[r];
+      const uint32_t nm = list_end[g] - list_begin[g];
+      const uint32_t nq = list_end[r] - list_begin[r];
       uint32_t d = dep[e];
       if (g != r)
         while (d < nm && d < nq && m[d] == rq[d]) ++d;
@@ -1260,7 +1387,7 @@ int ps_pre_rank_keys(const int* row_ptr, int rows, const int* col_ind, int nnz,
 int ps_pre_rank_sort(const int* row_ptr, int rows, const int* col_ind, int nnz,
                      const int* col_nnz, int max_count, int count_bits, uint64_t* keys,
                      uint32_t* vals, ps_stream_t stream) {
-  PS_CHECK_ARG(row_ptr && col_ind && col_nnz && keys && vals && nnz > 0 && rows > 0,
+  PS_CHECK_ARG(row_ptr && col_ind && col_nnz && vals && nnz > 0 && rows > 0,
                "ps_pre_rank_sort: bad argument");
   PS_CHECK_ARG(count_bits >= 0 && count_bits <= 32 &&
                    count_bits + ps::bits_for(uint64_t(rows - 1)) <= 64,
@@ -1352,6 +1479,17 @@ int ps_pre_rank_sort(const int* row_ptr, int rows, const int* col_ind, int nnz,
     PS_HIP(hipStreamSynchronize(st));
   }
   PS_HIP(hipStreamSynchronize(st));
+  return PS_OK;
+}
+
+int ps_pre_row_keys(const int* row_ptr, int rows, int count_bits, uint64_t* keys,
+                    ps_stream_t stream) {
+  PS_CHECK_ARG(row_ptr && keys && rows > 0 && count_bits >= 0 &&
+                   count_bits + ps::bits_for(uint64_t(rows - 1)) <= 64,
+               "ps_pre_row_keys: bad argument");
+  ps::row_keys_kernel<<<ps::grid_for(size_t(rows) * 64), ps::kThreads, 0, ps::to_hip(stream)>>>(
+      row_ptr, rows, count_bits, keys);
+  PS_LAUNCHED();
   return PS_OK;
 }
 
@@ -1610,6 +1748,57 @@ int ps_pre_locality_score(int count, const int* const* col_ind, const long long*
   return PS_OK;
 }
 
+int ps_pre_group_lists(int group_type_num, const int* group_num, const int* const* group_start,
+                       const int* residue_len, const uint32_t* ranked_vals, const int* col_ind,
+                       const int* sigbit, int signature_len, uint32_t* lists, uint32_t* list_at,
+                       uint32_t* list_end, ps_stream_t stream) {
+  PS_CHECK_ARG(group_num && group_start && ranked_vals && col_ind && sigbit &&
+                   lists && list_at && list_end && group_type_num >= 1 &&
+                   group_type_num <= PS_MAX_WORKSETS && signature_len >= 1,
+               "ps_pre_group_lists: bad argument");
+  hipStream_t st = ps::to_hip(stream);
+  int bit_bits = 1;
+  while (bit_bits < 31 && (uint32_t(signature_len) - 1u) >> bit_bits) ++bit_bits;
+  size_t base = 0;  // global number of the workset's first group
+  for (int s = 0; s < group_type_num; ++s) {
+    const int G = group_num[s];
+    if (G <= 0) continue;
+    const int gs = s == 0 ? 0 : 32 << (s - 1);
+    PS_CHECK_ARG(gs <= ps::kGatherTileMax, "ps_pre_group_lists: groups of more than " +
+                                               std::to_string(ps::kGatherTileMax) + " nonzeros");
+    PS_CHECK_ARG(group_start[s] && (s > 0 || residue_len),
+                 "ps_pre_group_lists: missing group starts or lengths");
+    uint32_t* const at = list_at + base;
+    uint32_t* const end = list_end + base;
+    if (gs <= 32) {
+      const size_t threads = size_t(G) * 32;
+      ps::group_lists_small_kernel<<<unsigned((threads + ps::kThreads - 1) / ps::kThreads),
+                                     ps::kThreads, 0, st>>>(G, group_start[s],
+                                                            s == 0 ? residue_len : nullptr,
+                                                            ranked_vals, col_ind, sigbit, lists,
+                                                            at, end);
+    } else {
+      const int log2 = __builtin_ctz(unsigned(gs));
+      const int tile = gs <= 2048 ? 2048 : gs;
+      int per_block = tile / gs;
+      while (per_block > 1 && uint64_t(per_block) << bit_bits > uint64_t(1) << 32) per_block /= 2;
+      const unsigned grid = unsigned((G + per_block - 1) / per_block);
+      auto launch = [&](auto nt) {
+        constexpr int NT = decltype(nt)::value;
+        ps::group_lists_tile_kernel<NT><<<grid, NT, 0, st>>>(log2, per_block, bit_bits, G,
+                                                             group_start[s], ranked_vals, col_ind,
+                                                             sigbit, lists, at, end);
+      };
+      if (tile == 8192) launch(std::integral_constant<int, 1024>{});
+      else if (tile == 4096) launch(std::integral_constant<int, 512>{});
+      else launch(std::integral_constant<int, 256>{});
+    }
+    PS_LAUNCHED();
+    base += size_t(G);
+  }
+  return PS_OK;
+}
+
 int ps_pre_signature_lists(const int* row_ptr, int rows, int group_type_num, int fine,
                            const uint64_t* ranked_keys, int count_bits,
                            const uint32_t* ranked_vals, int nnz, const int* col_ind,
@@ -1707,7 +1896,16 @@ extern "C" {
 int ps_pre_signature_order(const uint32_t* lists, const uint32_t* list_begin,
                            int group_type_num, const int* group_num, int signature_len,
                            uint32_t* const* perm, ps_stream_t stream) {
-  PS_CHECK_ARG(lists && list_begin && group_num && perm && group_type_num >= 1 &&
+  PS_CHECK_ARG(list_begin, "ps_pre_signature_order: bad argument");
+  return ps_pre_signature_order_spans(lists, list_begin, list_begin + 1, group_type_num, group_num,
+                                      signature_len, perm, stream);
+}
+
+int ps_pre_signature_order_spans(const uint32_t* lists, const uint32_t* list_begin,
+                                 const uint32_t* list_end, int group_type_num,
+                                 const int* group_num, int signature_len, uint32_t* const* perm,
+                                 ps_stream_t stream) {
+  PS_CHECK_ARG(lists && list_begin && list_end && group_num && perm && group_type_num >= 1 &&
                    group_type_num <= PS_MAX_WORKSETS && signature_len >= 1,
                "ps_pre_signature_order: bad argument");
   ps::GroupBase gb{};
@@ -1765,7 +1963,8 @@ int ps_pre_signature_order(const uint32_t* lists, const uint32_t* list_begin,
   PS_HIP(hipMemsetAsync(max_len_dev, 0, 4, st));
   {
     unsigned gx = ps::grid_for(n0);
-    ps::max_list_kernel<<<gx < 1024 ? gx : 1024, ps::kThreads, 0, st>>>(list_begin, total,
+    ps::max_list_kernel<<<gx < 1024 ? gx : 1024, ps::kThreads, 0, st>>>(list_begin, list_end,
+                                                                        total,
                                                                         max_len_dev);
     PS_LAUNCHED();
   }
@@ -1793,7 +1992,7 @@ int ps_pre_signature_order(const uint32_t* lists, const uint32_t* list_begin,
       PS_HIP(hipMemsetAsync(max_len_dev, 0, 4, st));
       const size_t lds = ps::kFinishLds;
       ps::order_finish_kernel<<<1, ps::kFinishThreads, lds, st>>>(
-          n, act_group, act_base, act_depth, lists, list_begin, end, max_len, lo_bits, gb, out,
+          n, act_group, act_base, act_depth, lists, list_begin, list_end, end, max_len, lo_bits, gb, out,
           max_len_dev);
       PS_LAUNCHED();
       PS_HIP(hipMemcpyAsync(&flag, max_len_dev, 4, hipMemcpyDeviceToHost, st));
@@ -1812,7 +2011,7 @@ int ps_pre_signature_order(const uint32_t* lists, const uint32_t* list_begin,
     ps::order_class_start_kernel<<<grid, ps::kThreads, 0, st>>>(n, head, rank, head_at);
     PS_LAUNCHED();
     ps::order_diverge_kernel<<<grid, ps::kThreads, 0, st>>>(
-        act_group, act_depth, n, lists, list_begin, head, rank, head_at, end, max_len, hi, lo,
+        act_group, act_depth, n, lists, list_begin, list_end, head, rank, head_at, end, max_len, hi, lo,
         lcp, idx);
     PS_LAUNCHED();
     // Sort by (hi, lo): one pass over the combined key when it fits 64 bits,

@@ -236,7 +236,6 @@ struct PowerSparseMatrixGPU::Prepared {
   std::vector<int> col_nnz_host, sigbit;
   int max_count = 0, count_bits = 0;
   // Each row's nonzeros ranked by column count (descending, ties in CSR order).
-  DeviceArray<uint64_t> keys;
   DeviceArray<uint32_t> vals;
   DeviceArray<int> sigbit_device;
   int signature_len = 0;
@@ -279,10 +278,9 @@ struct PowerSparseMatrixGPU::Prepared {
     });
 
     count_bits = BitsFor(uint64_t(max_count));
-    keys.Allocate(size_t(nnz));
     vals.Allocate(size_t(nnz));
     ThrowOnError(ps_pre_rank_sort(row_ptr.data(), rows, col_ind.data(), nnz, col_nnz.data(),
-                                  max_count, count_bits, keys.data(), vals.data(), st));
+                                  max_count, count_bits, nullptr, vals.data(), st));
     clock.Mark(&PreprocessTimings::rank_ms);
   }
 
@@ -365,7 +363,7 @@ PowerSparseMatrixGPU::PowerSparseMatrixGPU(int row_num, int col_num, int nnz_num
     // decides the order at the end of the build).
     const bool may_tune =
         policy.spmm_partition == SpmmPartition::kTuned && _task_order != TaskOrder::kRow;
-    Build(row_ptr, in, !may_tune);
+    Build(row_ptr, in);
     bool hub = false;
     if (may_tune && _task_order == TaskOrder::kSignature && _want_run_order &&
         policy.hub_block == HubBlock::kAuto)
@@ -380,7 +378,7 @@ PowerSparseMatrixGPU::PowerSparseMatrixGPU(int row_num, int col_num, int nnz_num
       tuned.spmm_partition = SpmmPartition::kParity;
       _spmm_tuned =
           new PowerSparseMatrixGPU(Unbuilt{}, row_num, col_num, nnz_num, _cu_count, tuned);
-      _spmm_tuned->Build(row_ptr, in, true);
+      _spmm_tuned->Build(row_ptr, in);
     }
     in.clock.Finish();
   } catch (...) {
@@ -389,7 +387,7 @@ PowerSparseMatrixGPU::PowerSparseMatrixGPU(int row_num, int col_num, int nnz_num
   }
 }
 
-void PowerSparseMatrixGPU::Build(const int* row_ptr, Prepared& in, bool last_partition) {
+void PowerSparseMatrixGPU::Build(const int* row_ptr, Prepared& in) {
   const int rows = _matrix_row, nnz = _matrix_nnz;
   const int fine = _group_fine_size;
   ps_stream_t st = nullptr;
@@ -405,8 +403,6 @@ void PowerSparseMatrixGPU::Build(const int* row_ptr, Prepared& in, bool last_par
   if (_max_group_types > 0 && S > _max_group_types) S = _max_group_types;
   if (S > PS_MAX_WORKSETS) throw std::runtime_error("Too many worksets");
   _group_type_num = S;
-  // No tuned partition follows a partition of at most its cap of worksets.
-  if (S <= kTunedSpmmGroupTypes) last_partition = true;
 
   // Group counts per workset, on the host from row_ptr (the split the device
   // kernels make), so the device arrays are sized without waiting.
@@ -496,7 +492,13 @@ void PowerSparseMatrixGPU::Build(const int* row_ptr, Prepared& in, bool last_par
     _signature_order = words <= kBitmapMaxWords ? SignatureOrder::kBitmapWords
                                                 : SignatureOrder::kBitLists;
   const int* d_sigbit = in.sigbit_device.data();
-  const uint64_t* keys = in.keys.data();
+  // the rows of the ranked positions, for the stages that start from them
+  DeviceArray<uint64_t> keys;
+  auto row_keys = [&] {
+    keys.Allocate(size_t(nnz));
+    ThrowOnError(ps_pre_row_keys(d_rp.data(), rows, count_bits, keys.data(), st));
+    return keys.data();
+  };
   std::vector<DeviceArray<uint32_t>> perm(static_cast<size_t>(S));
   std::vector<uint32_t*> perm_ptr(static_cast<size_t>(S), nullptr);
   for (int s = 0; s < S; ++s) {
@@ -509,14 +511,27 @@ void PowerSparseMatrixGPU::Build(const int* row_ptr, Prepared& in, bool last_par
     size_t total = 0;
     for (int s = 0; s < S; ++s) total += size_t(_group_num[s]);
     DeviceArray<uint32_t> lists(static_cast<size_t>(nnz)), list_begin(total + 1);
-    ThrowOnError(ps_pre_signature_lists(d_rp.data(), rows, S, fine, keys, count_bits,
-                                        vals.data(), nnz, d_ci.data(), d_sigbit,
-                                        _signature_len, prefix.data(), _group_num, lists.data(),
-                                        list_begin.data(), st));
-    if (last_partition) in.keys.Reset();
-    clock.Mark(&PreprocessTimings::signature_ms);
-    ThrowOnError(ps_pre_signature_order(lists.data(), list_begin.data(), S, _group_num,
-                                        _signature_len, perm_ptr.data(), st));
+    int largest = S - 1;  // the largest group size that occurs
+    while (largest > 0 && _group_num[largest] == 0) --largest;
+    if (largest > 0 && GROUP_SIZE(largest) > kGroupListMax) {
+      // groups beyond one workgroup's tile: a sort over every group's entries
+      ThrowOnError(ps_pre_signature_lists(d_rp.data(), rows, S, fine, row_keys(), count_bits,
+                                          vals.data(), nnz, d_ci.data(), d_sigbit,
+                                          _signature_len, prefix.data(), _group_num, lists.data(),
+                                          list_begin.data(), st));
+      keys.Reset();
+      clock.Mark(&PreprocessTimings::signature_ms);
+      ThrowOnError(ps_pre_signature_order(lists.data(), list_begin.data(), S, _group_num,
+                                          _signature_len, perm_ptr.data(), st));
+    } else {
+      DeviceArray<uint32_t> list_end(total);
+      ThrowOnError(ps_pre_group_lists(S, _group_num, start_ptr.data(), res_len.data(), vals.data(),
+                                      d_ci.data(), d_sigbit, _signature_len, lists.data(),
+                                      list_begin.data(), list_end.data(), st));
+      clock.Mark(&PreprocessTimings::signature_ms);
+      ThrowOnError(ps_pre_signature_order_spans(lists.data(), list_begin.data(), list_end.data(), S,
+                                                _group_num, _signature_len, perm_ptr.data(), st));
+    }
   } else {
     // Signature bitmaps, word-major per workset.
     std::vector<DeviceArray<uint32_t>> sig(static_cast<size_t>(S));
@@ -526,10 +541,10 @@ void PowerSparseMatrixGPU::Build(const int* row_ptr, Prepared& in, bool last_par
       sig[size_t(s)].Zero(st);
       sig_ptr[size_t(s)] = sig[size_t(s)].data();
     }
-    ThrowOnError(ps_pre_signatures(d_rp.data(), rows, S, fine, keys, count_bits,
+    ThrowOnError(ps_pre_signatures(d_rp.data(), rows, S, fine, row_keys(), count_bits,
                                    vals.data(), nnz, d_ci.data(), d_sigbit, prefix.data(),
                                    _group_num, sig_ptr.data(), st));
-    if (last_partition) in.keys.Reset();
+    keys.Reset();
     clock.Mark(&PreprocessTimings::signature_ms);
     // Stable sort of each workset's groups by signature, descending, word 0
     // most significant: one stable pass per word from the last word to the
@@ -862,7 +877,7 @@ bool PowerSparseMatrixGPU::BuildHub(const int* row_ptr, Prepared& in,
   tuned.hub_block = HubBlock::kOff;
   std::unique_ptr<PowerSparseMatrixGPU> part(
       new PowerSparseMatrixGPU(Unbuilt{}, rows, cols, nnz_rest, _cu_count, tuned));
-  part->Build(rp_host.data(), rest, true);
+  part->Build(rp_host.data(), rest);
   // hub rows add their remaining entries to the block's product
   for (const auto& t : hub->tiers)
     ThrowOnError(ps_hub_mark_atomic(&t->desc, part->_group_des[0], part->_group_num[0],

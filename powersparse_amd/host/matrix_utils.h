@@ -37,6 +37,9 @@ enum GroupSort { GroupNoSort = 0, GroupDoSort = 1 };
 // beyond (measured faster from 22 words up: C1, C3, C4).
 enum class SignatureOrder { kAuto = 0, kBitmapWords = 1, kBitLists = 2 };
 constexpr int kBitmapMaxWords = 4;
+// Largest group whose signature bits one workgroup sorts (ps_pre_group_lists);
+// a partition with larger groups lists them by one sort over all entries.
+constexpr int kGroupListMax = 8192;
 
 // The order in which the operators run the groups (their results do not depend
 // on it, beyond the order of FP32 atomic additions). kSignature runs the public
@@ -254,10 +257,8 @@ class PowerSparseMatrixGPU {
   PowerSparseMatrixGPU(Unbuilt, int row_num, int col_num, int nnz_num, int cu_count,
                        const PartitionPolicy& policy);
   void Configure(const PartitionPolicy& policy);
-  // The partition at this object's settings from the prepared stages; drops
-  // the per-row ranking from `in` once it is no longer needed when
-  // `last_partition` is set.
-  void Build(const int* row_ptr, Prepared& in, bool last_partition);
+  // The partition at this object's settings from the prepared stages.
+  void Build(const int* row_ptr, Prepared& in);
   void Release() noexcept;
   void ReleaseExecution() noexcept;
   void BuildRunOrders();

@@ -42,3 +42,47 @@ def test_gather_tiles(gs, groups, cols):
     np.testing.assert_array_equal(out[2].download(np.int32), pos)
     np.testing.assert_array_equal(out[0].download(np.int32), col[pos])
     np.testing.assert_array_equal(out[1].download(np.uint32), val[pos].view(np.uint32))
+
+
+@pytest.mark.parametrize("length", [1, 33, 3488, (1 << 31) - 1])
+@pytest.mark.parametrize("worksets", [1, 2, 9])
+def test_group_lists(length, worksets):
+    # each group's distinct signature bits: residue groups of 1..31 members, one
+    # and several groups per tile, all bits equal, none equal, already sorted
+    import ctypes
+    setup()
+    say(f"group lists L={length} worksets={worksets}")
+    rng = np.random.default_rng(length % 1000 + worksets)
+    num = [70] + [int(rng.choice([0, 1, 5, 67])) for _ in range(worksets - 1)]
+    if worksets == 9:
+        num[2], num[7], num[8] = 67, 3, 2  # 64: several a tile; 2048 and 4096
+    sizes = [rng.integers(1, 32, num[0])] + [np.full(num[s], 32 << (s - 1)) for s in range(1, worksets)]
+    begin = np.concatenate([[0], np.cumsum(np.concatenate(sizes))])
+    n = int(begin[-1])
+    cols = max(1, n // 3)
+    sigbit = rng.integers(0, length, cols).astype(np.int32)
+    if length == 3488:
+        sigbit.sort()  # sorted columns then give sorted bits
+    col = rng.integers(0, cols, n).astype(np.int32)
+    bounds = np.concatenate([[0], np.cumsum(num)])
+    starts = [begin[bounds[s]:bounds[s + 1]].astype(np.int32) for s in range(worksets)]
+    if length == 3488:
+        for a, b in zip(begin[:-1:2], begin[1::2]):
+            col[a:b].sort()
+    ranked = rng.permutation(n).astype(np.uint32)
+    by_rank = np.empty(n, np.int32)
+    by_rank[ranked] = col  # col_ind such that ranked position i holds column col[i]
+    d = [ps.DeviceBuffer(host=a) for a in (ranked, by_rank, sigbit, sizes[0].astype(np.int32))]
+    ds = [ps.DeviceBuffer(host=a if a.size else np.zeros(1, np.int32)) for a in starts]
+    total = int(bounds[-1])
+    lists, at, end = ps.DeviceBuffer(n * 4), ps.DeviceBuffer(total * 4), ps.DeviceBuffer(total * 4)
+    counts = (ctypes.c_int * worksets)(*num)
+    ptrs = (ctypes.c_void_p * worksets)(*[x.ptr for x in ds])
+    ps._hip_call(_native.hip().ps_pre_group_lists(
+        worksets, counts, ptrs, d[3].ptr, d[0].ptr, d[1].ptr, d[2].ptr, length, lists.ptr, at.ptr,
+        end.ptr, None))
+    got, a, e = lists.download(np.uint32), at.download(np.uint32), end.download(np.uint32)
+    for g in range(total):
+        want = np.unique(sigbit[col[begin[g]:begin[g + 1]]])
+        assert a[g] == begin[g]
+        np.testing.assert_array_equal(got[a[g]:e[g]], want, err_msg=f"group {g}")
