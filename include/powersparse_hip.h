@@ -333,6 +333,17 @@ int ps_hub_kept_counts(const ps_hub_block* hb, const int* row_ptr, const int* co
 int ps_hub_compact(const ps_hub_block* hb, const int* row_ptr, const int* col_ind,
                    const float* sp_data, const uint32_t* new_row_ptr, int* new_col,
                    float* new_val, ps_stream_t stream);
+/* The same over several tiers of disjoint rows, for a matrix whose rows are
+ * already ranked (ps_pre_rank_sort): counts[r] = entries of row r outside every
+ * tier's stored slots, and new_ranked[new_row_ptr[r] ..] = row r's ranked
+ * positions of those entries, in order; new_row_ptr is the exclusive scan of
+ * the counts. hubs: up to PS_HUB_MAX_TIERS descriptors (host array). */
+#define PS_HUB_MAX_TIERS 4
+int ps_hub_rest_counts(int tiers, const ps_hub_block* hubs, const int* row_ptr, uint32_t* counts,
+                       ps_stream_t stream);
+int ps_hub_rest_ranked(int tiers, const ps_hub_block* hubs, const int* row_ptr, const int* col_ind,
+                       const uint32_t* ranked, const uint32_t* new_row_ptr, uint32_t* new_ranked,
+                       ps_stream_t stream);
 /* residue_atomic[g] = 1 for every residue group g whose row (group_des[g]) is a
  * hub row (the rows of a partition without the block keep accumulating). */
 int ps_hub_mark_atomic(const ps_hub_block* hb, const int* group_des, int group_num,

@@ -164,6 +164,11 @@ HIP_API = [
     ("ps_hub_compact", ctypes.c_int,
      [ctypes.POINTER(HubBlock), c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
       c_void_p]),
+    ("ps_hub_rest_counts", ctypes.c_int,
+     [ctypes.c_int, ctypes.POINTER(HubBlock), c_void_p, c_void_p, c_void_p]),
+    ("ps_hub_rest_ranked", ctypes.c_int,
+     [ctypes.c_int, ctypes.POINTER(HubBlock), c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+      c_void_p]),
     ("ps_hub_mark_atomic", ctypes.c_int,
      [ctypes.POINTER(HubBlock), c_void_p, ctypes.c_int, c_void_p, c_void_p]),
     ("ps_hub_tile_flags", ctypes.c_int,

@@ -264,6 +264,88 @@ __global__ __launch_bounds__(kThreads) void compact_kernel(ps_hub_block hb,
   }
 }
 
+// ---- the matrix without the block, as a shorter ranking ----
+//
+// The rest of the matrix keeps the whole matrix's ranking (each row's nonzeros
+// by column count): leaving out the block's entries keeps the others in order,
+// so nothing is counted, ranked or uploaded again.
+struct HubSet {
+  ps_hub_block t[PS_HUB_MAX_TIERS];
+  int count;
+};
+
+// counts[r] = degree of row r.
+__global__ __launch_bounds__(kThreads) void degrees_kernel(const int* __restrict__ row_ptr, int rows,
+                                                            uint32_t* __restrict__ counts) {
+  for (int r = blockIdx.x * kThreads + threadIdx.x; r < rows; r += gridDim.x * kThreads)
+    counts[r] = uint32_t(row_ptr[r + 1] - row_ptr[r]);
+}
+
+// counts[hub row] -= the row's stored slots (each holds one entry). One wave
+// per hub row.
+__global__ __launch_bounds__(kThreads) void drop_stored_kernel(ps_hub_block hb,
+                                                                uint32_t* __restrict__ counts) {
+  const size_t words = (size_t(hb.cols) + 31) / 32;
+  const int waves = kThreads / kWave;
+  for (int i = blockIdx.x * waves + threadIdx.x / kWave; i < hb.rows; i += gridDim.x * waves) {
+    uint32_t n = 0;
+    for (size_t q = lane_id(); q < words; q += kWave) n += __popc(hb.stored[size_t(i) * words + q]);
+    for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
+    if (lane_id() == 0) counts[hb.hub_rows[i]] -= n;
+  }
+}
+
+// The rows outside every tier keep their whole ranking. One wave per row.
+__global__ __launch_bounds__(kThreads) void rest_rows_kernel(HubSet hs,
+                                                              const int* __restrict__ row_ptr,
+                                                              const uint32_t* __restrict__ ranked,
+                                                              const uint32_t* __restrict__ new_row_ptr,
+                                                              uint32_t* __restrict__ new_ranked) {
+  const int waves = kThreads / kWave, rows = hs.t[0].matrix_rows;
+  for (int r = blockIdx.x * waves + threadIdx.x / kWave; r < rows; r += gridDim.x * waves) {
+    bool hub = false;
+    for (int k = 0; k < hs.count; ++k) hub |= hs.t[k].hub_index[r] >= 0;
+    if (hub) continue;
+    const int b = row_ptr[r], e = row_ptr[r + 1];
+    const uint32_t out = new_row_ptr[r];
+    for (int p = b + lane_id(); p < e; p += kWave) new_ranked[out + uint32_t(p - b)] = ranked[p];
+  }
+}
+
+// A tier's rows: the entries outside the block's stored slots, in ranked
+// order. One workgroup per hub row.
+__global__ __launch_bounds__(kThreads) void rest_hub_rows_kernel(
+    ps_hub_block hb, const int* __restrict__ row_ptr, const int* __restrict__ col_ind,
+    const uint32_t* __restrict__ ranked, const uint32_t* __restrict__ new_row_ptr,
+    uint32_t* __restrict__ new_ranked) {
+  constexpr int kWaves = kThreads / kWave;
+  __shared__ uint32_t kept[2][kWaves];
+  const int w = threadIdx.x / kWave, lane = lane_id();
+  for (int i = blockIdx.x; i < hb.rows; i += gridDim.x) {
+    const int r = hb.hub_rows[i];
+    const int b = row_ptr[r], e = row_ptr[r + 1];
+    uint32_t out = new_row_ptr[r];
+    int flip = 0;  // the counts of a step are read after its barrier only
+    for (int p0 = b; p0 < e; p0 += kThreads, flip ^= 1) {
+      const int p = p0 + int(threadIdx.x);
+      const uint32_t at = p < e ? ranked[p] : 0u;
+      const bool keep = p < e && !in_block(hb, i, hb.hot_rank[col_ind[at]]);
+      const uint64_t m = __ballot(keep);
+      if (lane == 0) kept[flip][w] = uint32_t(__popcll(m));
+      __syncthreads();
+      uint32_t before = 0, all = 0;
+#pragma unroll
+      for (int q = 0; q < kWaves; ++q) {
+        if (q < w) before += kept[flip][q];
+        all += kept[flip][q];
+      }
+      if (keep) new_ranked[out + before + uint32_t(__popcll(m & ((1ull << lane) - 1ull)))] = at;
+      out += all;
+    }
+    __syncthreads();  // the next row's first step may reuse kept[0]
+  }
+}
+
 // flags[t] = 1 when the t-th 64-nonzero stretch of a block workset (groups of
 // 64 or more nonzeros, so a stretch lies in one group) lies inside the block:
 // its group's row is a hub row and all its 64 columns are hot. One wave per
@@ -1057,6 +1139,58 @@ int ps_hub_compact(const ps_hub_block* hb, const int* row_ptr, const int* col_in
                        ps::kThreads, 0, st>>>(*hb, row_ptr, col_ind, sp_data, new_row_ptr, new_col,
                                               new_val);
   PS_LAUNCHED();
+  return PS_OK;
+}
+
+static int hub_set(int tiers, const ps_hub_block* hubs, ps::HubSet* hs) {
+  PS_CHECK_ARG(tiers >= 1 && tiers <= PS_HUB_MAX_TIERS && hubs, "hub block: bad tier count");
+  hs->count = tiers;
+  for (int k = 0; k < tiers; ++k) {
+    const int rc = ps::check_block(&hubs[k]);
+    if (rc != PS_OK) return rc;
+    PS_CHECK_ARG(hubs[k].stored, "hub block: missing stored bits");
+    PS_CHECK_ARG(hubs[k].matrix_rows == hubs[0].matrix_rows, "hub block: tiers of two matrices");
+    hs->t[k] = hubs[k];
+  }
+  return PS_OK;
+}
+
+int ps_hub_rest_counts(int tiers, const ps_hub_block* hubs, const int* row_ptr, uint32_t* counts,
+                       ps_stream_t stream) {
+  ps::HubSet hs{};
+  const int rc = hub_set(tiers, hubs, &hs);
+  if (rc != PS_OK) return rc;
+  PS_CHECK_ARG(row_ptr && counts, "ps_hub_rest_counts: null argument");
+  hipStream_t st = ps::to_hip(stream);
+  const int rows = hs.t[0].matrix_rows;
+  ps::degrees_kernel<<<ps::grid_for(size_t(rows), ps::kThreads), ps::kThreads, 0, st>>>(row_ptr,
+                                                                                        rows, counts);
+  PS_LAUNCHED();
+  for (int k = 0; k < tiers; ++k) {
+    ps::drop_stored_kernel<<<ps::grid_for(size_t(hs.t[k].rows), ps::kThreads / ps::kWave),
+                             ps::kThreads, 0, st>>>(hs.t[k], counts);
+    PS_LAUNCHED();
+  }
+  return PS_OK;
+}
+
+int ps_hub_rest_ranked(int tiers, const ps_hub_block* hubs, const int* row_ptr, const int* col_ind,
+                       const uint32_t* ranked, const uint32_t* new_row_ptr, uint32_t* new_ranked,
+                       ps_stream_t stream) {
+  ps::HubSet hs{};
+  const int rc = hub_set(tiers, hubs, &hs);
+  if (rc != PS_OK) return rc;
+  PS_CHECK_ARG(row_ptr && col_ind && ranked && new_row_ptr && new_ranked,
+               "ps_hub_rest_ranked: null argument");
+  hipStream_t st = ps::to_hip(stream);
+  ps::rest_rows_kernel<<<ps::grid_for(size_t(hs.t[0].matrix_rows), ps::kThreads / ps::kWave),
+                         ps::kThreads, 0, st>>>(hs, row_ptr, ranked, new_row_ptr, new_ranked);
+  PS_LAUNCHED();
+  for (int k = 0; k < tiers; ++k) {
+    ps::rest_hub_rows_kernel<<<ps::grid_for(size_t(hs.t[k].rows), 1), ps::kThreads, 0, st>>>(
+        hs.t[k], row_ptr, col_ind, ranked, new_row_ptr, new_ranked);
+    PS_LAUNCHED();
+  }
   return PS_OK;
 }
 

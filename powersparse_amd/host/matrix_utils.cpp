@@ -250,11 +250,14 @@ struct PowerSparseMatrixGPU::Prepared {
     clock.Mark(&PreprocessTimings::upload_ms);
     Analyze(rows, cols, nnz);
   }
-  // From a CSR already on the device (stage times not recorded).
-  Prepared(int rows, int cols, int nnz, DeviceArray<int>&& rp, DeviceArray<int>&& ci,
-           DeviceArray<float>&& sv)
-      : clock(nullptr), row_ptr(std::move(rp)), col_ind(std::move(ci)), sp_data(std::move(sv)) {
-    Analyze(rows, cols, nnz);
+  // From here on only the nonzeros of a shorter ranking (positions in the same
+  // CSR arrays), with its row pointers and degree sums.
+  void Restrict(DeviceArray<int>&& rp, DeviceArray<uint32_t>&& ranked,
+                const unsigned long long (&sums)[32]) {
+    row_ptr = std::move(rp);
+    vals = std::move(ranked);
+    ranked.Reset();  // the whole ranking
+    std::copy(std::begin(sums), std::end(sums), degree_sums);
   }
 
   void Analyze(int rows, int cols, int nnz) {
@@ -834,40 +837,36 @@ bool PowerSparseMatrixGPU::BuildHub(const int* row_ptr, Prepared& in,
   }
   if (hub->tiers.empty()) return false;
 
-  // SpMM: a tuned partition of the matrix without the block, the tiers taken
-  // out one after another (their rows are disjoint).
-  DeviceArray<int> rp, ci;
-  DeviceArray<float> sv;
-  std::vector<int> rp_host(size_t(rows) + 1);
-  int nnz_rest = _matrix_nnz;
-  for (const auto& t : hub->tiers) {
-    const int* cur_rp = rp.size() ? rp.data() : in.row_ptr.data();
-    const int* cur_ci = ci.size() ? ci.data() : in.col_ind.data();
-    const float* cur_sv = sv.size() ? sv.data() : in.sp_data.data();
+  // SpMM: a tuned partition of the matrix without the block. It keeps the
+  // whole matrix's column counts, ranking and signature bits: which of a row's
+  // nonzeros share a group moves with the counts, the products do not.
+  static_assert(kHubMaxTiers <= PS_HUB_MAX_TIERS, "tiers of one matrix");
+  std::vector<ps_hub_block> descs;
+  for (const auto& t : hub->tiers) descs.push_back(t->desc);
+  DeviceArray<int> rest_ptr(size_t(rows) + 1);
+  {
     DeviceArray<uint32_t> kept(size_t(rows) + 1);
     ThrowOnError(ps_memset_async(kept.data() + rows, 0, sizeof(uint32_t), nullptr));
-    ThrowOnError(ps_hub_kept_counts(&t->desc, cur_rp, cur_ci, kept.data(), nullptr));
-    DeviceArray<int> next_rp(size_t(rows) + 1);
-    {
-      DeviceArray<char> scan_ws(ps_scan_workspace_bytes(size_t(rows) + 1));
-      ThrowOnError(ps_exclusive_scan_u32(kept.data(), reinterpret_cast<uint32_t*>(next_rp.data()),
-                                         size_t(rows) + 1, scan_ws.data(), nullptr));
-    }
-    ThrowOnError(ps_memcpy_dtoh(&nnz_rest, next_rp.data() + rows, sizeof(int)));
-    if (nnz_rest <= 0) return false;  // the block would hold every nonzero
-    DeviceArray<int> next_ci{static_cast<size_t>(nnz_rest)};
-    DeviceArray<float> next_sv{static_cast<size_t>(nnz_rest)};
-    ThrowOnError(ps_hub_compact(&t->desc, cur_rp, cur_ci, cur_sv,
-                                reinterpret_cast<const uint32_t*>(next_rp.data()), next_ci.data(),
-                                next_sv.data(), nullptr));
-    rp = std::move(next_rp);
-    ci = std::move(next_ci);
-    sv = std::move(next_sv);
+    ThrowOnError(ps_hub_rest_counts(int(descs.size()), descs.data(), in.row_ptr.data(),
+                                    kept.data(), nullptr));
+    DeviceArray<char> scan_ws(ps_scan_workspace_bytes(size_t(rows) + 1));
+    ThrowOnError(ps_exclusive_scan_u32(kept.data(), reinterpret_cast<uint32_t*>(rest_ptr.data()),
+                                       size_t(rows) + 1, scan_ws.data(), nullptr));
   }
-  rp.Download(rp_host.data(), rp_host.size());
-  Prepared rest(rows, cols, nnz_rest, std::move(rp), std::move(ci), std::move(sv));
+  std::vector<int> rp_host(size_t(rows) + 1);
+  rest_ptr.Download(rp_host.data(), rp_host.size());
+  const int nnz_rest = rp_host.back();
+  if (nnz_rest <= 0) return false;  // the block would hold every nonzero
   // the rest must keep the public partition's store rule: more than one workset
-  if (std::min(WorksetCount(rest.degree_sums, _cu_count), kTunedSpmmGroupTypes) < 2) return false;
+  unsigned long long rest_sums[32] = {};
+  ThrowOnError(ps_pre_degree_sums(rest_ptr.data(), rows, rest_sums, nullptr));
+  if (std::min(WorksetCount(rest_sums, _cu_count), kTunedSpmmGroupTypes) < 2) return false;
+  DeviceArray<uint32_t> rest_vals{static_cast<size_t>(nnz_rest)};
+  ThrowOnError(ps_hub_rest_ranked(int(descs.size()), descs.data(), in.row_ptr.data(),
+                                  in.col_ind.data(), in.vals.data(),
+                                  reinterpret_cast<const uint32_t*>(rest_ptr.data()),
+                                  rest_vals.data(), nullptr));
+  in.Restrict(std::move(rest_ptr), std::move(rest_vals), rest_sums);
   PartitionPolicy tuned;
   tuned.cu_count = _cu_count;
   tuned.task_order = TaskOrder::kSignature;
@@ -877,7 +876,7 @@ bool PowerSparseMatrixGPU::BuildHub(const int* row_ptr, Prepared& in,
   tuned.hub_block = HubBlock::kOff;
   std::unique_ptr<PowerSparseMatrixGPU> part(
       new PowerSparseMatrixGPU(Unbuilt{}, rows, cols, nnz_rest, _cu_count, tuned));
-  part->Build(rp_host.data(), rest);
+  part->Build(rp_host.data(), in);
   // hub rows add their remaining entries to the block's product
   for (const auto& t : hub->tiers)
     ThrowOnError(ps_hub_mark_atomic(&t->desc, part->_group_des[0], part->_group_num[0],
