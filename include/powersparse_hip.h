@@ -440,6 +440,9 @@ int ps_pre_degree_sums(const int* row_ptr, int rows, unsigned long long* sums_ho
 /* col_nnz[c] += number of nonzeros in column c (col_nnz pre-zeroed).
  * Replaces: the OpenMP histogram (matrix_utils.cu:508-514). */
 int ps_pre_col_histogram(const int* col_ind, int nnz, int* col_nnz, ps_stream_t stream);
+/* The same for a matrix of `cols` columns (every column id below it). */
+int ps_pre_col_histogram_cols(const int* col_ind, int nnz, int cols, int* col_nnz,
+                              ps_stream_t stream);
 
 /* keys[p] = (row(p) << count_bits) | (max_count - col_nnz[col_ind[p]]), vals[p] = p:
  * the stable sort of these pairs gives each row's nonzeros by column count

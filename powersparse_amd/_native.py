@@ -222,6 +222,8 @@ HIP_API = [
     ("ps_iota_u32", ctypes.c_int, [c_void_p, ctypes.c_int, c_void_p]),
     ("ps_pre_degree_sums", ctypes.c_int, [c_void_p, ctypes.c_int, c_u64_p, c_void_p]),
     ("ps_pre_col_histogram", ctypes.c_int, [c_void_p, ctypes.c_int, c_void_p, c_void_p]),
+    ("ps_pre_col_histogram_cols", ctypes.c_int,
+     [c_void_p, ctypes.c_int, ctypes.c_int, c_void_p, c_void_p]),
     ("ps_pre_rank_keys", ctypes.c_int,
      [c_void_p, ctypes.c_int, c_void_p, ctypes.c_int, c_void_p, ctypes.c_int, ctypes.c_int,
       c_void_p, c_void_p, c_void_p]),

@@ -266,7 +266,7 @@ struct PowerSparseMatrixGPU::Prepared {
     ThrowOnError(ps_pre_degree_sums(row_ptr.data(), rows, degree_sums, st));
     col_nnz.Allocate(size_t(cols));
     col_nnz.Zero(st);
-    ThrowOnError(ps_pre_col_histogram(col_ind.data(), nnz, col_nnz.data(), st));
+    ThrowOnError(ps_pre_col_histogram_cols(col_ind.data(), nnz, cols, col_nnz.data(), st));
     col_nnz_host.resize(size_t(cols));
     col_nnz.Download(col_nnz_host.data(), size_t(cols));
     max_count = *std::max_element(col_nnz_host.begin(), col_nnz_host.end());

@@ -86,3 +86,21 @@ def test_group_lists(length, worksets):
         want = np.unique(sigbit[col[begin[g]:begin[g + 1]]])
         assert a[g] == begin[g]
         np.testing.assert_array_equal(got[a[g]:e[g]], want, err_msg=f"group {g}")
+
+
+@pytest.mark.parametrize("cols", [1, 255, 256, 257, 100000, (1 << 23), (1 << 23) + 1])
+@pytest.mark.parametrize("nnz", [1, 2047, 2049, 1 << 20, (1 << 26) + 5])
+def test_col_histogram(cols, nnz):
+    # one class, all classes, the most columns the split takes and one beyond;
+    # one nonzero, chunk remainders, more than one slab
+    setup()
+    say(f"column histogram cols={cols} nnz={nnz}")
+    rng = np.random.default_rng(cols + nnz)
+    if nnz > 1 << 21 and cols < 100000:
+        pytest.skip("the slab edge needs one column range")
+    c = rng.integers(0, cols, nnz, dtype=np.int32)
+    c[::3] //= 1 + cols // 50  # popular columns
+    c[-1] = cols - 1
+    d, out = ps.DeviceBuffer(host=c), ps.DeviceBuffer.zeros(cols * 4)
+    ps._hip_call(_native.hip().ps_pre_col_histogram_cols(d.ptr, nnz, cols, out.ptr, None))
+    np.testing.assert_array_equal(out.download(np.int32), np.bincount(c, minlength=cols))
