@@ -677,12 +677,16 @@ __global__ __launch_bounds__(NT, 8) void group_lists_tile_kernel(
 }
 
 // Refinement. The active groups (still tied with another group of their
-// class) are kept in class order, each with its class base (final position
-// of the class's first member) and class depth (all members have equal lists
-// before it). Initially every group is active, the classes are the worksets
-// and the depth is 0. Each round compares every member with its class's first
-// member r (the reference) from the class depth on: the first position where
-// they differ, `lcp`, and which way the member goes:
+// class) are kept in class order, each with the active position of its class's
+// first member, its class base (the final position of that member) and its
+// class depth (all members have equal lists before it).
+//
+// The first round's classes are the worksets: their groups are sorted by as
+// many leading list elements as a 64-bit key holds beside the class (4 of 10
+// bits on C1), the end of a list after every element. Each later round
+// compares every member with its class's first member r (the reference) from
+// the class depth on: the first position where they differ, `lcp`, and which
+// way the member goes:
 //   EQ     identical list to r;
 //   BEFORE the member's element at lcp is smaller than r's, or r's list ends;
 //   AFTER  the member's list ends at lcp, or its element is larger.
@@ -693,11 +697,28 @@ __global__ __launch_bounds__(NT, 8) void group_lists_tile_kernel(
 // lists ended, and single members are placed. Every class loses at least its
 // reference each round, and in practice a whole nest of prefix-related lists
 // separates in one round.
+//
+// A round is bound by its launches and the host's wait for the next round's
+// size (thousands of groups, a dozen rounds), so it has few of both (the order
+// stage of both partitions: C1 13.7 -> 9.5 ms, C3 24.5 -> 18.1 ms, a 10 k-node
+// graph 1.40 -> 0.63 ms against rounds of 17 launches and two waits): a class
+// keeps its place in the active list when that is sorted, so a member's class
+// start is its class's first position, a run's start is found by bisection
+// in the sorted keys, and the next round's keys are made before the one copy
+// that brings the host its size and the key bits that vary.
 constexpr uint32_t kBefore = 0, kEq = 1, kAfter = 2;
+
+// What the host reads each round.
+struct OrderState {
+  uint32_t n;        // active groups
+  uint32_t max_len;  // longest list
+  unsigned long long any, all;  // OR and AND of the sort keys
+};
 
 __global__ void order_init_kernel(uint32_t n, GroupBase gb, uint32_t* __restrict__ act_group,
                                   uint32_t* __restrict__ act_base,
-                                  uint32_t* __restrict__ act_depth) {
+                                  uint32_t* __restrict__ act_depth, OrderState* __restrict__ st) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *st = OrderState{n, 0u, 0ull, ~0ull};
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     act_group[i] = i;
     act_base[i] = gb.base[workset_of(gb, i)];
@@ -708,48 +729,75 @@ __global__ void order_init_kernel(uint32_t n, GroupBase gb, uint32_t* __restrict
 // Longest list (bounds the divergence depth).
 __global__ void max_list_kernel(const uint32_t* __restrict__ list_begin,
                                 const uint32_t* __restrict__ list_end, uint32_t groups,
-                                uint32_t* __restrict__ out) {
+                                OrderState* __restrict__ st) {
   uint32_t m = 0;
   for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < groups;
        g += gridDim.x * blockDim.x)
     m = max(m, list_end[g] - list_begin[g]);
   for (int d = 1; d < kWave; d <<= 1) m = max(m, uint32_t(__shfl_xor(int(m), d, kWave)));
-  if (lane_id() == 0) atomicMax(out, m);
+  if (lane_id() == 0) atomicMax(&st->max_len, m);
 }
 
-// head[i] = 1 where a class starts.
-__global__ void order_class_heads_kernel(const uint32_t* __restrict__ act_base, uint32_t n,
-                                         uint32_t* __restrict__ head) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-    head[i] = (i == 0 || act_base[i] != act_base[i - 1]) ? 1u : 0u;
+// One atomic per workgroup for the OR and AND of its threads' keys.
+__device__ __forceinline__ void span_add(unsigned long long any, unsigned long long all,
+                                         OrderState* st) {
+  __shared__ unsigned long long part[2];
+  if (threadIdx.x == 0) {
+    part[0] = 0ull;
+    part[1] = ~0ull;
+  }
+  __syncthreads();
+  for (int d = 1; d < kWave; d <<= 1) {
+    any |= __shfl_xor(any, d, kWave);
+    all &= __shfl_xor(all, d, kWave);
+  }
+  if (lane_id() == 0) {
+    atomicOr(&part[0], any);
+    atomicAnd(&part[1], all);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    atomicOr(&st->any, part[0]);
+    atomicAnd(&st->all, part[1]);
+  }
 }
 
-// head_at[c] = index of class c's first member (its reference).
-__global__ void order_class_start_kernel(uint32_t n, const uint32_t* __restrict__ head,
-                                         const uint32_t* __restrict__ rank,
-                                         uint32_t* __restrict__ head_at) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-    if (head[i]) head_at[rank[i]] = i;
+// First round's keys: the class's first position, then the list's first
+// `elems` elements of elem_bits bits each.
+__global__ __launch_bounds__(kThreads) void order_pack_kernel(
+    uint32_t n, GroupBase gb, const uint32_t* __restrict__ lists,
+    const uint32_t* __restrict__ list_begin, const uint32_t* __restrict__ list_end, uint32_t end,
+    int elems, int elem_bits, uint64_t* __restrict__ key, uint32_t* __restrict__ idx,
+    OrderState* __restrict__ st) {
+  unsigned long long any = 0ull, all = ~0ull;
+  for (uint32_t i = blockIdx.x * kThreads + threadIdx.x; i < n; i += gridDim.x * kThreads) {
+    const uint32_t b = list_begin[i], len = list_end[i] - b;
+    uint64_t k = gb.base[workset_of(gb, i)];
+    for (int e = 0; e < elems; ++e) k = (k << elem_bits) | (uint32_t(e) < len ? lists[b + e] : end);
+    key[i] = k;
+    idx[i] = i;
+    any |= k;
+    all &= k;
+  }
+  span_add(any, all, st);
 }
 
-// Sort keys of every active member: hi = class * 3 + side; lo = divergence
-// key * (end + 1) + element (end for a list that ended). lcp[i] = divergence
-// position; idx[i] = i.
-__global__ void order_diverge_kernel(const uint32_t* __restrict__ act_group,
-                                     const uint32_t* __restrict__ act_depth, uint32_t n,
-                                     const uint32_t* __restrict__ lists,
-                                     const uint32_t* __restrict__ list_begin,
-                                     const uint32_t* __restrict__ list_end,
-                                     const uint32_t* __restrict__ head,
-                                     const uint32_t* __restrict__ rank,
-                                     const uint32_t* __restrict__ head_at, uint32_t end,
-                                     uint32_t max_len, uint64_t* __restrict__ hi,
-                                     uint64_t* __restrict__ lo, uint32_t* __restrict__ lcp_out,
-                                     uint32_t* __restrict__ idx) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const uint32_t c = rank[i] + head[i] - 1;
+// Later rounds' keys, for the st->n active members: hi = class first * 3 +
+// side; lo = divergence key * (end + 1) + element (end for a list that ended);
+// one key hi << lo_bits | lo, or hi and lo apart when `hi` is given. lcp[i] =
+// divergence position; idx[i] = i.
+__global__ __launch_bounds__(kThreads) void order_diverge_kernel(
+    const uint32_t* __restrict__ act_group, const uint32_t* __restrict__ act_depth,
+    const uint32_t* __restrict__ act_first, const uint32_t* __restrict__ lists,
+    const uint32_t* __restrict__ list_begin, const uint32_t* __restrict__ list_end, uint32_t end,
+    uint32_t max_len, int lo_bits, uint64_t* __restrict__ key, uint64_t* __restrict__ hi,
+    uint32_t* __restrict__ lcp_out, uint32_t* __restrict__ idx, OrderState* __restrict__ st) {
+  const uint32_t n = st->n;
+  unsigned long long any = 0ull, all = ~0ull;
+  for (uint32_t i = blockIdx.x * kThreads + threadIdx.x; i < n; i += gridDim.x * kThreads) {
+    const uint32_t first = act_first[i];
     const uint32_t g = act_group[i];
-    const uint32_t r = act_group[head_at[c]];
+    const uint32_t r = act_group[first];
     const uint32_t* m = lists + list_begin[g];
     const uint32_t* q = lists + list_begin[r];
     const uint32_t nm = list_end[g] - list_begin[g];
@@ -757,28 +805,34 @@ __global__ void order_diverge_kernel(const uint32_t* __restrict__ act_group,
     uint32_t d = act_depth[i];
     if (g != r)
       while (d < nm && d < nq && m[d] == q[d]) ++d;
-    uint32_t side, key = 0, elem = 0;
+    uint32_t side, div = 0, elem = 0;
     if (g == r || (d == nm && d == nq)) {
       side = kEq;
       d = nm;
     } else if (d == nm) {
       side = kAfter;
-      key = max_len - d;
+      div = max_len - d;
       elem = end;
     } else if (d == nq || m[d] < q[d]) {
       side = kBefore;
-      key = d;
+      div = d;
       elem = m[d];
     } else {
       side = kAfter;
-      key = max_len - d;
+      div = max_len - d;
       elem = m[d];
     }
-    hi[i] = uint64_t(c) * 3u + side;
-    lo[i] = uint64_t(key) * (uint64_t(end) + 1u) + elem;
+    const uint64_t h = uint64_t(first) * 3u + side;
+    const uint64_t l = uint64_t(div) * (uint64_t(end) + 1u) + elem;
+    const uint64_t k = hi ? l : (h << lo_bits) | l;
+    key[i] = k;
+    if (hi) hi[i] = h;
     lcp_out[i] = d;
     idx[i] = i;
+    any |= k;
+    all &= k;
   }
+  span_add(any, all, st);
 }
 
 // ---- refinement tail in one workgroup ----
@@ -787,8 +841,10 @@ __global__ void order_diverge_kernel(const uint32_t* __restrict__ act_group,
 // runs the remaining rounds with the whole state in LDS (no host round trip
 // per round): the same rounds as above, the sort being an LDS bitonic sort of
 // (key, slot) pairs (slots unique, so equal keys keep their class order) and
-// run / class starts coming from block max-scans.
-constexpr int kFinishMax = 2048;
+// run / class starts coming from block max-scans. 4096 groups fill 144 KB of
+// the LDS; C3's public partition loses its groups a few dozen a round there
+// (17 rounds from 4096 to 2048).
+constexpr int kFinishMax = 4096;
 constexpr int kFinishThreads = 1024;
 constexpr int kFinishPer = kFinishMax / kFinishThreads;  // elements per thread
 // LDS of order_finish_kernel: one uint64 key and seven uint32 arrays per
@@ -1020,32 +1076,6 @@ __global__ __launch_bounds__(kFinishThreads) void order_finish_kernel(
   }
 }
 
-// or_and[0] |= OR of the keys, or_and[1] &= AND of the keys.
-__global__ void key_span_kernel(const uint64_t* __restrict__ keys, uint32_t n,
-                                unsigned long long* __restrict__ or_and) {
-  unsigned long long o = 0ull, a = ~0ull;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    o |= keys[i];
-    a &= keys[i];
-  }
-  for (int d = 1; d < kWave; d <<= 1) {
-    o |= __shfl_xor(o, d, kWave);
-    a &= __shfl_xor(a, d, kWave);
-  }
-  if (lane_id() == 0) {
-    atomicOr(&or_and[0], o);
-    atomicAnd(&or_and[1], a);
-  }
-}
-
-// Combined key when both parts fit: hi << lo_bits | lo.
-__global__ void order_combine_kernel(uint32_t n, const uint64_t* __restrict__ hi,
-                                     const uint64_t* __restrict__ lo, int lo_bits,
-                                     uint64_t* __restrict__ key) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-    key[i] = (hi[i] << lo_bits) | lo[i];
-}
-
 // key[j] = part[src[j]] (the second key of a two-pass sort, in first-pass order).
 __global__ void order_permute_key_kernel(uint32_t n, const uint32_t* __restrict__ src,
                                          const uint64_t* __restrict__ part,
@@ -1054,92 +1084,94 @@ __global__ void order_permute_key_kernel(uint32_t n, const uint32_t* __restrict_
     key[j] = part[src[j]];
 }
 
-// After the sort: new_head / old_head flag the starts of runs of equal keys and
-// of classes; the members' group, base and lcp follow their sorted positions.
-__global__ void order_runs_kernel(uint32_t n, const uint32_t* __restrict__ src,
-                                  const uint64_t* __restrict__ hi, const uint64_t* __restrict__ lo,
-                                  uint32_t* __restrict__ new_head, uint32_t* __restrict__ old_head) {
-  for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
-    const uint32_t i = src[j];
-    if (j == 0) {
-      new_head[j] = 1u;
-      old_head[j] = 1u;
-      continue;
-    }
-    const uint32_t p = src[j - 1];
-    new_head[j] = (hi[i] != hi[p] || lo[i] != lo[p]) ? 1u : 0u;
-    old_head[j] = (hi[i] / 3u != hi[p] / 3u) ? 1u : 0u;
+// The sorted keys of a round, by sorted position.
+struct OrderKeys {
+  const uint64_t* key;  // first round and one-key rounds: sorted
+  const uint64_t* hi;   // two-key rounds: hi and lo by active position (else null)
+  const uint64_t* lo;
+  const uint32_t* src;  // sorted position -> active position
+  uint32_t end;
+  int lo_bits;
+  int elem_bits;  // first round: bits of one packed element, else 0
+  __device__ __forceinline__ uint64_t hi_of(uint32_t j) const {
+    return hi ? hi[src[j]] : key[j] >> lo_bits;
   }
-}
-
-// new_at[c] / old_at[c] = sorted index where run c begins (runs numbered by the
-// exclusive scans of the head flags).
-__global__ void order_heads_kernel(uint32_t n, const uint32_t* __restrict__ new_head,
-                                   const uint32_t* __restrict__ new_rank,
-                                   const uint32_t* __restrict__ old_head,
-                                   const uint32_t* __restrict__ old_rank,
-                                   uint32_t* __restrict__ new_at, uint32_t* __restrict__ old_at) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    if (new_head[i]) new_at[new_rank[i]] = i;
-    if (old_head[i]) old_at[old_rank[i]] = i;
+  __device__ __forceinline__ uint64_t lo_of(uint32_t j) const {
+    return hi ? lo[src[j]] : key[j] & ((uint64_t(1) << lo_bits) - 1u);
   }
-}
+  __device__ __forceinline__ bool equal(uint32_t i, uint32_t j) const {
+    return hi ? hi_of(i) == hi_of(j) && lo_of(i) == lo_of(j) : key[i] == key[j];
+  }
+  __device__ __forceinline__ uint32_t class_first(uint32_t j) const {
+    return uint32_t(elem_bits ? hi_of(j) : hi_of(j) / 3u);
+  }
+  // the lists of this key ended inside it: members of a run are identical
+  __device__ __forceinline__ bool ended(uint32_t j) const {
+    if (elem_bits) return (key[j] & ((uint64_t(1) << elem_bits) - 1u)) == end;
+    return uint32_t(hi_of(j) % 3u) == kEq || lo_of(j) % (uint64_t(end) + 1u) == end;
+  }
+};
 
 // A run's base = its class base + the run's offset inside the class. Placed
 // members write the permutation; the others (keep = 1) carry their new class
-// base and depth lcp + 1.
-__global__ void order_resolve_kernel(uint32_t n, const uint32_t* __restrict__ src,
-                                     const uint64_t* __restrict__ hi,
-                                     const uint64_t* __restrict__ lo, uint32_t end,
-                                     const uint32_t* __restrict__ act_group,
-                                     const uint32_t* __restrict__ act_base,
-                                     const uint32_t* __restrict__ lcp,
-                                     const uint32_t* __restrict__ new_head,
-                                     const uint32_t* __restrict__ new_rank,
-                                     const uint32_t* __restrict__ old_head,
-                                     const uint32_t* __restrict__ old_rank,
-                                     const uint32_t* __restrict__ new_at,
-                                     const uint32_t* __restrict__ old_at, GroupBase gb,
-                                     SigTable perm, uint32_t* __restrict__ keep,
-                                     uint32_t* __restrict__ next_group,
-                                     uint32_t* __restrict__ next_base,
-                                     uint32_t* __restrict__ next_depth) {
-  for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
-    const uint32_t i = src[j];
-    const uint32_t hn = new_at[new_rank[j] + new_head[j] - 1];
-    const uint32_t ho = old_at[old_rank[j] + old_head[j] - 1];
+// base, depth (lcp + 1, or `depth` after the first round) and their run's
+// first sorted position. Also resets the key span for the next round's keys.
+__global__ __launch_bounds__(kThreads) void order_resolve_kernel(
+    uint32_t n, OrderKeys k, uint32_t depth, const uint32_t* __restrict__ act_group,
+    const uint32_t* __restrict__ act_base, const uint32_t* __restrict__ lcp, GroupBase gb,
+    SigTable perm, uint32_t* __restrict__ keep, uint32_t* __restrict__ next_group,
+    uint32_t* __restrict__ next_base, uint32_t* __restrict__ next_depth,
+    uint32_t* __restrict__ run_first, OrderState* __restrict__ st) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    st->any = 0ull;
+    st->all = ~0ull;
+  }
+  for (uint32_t j = blockIdx.x * kThreads + threadIdx.x; j < n; j += gridDim.x * kThreads) {
+    const uint32_t i = k.src[j];
+    const uint32_t ho = k.class_first(j);
+    uint32_t hn = j;  // the run's first position: bisection over [ho, j]
+    if (j > ho && k.equal(j - 1, j)) {
+      uint32_t lo = ho, hi = j - 1;  // position hi has j's key
+      while (lo < hi) {
+        const uint32_t mid = lo + (hi - lo) / 2;
+        if (k.equal(mid, j)) hi = mid;
+        else lo = mid + 1;
+      }
+      hn = hi;
+    }
     const uint32_t base = act_base[i] + (hn - ho);
-    const bool single = new_head[j] && (j + 1 == n || new_head[j + 1]);
-    const bool ended = uint32_t(hi[i] % 3u) == kEq || lo[i] % (uint64_t(end) + 1u) == end;
+    const bool single = hn == j && (j + 1 == n || !k.equal(j + 1, j));
     const uint32_t g = act_group[i];
-    if (single || ended) {
+    const bool placed = single || k.ended(j);
+    if (placed) {
       const int s = workset_of(gb, g);
       const uint32_t at = base + (j - hn) - gb.base[s];
       if (at < uint32_t(perm.groups[s])) perm.p[s][at] = g - gb.base[s];  // always, if correct
-      keep[j] = 0u;
-    } else {
-      keep[j] = 1u;
     }
+    keep[j] = placed ? 0u : 1u;
     next_group[j] = g;
     next_base[j] = base;
-    next_depth[j] = lcp[i] + 1u;
+    next_depth[j] = depth ? depth : lcp[i] + 1u;
+    run_first[j] = hn;
   }
 }
 
-__global__ void order_compact_kernel(uint32_t n, const uint32_t* __restrict__ keep,
-                                     const uint32_t* __restrict__ slot,
-                                     const uint32_t* __restrict__ next_group,
-                                     const uint32_t* __restrict__ next_base,
-                                     const uint32_t* __restrict__ next_depth,
-                                     uint32_t* __restrict__ act_group,
-                                     uint32_t* __restrict__ act_base,
-                                     uint32_t* __restrict__ act_depth) {
-  for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
+// The kept members close up (a run is kept or placed as a whole).
+__global__ __launch_bounds__(kThreads) void order_compact_kernel(
+    uint32_t n, const uint32_t* __restrict__ keep, const uint32_t* __restrict__ slot,
+    const uint32_t* __restrict__ next_group, const uint32_t* __restrict__ next_base,
+    const uint32_t* __restrict__ next_depth, const uint32_t* __restrict__ run_first,
+    uint32_t* __restrict__ act_group, uint32_t* __restrict__ act_base,
+    uint32_t* __restrict__ act_depth, uint32_t* __restrict__ act_first,
+    OrderState* __restrict__ st) {
+  for (uint32_t j = blockIdx.x * kThreads + threadIdx.x; j < n; j += gridDim.x * kThreads) {
     if (keep[j]) {
       act_group[slot[j]] = next_group[j];
       act_base[slot[j]] = next_base[j];
       act_depth[slot[j]] = next_depth[j];
+      act_first[slot[j]] = slot[run_first[j]];
     }
+    if (j == n - 1) st->n = slot[j] + keep[j];
   }
 }
 
@@ -1990,21 +2022,12 @@ namespace ps {
 namespace {
 
 // Stable radix sort of (key, index) pairs over the bits where the keys differ
-// (found by an OR/AND reduction); *k / *v point at the sorted data.
+// (`diff`); *k / *v point at the sorted data.
 int sort_varying(uint64_t* keys, uint64_t* keys_alt, uint32_t* vals, uint32_t* vals_alt,
-                 uint32_t n, unsigned long long* span, void* radix_ws, hipStream_t st,
-                 const uint64_t** k, const uint32_t** v) {
-  static const unsigned long long span_init[2] = {0ull, ~0ull};
-  unsigned long long host_span[2] = {0ull, 0ull};
+                 uint32_t n, uint64_t diff, void* radix_ws, hipStream_t st, const uint64_t** k,
+                 uint32_t** v) {
   *k = keys;
   *v = vals;
-  PS_HIP(hipMemcpyAsync(span, span_init, sizeof(span_init), hipMemcpyHostToDevice, st));
-  const unsigned grid = grid_for(n);
-  key_span_kernel<<<grid < 1024 ? grid : 1024, kThreads, 0, st>>>(keys, n, span);
-  PS_LAUNCHED();
-  PS_HIP(hipMemcpyAsync(host_span, span, sizeof(host_span), hipMemcpyDeviceToHost, st));
-  PS_HIP(hipStreamSynchronize(st));
-  const uint64_t diff = host_span[0] ^ host_span[1];
   if (diff == 0) return PS_OK;
   const int lo = __builtin_ctzll(diff) / 8 * 8;
   const int hi = 64 - __builtin_clzll(diff);
@@ -2054,141 +2077,128 @@ int ps_pre_signature_order_spans(const uint32_t* lists, const uint32_t* list_beg
   const uint32_t end = uint32_t(signature_len);
   const size_t n0 = total;
   using S = ps::Scratch;
-  S ws(6 * S::bytes(n0, 8) + 17 * S::bytes(n0, 4) + S::bytes(2, 8) + S::bytes(1, 4) +
+  S ws(4 * S::bytes(n0, 8) + 13 * S::bytes(n0, 4) + S::bytes(sizeof(ps::OrderState), 1) +
        ps_radix_workspace_bytes(n0) + ps_scan_workspace_bytes(n0));
   PS_HIP(ws.error());
-  uint64_t* hi = ws.take<uint64_t>(n0);
-  uint64_t* lo = ws.take<uint64_t>(n0);
   uint64_t* keys = ws.take<uint64_t>(n0);
   uint64_t* keys_alt = ws.take<uint64_t>(n0);
-  uint64_t* keys2 = ws.take<uint64_t>(n0);
-  uint64_t* keys2_alt = ws.take<uint64_t>(n0);
+  uint64_t* hi = ws.take<uint64_t>(n0);
+  uint64_t* lo = ws.take<uint64_t>(n0);
   uint32_t* act_group = ws.take<uint32_t>(n0);
   uint32_t* act_base = ws.take<uint32_t>(n0);
   uint32_t* act_depth = ws.take<uint32_t>(n0);
-  uint32_t* head = ws.take<uint32_t>(n0);
-  uint32_t* rank = ws.take<uint32_t>(n0);
-  uint32_t* head_at = ws.take<uint32_t>(n0);
+  uint32_t* act_first = ws.take<uint32_t>(n0);
+  uint32_t* next_group = ws.take<uint32_t>(n0);
+  uint32_t* next_base = ws.take<uint32_t>(n0);
+  uint32_t* next_depth = ws.take<uint32_t>(n0);
+  uint32_t* run_first = ws.take<uint32_t>(n0);
   uint32_t* lcp = ws.take<uint32_t>(n0);
   uint32_t* idx = ws.take<uint32_t>(n0);
   uint32_t* idx_alt = ws.take<uint32_t>(n0);
-  uint32_t* new_head = ws.take<uint32_t>(n0);
-  uint32_t* old_head = ws.take<uint32_t>(n0);
-  uint32_t* new_rank = ws.take<uint32_t>(n0);
-  uint32_t* old_rank = ws.take<uint32_t>(n0);
-  uint32_t* new_at = ws.take<uint32_t>(n0);
-  uint32_t* old_at = ws.take<uint32_t>(n0);
   uint32_t* keep = ws.take<uint32_t>(n0);
   uint32_t* slot = ws.take<uint32_t>(n0);
-  unsigned long long* span = ws.take<unsigned long long>(2);
-  uint32_t* max_len_dev = ws.take<uint32_t>(1);
+  ps::OrderState* dev = ws.take<ps::OrderState>(1);
   void* radix_ws = ws.take<char>(ps_radix_workspace_bytes(n0));
   void* scan_ws = ws.take<char>(ps_scan_workspace_bytes(n0));
-  // next_group / next_base / next_depth reuse buffers free after the sort
-  uint32_t* next_group = head;
-  uint32_t* next_base = head_at;
-  uint32_t* next_depth = rank;
   hipStream_t st = ps::to_hip(stream);
+  ps::OrderState now{};
 
-  uint32_t max_len = 0;
-  PS_HIP(hipMemsetAsync(max_len_dev, 0, 4, st));
-  {
-    unsigned gx = ps::grid_for(n0);
-    ps::max_list_kernel<<<gx < 1024 ? gx : 1024, ps::kThreads, 0, st>>>(list_begin, list_end,
-                                                                        total,
-                                                                        max_len_dev);
-    PS_LAUNCHED();
-  }
-  PS_HIP(hipMemcpyAsync(&max_len, max_len_dev, 4, hipMemcpyDeviceToHost, st));
-  ps::order_init_kernel<<<ps::grid_for(n0), ps::kThreads, 0, st>>>(total, gb, act_group,
-                                                                   act_base, act_depth);
+  // The first round's keys: the class in the bits of `total`, as many elements
+  // of elem_bits as the rest holds (at least one: either takes at most 31 bits).
+  const unsigned grid0 = ps::grid_for(n0);
+  const int elem_bits = ps::bits_for(uint64_t(end));
+  const int class_bits = total > 1 ? ps::bits_for(uint64_t(total - 1)) : 1;
+  const int elems = (64 - class_bits) / elem_bits;
+  ps::order_init_kernel<<<grid0, ps::kThreads, 0, st>>>(total, gb, act_group, act_base, act_depth,
+                                                        dev);
   PS_LAUNCHED();
+  ps::max_list_kernel<<<grid0 < 1024 ? grid0 : 1024, ps::kThreads, 0, st>>>(list_begin, list_end,
+                                                                            total, dev);
+  PS_LAUNCHED();
+  ps::order_pack_kernel<<<grid0, ps::kThreads, 0, st>>>(total, gb, lists, list_begin, list_end, end,
+                                                        elems, elem_bits, keys, idx, dev);
+  PS_LAUNCHED();
+  PS_HIP(hipMemcpyAsync(&now, dev, sizeof(now), hipMemcpyDeviceToHost, st));
   PS_HIP(hipStreamSynchronize(st));
+  const uint32_t max_len = now.max_len;
   const int lo_bits = ps::bits_for(uint64_t(max_len) * (uint64_t(end) + 1u) + end);
-  uint32_t n = total;
-  // The finisher holds class ranks < kFinishMax in 13 bits of its keys.
-  const bool finisher = 13 + lo_bits <= 64;
+  // The finisher holds class ranks < kFinishMax in 14 bits of its keys.
+  static_assert(3 * ps::kFinishMax <= 1 << 14, "class ranks of the finisher's keys");
+  const bool finisher = 14 + lo_bits <= 64;
   if (finisher) {
     const size_t lds = ps::kFinishLds;
     PS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&ps::order_finish_kernel),
                                hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
   }
-  // Every round places at least each class's reference, so a class of k
-  // groups needs at most k rounds.
-  for (uint32_t round = 0; n > 0; ++round) {
+  // The last rounds in one workgroup, which clears and reports its own flag.
+  auto finish = [&](uint32_t n) {
+    uint32_t flag = 0;
+    uint32_t* const flag_dev = keep;  // free between rounds
+    PS_HIP(hipMemsetAsync(flag_dev, 0, 4, st));
+    ps::order_finish_kernel<<<1, ps::kFinishThreads, ps::kFinishLds, st>>>(
+        n, act_group, act_base, act_depth, lists, list_begin, list_end, end, max_len, lo_bits, gb,
+        out, flag_dev);
+    PS_LAUNCHED();
+    PS_HIP(hipMemcpyAsync(&flag, flag_dev, 4, hipMemcpyDeviceToHost, st));
+    PS_HIP(hipStreamSynchronize(st));
+    if (flag)
+      return ps::fail(PS_ERR_RUNTIME, flag == 1u
+                                          ? "ps_pre_signature_order: refinement did not converge"
+                                          : "ps_pre_signature_order: position out of range");
+    return int(PS_OK);
+  };
+  // Every later round places at least each class's reference, so a class of k
+  // groups needs at most k of them.
+  bool split = false;  // this round's keys take two passes
+  for (uint32_t round = 0; now.n > 0; ++round) {
+    const uint32_t n = now.n;
     if (round > total)
       return ps::fail(PS_ERR_RUNTIME, "ps_pre_signature_order: refinement did not converge");
-    if (finisher && n <= uint32_t(ps::kFinishMax)) {
-      uint32_t flag = 0;
-      PS_HIP(hipMemsetAsync(max_len_dev, 0, 4, st));
-      const size_t lds = ps::kFinishLds;
-      ps::order_finish_kernel<<<1, ps::kFinishThreads, lds, st>>>(
-          n, act_group, act_base, act_depth, lists, list_begin, list_end, end, max_len, lo_bits, gb, out,
-          max_len_dev);
-      PS_LAUNCHED();
-      PS_HIP(hipMemcpyAsync(&flag, max_len_dev, 4, hipMemcpyDeviceToHost, st));
-      PS_HIP(hipStreamSynchronize(st));
-      if (flag)
-        return ps::fail(PS_ERR_RUNTIME, flag == 1u
-                                            ? "ps_pre_signature_order: refinement did not converge"
-                                            : "ps_pre_signature_order: position out of range");
-      break;
-    }
+    if (finisher && n <= uint32_t(ps::kFinishMax)) return finish(n);
     const unsigned grid = ps::grid_for(n);
-    ps::order_class_heads_kernel<<<grid, ps::kThreads, 0, st>>>(act_base, n, head);
-    PS_LAUNCHED();
-    int rc = ps_exclusive_scan_u32(head, rank, n, scan_ws, stream);
-    if (rc != PS_OK) return rc;
-    ps::order_class_start_kernel<<<grid, ps::kThreads, 0, st>>>(n, head, rank, head_at);
-    PS_LAUNCHED();
-    ps::order_diverge_kernel<<<grid, ps::kThreads, 0, st>>>(
-        act_group, act_depth, n, lists, list_begin, list_end, head, rank, head_at, end, max_len, hi, lo,
-        lcp, idx);
-    PS_LAUNCHED();
-    // Sort by (hi, lo): one pass over the combined key when it fits 64 bits,
-    // else lo first and hi second (both stable).
-    const int hi_bits = ps::bits_for(3ull * n);
+    // Sort by the whole key, or lo first and hi second (both stable).
     const uint64_t* k = nullptr;
-    const uint32_t* src = nullptr;
-    if (hi_bits + lo_bits <= 64) {
-      ps::order_combine_kernel<<<grid, ps::kThreads, 0, st>>>(n, hi, lo, lo_bits, keys);
-      PS_LAUNCHED();
-      rc = ps::sort_varying(keys, keys_alt, idx, idx_alt, n, span, radix_ws, st, &k, &src);
-      if (rc != PS_OK) return rc;
-    } else {
-      ps::order_permute_key_kernel<<<grid, ps::kThreads, 0, st>>>(n, idx, lo, keys);
-      PS_LAUNCHED();
-      rc = ps::sort_varying(keys, keys_alt, idx, idx_alt, n, span, radix_ws, st, &k, &src);
-      if (rc != PS_OK) return rc;
-      uint32_t* first = const_cast<uint32_t*>(src);
-      uint32_t* first_alt = first == idx ? idx_alt : idx;
-      ps::order_permute_key_kernel<<<grid, ps::kThreads, 0, st>>>(n, first, hi, keys2);
-      PS_LAUNCHED();
-      rc = ps::sort_varying(keys2, keys2_alt, first, first_alt, n, span, radix_ws, st, &k, &src);
-      if (rc != PS_OK) return rc;
-    }
-    ps::order_runs_kernel<<<grid, ps::kThreads, 0, st>>>(n, src, hi, lo, new_head, old_head);
-    PS_LAUNCHED();
-    rc = ps_exclusive_scan_u32(new_head, new_rank, n, scan_ws, stream);
-    if (rc == PS_OK) rc = ps_exclusive_scan_u32(old_head, old_rank, n, scan_ws, stream);
+    uint32_t* src = nullptr;
+    const bool packed = round == 0;
+    ps::OrderKeys sorted{};
+    if (split) PS_HIP(hipMemcpyAsync(lo, keys, size_t(n) * 8, hipMemcpyDeviceToDevice, st));
+    int rc = ps::sort_varying(keys, keys_alt, idx, idx_alt, n, now.any ^ now.all, radix_ws, st, &k,
+                              &src);
     if (rc != PS_OK) return rc;
-    ps::order_heads_kernel<<<grid, ps::kThreads, 0, st>>>(n, new_head, new_rank, old_head,
-                                                          old_rank, new_at, old_at);
-    PS_LAUNCHED();
+    if (split) {
+      uint32_t* const src_alt = src == idx ? idx_alt : idx;
+      ps::order_permute_key_kernel<<<grid, ps::kThreads, 0, st>>>(n, src, hi, keys);
+      PS_LAUNCHED();
+      // (the classes and sides vary over all their bits: no span to wait for)
+      const uint64_t all_bits = (uint64_t(1) << ps::bits_for(3ull * n)) - 1u;
+      rc = ps::sort_varying(keys, keys_alt, src, src_alt, n, all_bits, radix_ws, st, &k, &src);
+      if (rc != PS_OK) return rc;
+      sorted.hi = hi;
+      sorted.lo = lo;
+    }
+    sorted.key = k;
+    sorted.src = src;
+    sorted.end = end;
+    sorted.lo_bits = packed ? elems * elem_bits : lo_bits;
+    sorted.elem_bits = packed ? elem_bits : 0;
     ps::order_resolve_kernel<<<grid, ps::kThreads, 0, st>>>(
-        n, src, hi, lo, end, act_group, act_base, lcp, new_head, new_rank, old_head, old_rank,
-        new_at, old_at, gb, out, keep, next_group, next_base, next_depth);
+        n, sorted, packed ? uint32_t(elems) : 0u, act_group, act_base, lcp, gb, out, keep,
+        next_group, next_base, next_depth, run_first, dev);
     PS_LAUNCHED();
     rc = ps_exclusive_scan_u32(keep, slot, n, scan_ws, stream);
     if (rc != PS_OK) return rc;
     ps::order_compact_kernel<<<grid, ps::kThreads, 0, st>>>(
-        n, keep, slot, next_group, next_base, next_depth, act_group, act_base, act_depth);
+        n, keep, slot, next_group, next_base, next_depth, run_first, act_group, act_base,
+        act_depth, act_first, dev);
     PS_LAUNCHED();
-    uint32_t tail[2] = {0u, 0u};
-    PS_HIP(hipMemcpyAsync(&tail[0], slot + (n - 1), sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-    PS_HIP(hipMemcpyAsync(&tail[1], keep + (n - 1), sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+    // the next round's keys, for as many members as `dev` says (at most n)
+    split = ps::bits_for(3ull * n) + lo_bits > 64;
+    ps::order_diverge_kernel<<<grid, ps::kThreads, 0, st>>>(
+        act_group, act_depth, act_first, lists, list_begin, list_end, end, max_len, lo_bits, keys,
+        split ? hi : nullptr, lcp, idx, dev);
+    PS_LAUNCHED();
+    PS_HIP(hipMemcpyAsync(&now, dev, sizeof(now), hipMemcpyDeviceToHost, st));
     PS_HIP(hipStreamSynchronize(st));
-    n = tail[0] + tail[1];
   }
   return PS_OK;
 }
