@@ -399,6 +399,11 @@ int ps_hub_sddmm_launch(const ps_hub_block* hb, int workset_count, const ps_work
 size_t ps_scan_workspace_bytes(size_t n);
 int ps_exclusive_scan_u32(const uint32_t* in, uint32_t* out, size_t n, void* workspace,
                           ps_stream_t stream);
+/* The same over `batch` arrays of n values, one after another, each scanned on
+ * its own. workspace: ps_scan_batch_workspace_bytes(n, batch) bytes. */
+size_t ps_scan_batch_workspace_bytes(size_t n, int batch);
+int ps_exclusive_scan_u32_batch(const uint32_t* in, uint32_t* out, size_t n, int batch,
+                                void* workspace, ps_stream_t stream);
 /* ps_exclusive_scan_u32 without a workspace and without any allocation: the
  * tile sums live in a 256 KiB array the library keeps in each GPU's memory
  * for the life of the process, so n is limited to what it holds
@@ -473,6 +478,11 @@ int ps_pre_row_keys(const int* row_ptr, int rows, int count_bits, uint64_t* keys
  * (s = 0 residue). Replaces: GetGroupNumArray (matrix_utils.cu:132-156). */
 int ps_pre_group_counts(const int* row_ptr, int rows, int group_type_num, int fine,
                         uint32_t* counts, ps_stream_t stream);
+/* The counts of ps_pre_group_counts scanned (exclusively) workset by workset,
+ * prefix[s * (rows + 1) + r] = groups of workset s before row r, and each
+ * workset's total on the host. Synchronises the stream. */
+int ps_pre_group_prefix(const int* row_ptr, int rows, int group_type_num, int fine,
+                        uint32_t* prefix, uint32_t* totals_host, ps_stream_t stream);
 
 /* Per-group metadata in initial (row) order from the exclusive prefix of the
  * counts (prefix[s * rows + r]): destination row, first ranked index, and for

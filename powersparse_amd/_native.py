@@ -210,6 +210,9 @@ HIP_API = [
     ("ps_scan_workspace_bytes", ctypes.c_size_t, [ctypes.c_size_t]),
     ("ps_exclusive_scan_u32", ctypes.c_int,
      [c_void_p, c_void_p, ctypes.c_size_t, c_void_p, c_void_p]),
+    ("ps_scan_batch_workspace_bytes", ctypes.c_size_t, [ctypes.c_size_t, ctypes.c_int]),
+    ("ps_exclusive_scan_u32_batch", ctypes.c_int,
+     [c_void_p, c_void_p, ctypes.c_size_t, ctypes.c_int, c_void_p, c_void_p]),
     ("ps_exclusive_scan_u32_noalloc", ctypes.c_int,
      [c_void_p, c_void_p, ctypes.c_size_t, c_void_p]),
     ("ps_radix_workspace_bytes", ctypes.c_size_t, [ctypes.c_size_t]),
@@ -232,6 +235,8 @@ HIP_API = [
       c_void_p, c_void_p, c_void_p]),
     ("ps_pre_group_counts", ctypes.c_int,
      [c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int, c_void_p, c_void_p]),
+    ("ps_pre_group_prefix", ctypes.c_int,
+     [c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int, c_void_p, c_u32_p, c_void_p]),
     ("ps_pre_group_meta", ctypes.c_int,
      [c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int, c_void_p, ctypes.POINTER(c_void_p),
       ctypes.POINTER(c_void_p), c_void_p, c_void_p, c_void_p]),

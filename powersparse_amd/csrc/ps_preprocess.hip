@@ -406,6 +406,13 @@ __global__ void group_counts_kernel(const int* __restrict__ row_ptr, int rows, i
   }
 }
 
+// totals[s] = groups of workset s, from the scanned counts.
+__global__ void group_totals_kernel(const uint32_t* __restrict__ prefix, int rows, int S,
+                                    uint32_t* __restrict__ totals) {
+  const int s = threadIdx.x;
+  if (s < S) totals[s] = prefix[size_t(s) * (size_t(rows) + 1) + size_t(rows)];
+}
+
 struct PtrTable {
   int* p[PS_MAX_WORKSETS];
 };
@@ -1664,6 +1671,28 @@ int ps_pre_group_counts(const int* row_ptr, int rows, int group_type_num, int fi
   ps::group_counts_kernel<<<ps::grid_for(size_t(rows) + 1), ps::kThreads, 0,
                             ps::to_hip(stream)>>>(row_ptr, rows, group_type_num, fine, counts);
   PS_LAUNCHED();
+  return PS_OK;
+}
+
+int ps_pre_group_prefix(const int* row_ptr, int rows, int group_type_num, int fine,
+                        uint32_t* prefix, uint32_t* totals_host, ps_stream_t stream) {
+  PS_CHECK_ARG(totals_host, "ps_pre_group_prefix: bad argument");
+  int rc = ps_pre_group_counts(row_ptr, rows, group_type_num, fine, prefix, stream);
+  if (rc != PS_OK) return rc;
+  const size_t n = size_t(rows) + 1;
+  using S = ps::Scratch;
+  const size_t scan_bytes = ps_scan_batch_workspace_bytes(n, group_type_num);
+  S ws(S::bytes(PS_MAX_WORKSETS, 4) + S::bytes(scan_bytes, 1));
+  PS_HIP(ws.error());
+  uint32_t* totals = ws.take<uint32_t>(PS_MAX_WORKSETS);
+  rc = ps_exclusive_scan_u32_batch(prefix, prefix, n, group_type_num, ws.take<char>(scan_bytes),
+                                   stream);
+  if (rc != PS_OK) return rc;
+  hipStream_t st = ps::to_hip(stream);
+  ps::group_totals_kernel<<<1, ps::kWave, 0, st>>>(prefix, rows, group_type_num, totals);
+  PS_LAUNCHED();
+  PS_HIP(hipMemcpyAsync(totals_host, totals, size_t(group_type_num) * 4, hipMemcpyDeviceToHost, st));
+  PS_HIP(hipStreamSynchronize(st));
   return PS_OK;
 }
 

@@ -39,6 +39,8 @@ __global__ __launch_bounds__(kThreads) void scan_reduce_kernel(const uint32_t* _
                                                                size_t n,
                                                                uint32_t* __restrict__ sums) {
   __shared__ uint32_t wave_sum[kThreads / kWave];
+  in += size_t(blockIdx.y) * n;  // the batch's arrays follow one another
+  sums += size_t(blockIdx.y) * gridDim.x;
   const size_t base = size_t(blockIdx.x) * kTile;
   uint32_t s = 0;
 #pragma unroll
@@ -62,6 +64,9 @@ __global__ __launch_bounds__(kThreads) void scan_apply_kernel(const uint32_t* in
                                                               size_t n,
                                                               const uint32_t* __restrict__ offsets) {
   __shared__ uint32_t wave_sum[kThreads / kWave];
+  in += size_t(blockIdx.y) * n;
+  out += size_t(blockIdx.y) * n;
+  if (offsets) offsets += size_t(blockIdx.y) * gridDim.x;
   const size_t base = size_t(blockIdx.x) * kTile + size_t(threadIdx.x) * kItems;
   uint32_t v[kItems];
   uint32_t total = 0;
@@ -87,27 +92,31 @@ __global__ __launch_bounds__(kThreads) void scan_apply_kernel(const uint32_t* in
 
 size_t align_up(size_t x) { return (x + 255) & ~size_t(255); }
 
-size_t scan_ws(size_t n) {
+size_t scan_ws(size_t n, unsigned batch = 1) {
   if (n <= size_t(kTile)) return 0;
   const size_t b = (n + kTile - 1) / kTile;
-  return align_up(b * sizeof(uint32_t)) + scan_ws(b);
+  return align_up(batch * b * sizeof(uint32_t)) + scan_ws(b, batch);
 }
 
-int scan(const uint32_t* in, uint32_t* out, size_t n, char* ws, hipStream_t stream) {
+// `batch` arrays of n values, one after another, each scanned on its own.
+int scan(const uint32_t* in, uint32_t* out, size_t n, char* ws, hipStream_t stream,
+         unsigned batch = 1) {
   if (n == 0) return PS_OK;
   const size_t blocks = (n + kTile - 1) / kTile;
-  PS_CHECK_ARG(blocks < (1u << 31), "scan too large");
+  PS_CHECK_ARG(blocks < (1u << 31) && batch <= 65535, "scan too large");
+  const dim3 grid(unsigned(blocks), batch);
   if (blocks == 1) {
-    scan_apply_kernel<<<1, kThreads, 0, stream>>>(in, out, n, nullptr);
+    scan_apply_kernel<<<grid, kThreads, 0, stream>>>(in, out, n, nullptr);
     PS_LAUNCHED();
     return PS_OK;
   }
   uint32_t* sums = reinterpret_cast<uint32_t*>(ws);
-  scan_reduce_kernel<<<unsigned(blocks), kThreads, 0, stream>>>(in, n, sums);
+  scan_reduce_kernel<<<grid, kThreads, 0, stream>>>(in, n, sums);
   PS_LAUNCHED();
-  const int rc = scan(sums, sums, blocks, ws + align_up(blocks * sizeof(uint32_t)), stream);
+  const int rc = scan(sums, sums, blocks, ws + align_up(batch * blocks * sizeof(uint32_t)), stream,
+                      batch);
   if (rc != PS_OK) return rc;
-  scan_apply_kernel<<<unsigned(blocks), kThreads, 0, stream>>>(in, out, n, sums);
+  scan_apply_kernel<<<grid, kThreads, 0, stream>>>(in, out, n, sums);
   PS_LAUNCHED();
   return PS_OK;
 }
@@ -304,6 +313,19 @@ int ps_exclusive_scan_u32(const uint32_t* in, uint32_t* out, size_t n, void* wor
   PS_CHECK_ARG(in && out, "ps_exclusive_scan_u32: null buffer");
   PS_CHECK_ARG(workspace || ps::scan_ws(n) == 0, "ps_exclusive_scan_u32: null workspace");
   return ps::scan(in, out, n, reinterpret_cast<char*>(workspace), ps::to_hip(stream));
+}
+
+size_t ps_scan_batch_workspace_bytes(size_t n, int batch) {
+  return batch > 0 ? ps::scan_ws(n, unsigned(batch)) + 256 : 0;
+}
+
+int ps_exclusive_scan_u32_batch(const uint32_t* in, uint32_t* out, size_t n, int batch,
+                                void* workspace, ps_stream_t stream) {
+  if (n == 0 || batch == 0) return PS_OK;
+  PS_CHECK_ARG(in && out && batch > 0, "ps_exclusive_scan_u32_batch: bad argument");
+  PS_CHECK_ARG(workspace || ps::scan_ws(n) == 0, "ps_exclusive_scan_u32_batch: null workspace");
+  return ps::scan(in, out, n, reinterpret_cast<char*>(workspace), ps::to_hip(stream),
+                  unsigned(batch));
 }
 
 size_t ps_radix_workspace_bytes(size_t n) { return ps::radix_ws(n) + 256; }

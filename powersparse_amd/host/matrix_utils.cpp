@@ -162,38 +162,6 @@ int WorksetCount(const unsigned long long* degree_sums, int cu_count) {
 
 namespace {
 
-// Groups per workset, as the device kernels split each row (matrix_utils.cu:
-// 132-156): S == 1 cuts rows into chunks of `fine`; otherwise the block sizes
-// are taken greedily from the largest and the rest is one residue group.
-void HostGroupCounts(const int* row_ptr, int rows, int S, int fine, int* group_num) {
-  std::vector<long long> total(static_cast<size_t>(S), 0);
-#pragma omp parallel
-  {
-    std::vector<long long> mine(static_cast<size_t>(S), 0);
-#pragma omp for schedule(static)
-    for (int r = 0; r < rows; ++r) {
-      long long d = row_ptr[r + 1] - row_ptr[r];
-      if (S == 1) {
-        mine[0] += (d + fine - 1) / fine;
-        continue;
-      }
-      for (int s = S - 1; s > 0; --s) {
-        const long long n = d / GROUP_SIZE(s);
-        mine[size_t(s)] += n;
-        d -= n * GROUP_SIZE(s);
-      }
-      mine[0] += d > 0;
-    }
-#pragma omp critical
-    for (int s = 0; s < S; ++s) total[size_t(s)] += mine[size_t(s)];
-  }
-  for (int s = 0; s < S; ++s) {
-    if (total[size_t(s)] > std::numeric_limits<int>::max())
-      throw std::runtime_error("Too many groups in one workset");
-    group_num[s] = int(total[size_t(s)]);
-  }
-}
-
 int BitsFor(uint64_t v) {
   int b = 0;
   while (b < 64 && (v >> b) != 0) ++b;
@@ -366,7 +334,7 @@ PowerSparseMatrixGPU::PowerSparseMatrixGPU(int row_num, int col_num, int nnz_num
     // decides the order at the end of the build).
     const bool may_tune =
         policy.spmm_partition == SpmmPartition::kTuned && _task_order != TaskOrder::kRow;
-    Build(row_ptr, in);
+    Build(in);
     bool hub = false;
     if (may_tune && _task_order == TaskOrder::kSignature && _want_run_order &&
         policy.hub_block == HubBlock::kAuto)
@@ -381,7 +349,7 @@ PowerSparseMatrixGPU::PowerSparseMatrixGPU(int row_num, int col_num, int nnz_num
       tuned.spmm_partition = SpmmPartition::kParity;
       _spmm_tuned =
           new PowerSparseMatrixGPU(Unbuilt{}, row_num, col_num, nnz_num, _cu_count, tuned);
-      _spmm_tuned->Build(row_ptr, in);
+      _spmm_tuned->Build(in);
     }
     in.clock.Finish();
   } catch (...) {
@@ -390,7 +358,7 @@ PowerSparseMatrixGPU::PowerSparseMatrixGPU(int row_num, int col_num, int nnz_num
   }
 }
 
-void PowerSparseMatrixGPU::Build(const int* row_ptr, Prepared& in) {
+void PowerSparseMatrixGPU::Build(Prepared& in) {
   const int rows = _matrix_row, nnz = _matrix_nnz;
   const int fine = _group_fine_size;
   ps_stream_t st = nullptr;
@@ -407,10 +375,18 @@ void PowerSparseMatrixGPU::Build(const int* row_ptr, Prepared& in) {
   if (S > PS_MAX_WORKSETS) throw std::runtime_error("Too many worksets");
   _group_type_num = S;
 
-  // Group counts per workset, on the host from row_ptr (the split the device
-  // kernels make), so the device arrays are sized without waiting.
+  // Per-row group counts, their exclusive scans (group ids in row order) and
+  // the groups per workset.
+  const size_t stride = size_t(rows) + 1;
+  DeviceArray<uint32_t> prefix(static_cast<size_t>(S) * stride);
+  uint32_t totals[PS_MAX_WORKSETS] = {};
+  ThrowOnError(ps_pre_group_prefix(d_rp.data(), rows, S, fine, prefix.data(), totals, st));
   _group_num = new int[S]();
-  HostGroupCounts(row_ptr, rows, S, fine, _group_num);
+  for (int s = 0; s < S; ++s) {
+    if (totals[s] > uint32_t(std::numeric_limits<int>::max()))
+      throw std::runtime_error("Too many groups in one workset");
+    _group_num[s] = int(totals[s]);
+  }
   const int G0 = _group_num[0];
   std::vector<long long> lengths(static_cast<size_t>(S), 0);  // nonzeros per workset
   lengths[0] = nnz;
@@ -418,15 +394,6 @@ void PowerSparseMatrixGPU::Build(const int* row_ptr, Prepared& in) {
     lengths[size_t(s)] = (long long)_group_num[s] * GROUP_SIZE(s);
     lengths[0] -= lengths[size_t(s)];
   }
-
-  // Per-row group counts and their exclusive scans (group ids in row order).
-  const size_t stride = size_t(rows) + 1;
-  DeviceArray<uint32_t> prefix(static_cast<size_t>(S) * stride);
-  ThrowOnError(ps_pre_group_counts(d_rp.data(), rows, S, fine, prefix.data(), st));
-  DeviceArray<char> scan_ws(ps_scan_workspace_bytes(stride));
-  for (int s = 0; s < S; ++s)
-    ThrowOnError(ps_exclusive_scan_u32(prefix.data() + s * stride, prefix.data() + s * stride,
-                                       stride, scan_ws.data(), st));
 
   std::vector<DeviceArray<int>> des0(static_cast<size_t>(S)), start(static_cast<size_t>(S));
   std::vector<int*> des_ptr(static_cast<size_t>(S), nullptr), start_ptr(static_cast<size_t>(S), nullptr);
@@ -853,9 +820,8 @@ bool PowerSparseMatrixGPU::BuildHub(const int* row_ptr, Prepared& in,
     ThrowOnError(ps_exclusive_scan_u32(kept.data(), reinterpret_cast<uint32_t*>(rest_ptr.data()),
                                        size_t(rows) + 1, scan_ws.data(), nullptr));
   }
-  std::vector<int> rp_host(size_t(rows) + 1);
-  rest_ptr.Download(rp_host.data(), rp_host.size());
-  const int nnz_rest = rp_host.back();
+  int nnz_rest = 0;
+  ThrowOnError(ps_memcpy_dtoh(&nnz_rest, rest_ptr.data() + rows, sizeof(int)));
   if (nnz_rest <= 0) return false;  // the block would hold every nonzero
   // the rest must keep the public partition's store rule: more than one workset
   unsigned long long rest_sums[32] = {};
@@ -876,7 +842,7 @@ bool PowerSparseMatrixGPU::BuildHub(const int* row_ptr, Prepared& in,
   tuned.hub_block = HubBlock::kOff;
   std::unique_ptr<PowerSparseMatrixGPU> part(
       new PowerSparseMatrixGPU(Unbuilt{}, rows, cols, nnz_rest, _cu_count, tuned));
-  part->Build(rp_host.data(), in);
+  part->Build(in);
   // hub rows add their remaining entries to the block's product
   for (const auto& t : hub->tiers)
     ThrowOnError(ps_hub_mark_atomic(&t->desc, part->_group_des[0], part->_group_num[0],

@@ -258,7 +258,7 @@ class PowerSparseMatrixGPU {
                        const PartitionPolicy& policy);
   void Configure(const PartitionPolicy& policy);
   // The partition at this object's settings from the prepared stages.
-  void Build(const int* row_ptr, Prepared& in);
+  void Build(Prepared& in);
   void Release() noexcept;
   void ReleaseExecution() noexcept;
   void BuildRunOrders();
