@@ -69,6 +69,12 @@ int ps_device_synchronize(void);
  * benchmark_utils.h:13-37). ps_free(NULL) is a no-op. */
 int ps_malloc(void** ptr, size_t bytes);
 int ps_free(void* ptr);
+/* ps_free keeps blocks of 2 MB and more for later ps_malloc calls, up to a
+ * sixteenth of the device's memory: they are given back to the driver after
+ * ten seconds unused (at a later ps_free), when an allocation fails, by
+ * ps_mem_get_info, and by this call (the current device's). No reference
+ * counterpart. */
+int ps_mem_trim(void);
 /* Debugging aid, no reference counterpart. With the environment variable
  * PS_DEVICE_GUARD set to a byte count when the library is first used, every
  * device block the library allocates (ps_malloc, and the temporaries of the
@@ -79,7 +85,8 @@ int ps_free(void* ptr);
  * (each run is also reported on stderr); -1 when guards are off, -2 when the
  * device cannot be synchronised. */
 long long ps_guard_violations(void);
-/* Free and total device memory of the current device, in bytes (hipMemGetInfo).
+/* Free and total device memory of the current device, in bytes (hipMemGetInfo
+ * after ps_mem_trim).
  * No reference counterpart: callers and tests use it to check that a matrix
  * releases every device allocation it made. */
 int ps_mem_get_info(size_t* free_bytes, size_t* total_bytes);

@@ -1,0 +1,87 @@
+"""Device blocks kept between ps_free and ps_malloc: reuse, the size rule, and
+giving them back."""
+from concurrent.futures import ThreadPoolExecutor
+
+import numpy as np
+import pytest
+
+import powersparse_amd as ps
+from powersparse_amd import _native
+from gpu_util import say, setup
+
+pytestmark = pytest.mark.gpu
+
+MB = 1 << 20
+
+
+def raw_free_bytes():
+    """The driver's free memory, asked for without ps_mem_get_info's trim."""
+    import torch
+    return torch.cuda.mem_get_info()[0]
+
+
+@pytest.mark.parametrize("first,second,same", [
+    (64 * MB, 64 * MB, True), (64 * MB, 63 * MB + 5, True), (64 * MB, 52 * MB, True),
+    (64 * MB, 50 * MB, False), (64 * MB, 65 * MB, False), (2 * MB, 2 * MB, True)])
+def test_reuse_rule(first, second, same):
+    # a kept block serves requests from four fifths of its size up to it
+    setup()
+    assert _native.hip().ps_mem_trim() == _native.PS_OK
+    a = ps.DeviceBuffer(first)
+    ptr = a.ptr
+    a.free()
+    b = ps.DeviceBuffer(second)
+    say(f"{first} then {second}: {'same' if b.ptr == ptr else 'another'} block")
+    got = b.ptr
+    x = np.arange(second // 4, dtype=np.uint32)
+    b.upload(x)
+    np.testing.assert_array_equal(b.download(np.uint32, x.size), x)
+    b.free()
+    assert (got == ptr) == same
+
+
+def test_given_back():
+    setup()
+    _native.hip().ps_mem_trim()
+    free0 = raw_free_bytes()
+    a = ps.DeviceBuffer(512 * MB)
+    assert raw_free_bytes() <= free0 - 500 * MB
+    a.free()
+    assert raw_free_bytes() <= free0 - 500 * MB  # kept
+    assert ps.mem_get_info()[0] >= free0 - 4 * MB  # counted as free, and given back
+    assert raw_free_bytes() >= free0 - 4 * MB
+
+
+def test_bounded():
+    # blocks beyond a sixteenth of the device go back to the driver, oldest first
+    setup()
+    _native.hip().ps_mem_trim()
+    total = ps.mem_get_info()[1]
+    free0 = raw_free_bytes()
+    n = total // 16 // (1024 * MB) + 3
+    blocks = [ps.DeviceBuffer(1024 * MB) for _ in range(n)]
+    for b in blocks:
+        b.free()
+    kept = free0 - raw_free_bytes()
+    say(f"kept {kept >> 20} MB of {total >> 20} MB")
+    assert total // 16 - 2048 * MB <= kept <= total // 16 + 4 * MB
+    _native.hip().ps_mem_trim()
+
+
+def test_threads_never_share_a_block():
+    setup()
+
+    def work(t):
+        ps.set_device(0)
+        rng = np.random.default_rng(t)
+        for _ in range(30):
+            n = int(rng.integers(2 * MB, 8 * MB)) // 4
+            b = ps.DeviceBuffer(n * 4)
+            x = rng.integers(0, 1 << 32, n, dtype=np.uint32)
+            b.upload(x)
+            np.testing.assert_array_equal(b.download(np.uint32, n), x)
+            b.free()
+        return True
+
+    with ThreadPoolExecutor(8) as ex:
+        assert all(ex.map(work, range(8)))
