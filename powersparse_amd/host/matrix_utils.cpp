@@ -716,6 +716,7 @@ bool PowerSparseMatrixGPU::BuildHub(const int* row_ptr, Prepared& in,
       specs.push_back({policy.hub_min_degree[k], hi, policy.hub_min_count[k]});
     }
   } else {
+    if (double(_matrix_nnz) < kHubMinGainNonzeros) return false;
     // nonzeros of rows of degree >= 2^a (a >= 8) in columns of count >= 2^b
     DeviceArray<unsigned long long> hist(32 * 32);
     ThrowOnError(ps_hub_histogram(in.row_ptr.data(), rows, in.col_ind.data(), in.col_nnz.data(),
@@ -745,7 +746,9 @@ bool PowerSparseMatrixGPU::BuildHub(const int* row_ptr, Prepared& in,
             bb = b;
           }
         }
-      if (ba < 0 || best < (k == 0 ? kHubMinGain : kHubMinTierGain) * double(_matrix_nnz)) break;
+      if (ba < 0 || best < (k == 0 ? kHubMinGain : kHubMinTierGain) * double(_matrix_nnz) ||
+          (k == 0 && best < kHubMinGainNonzeros))
+        break;
       specs.push_back({1LL << ba, top < 32 ? (1LL << top) : std::numeric_limits<long long>::max(),
                        1LL << bb});
       top = ba;

@@ -86,8 +86,14 @@ constexpr int kTunedSpmmGroupTypes = 3;
 // kHubMaxTiers tiers of disjoint row ranges, each with its own columns: the
 // first tier is the pair of power-of-two thresholds (row degree >= 2^a,
 // column count >= 2^b) that maximises block nonzeros - kHubDenseCost * rows
-// * columns, kept when that gain is at least kHubMinGain of the nonzeros; the
-// next tier takes the rows below 2^a the same way, kept from kHubMinTierGain
+// * columns, kept when that gain is at least kHubMinGain of the nonzeros and
+// kHubMinGainNonzeros: below it the block's extra launches and the cheaper
+// gathers of a smaller graph cost more than the block saves. Chung-Lu graphs,
+// with against without the block, SpMM N = 32 / 128, SDDMM N = 32 / 128: gain
+// 22.8 M (128 M nonzeros) 0.94 / 0.86, 1.01 / 1.00; 12.7 M (66 M) 1.01 / 0.87,
+// 1.05 / 0.94; 7.9 M (100 M) 1.05 / 0.97, 1.00 / 1.00; 6.3 M (32 M) 1.16 / 0.94,
+// 1.14 / 0.94; 3.6 M (16.5 M) 1.38 / 0.98, 1.08 / 0.93; 0.9 M (4 M) 2.34 /
+// 1.57, 1.74 / 1.17. The next tier takes the rows below 2^a the same way, kept from kHubMinTierGain
 // (kHubDenseCost: the dense element's cost relative to the sparse nonzero it
 // replaces, measured on MI355X). SDDMM computes a tier's dense dots whole and
 // takes from it only the tiles lying inside it, so it uses a tier when those
@@ -105,6 +111,7 @@ constexpr int kTunedSpmmGroupTypes = 3;
 enum class HubBlock { kAuto = 0, kOff = 1 };
 constexpr int kHubMaxTiers = 3;
 constexpr double kHubDenseCost = 0.12, kHubMinGain = 0.05, kHubMinTierGain = 0.02;
+constexpr double kHubMinGainNonzeros = 10e6;
 constexpr double kHubSddmmMinFill = 0.25;
 constexpr int kHubMinRows = 256, kHubMinCols = 1024;
 constexpr long long kHubMaxElements = 1LL << 29;
