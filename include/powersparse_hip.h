@@ -116,6 +116,8 @@ int ps_fill_random_async(float* dst, size_t count, uint64_t seed, float lo, floa
 int ps_stream_create(ps_stream_t* stream);
 int ps_stream_destroy(ps_stream_t stream);
 int ps_stream_synchronize(ps_stream_t stream);
+/* *idle = 1 when everything enqueued on the stream so far has run, else 0. */
+int ps_stream_idle(ps_stream_t stream, int* idle);
 /* Replaces: cudaEventCreate/Record/Synchronize/ElapsedTime (benchmark_utils.h:68-88). */
 int ps_event_create(ps_event_t* event);
 int ps_event_destroy(ps_event_t event);

@@ -121,6 +121,7 @@ HIP_API = [
       c_void_p]),
     ("ps_stream_create", ctypes.c_int, [ctypes.POINTER(c_void_p)]),
     ("ps_stream_destroy", ctypes.c_int, [c_void_p]),
+    ("ps_stream_idle", ctypes.c_int, [c_void_p, c_int_p]),
     ("ps_stream_synchronize", ctypes.c_int, [c_void_p]),
     ("ps_event_create", ctypes.c_int, [ctypes.POINTER(c_void_p)]),
     ("ps_event_destroy", ctypes.c_int, [c_void_p]),

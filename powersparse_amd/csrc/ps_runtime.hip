@@ -469,6 +469,16 @@ int ps_stream_synchronize(ps_stream_t stream) {
   return PS_OK;
 }
 
+int ps_stream_idle(ps_stream_t stream, int* idle) {
+  PS_CHECK_ARG(idle, "ps_stream_idle: null output");
+  const hipError_t e = hipStreamQuery(ps::to_hip(stream));
+  if (e != hipSuccess) (void)hipGetLastError();  // not ready is an answer, not a failure
+  *idle = e == hipSuccess ? 1 : 0;
+  if (e == hipErrorNotReady) return PS_OK;
+  PS_HIP(e);
+  return PS_OK;
+}
+
 int ps_event_create(ps_event_t* event) {
   PS_CHECK_ARG(event, "ps_event_create: null output");
   hipEvent_t e = nullptr;
