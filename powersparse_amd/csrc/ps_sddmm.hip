@@ -28,6 +28,9 @@
 // signature-ordered worksets. A task's work, and so every output, is the same
 // in any order; residue tasks keep their 8 consecutive groups.
 //
+// Wide features run as slices, one launch after another: the first stores
+// a_p * <its features>, the others add theirs (kSliceWide / kSliceNarrow).
+//
 // Store modes (kMode): 0 = at the nonzero's own position (as above); 1 = per
 // nonzero map, out[s][map[s][p]]: CSR order (every out[s] is the one
 // CSR-order array, map = CSR positions, plain stores: each position is
@@ -46,6 +49,25 @@ constexpr int kTaskOut = 256;  // residue results of one task collected in LDS
 // C3 N = 128: runs of 256 workgroups 1.4% faster than the round robin, 1024
 // slower on C1).
 constexpr int kAutoChunkMax = 256;
+// Most features per launch. One launch over all of N = 512 holds 64 VGPRs of X
+// and few loads in flight, and its Y rows crowd the L2; slices re-read 12
+// bytes per nonzero each instead. 128 features where Y is larger than
+// kWideRhsBytes, else 256; in CSR order, where every further slice costs a
+// scattered read and write per nonzero, 256 and 320 (us, N = 256 / 512):
+//   C1, one launch -> slices of 128        4880 / 10613 -> 4486 / 8975
+//   100 k nodes, 5 M nonzeros              437 / 987 -> 384 / 764
+//   community graph, 13 M                  1230 / 2694 -> 1150 / 2285
+//   100 k x 5 k uniform, N = 512           716 -> 536 (256), 568 (128)
+//   20 k nodes, 1 M, N = 256 / 512         87 / 182 -> 81 / 161 (256), 92 / 184 (128)
+//   100 k nodes in CSR order, N = 192      334 -> 385 (128)
+//   the same, N = 320 / 512                585 / 1005 -> 564 / 919 (256)
+//   20 k nodes in CSR order, N = 288       98 -> 103 (256)
+// Launches that gather less than kSliceMinGather (an upper bound: every task
+// full) are not cut: another launch costs about 3.5 us (61 k nonzeros, N = 448:
+// 25.9 us in one launch, 29.3 in two).
+constexpr int kSliceNarrow = 128, kSliceWide = 256, kSliceCsr = 320;
+constexpr uint64_t kWideRhsBytes = uint64_t(48) << 20;
+constexpr uint64_t kSliceMinGather = uint64_t(512) << 20;
 static_assert(kTaskOut >= 8 * kStage, "a task's slots each collect up to kStage results");
 
 struct SddmmArgs {
@@ -53,7 +75,8 @@ struct SddmmArgs {
   float* out[PS_MAX_WORKSETS];
   uint32_t task_begin[PS_MAX_WORKSETS + 1];
   int32_t count;
-  int32_t N;
+  uint32_t row_bytes;     // bytes from one X / Y row to the next
+  int32_t accumulate;     // add to the outputs stored by an earlier feature slice
   uint32_t total_tasks;   // tasks of the worksets
   uint32_t launch_tasks;  // waves with work: total_tasks, or the task map's length
   const int* residue_offset;
@@ -67,16 +90,59 @@ struct SddmmArgs {
   const uint32_t* task_map;             // run order of the tasks, or null
 };
 
-// Transposing reduction over the 8 lanes of a slot: in p[j] each lane holds
-// its partial for nonzero j of the slot; returns the full sum for j == sub.
-__device__ __forceinline__ float slot_transpose_sum(const float (&p)[8], int sub) {
+// The full dot of nonzero `sub` of this lane's slot, whose 8 nonzeros have
+// the columns col_of(0 .. 7). In p[j] of a transposing butterfly each lane
+// would hold its partial for nonzero j; the nonzeros are taken in pairs
+// (j, j + 4), P pairs per batch, and each pair's partials pass the
+// butterfly's first (xor 4) exchange at once, so a lane keeps 4 partials
+// instead of 8 and no row offsets (the same sums, bit for bit; with one pair
+// per batch the K = 128 kernel took 69 VGPRs instead of 79 and ran C3 SDDMM
+// N=128 in 6.26 instead of 6.29 ms).
+template <int KQ, bool kBuf, typename ColOf>
+__device__ __forceinline__ float slot_dot(const Rows<kBuf>& Y, uint32_t row_bytes, uint32_t piece,
+                                          const float4 (&x)[KQ], int sub, ColOf col_of) {
+  using Off = typename Rows<kBuf>::Off;
+  // pairs per batch: 8 KQ loads in flight up to K = 64, 16 at K = 128
+  // (C3 SDDMM N=128 6.234 -> 6.195 ms, C1 2.250 -> 2.230 ms against 8
+  // loads, although the kernel then holds 100 VGPRs, 4 waves per SIMD; 32
+  // loads: 6.494 ms; K = 64 with 8 loads instead of 16: C4 1.347 -> 1.372
+  // ms), 2 KQ otherwise
+  constexpr int P = KQ <= 2 ? 4 : (KQ == 4 ? 2 : 1);
   const bool b2 = sub & 4, b1 = sub & 2, b0 = sub & 1;
   float q[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float keep = b2 ? p[i + 4] : p[i];
-    const float send = b2 ? p[i] : p[i + 4];
-    q[i] = keep + xor_shfl<4>(send);
+  for (int i0 = 0; i0 < 4; i0 += P) {
+    float4 y[P][2][KQ];
+#pragma unroll
+    for (int u = 0; u < P; ++u) {
+      const Off o0 = Off(uint32_t(col_of(i0 + u))) * row_bytes + piece;
+      const Off o1 = Off(uint32_t(col_of(i0 + u + 4))) * row_bytes + piece;
+#pragma unroll
+      for (int k = 0; k < KQ; ++k) {
+        y[u][0][k] = Y.load(o0 + 128u * uint32_t(k));
+        y[u][1][k] = Y.load(o1 + 128u * uint32_t(k));
+      }
+    }
+    // keep the whole batch of loads in flight before the first use
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < P; ++u) {
+      float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+      for (int k = 0; k < KQ; ++k) {
+        s0 = fmaf(x[k].x, y[u][0][k].x, s0);
+        s0 = fmaf(x[k].y, y[u][0][k].y, s0);
+        s0 = fmaf(x[k].z, y[u][0][k].z, s0);
+        s0 = fmaf(x[k].w, y[u][0][k].w, s0);
+        s1 = fmaf(x[k].x, y[u][1][k].x, s1);
+        s1 = fmaf(x[k].y, y[u][1][k].y, s1);
+        s1 = fmaf(x[k].z, y[u][1][k].z, s1);
+        s1 = fmaf(x[k].w, y[u][1][k].w, s1);
+      }
+      // the butterfly's first exchange for nonzeros i and i + 4
+      const float keep = b2 ? s1 : s0, send = b2 ? s0 : s1;
+      q[i0 + u] = keep + xor_shfl<4>(send);
+    }
   }
   float r[2];
 #pragma unroll
@@ -90,115 +156,9 @@ __device__ __forceinline__ float slot_transpose_sum(const float (&p)[8], int sub
   return keep + xor_shfl<1>(send);
 }
 
-// Partial dots of the 8 nonzeros of this lane's slot (Y row byte offsets in
-// yoff[]), `kSteps` nonzeros per batch: 8-16 loads in flight per lane.
-template <int KQ, bool kBuf>
-__device__ __forceinline__ void slot_dots(const Rows<kBuf>& Y,
-                                          const typename Rows<kBuf>::Off (&yoff)[8],
-                                          const float4 (&x)[KQ], float (&p)[8]) {
-  // a power of two dividing the 8 steps: 16 loads for K <= 64, 8 for K = 96,
-  // 128 (in the run order, C3 N = 128: 7.69 ms with 16, 7.50 with 8, 7.74
-  // with 4; C1 2.272 / 2.278 / 2.342 ms), 16 for K <= 256, 16-32 beyond
-  constexpr int kSteps = KQ <= 2 ? 8 : (KQ <= 4 ? 2 : (KQ <= 8 ? 2 : 1));
-  static_assert(8 % kSteps == 0, "batches must tile the slot's 8 nonzeros");
-#pragma unroll
-  for (int b = 0; b < 8; b += kSteps) {
-    float4 y[kSteps][KQ];
-#pragma unroll
-    for (int u = 0; u < kSteps; ++u)
-#pragma unroll
-      for (int q = 0; q < KQ; ++q) y[u][q] = Y.load(yoff[b + u] + 128u * uint32_t(q));
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int u = 0; u < kSteps; ++u) {
-      float s = 0.f;
-#pragma unroll
-      for (int q = 0; q < KQ; ++q) {
-        s = fmaf(x[q].x, y[u][q].x, s);
-        s = fmaf(x[q].y, y[u][q].y, s);
-        s = fmaf(x[q].z, y[u][q].z, s);
-        s = fmaf(x[q].w, y[u][q].w, s);
-      }
-      p[b + u] = s;
-    }
-  }
-}
-
-// The full dot of nonzero `sub` of this lane's slot, whose 8 nonzeros have
-// the columns col_of(0 .. 7). Up to K = 256 the nonzeros are taken in pairs
-// (j, j + 4), P pairs per batch, and each pair's partials pass the
-// butterfly's first (xor 4) exchange at once, so a lane keeps 4 partials
-// instead of 8 and no row offsets (the same sums, bit for bit; with one pair
-// per batch the K = 128 kernel took 69 VGPRs instead of 79 and ran C3 SDDMM
-// N=128 in 6.26 instead of 6.29 ms).
-template <int KQ, bool kBuf, typename ColOf>
-__device__ __forceinline__ float slot_dot(const Rows<kBuf>& Y, uint32_t row_bytes, uint32_t piece,
-                                          const float4 (&x)[KQ], int sub, ColOf col_of) {
-  using Off = typename Rows<kBuf>::Off;
-  if constexpr (KQ > 8) {
-    float p[8];
-    Off yoff[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) yoff[j] = Off(uint32_t(col_of(j))) * row_bytes + piece;
-    slot_dots<KQ, kBuf>(Y, yoff, x, p);
-    return slot_transpose_sum(p, sub);
-  } else {
-    // pairs per batch: 8 KQ loads in flight up to K = 64, 16 at K = 128
-    // (C3 SDDMM N=128 6.234 -> 6.195 ms, C1 2.250 -> 2.230 ms against 8
-    // loads, although the kernel then holds 100 VGPRs, 4 waves per SIMD; 32
-    // loads: 6.494 ms; K = 64 with 8 loads instead of 16: C4 1.347 -> 1.372
-    // ms), 2 KQ otherwise
-    constexpr int P = KQ <= 2 ? 4 : (KQ == 4 ? 2 : 1);
-    const bool b2 = sub & 4, b1 = sub & 2, b0 = sub & 1;
-    float q[4];
-#pragma unroll
-    for (int i0 = 0; i0 < 4; i0 += P) {
-      float4 y[P][2][KQ];
-#pragma unroll
-      for (int u = 0; u < P; ++u) {
-        const Off o0 = Off(uint32_t(col_of(i0 + u))) * row_bytes + piece;
-        const Off o1 = Off(uint32_t(col_of(i0 + u + 4))) * row_bytes + piece;
-#pragma unroll
-        for (int k = 0; k < KQ; ++k) {
-          y[u][0][k] = Y.load(o0 + 128u * uint32_t(k));
-          y[u][1][k] = Y.load(o1 + 128u * uint32_t(k));
-        }
-      }
-      // keep the whole batch of loads in flight before the first use
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int u = 0; u < P; ++u) {
-        float s0 = 0.f, s1 = 0.f;
-#pragma unroll
-        for (int k = 0; k < KQ; ++k) {
-          s0 = fmaf(x[k].x, y[u][0][k].x, s0);
-          s0 = fmaf(x[k].y, y[u][0][k].y, s0);
-          s0 = fmaf(x[k].z, y[u][0][k].z, s0);
-          s0 = fmaf(x[k].w, y[u][0][k].w, s0);
-          s1 = fmaf(x[k].x, y[u][1][k].x, s1);
-          s1 = fmaf(x[k].y, y[u][1][k].y, s1);
-          s1 = fmaf(x[k].z, y[u][1][k].z, s1);
-          s1 = fmaf(x[k].w, y[u][1][k].w, s1);
-        }
-        // slot_transpose_sum's first exchange for nonzeros i and i + 4
-        const float keep = b2 ? s1 : s0, send = b2 ? s0 : s1;
-        q[i0 + u] = keep + xor_shfl<4>(send);
-      }
-    }
-    float r[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const float keep = b1 ? q[i + 2] : q[i];
-      const float send = b1 ? q[i] : q[i + 2];
-      r[i] = keep + xor_shfl<2>(send);
-    }
-    const float keep = b0 ? r[1] : r[0];
-    const float send = b0 ? r[0] : r[1];
-    return keep + xor_shfl<1>(send);
-  }
-}
-
-template <int KQ, bool kBuf, int kMode>
+// kSliced: one of several feature slices (rows further apart than the slice is
+// wide; all but the first add to the outputs).
+template <int KQ, bool kBuf, int kMode, bool kSliced>
 __global__ __launch_bounds__(kWave* kWavesPerBlock) void sddmm_kernel(SddmmArgs args) {
   constexpr int K = 32 * KQ;
   __shared__ __attribute__((aligned(16))) int stage[kWavesPerBlock][8 * kStage];
@@ -224,7 +184,8 @@ __global__ __launch_bounds__(kWave* kWavesPerBlock) void sddmm_kernel(SddmmArgs 
   const int slot = lane / 8, sub = lane % 8;
   const Rows<kBuf> X(args.lhs, args.lhs_bytes), Y(args.rhs, args.rhs_bytes);
   using Off = typename Rows<kBuf>::Off;
-  const uint32_t row_bytes = uint32_t(K) * 4u;
+  const uint32_t row_bytes = kSliced ? args.row_bytes : uint32_t(K) * 4u;
+  const bool accumulate = kSliced && args.accumulate;
   const uint32_t piece = uint32_t(sub) * 16u;
   float4 x[KQ];
   int* const wave_stage = stage[threadIdx.x / kWave];
@@ -252,6 +213,7 @@ __global__ __launch_bounds__(kWave* kWavesPerBlock) void sddmm_kernel(SddmmArgs 
       const int gl = pos >> gs_shift;
       if (valid) dst = out_pos[gl] + (pos - gl * ws.group_size);
     }
+    const float before = valid && accumulate ? __builtin_nontemporal_load(out + dst) : 0.f;
 #pragma unroll
     for (int q = 0; q < KQ; ++q) x[q] = X.load(Off(uint32_t(row)) * row_bytes + piece + 128u * q);
     wave_lds_sync();
@@ -262,7 +224,8 @@ __global__ __launch_bounds__(kWave* kWavesPerBlock) void sddmm_kernel(SddmmArgs 
       // every output is written once and not read back by the launch:
       // non-temporal stores keep them from displacing Y rows in the L2 (C3
       // SDDMM N=128 6.374 -> 6.348 ms)
-      __builtin_nontemporal_store(dot * a_val, out + dst);
+      __builtin_nontemporal_store(accumulate ? fmaf(dot, a_val, before) : dot * a_val,
+                                  out + dst);
     }
   } else {
     // One slot per group (the run order's entry local * 8 + slot: order[]
@@ -327,11 +290,11 @@ __global__ __launch_bounds__(kWave* kWavesPerBlock) void sddmm_kernel(SddmmArgs 
         if constexpr (kMode == 2) {
           if (group_collect) res_lds[slot * kStage + k] = v;
           else if (args.residue_add) unsafeAtomicAdd(out + out_pos[g] + k, v);
-          else out[out_pos[g] + k] = v;
+          else out[out_pos[g] + k] = accumulate ? out[out_pos[g] + k] + v : v;
         } else if constexpr (kMode == 1) {
           const int at = out_pos[beg + k];
           if (args.residue_add) unsafeAtomicAdd(out + at, v);
-          else out[at] = v;
+          else out[at] = accumulate ? out[at] + v : v;
         } else if (collect) {
           res_lds[beg + k - out0] = v;
         } else {
@@ -372,19 +335,33 @@ __global__ void to_csr_kernel(const float* __restrict__ in, const int* __restric
     out[pos[e]] = in[e];
 }
 
-template <int KQ>
-void launch_kq(const SddmmArgs& a, bool buf, int mode, unsigned grid, hipStream_t stream) {
+template <int KQ, bool kSliced>
+void launch_mode(const SddmmArgs& a, bool buf, int mode, unsigned grid, hipStream_t stream) {
   constexpr unsigned kBlock = kWave * kWavesPerBlock;
   if (mode == 1) {
-    if (buf) sddmm_kernel<KQ, true, 1><<<grid, kBlock, 0, stream>>>(a);
-    else sddmm_kernel<KQ, false, 1><<<grid, kBlock, 0, stream>>>(a);
+    if (buf) sddmm_kernel<KQ, true, 1, kSliced><<<grid, kBlock, 0, stream>>>(a);
+    else sddmm_kernel<KQ, false, 1, kSliced><<<grid, kBlock, 0, stream>>>(a);
   } else if (mode == 2) {
-    if (buf) sddmm_kernel<KQ, true, 2><<<grid, kBlock, 0, stream>>>(a);
-    else sddmm_kernel<KQ, false, 2><<<grid, kBlock, 0, stream>>>(a);
+    if (buf) sddmm_kernel<KQ, true, 2, kSliced><<<grid, kBlock, 0, stream>>>(a);
+    else sddmm_kernel<KQ, false, 2, kSliced><<<grid, kBlock, 0, stream>>>(a);
   } else {
-    if (buf) sddmm_kernel<KQ, true, 0><<<grid, kBlock, 0, stream>>>(a);
-    else sddmm_kernel<KQ, false, 0><<<grid, kBlock, 0, stream>>>(a);
+    if (buf) sddmm_kernel<KQ, true, 0, kSliced><<<grid, kBlock, 0, stream>>>(a);
+    else sddmm_kernel<KQ, false, 0, kSliced><<<grid, kBlock, 0, stream>>>(a);
   }
+}
+
+template <int KQ>
+void launch_kq(const SddmmArgs& a, bool sliced, bool buf, int mode, unsigned grid,
+               hipStream_t stream) {
+  // slices are 96 features wide at least (N > 128 in nearly equal parts), the
+  // last one perhaps less, and kSliceCsr at most
+  if constexpr (KQ <= kSliceCsr / 32) {
+    if (sliced) {
+      launch_mode<KQ, true>(a, buf, mode, grid, stream);
+      return;
+    }
+  }
+  launch_mode<KQ, false>(a, buf, mode, grid, stream);
 }
 
 // Workset q writes outs[q] at its own positions (mode 0), through the
@@ -404,14 +381,10 @@ int launch(int count, const int* order, const ps_workset* worksets, float* const
                "SDDMM task_chunk must be PS_TASK_CHUNK_AUTO, 0 or a power of two up to 4096");
   SddmmArgs a{};
   a.residue_add = residue_add;
-  a.N = N;
-  a.lhs = lhs;
-  a.rhs = rhs;
+  a.row_bytes = uint32_t(N) * 4u;
   const uint64_t lhs_bytes = uint64_t(rows) * uint64_t(N) * 4u;
   const uint64_t rhs_bytes = uint64_t(cols) * uint64_t(N) * 4u;
   const bool buf = lhs_bytes <= 0xFFFFFFFFull && rhs_bytes <= 0xFFFFFFFFull;
-  a.lhs_bytes = lhs_bytes;
-  a.rhs_bytes = rhs_bytes;
   a.residue_offset = residue_offset;
   uint64_t tasks = 0;
   int n = 0;
@@ -466,25 +439,40 @@ int launch(int count, const int* order, const ps_workset* worksets, float* const
   if (a.launch_tasks == 0) return PS_OK;
   const unsigned grid = unsigned((uint64_t(a.launch_tasks) + kWavesPerBlock - 1) / kWavesPerBlock);
   a.chunk_log2 = uint32_t(task_chunk_log2(task_chunk, grid, kAutoChunkMax));
-  switch (N / 32) {
-    case 1: launch_kq<1>(a, buf, mode, grid, stream); break;
-    case 2: launch_kq<2>(a, buf, mode, grid, stream); break;
-    case 3: launch_kq<3>(a, buf, mode, grid, stream); break;
-    case 4: launch_kq<4>(a, buf, mode, grid, stream); break;
-    case 5: launch_kq<5>(a, buf, mode, grid, stream); break;
-    case 6: launch_kq<6>(a, buf, mode, grid, stream); break;
-    case 7: launch_kq<7>(a, buf, mode, grid, stream); break;
-    case 8: launch_kq<8>(a, buf, mode, grid, stream); break;
-    case 9: launch_kq<9>(a, buf, mode, grid, stream); break;
-    case 10: launch_kq<10>(a, buf, mode, grid, stream); break;
-    case 11: launch_kq<11>(a, buf, mode, grid, stream); break;
-    case 12: launch_kq<12>(a, buf, mode, grid, stream); break;
-    case 13: launch_kq<13>(a, buf, mode, grid, stream); break;
-    case 14: launch_kq<14>(a, buf, mode, grid, stream); break;
-    case 15: launch_kq<15>(a, buf, mode, grid, stream); break;
-    default: launch_kq<16>(a, buf, mode, grid, stream); break;
+  // slices of nearly equal width, multiples of 32 features
+  const uint64_t gathered = uint64_t(a.launch_tasks) * 64 * uint64_t(N) * 4u;
+  const int most = gathered < kSliceMinGather ? 512
+                   : mode == 1 ? (rhs_bytes > kWideRhsBytes ? kSliceWide : kSliceCsr)
+                   : rhs_bytes > kWideRhsBytes ? kSliceNarrow
+                                               : kSliceWide;
+  const int slices = (N + most - 1) / most;
+  const int width = (N / 32 + slices - 1) / slices * 32;
+  for (int f0 = 0; f0 < N; f0 += width) {
+    a.lhs = lhs + f0;
+    a.rhs = rhs + f0;
+    a.lhs_bytes = lhs_bytes - uint64_t(f0) * 4u;
+    a.rhs_bytes = rhs_bytes - uint64_t(f0) * 4u;
+    a.accumulate = f0 > 0;
+    switch ((N - f0 < width ? N - f0 : width) / 32) {
+      case 1: launch_kq<1>(a, slices > 1, buf, mode, grid, stream); break;
+      case 2: launch_kq<2>(a, slices > 1, buf, mode, grid, stream); break;
+      case 3: launch_kq<3>(a, slices > 1, buf, mode, grid, stream); break;
+      case 4: launch_kq<4>(a, slices > 1, buf, mode, grid, stream); break;
+      case 5: launch_kq<5>(a, slices > 1, buf, mode, grid, stream); break;
+      case 6: launch_kq<6>(a, slices > 1, buf, mode, grid, stream); break;
+      case 7: launch_kq<7>(a, slices > 1, buf, mode, grid, stream); break;
+      case 8: launch_kq<8>(a, slices > 1, buf, mode, grid, stream); break;
+      case 9: launch_kq<9>(a, slices > 1, buf, mode, grid, stream); break;
+      case 10: launch_kq<10>(a, slices > 1, buf, mode, grid, stream); break;
+      case 11: launch_kq<11>(a, slices > 1, buf, mode, grid, stream); break;
+      case 12: launch_kq<12>(a, slices > 1, buf, mode, grid, stream); break;
+      case 13: launch_kq<13>(a, slices > 1, buf, mode, grid, stream); break;
+      case 14: launch_kq<14>(a, slices > 1, buf, mode, grid, stream); break;
+      case 15: launch_kq<15>(a, slices > 1, buf, mode, grid, stream); break;
+      default: launch_kq<16>(a, slices > 1, buf, mode, grid, stream); break;
+    }
+    PS_LAUNCHED();
   }
-  PS_LAUNCHED();
   return PS_OK;
 }
 
