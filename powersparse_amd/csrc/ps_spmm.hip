@@ -239,6 +239,10 @@ __global__ __launch_bounds__(kWave* waves_per_block(LPN)) void spmm_kernel(SpmmA
     int g = kq < ws.group_num ? (ws.order ? ws.order[kq] : kq) : -1;
     const bool has = g >= 0 && g < ws.group_num;  // order entries out of range are skipped
     if (!has) g = 0;
+    // the row and its flag with the offsets, not after the walk: a small
+    // launch is one chain of loads (65 k nonzeros, N = 32: 5.4 -> 5.1 us)
+    const int row = ws.group_des[g];
+    const bool add = args.residue_atomic[g] != 0;
     const int start = has ? args.residue_offset[g] : 0;
     const int len = has ? args.residue_offset[g + 1] - start : 0;
     int* const slot_lds = my_lds + slot * kSlotWords;
@@ -280,8 +284,7 @@ __global__ __launch_bounds__(kWave* waves_per_block(LPN)) void spmm_kernel(SpmmA
     }
     int atomic_row = -1;
     if (has && len > 0) {
-      const int row = ws.group_des[g];
-      if (args.residue_atomic[g])
+      if (add)
         atomic_row = row;
       else
         // written once per launch: a non-temporal store keeps the row from
