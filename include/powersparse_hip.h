@@ -114,6 +114,8 @@ int ps_fill_random_async(float* dst, size_t count, uint64_t seed, float lo, floa
 /* ------------------------------------------------------- streams, events */
 /* Replaces: cudaStreamCreate / cudaStreamDestroy (benchmark_utils.h:48-66). */
 int ps_stream_create(ps_stream_t* stream);
+/* A stream that does not order itself against the null stream. */
+int ps_stream_create_nonblocking(ps_stream_t* stream);
 int ps_stream_destroy(ps_stream_t stream);
 int ps_stream_synchronize(ps_stream_t stream);
 /* *idle = 1 when everything enqueued on the stream so far has run, else 0. */
@@ -451,6 +453,12 @@ int ps_iota_u32(uint32_t* out, int n, ps_stream_t stream);
 int ps_pre_degree_sums(const int* row_ptr, int rows, unsigned long long* sums_host,
                        ps_stream_t stream);
 
+/* *bad = 1 when a column id lies outside [0, cols) (col_ind given) or a value
+ * is not finite (values given; n of either), else 0. `flag`: 4 bytes of
+ * scratch. Synchronises the stream.
+ * Replaces: the host loop over the nonzeros (matrix_utils.cu:484-488). */
+int ps_pre_check_csr(const int* col_ind, const float* values, int n, int cols, uint32_t* flag,
+                     int* bad, ps_stream_t stream);
 /* col_nnz[c] += number of nonzeros in column c (col_nnz pre-zeroed).
  * Replaces: the OpenMP histogram (matrix_utils.cu:508-514). */
 int ps_pre_col_histogram(const int* col_ind, int nnz, int* col_nnz, ps_stream_t stream);

@@ -120,6 +120,7 @@ HIP_API = [
      [c_void_p, ctypes.c_size_t, ctypes.c_uint64, ctypes.c_float, ctypes.c_float, ctypes.c_int,
       c_void_p]),
     ("ps_stream_create", ctypes.c_int, [ctypes.POINTER(c_void_p)]),
+    ("ps_stream_create_nonblocking", ctypes.c_int, [ctypes.POINTER(c_void_p)]),
     ("ps_stream_destroy", ctypes.c_int, [c_void_p]),
     ("ps_stream_idle", ctypes.c_int, [c_void_p, c_int_p]),
     ("ps_stream_synchronize", ctypes.c_int, [c_void_p]),
@@ -227,6 +228,8 @@ HIP_API = [
     ("ps_iota_u32", ctypes.c_int, [c_void_p, ctypes.c_int, c_void_p]),
     ("ps_pre_degree_sums", ctypes.c_int, [c_void_p, ctypes.c_int, c_u64_p, c_void_p]),
     ("ps_pre_col_histogram", ctypes.c_int, [c_void_p, ctypes.c_int, c_void_p, c_void_p]),
+    ("ps_pre_check_csr", ctypes.c_int,
+     [c_void_p, c_void_p, ctypes.c_int, ctypes.c_int, c_void_p, c_int_p, c_void_p]),
     ("ps_pre_col_histogram_cols", ctypes.c_int,
      [c_void_p, ctypes.c_int, ctypes.c_int, c_void_p, c_void_p]),
     ("ps_pre_rank_keys", ctypes.c_int,

@@ -49,10 +49,11 @@ void ParallelCopy(void* dst, const void* src, size_t bytes) {
   }
 }
 
-// Waits for the null stream on scope exit, so that no DMA still reads a
-// staging buffer when the pool is released (also on an error path).
+// Waits for the stream on scope exit, so that no DMA still reads a staging
+// buffer when the pool is released (also on an error path).
 struct DrainOnExit {
-  ~DrainOnExit() { (void)ps_stream_synchronize(nullptr); }
+  ps_stream_t stream;
+  ~DrainOnExit() { (void)ps_stream_synchronize(stream); }
 };
 
 struct Events {
@@ -65,7 +66,7 @@ struct Events {
 
 }  // namespace
 
-void StagedUpload(void* dst, const void* src, size_t bytes) {
+void StagedUpload(void* dst, const void* src, size_t bytes, ps_stream_t stream) {
   if (bytes < kMinStaged) {
     ThrowOnError(ps_memcpy_htod(dst, src, bytes));
     return;
@@ -84,7 +85,7 @@ void StagedUpload(void* dst, const void* src, size_t bytes) {
   }
   Events ev;
   for (ps_event_t& x : ev.e) ThrowOnError(ps_event_create(&x));
-  DrainOnExit drain;
+  DrainOnExit drain{stream};
   const char* s = static_cast<const char*>(src);
   char* d = static_cast<char*>(dst);
   size_t k = 0;
@@ -93,10 +94,10 @@ void StagedUpload(void* dst, const void* src, size_t bytes) {
     const size_t len = std::min(kChunk, bytes - off);
     if (k >= 2) ThrowOnError(ps_event_synchronize(ev.e[b]));  // buffer b's DMA is done
     ParallelCopy(pool.buf[b], s + off, len);
-    ThrowOnError(ps_memcpy_htod_async(d + off, pool.buf[b], len, nullptr));
-    ThrowOnError(ps_event_record(ev.e[b], nullptr));
+    ThrowOnError(ps_memcpy_htod_async(d + off, pool.buf[b], len, stream));
+    ThrowOnError(ps_event_record(ev.e[b], stream));
   }
-  ThrowOnError(ps_stream_synchronize(nullptr));
+  ThrowOnError(ps_stream_synchronize(stream));
 }
 
 }  // namespace PowerSparse

@@ -104,3 +104,31 @@ def test_col_histogram(cols, nnz):
     d, out = ps.DeviceBuffer(host=c), ps.DeviceBuffer.zeros(cols * 4)
     ps._hip_call(_native.hip().ps_pre_col_histogram_cols(d.ptr, nnz, cols, out.ptr, None))
     np.testing.assert_array_equal(out.download(np.int32), np.bincount(c, minlength=cols))
+
+
+@pytest.mark.parametrize("at", [0, (1 << 24) - 1, 1 << 24, (1 << 24) + 4])
+@pytest.mark.parametrize("what", ["column", "negative", "nan", "inf"])
+def test_large_csr_is_checked_on_the_device(at, what):
+    # a matrix large enough for the device's checks, one bad entry: refused with
+    # the host check's message; the same matrix without it is built
+    setup()
+    rows, cols, n = 1 << 18, 1000, (1 << 24) + 5
+    rp = np.minimum(np.arange(rows + 1, dtype=np.int64) * 65, n).astype(np.int32)
+    rp[-1] = n
+    ci = (np.arange(n, dtype=np.int64) * 7 % cols).astype(np.int32)
+    va = np.ones(n, np.float32)
+    say(f"check {what} at {at}")
+    ok = (ci[at], va[at])
+    if what == "column":
+        ci[at] = cols
+    elif what == "negative":
+        ci[at] = -1
+    else:
+        va[at] = np.nan if what == "nan" else -np.inf
+    with pytest.raises(ValueError, match="Invalid CSR column index or sparse value"):
+        ps.PowerSparseMatrixGPU(rows, cols, n, rp, ci, va)
+    ci[at], va[at] = ok
+    if at == 0:
+        m = ps.PowerSparseMatrixGPU(rows, cols, n, rp, ci, va)
+        assert m.MatrixNNZ() == n
+        m.close()
