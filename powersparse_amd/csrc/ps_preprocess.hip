@@ -731,6 +731,30 @@ __global__ __launch_bounds__(NT, 8) void group_lists_tile_kernel(
 // that brings the host its size and the key bits that vary.
 constexpr uint32_t kBefore = 0, kEq = 1, kAfter = 2;
 
+// First position from d on where the lists m and q differ or one ends. Nested
+// hub lists agree over hundreds of elements, and one step is two dependent
+// loads, so eight steps' loads are in flight at once.
+__device__ __forceinline__ uint32_t list_lcp(const uint32_t* __restrict__ m, uint32_t nm,
+                                             const uint32_t* __restrict__ q, uint32_t nq,
+                                             uint32_t d) {
+  constexpr uint32_t kStep = 8;
+  const uint32_t n = nm < nq ? nm : nq;
+  for (; d + kStep <= n; d += kStep) {
+    uint32_t a[kStep], b[kStep];
+#pragma unroll
+    for (uint32_t u = 0; u < kStep; ++u) {
+      a[u] = m[d + u];
+      b[u] = q[d + u];
+    }
+    uint32_t differ = 0;
+#pragma unroll
+    for (uint32_t u = 0; u < kStep; ++u) differ |= uint32_t(a[u] != b[u]) << u;
+    if (differ) return d + uint32_t(__builtin_ctz(differ));
+  }
+  while (d < n && m[d] == q[d]) ++d;
+  return d;
+}
+
 // What the host reads each round.
 struct OrderState {
   uint32_t n;        // active groups
@@ -826,8 +850,7 @@ __global__ __launch_bounds__(kThreads) void order_diverge_kernel(
     const uint32_t nm = list_end[g] - list_begin[g];
     const uint32_t nq = list_end[r] - list_begin[r];
     uint32_t d = act_depth[i];
-    if (g != r)
-      while (d < nm && d < nq && m[d] == q[d]) ++d;
+    if (g != r) d = list_lcp(m, nm, q, nq, d);
     uint32_t side, div = 0, elem = 0;
     if (g == r || (d == nm && d == nq)) {
       side = kEq;
@@ -985,8 +1008,7 @@ __global__ __launch_bounds__(kFinishThreads) void order_finish_kernel(
       const uint32_t nm = list_end[g] - list_begin[g];
       const uint32_t nq = list_end[r] - list_begin[r];
       uint32_t d = dep[e];
-      if (g != r)
-        while (d < nm && d < nq && m[d] == rq[d]) ++d;
+      if (g != r) d = list_lcp(m, nm, rq, nq, d);
       uint32_t side, kk = 0, el = 0;
       if (g == r || (d == nm && d == nq)) {
         side = kEq;
