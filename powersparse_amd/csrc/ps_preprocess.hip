@@ -219,12 +219,12 @@ __global__ void rank_keys_kernel(const int* __restrict__ row_ptr, int rows,
 // Rows arrive in order, so ranking only sorts inside each row: by count key
 // (max_count - col_nnz, ascending = column count descending), ties in CSR
 // order. Rows of up to 256 nonzeros: one wave per row, each element's rank
-// counted against the others. 257 .. 8192: one workgroup per row, bitonic sort of
-// (count key, index) pairs in LDS. Longer rows: their elements are compacted
-// and radix-sorted (stable) with the row's list index in the high bits.
+// counted against the others. 257 .. 8192: one workgroup per row, an LDS radix
+// sort (BlockSort; rows up to 2048 in quarter-size tiles). Longer rows: one
+// workgroup per row, the same sort tile by tile.
 // Output as the stable sort of (row, count key): keys (when asked for) = row <<
 // count_bits | count key, vals = CSR position.
-constexpr int kRankTileSmall = 1024, kRankTileLarge = 8192;
+constexpr int kRankTileSmall = 256 * kSortItems, kRankTileLarge = 1024 * kSortItems;
 
 __device__ __forceinline__ uint32_t count_key(const int* __restrict__ col_ind,
                                               const int* __restrict__ col_nnz, int max_count,
@@ -279,40 +279,34 @@ __global__ void rank_small_kernel(const int* __restrict__ row_ptr, int rows,
   }
 }
 
-// One workgroup per listed row (degree <= tile).
-__global__ __launch_bounds__(kThreads) void rank_tile_kernel(
+// One workgroup per listed row of at most one LDS tile.
+template <int NT>
+__global__ __launch_bounds__(NT, 8) void rank_tile_kernel(
     const uint32_t* __restrict__ row_list, const int* __restrict__ row_ptr,
     const int* __restrict__ col_ind, const int* __restrict__ col_nnz, int max_count,
     int count_bits, uint64_t* __restrict__ keys, uint32_t* __restrict__ vals) {
-  extern __shared__ uint64_t pairs[];
+  using Sort = BlockSort<NT, true>;
+  __shared__ typename Sort::Lds lds;
   const int r = int(row_list[blockIdx.x]);
   const int b = row_ptr[r];
   const int d = row_ptr[r + 1] - b;
-  int pw = 2;
-  while (pw < d) pw <<= 1;
-  for (int e = threadIdx.x; e < pw; e += blockDim.x)
-    pairs[e] = e < d ? (uint64_t(count_key(col_ind, col_nnz, max_count, b + e)) << 32) | uint32_t(e)
-                     : ~0ull;
-  __syncthreads();
-  for (int k2 = 2; k2 <= pw; k2 <<= 1) {
-    for (int j = k2 >> 1; j > 0; j >>= 1) {
-      for (int e = threadIdx.x; e < pw / 2; e += blockDim.x) {
-        const int i = (e / j) * 2 * j + (e % j);
-        const int l = i + j;
-        const bool asc = (i & k2) == 0;
-        const uint64_t x = pairs[i], y = pairs[l];
-        if ((x > y) == asc) {
-          pairs[i] = y;
-          pairs[l] = x;
-        }
-      }
-      __syncthreads();
-    }
+  uint32_t key[kSortItems], val[kSortItems];
+#pragma unroll
+  for (int q = 0; q < kSortItems; ++q) {
+    const int e = Sort::at(q);
+    key[q] = uint32_t(col_ind[b + (e < d ? e : d - 1)]);
+    val[q] = uint32_t(e);
   }
-  for (int e = threadIdx.x; e < d; e += blockDim.x) {
-    const uint64_t v = pairs[e];
-    if (keys) keys[b + e] = (uint64_t(r) << count_bits) | (v >> 32);
-    vals[b + e] = uint32_t(b) + uint32_t(v & 0xFFFFFFFFu);
+#pragma unroll
+  for (int q = 0; q < kSortItems; ++q)
+    key[q] = Sort::at(q) < d ? uint32_t(max_count - col_nnz[key[q]]) : Sort::kPad;
+  Sort::sort(lds, key, val, d);
+#pragma unroll
+  for (int q = 0; q < kSortItems; ++q) {
+    const int e = Sort::at(q);
+    if (e >= d) continue;
+    if (keys) keys[b + e] = (uint64_t(r) << count_bits) | key[q];
+    vals[b + e] = uint32_t(b) + val[q];
   }
 }
 
@@ -350,42 +344,109 @@ __global__ void permute_long_degrees_kernel(const uint32_t* __restrict__ list, u
   }
 }
 
-// Long rows: compacted keys (list index << count_bits | count key), values =
-// CSR positions; one workgroup per long row.
-__global__ void rank_long_keys_kernel(const uint32_t* __restrict__ list,
-                                      const uint32_t* __restrict__ seg_start,
-                                      const int* __restrict__ row_ptr,
-                                      const int* __restrict__ col_ind,
-                                      const int* __restrict__ col_nnz, int max_count,
-                                      int count_bits, uint64_t* __restrict__ ck,
-                                      uint32_t* __restrict__ cv) {
-  const uint32_t i = blockIdx.x;
-  const int r = int(list[i]);
+// Long rows, one workgroup per row: a stable radix sort over the row's tiles,
+// from one scratch copy of the row to the other (seg_start[i] = where row
+// list[i]'s share of the scratch begins), a pass counting the row's digits
+// first. Each tile is put in digit order in LDS, so that its elements leave as
+// runs, one per digit. The row's 8 to 16 bytes per element stay in the caches.
+constexpr int kRankLongThreads = 1024;
+__global__ __launch_bounds__(kRankLongThreads, 8) void rank_long_kernel(
+    const uint32_t* __restrict__ list, const uint32_t* __restrict__ seg_start,
+    const int* __restrict__ row_ptr, const int* __restrict__ col_ind,
+    const int* __restrict__ col_nnz, int max_count, int count_bits, uint32_t* __restrict__ key_a,
+    uint32_t* __restrict__ key_b, uint32_t* __restrict__ val_a, uint32_t* __restrict__ val_b,
+    uint64_t* __restrict__ keys, uint32_t* __restrict__ vals) {
+  using Sort = BlockSort<kRankLongThreads, true>;
+  __shared__ typename Sort::Lds lds;
+  __shared__ uint32_t next[kSortBins];  // where a digit's next element goes
+  const int r = int(list[blockIdx.x]);
   const int b = row_ptr[r];
   const int d = row_ptr[r + 1] - b;
-  const size_t o = seg_start[i];
-  for (int e = threadIdx.x; e < d; e += blockDim.x) {
-    ck[o + e] = (uint64_t(i) << count_bits) | count_key(col_ind, col_nnz, max_count, b + e);
-    cv[o + e] = uint32_t(b + e);
+  const size_t o = seg_start[blockIdx.x];
+  const int t = int(threadIdx.x), lane = lane_id();
+  uint32_t* ks = key_a + o;
+  uint32_t* kd = key_b + o;
+  uint32_t* vs = val_a + o;
+  uint32_t* vd = val_b + o;
+  if (t == 0) lds.diff = 0;
+  __syncthreads();
+  uint32_t diff = 0;
+  const uint32_t first = uint32_t(max_count - col_nnz[col_ind[b]]);
+  for (int e = t; e < d; e += kRankLongThreads) {
+    const uint32_t k = uint32_t(max_count - col_nnz[col_ind[b + e]]);
+    ks[e] = k;
+    vs[e] = uint32_t(e);
+    diff |= k ^ first;
   }
-}
-
-// After the stable sort the elements of long row i occupy the same compacted
-// range as before: element j of it goes to row_ptr[row] + (j - seg_start[i]).
-__global__ void rank_long_write_kernel(size_t total, const uint64_t* __restrict__ ck,
-                                       const uint32_t* __restrict__ cv,
-                                       const uint32_t* __restrict__ list,
-                                       const uint32_t* __restrict__ seg_start,
-                                       const int* __restrict__ row_ptr, int count_bits,
-                                       uint64_t* __restrict__ keys, uint32_t* __restrict__ vals) {
-  const uint64_t mask = (uint64_t(1) << count_bits) - 1;
-  for (size_t j = size_t(blockIdx.x) * blockDim.x + threadIdx.x; j < total;
-       j += size_t(gridDim.x) * blockDim.x) {
-    const uint32_t i = uint32_t(ck[j] >> count_bits);
-    const int r = int(list[i]);
-    const size_t out = size_t(row_ptr[r]) + (j - seg_start[i]);
-    if (keys) keys[out] = (uint64_t(r) << count_bits) | (ck[j] & mask);
-    vals[out] = cv[j];
+  for (int s = 1; s < kWave; s <<= 1) diff |= uint32_t(__shfl_xor(int(diff), s, kWave));
+  if (lane == 0) atomicOr(&lds.diff, diff);
+  __syncthreads();
+  diff = lds.diff;
+  const int lo = diff ? __builtin_ctz(diff) : 0, hi = diff ? 32 - __builtin_clz(diff) : 0;
+  const int passes = (hi - lo + 7) / 8;
+  const int bits = passes ? (hi - lo + passes - 1) / passes : 0;
+  const uint32_t mask = (1u << bits) - 1u;
+  for (int shift = lo; shift < hi; shift += bits) {
+    for (int q = t; q < kSortBins; q += kRankLongThreads) next[q] = 0;
+    __syncthreads();  // also: the last pass's writes are visible to the workgroup
+    for (int e = t; e < d; e += kRankLongThreads) atomicAdd(&next[(ks[e] >> shift) & mask], 1u);
+    __syncthreads();
+    uint32_t own = 0, incl = 0;
+    if (t < kSortBins) {
+      own = incl = next[t];
+      for (int s = 1; s < kWave; s <<= 1) {
+        const uint32_t v = uint32_t(__shfl_up(int(incl), s, kWave));
+        if (lane >= s) incl += v;
+      }
+      if (lane == kWave - 1) lds.wave_sum[t / kWave] = incl;
+    }
+    __syncthreads();
+    if (t < kSortBins) {
+      for (int q = 0; q < t / kWave; ++q) incl += lds.wave_sum[q];
+      next[t] = incl - own;
+    }
+    __syncthreads();
+    for (int e0 = 0; e0 < d; e0 += Sort::kTile) {
+      const int valid = d - e0 < Sort::kTile ? d - e0 : Sort::kTile;
+      uint32_t key[kSortItems], val[kSortItems], pos[kSortItems];
+#pragma unroll
+      for (int q = 0; q < kSortItems; ++q) {
+        const int e = Sort::at(q) < valid ? Sort::at(q) : valid - 1;
+        key[q] = Sort::at(q) < valid ? ks[e0 + e] : Sort::kPad;
+        val[q] = vs[e0 + e];
+      }
+      Sort::positions(lds, key, shift, bits, pos);
+#pragma unroll
+      for (int q = 0; q < kSortItems; ++q) {
+        lds.key[pos[q]] = key[q];
+        lds.val[pos[q]] = val[q];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < kSortItems; ++q) {
+        const int p = Sort::at(q);  // (padding comes last)
+        if (p >= valid) continue;
+        const uint32_t k = lds.key[p], dig = (k >> shift) & mask;
+        const uint32_t to = next[dig] + uint32_t(p) - lds.start[dig];
+        kd[to] = k;
+        vd[to] = lds.val[p];
+      }
+      __syncthreads();
+      if (t < kSortBins)  // the digit's elements in this tile
+        next[t] += (t + 1 < kSortBins ? lds.start[t + 1] : uint32_t(Sort::kTile)) - lds.start[t];
+      __syncthreads();
+    }
+    uint32_t* const k2 = ks;
+    ks = kd;
+    kd = k2;
+    uint32_t* const v2 = vs;
+    vs = vd;
+    vd = v2;
+  }
+  __syncthreads();
+  for (int e = t; e < d; e += kRankLongThreads) {
+    if (keys) keys[b + e] = (uint64_t(r) << count_bits) | ks[e];
+    vals[b + e] = uint32_t(b) + vs[e];
   }
 }
 
@@ -1658,16 +1719,13 @@ int ps_pre_rank_sort(const int* row_ptr, int rows, const int* col_ind, int nnz,
   const uint32_t n3 = tail_slot[2] + tail_flag[2];
   int rc = PS_OK;
   if (n1 > 0) {
-    ps::rank_tile_kernel<<<n1, ps::kThreads, ps::kRankTileSmall * sizeof(uint64_t), st>>>(
-        list1, row_ptr, col_ind, col_nnz, max_count, count_bits, keys, vals);
+    ps::rank_tile_kernel<256><<<n1, 256, 0, st>>>(list1, row_ptr, col_ind, col_nnz, max_count,
+                                                  count_bits, keys, vals);
     PS_LAUNCHED();
   }
   if (n2 > 0) {
-    const size_t lds = size_t(ps::kRankTileLarge) * sizeof(uint64_t);
-    PS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&ps::rank_tile_kernel),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-    ps::rank_tile_kernel<<<n2, ps::kThreads, lds, st>>>(list2, row_ptr, col_ind, col_nnz,
-                                                        max_count, count_bits, keys, vals);
+    ps::rank_tile_kernel<1024><<<n2, 1024, 0, st>>>(list2, row_ptr, col_ind, col_nnz, max_count,
+                                                    count_bits, keys, vals);
     PS_LAUNCHED();
   }
   if (n3 > 0) {
@@ -1681,25 +1739,15 @@ int ps_pre_rank_sort(const int* row_ptr, int rows, const int* col_ind, int nnz,
     uint32_t total = 0;
     PS_HIP(hipMemcpyAsync(&total, long_start + n3, 4, hipMemcpyDeviceToHost, st));
     PS_HIP(hipStreamSynchronize(st));
-    const int list_bits = ps::bits_for(uint64_t(n3 - 1));
-    PS_CHECK_ARG(list_bits + count_bits <= 64, "ps_pre_rank_sort: key does not fit 64 bits");
-    S lw(2 * S::bytes(total, 8) + 2 * S::bytes(total, 4) + ps_radix_workspace_bytes(total));
+    S lw(4 * S::bytes(total, 4));
     PS_HIP(lw.error());
-    uint64_t* ck = lw.take<uint64_t>(total);
-    uint64_t* ck_alt = lw.take<uint64_t>(total);
-    uint32_t* cv = lw.take<uint32_t>(total);
-    uint32_t* cv_alt = lw.take<uint32_t>(total);
-    void* radix_ws = lw.take<char>(ps_radix_workspace_bytes(total));
-    ps::rank_long_keys_kernel<<<n3, ps::kThreads, 0, st>>>(list3, long_start, row_ptr, col_ind,
-                                                           col_nnz, max_count, count_bits, ck, cv);
-    PS_LAUNCHED();
-    int alt = 0;
-    rc = ps_radix_sort_pairs_u64(ck, ck_alt, cv, cv_alt, total, 0, list_bits + count_bits,
-                                 radix_ws, &alt, stream);
-    if (rc != PS_OK) return rc;
-    ps::rank_long_write_kernel<<<ps::grid_for(total), ps::kThreads, 0, st>>>(
-        total, alt ? ck_alt : ck, alt ? cv_alt : cv, list3, long_start, row_ptr, count_bits,
-        keys, vals);
+    uint32_t* key_a = lw.take<uint32_t>(total);
+    uint32_t* key_b = lw.take<uint32_t>(total);
+    uint32_t* val_a = lw.take<uint32_t>(total);
+    uint32_t* val_b = lw.take<uint32_t>(total);
+    ps::rank_long_kernel<<<n3, ps::kRankLongThreads, 0, st>>>(
+        list3, long_start, row_ptr, col_ind, col_nnz, max_count, count_bits, key_a, key_b, val_a,
+        val_b, keys, vals);
     PS_LAUNCHED();
     PS_HIP(hipStreamSynchronize(st));
   }
