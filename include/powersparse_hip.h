@@ -548,6 +548,18 @@ int ps_pre_exec_positions(int group_size, const uint32_t* perm, int groups,
 int ps_pre_locality_score(int count, const int* const* col_ind, const long long* lengths,
                           int window, int max_windows, double* score, ps_stream_t stream);
 
+/* The score that ps_pre_locality_score gives the row-ordered copy of the
+ * worksets (largest groups first, the residue last; every group's members by
+ * column), from the groups themselves: group_start[s][g] = first ranked position,
+ * residue_offset the scanned residue lengths, lengths[s] the workset's
+ * nonzeros. window: a power of two, at least the largest group that occurs.
+ * Synchronises the stream. No reference counterpart. */
+int ps_pre_row_locality_score(int group_type_num, const int* group_num,
+                              const int* const* group_start, const int* residue_offset,
+                              const long long* lengths, const uint32_t* ranked_vals,
+                              const int* col_ind, int window, int max_windows, double* score,
+                              ps_stream_t stream);
+
 /* Sparse form of the signatures, for long signatures where the bitmaps of
  * ps_pre_signatures would not fit: the ascending list of distinct signature
  * bits of every group. Groups are numbered globally, workset after workset

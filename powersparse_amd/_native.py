@@ -204,6 +204,10 @@ HIP_API = [
       ctypes.c_uint32, c_void_p]),
     ("ps_pre_exec_positions", ctypes.c_int,
      [ctypes.c_int, c_void_p, ctypes.c_int, c_void_p, c_void_p, c_void_p]),
+    ("ps_pre_row_locality_score", ctypes.c_int,
+     [ctypes.c_int, c_int_p, ctypes.POINTER(c_void_p), c_void_p,
+      ctypes.POINTER(ctypes.c_longlong), c_void_p, c_void_p, ctypes.c_int, ctypes.c_int,
+      ctypes.POINTER(ctypes.c_double), c_void_p]),
     ("ps_pre_locality_score", ctypes.c_int,
      [ctypes.c_int, ctypes.POINTER(c_void_p), ctypes.POINTER(ctypes.c_longlong), ctypes.c_int,
       ctypes.c_int, c_double_p, c_void_p]),

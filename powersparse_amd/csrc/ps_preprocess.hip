@@ -1467,12 +1467,29 @@ struct SeqTable {
   int count;
 };
 
+// 1 when the key is new in the table.
+__device__ __forceinline__ uint32_t table_insert(uint32_t* table, uint32_t slots_log2,
+                                                 uint32_t col) {
+  const uint32_t mask = (1u << slots_log2) - 1, key = col + 1u;
+  uint32_t h = (key * 2654435761u) >> (32 - slots_log2);
+  for (;;) {  // load factor <= 1/2: a free slot or the key is always found
+    const uint32_t prev = atomicCAS(&table[h], 0u, key);
+    if (prev == 0u) return 1u;
+    if (prev == key) return 0u;
+    h = (h + 1) & mask;
+  }
+}
+
+__device__ __forceinline__ void add_distinct(uint32_t added, unsigned long long* distinct) {
+  for (int d = 1; d < kWave; d <<= 1) added += __shfl_xor(added, d, kWave);
+  if (lane_id() == 0 && added) atomicAdd(&distinct[0], (unsigned long long)added);
+}
+
 __global__ void window_distinct_kernel(SeqTable seq, uint64_t stride, uint32_t window,
                                        uint32_t slots_log2, uint32_t* __restrict__ tables,
                                        unsigned long long* __restrict__ distinct) {
   const uint32_t w = blockIdx.y;
   uint32_t* table = tables + (size_t(w) << slots_log2);
-  const uint32_t mask = (1u << slots_log2) - 1;
   const uint64_t first = uint64_t(w) * stride;
   uint32_t added = 0;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < window;
@@ -1480,20 +1497,71 @@ __global__ void window_distinct_kernel(SeqTable seq, uint64_t stride, uint32_t w
     const uint64_t e = first + i;
     int a = 0;
     while (a + 1 < seq.count && e >= seq.begin[a + 1]) ++a;
-    const uint32_t key = uint32_t(seq.p[a][e - seq.begin[a]]) + 1u;
-    uint32_t h = (key * 2654435761u) >> (32 - slots_log2);
-    for (;;) {  // load factor <= 1/2: a free slot or the key is always found
-      const uint32_t prev = atomicCAS(&table[h], 0u, key);
-      if (prev == 0u) {
-        ++added;
-        break;
+    added += table_insert(table, slots_log2, uint32_t(seq.p[a][e - seq.begin[a]]));
+  }
+  add_distinct(added, distinct);
+}
+
+// The same score for the groups in row order, whose sorted copy does not exist.
+// A piece is a stretch of one workset's elements [begin, end) inside one
+// window. The windows start at multiples of their length, which every block
+// group divides, so they hold whole block groups (a set of columns whatever
+// their order); only residue groups are cut, and ranked to know which of their
+// columns lie inside. The copy itself cost C3 4 ms of kernels, 2.1 GB, and a wait
+// for the values' upload.
+constexpr int kWindowThreads = 1024;
+constexpr int kWindowPiece = 8192;
+struct WindowPiece {
+  uint32_t window;
+  int32_t workset;  // 0: the residue
+  uint32_t begin, end;
+};
+struct RowGroups {
+  const int* start[PS_MAX_WORKSETS];  // first ranked position of each group
+  int groups[PS_MAX_WORKSETS];
+};
+
+__global__ __launch_bounds__(kWindowThreads) void row_window_kernel(
+    const WindowPiece* __restrict__ pieces, RowGroups rg, const int* __restrict__ residue_offset,
+    const uint32_t* __restrict__ ranked_vals, const int* __restrict__ col_ind,
+    uint32_t slots_log2, uint32_t* __restrict__ tables, unsigned long long* __restrict__ distinct) {
+  const WindowPiece w = pieces[blockIdx.x];
+  uint32_t* const table = tables + (size_t(w.window) << slots_log2);
+  const int* const start = rg.start[w.workset];
+  uint32_t added = 0;
+  if (w.workset > 0) {
+    const int gs_log2 = w.workset + 4;
+    for (uint32_t e = w.begin + threadIdx.x; e < w.end; e += kWindowThreads) {
+      const uint32_t k = e >> gs_log2;
+      added += table_insert(table, slots_log2,
+                            uint32_t(col_ind[ranked_vals[start[k] + int(e - (k << gs_log2))]]));
+    }
+  } else {
+    // half a wave per group, from the group that holds element `begin` on
+    int lo = 0, hi = rg.groups[0];  // residue_offset[lo] <= begin < residue_offset[hi]
+    while (hi - lo > 1) {
+      const int mid = lo + (hi - lo) / 2;
+      if (uint32_t(residue_offset[mid]) <= w.begin) lo = mid;
+      else hi = mid;
+    }
+    const int t = int(threadIdx.x) & 31, half = lane_id() & 32;
+    for (int g0 = lo; g0 < rg.groups[0]; g0 += kWindowThreads / 32) {
+      if (uint32_t(residue_offset[g0]) >= w.end) break;  // uniform
+      const int g = g0 + int(threadIdx.x) / 32;
+      const bool has = g < rg.groups[0];
+      const uint32_t at = has ? uint32_t(residue_offset[g]) : 0u;
+      const int len = has ? residue_offset[g + 1] - int(at) : 0;
+      const int col = t < len ? col_ind[ranked_vals[start[g] + t]] : 0x7fffffff;
+      uint32_t rank = 0;
+      for (int u = 0; u < 32; ++u) {
+        const int other = __shfl(col, half + u, kWave);
+        rank += u < len && (other < col || (other == col && u < t));
       }
-      if (prev == key) break;
-      h = (h + 1) & mask;
+      if (t < len && at + rank >= w.begin && at + rank < w.end)
+        added += table_insert(table, slots_log2, uint32_t(col));
     }
   }
-  for (int d = 1; d < kWave; d <<= 1) added += __shfl_xor(added, d, kWave);
-  if (lane_id() == 0 && added) atomicAdd(&distinct[0], (unsigned long long)added);
+  add_distinct(added, distinct);
 }
 
 // Largest group sorted in LDS: one 1024-thread tile.
@@ -2091,6 +2159,73 @@ int ps_pre_group_lists(int group_type_num, const int* group_num, const int* cons
     PS_LAUNCHED();
     base += size_t(G);
   }
+  return PS_OK;
+}
+
+int ps_pre_row_locality_score(int group_type_num, const int* group_num,
+                              const int* const* group_start, const int* residue_offset,
+                              const long long* lengths, const uint32_t* ranked_vals,
+                              const int* col_ind, int window, int max_windows, double* score,
+                              ps_stream_t stream) {
+  PS_CHECK_ARG(group_type_num >= 1 && group_type_num <= PS_MAX_WORKSETS && group_num &&
+                   group_start && residue_offset && lengths && ranked_vals && col_ind && score &&
+                   window >= 64 && window <= (1 << 24) && max_windows >= 1 && max_windows <= 65535,
+               "ps_pre_row_locality_score: bad argument");
+  PS_CHECK_ARG((window & (window - 1)) == 0, "ps_pre_row_locality_score: window must be a power of two");
+  ps::RowGroups rg{};
+  uint64_t total = 0;
+  for (int s = 0; s < group_type_num; ++s) {
+    PS_CHECK_ARG(group_num[s] >= 0 && lengths[s] >= 0 &&
+                     (group_num[s] == 0 || (group_start[s] && (s == 0 || window >> (s + 4) != 0))),
+                 "ps_pre_row_locality_score: bad workset");
+    rg.start[s] = group_start[s];
+    rg.groups[s] = group_num[s];
+    total += uint64_t(lengths[s]);
+  }
+  *score = 0.0;
+  const uint64_t nwin = total / uint64_t(window);
+  if (nwin == 0) return PS_OK;  // as ps_pre_locality_score
+  const uint32_t windows = uint32_t(nwin < uint64_t(max_windows) ? nwin : uint64_t(max_windows));
+  const uint64_t stride = nwin / windows * uint64_t(window);
+  // the windows' pieces: worksets from the largest groups down, the residue last
+  std::vector<ps::WindowPiece> pieces;
+  for (uint32_t w = 0; w < windows; ++w) {
+    const uint64_t first = uint64_t(w) * stride, last = first + uint64_t(window);
+    uint64_t base = 0;
+    for (int s = group_type_num - 1; s >= 0; --s) {
+      const uint64_t len = uint64_t(lengths[s]);
+      uint64_t b = first > base ? first - base : 0;
+      const uint64_t e = last > base ? (last - base < len ? last - base : len) : 0;
+      while (b < e) {
+        const uint64_t cut = (b / ps::kWindowPiece + 1) * ps::kWindowPiece;
+        const uint64_t end = cut < e ? cut : e;
+        pieces.push_back({w, s, uint32_t(b), uint32_t(end)});
+        b = end;
+      }
+      base += len;
+    }
+  }
+  uint32_t slots_log2 = 1;
+  while ((1u << slots_log2) < 2u * uint32_t(window)) ++slots_log2;
+  const size_t table_words = size_t(windows) << slots_log2;
+  using S = ps::Scratch;
+  S ws(S::bytes(table_words, 4) + S::bytes(1, 8) + S::bytes(pieces.size(), sizeof(ps::WindowPiece)));
+  PS_HIP(ws.error());
+  uint32_t* tables = ws.take<uint32_t>(table_words);
+  unsigned long long* distinct = ws.take<unsigned long long>(1);
+  ps::WindowPiece* dev = ws.take<ps::WindowPiece>(pieces.size());
+  hipStream_t st = ps::to_hip(stream);
+  PS_HIP(hipMemsetAsync(tables, 0, table_words * 4, st));
+  PS_HIP(hipMemsetAsync(distinct, 0, 8, st));
+  PS_HIP(hipMemcpyAsync(dev, pieces.data(), pieces.size() * sizeof(ps::WindowPiece),
+                        hipMemcpyHostToDevice, st));
+  ps::row_window_kernel<<<unsigned(pieces.size()), ps::kWindowThreads, 0, st>>>(
+      dev, rg, residue_offset, ranked_vals, col_ind, slots_log2, tables, distinct);
+  PS_LAUNCHED();
+  unsigned long long host = 0;
+  PS_HIP(hipMemcpyAsync(&host, distinct, 8, hipMemcpyDeviceToHost, st));
+  PS_HIP(hipStreamSynchronize(st));
+  *score = double(host) / (double(windows) * double(window));
   return PS_OK;
 }
 

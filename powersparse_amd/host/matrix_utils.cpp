@@ -457,51 +457,6 @@ void PowerSparseMatrixGPU::Build(Prepared& in) {
                                  start_ptr.data(), res_len.data(), res_atomic0.data(), st));
   clock.Mark(&PreprocessTimings::groups_ms);
 
-  // The row-ordered execution copy (task order) does not depend on the
-  // signature order either: build it now, decide whether to keep it later.
-  DeviceArray<uint32_t> iota, exec_len;
-  DeviceArray<char> exec_ws;
-  if (_task_order != TaskOrder::kSignature) {
-    size_t gmax = 0;
-    for (int s = 0; s < S; ++s) gmax = std::max(gmax, size_t(_group_num[s]));
-    iota.Allocate(gmax);
-    ThrowOnError(ps_iota_u32(iota.data(), int(gmax), st));
-    _exec_col_ind = new int*[S]();
-    _exec_sp_data = new float*[S]();
-    _exec_group_des = new int*[S]();
-    _exec_out_base = new int*[S]();
-    if (_keep_csr_pos) _exec_csr_pos = new int*[S]();
-    // residue offsets in the initial (row) order
-    ThrowOnError(ps_malloc(reinterpret_cast<void**>(&_exec_residue_offset),
-                           sizeof(int) * (size_t(G0) + 1)));
-    ThrowOnError(ps_memset_async(_exec_residue_offset, 0, sizeof(int) * (size_t(G0) + 1), st));
-    if (G0 > 0) {
-      exec_len.Allocate(size_t(G0) + 1);
-      ThrowOnError(ps_memcpy_dtod_async(exec_len.data(), res_len.data(), sizeof(int) * size_t(G0),
-                                        st));
-      ThrowOnError(ps_memset_async(exec_len.data() + G0, 0, sizeof(uint32_t), st));
-      exec_ws.Allocate(ps_scan_workspace_bytes(size_t(G0) + 1));
-      ThrowOnError(ps_exclusive_scan_u32(exec_len.data(),
-                                         reinterpret_cast<uint32_t*>(_exec_residue_offset),
-                                         size_t(G0) + 1, exec_ws.data(), st));
-    }
-    for (int s = 0; s < S; ++s) {
-      const int G = _group_num[s];
-      if (G == 0) continue;
-      const size_t size = size_t(lengths[size_t(s)]);
-      ThrowOnError(ps_malloc(reinterpret_cast<void**>(&_exec_col_ind[s]), sizeof(int) * size));
-      ThrowOnError(ps_malloc(reinterpret_cast<void**>(&_exec_sp_data[s]), sizeof(float) * size));
-      if (_keep_csr_pos)
-        ThrowOnError(ps_malloc(reinterpret_cast<void**>(&_exec_csr_pos[s]), sizeof(int) * size));
-      ThrowOnError(ps_pre_gather_workset_cols(s == 0 ? 0 : GROUP_SIZE(s), _matrix_col, iota.data(), G,
-                                         start[size_t(s)].data(),
-                                         s == 0 ? _exec_residue_offset : nullptr, vals.data(),
-                                         d_ci.data(), in.Values(), _exec_col_ind[s],
-                                         _exec_sp_data[s],
-                                         _keep_csr_pos ? _exec_csr_pos[s] : nullptr, st));
-    }
-  }
-
   _signature_len = in.SignatureLen();
 
   // Groups in signature order: perm[s][k] = initial group at position k.
@@ -634,33 +589,56 @@ void PowerSparseMatrixGPU::Build(Prepared& in) {
                                        _keep_csr_pos ? _workset_csr_pos[s] : nullptr, st));
   }
 
-  // Task order: keep the row-ordered copy when asked for, or when it scores
-  // clearly better than the signature order.
+  // Task order: a row-ordered execution copy when asked for, or when the row
+  // order scores clearly better than the signature order.
   if (_task_order != TaskOrder::kSignature) {
-    if (G0 > 0) _exec_residue_atomic = reinterpret_cast<bool*>(res_atomic0.Release());
-    for (int s = 0; s < S; ++s)
-      if (_group_num[s] > 0) _exec_group_des[s] = des0[size_t(s)].Release();
-    bool keep = _task_order == TaskOrder::kRow;
+    // residue offsets in the initial (row) order
+    DeviceArray<int> row_offset(size_t(G0) + 1);
+    ThrowOnError(ps_memset_async(row_offset.data() + G0, 0, sizeof(int), st));
+    if (G0 > 0) {
+      ThrowOnError(ps_memcpy_dtod_async(row_offset.data(), res_len.data(), sizeof(int) * size_t(G0),
+                                        st));
+      DeviceArray<char> ws(ps_scan_workspace_bytes(size_t(G0) + 1));
+      uint32_t* const off = reinterpret_cast<uint32_t*>(row_offset.data());
+      ThrowOnError(ps_exclusive_scan_u32(off, off, size_t(G0) + 1, ws.data(), st));
+    }
+    bool row = _task_order == TaskOrder::kRow;
     if (_task_order == TaskOrder::kAuto) {
       // Launch order of the worksets: largest groups first, the residue last.
-      std::vector<const int*> pub(static_cast<size_t>(S)), row(static_cast<size_t>(S));
+      std::vector<const int*> pub(static_cast<size_t>(S));
       std::vector<long long> len(static_cast<size_t>(S));
       for (int q = 0; q < S; ++q) {
         pub[size_t(q)] = _workset_col_ind[S - 1 - q];
-        row[size_t(q)] = _exec_col_ind[S - 1 - q];
         len[size_t(q)] = lengths[size_t(S - 1 - q)];
       }
       ThrowOnError(ps_pre_locality_score(S, pub.data(), len.data(), kLocalityWindow,
                                          kLocalityWindows, &_locality[0], st));
-      ThrowOnError(ps_pre_locality_score(S, row.data(), len.data(), kLocalityWindow,
-                                         kLocalityWindows, &_locality[1], st));
-      keep = _locality[1] < kRowOrderGain * _locality[0];
+      int largest = S - 1;
+      while (largest > 0 && _group_num[largest] == 0) --largest;
+      if (largest > 0 && GROUP_SIZE(largest) > kLocalityWindow) {
+        // windows that cut block groups: score the copy itself
+        BuildExecution(in, start_ptr, lengths, row_offset.data());
+        std::vector<const int*> cols(static_cast<size_t>(S));
+        for (int q = 0; q < S; ++q) cols[size_t(q)] = _exec_col_ind[S - 1 - q];
+        ThrowOnError(ps_pre_locality_score(S, cols.data(), len.data(), kLocalityWindow,
+                                           kLocalityWindows, &_locality[1], st));
+      } else {
+        ThrowOnError(ps_pre_row_locality_score(S, _group_num, start_ptr.data(), row_offset.data(),
+                                               lengths.data(), vals.data(), d_ci.data(),
+                                               kLocalityWindow, kLocalityWindows, &_locality[1],
+                                               st));
+      }
+      row = _locality[1] < kRowOrderGain * _locality[0];
     }
-    if (keep) {
+    if (row) {
       _task_order = TaskOrder::kRow;
+      if (!_exec_col_ind) BuildExecution(in, start_ptr, lengths, row_offset.data());
+      _exec_residue_offset = row_offset.Release();
+      if (G0 > 0) _exec_residue_atomic = reinterpret_cast<bool*>(res_atomic0.Release());
       for (int s = 0; s < S; ++s) {
         const int G = _group_num[s];
         if (G == 0) continue;
+        _exec_group_des[s] = des0[size_t(s)].Release();
         ThrowOnError(ps_malloc(reinterpret_cast<void**>(&_exec_out_base[s]),
                                sizeof(int) * size_t(G)));
         ThrowOnError(ps_pre_exec_positions(s == 0 ? 0 : GROUP_SIZE(s), perm[size_t(s)].data(), G,
@@ -675,6 +653,35 @@ void PowerSparseMatrixGPU::Build(Prepared& in) {
   if (_task_order == TaskOrder::kSignature && _want_run_order) BuildRunOrders();
   ThrowOnError(ps_device_synchronize());
   clock.Mark(&PreprocessTimings::gather_ms);
+}
+
+// The worksets with their groups in row order, members by column.
+void PowerSparseMatrixGPU::BuildExecution(Prepared& in, const std::vector<int*>& group_start,
+                                          const std::vector<long long>& lengths,
+                                          const int* residue_offset) {
+  const int S = _group_type_num;
+  size_t most = 0;
+  for (int s = 0; s < S; ++s) most = std::max(most, size_t(_group_num[s]));
+  DeviceArray<uint32_t> iota(most);
+  ThrowOnError(ps_iota_u32(iota.data(), int(most), nullptr));
+  _exec_col_ind = new int*[S]();
+  _exec_sp_data = new float*[S]();
+  _exec_group_des = new int*[S]();
+  _exec_out_base = new int*[S]();
+  if (_keep_csr_pos) _exec_csr_pos = new int*[S]();
+  for (int s = 0; s < S; ++s) {
+    const int G = _group_num[s];
+    if (G == 0) continue;
+    const size_t size = size_t(lengths[size_t(s)]);
+    ThrowOnError(ps_malloc(reinterpret_cast<void**>(&_exec_col_ind[s]), sizeof(int) * size));
+    ThrowOnError(ps_malloc(reinterpret_cast<void**>(&_exec_sp_data[s]), sizeof(float) * size));
+    if (_keep_csr_pos)
+      ThrowOnError(ps_malloc(reinterpret_cast<void**>(&_exec_csr_pos[s]), sizeof(int) * size));
+    ThrowOnError(ps_pre_gather_workset_cols(
+        s == 0 ? 0 : GROUP_SIZE(s), _matrix_col, iota.data(), G, group_start[size_t(s)],
+        s == 0 ? residue_offset : nullptr, in.vals.data(), in.col_ind.data(), in.Values(),
+        _exec_col_ind[s], _exec_sp_data[s], _keep_csr_pos ? _exec_csr_pos[s] : nullptr, nullptr));
+  }
 }
 
 // ------------------------------------------------------------ hub block

@@ -268,6 +268,8 @@ class PowerSparseMatrixGPU {
   void Build(Prepared& in);
   void Release() noexcept;
   void ReleaseExecution() noexcept;
+  void BuildExecution(Prepared& in, const std::vector<int*>& group_start,
+                      const std::vector<long long>& lengths, const int* residue_offset);
   void BuildRunOrders();
   // Chooses and builds the dense hub block and the tuned SpMM partition of
   // the rest; false (nothing built) when no block qualifies.

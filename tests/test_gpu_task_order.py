@@ -133,3 +133,58 @@ def test_locality_score_exact():
     # sampling: every other window of 8 when 4 may be sampled
     eight = np.concatenate([w0, w1] * 4)
     assert locality([eight], W, max_windows=4) == pytest.approx(1 / W)
+
+
+@pytest.mark.parametrize("cfg,scale,cu,window", [("C1", 20, 4, 1024), ("C3", 100, 2, 4096),
+                                                 ("C4", 32, 1, 1024), ("C0", 1, 256, 64),
+                                                 ("C0", 1, 256, 1 << 17)])
+def test_row_locality_score_is_the_copys(cfg, scale, cu, window):
+    """The row order's score from the groups equals the score of its gathered
+    copy: windows across worksets, residue groups cut by them, fine mode, and a
+    matrix shorter than one window."""
+    from powersparse_amd import _native as nat
+    setup()
+    csr = ps.synth(cfg, seed=9, scale=scale)
+    w = oracle.preprocess(csr.rows, csr.cols, csr.row_ptr, csr.col_ind, csr.values, cu)
+    S = w.S
+    if window < 32 << max(S - 2, 0):
+        window = 32 << (S - 2)
+    # groups in row order from the CSR: block sizes greedily from the largest
+    starts, lens = [[] for _ in range(S)], []
+    cnt = np.bincount(csr.col_ind, minlength=csr.cols)
+    ranked = np.empty(csr.nnz, np.uint32)
+    for r in range(csr.rows):
+        b, e = csr.row_ptr[r], csr.row_ptr[r + 1]
+        ranked[b:e] = b + np.argsort(-cnt[csr.col_ind[b:e]], kind="stable")
+        p = b
+        if S == 1:
+            while p < e:
+                starts[0].append(p)
+                lens.append(min(16, e - p))
+                p += 16
+            continue
+        for s in range(S - 1, 0, -1):
+            while e - p >= 32 << (s - 1):
+                starts[s].append(p)
+                p += 32 << (s - 1)
+        if p < e:
+            starts[0].append(p)
+            lens.append(e - p)
+    assert [len(x) for x in starts] == list(w.group_num)
+    sizes = [lens] + [[32 << (s - 1)] * len(starts[s]) for s in range(1, S)]
+    seq = []
+    for s in range(S - 1, -1, -1):
+        for b, n in zip(starts[s], sizes[s]):
+            seq.append(np.sort(csr.col_ind[ranked[b:b + n]]))
+    want = locality([np.concatenate(seq)], window, 16)
+    offset = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    dev = [ps.DeviceBuffer(host=np.asarray(x or [0], np.int32)) for x in starts]
+    d = [ps.DeviceBuffer(host=a) for a in (offset, ranked, csr.col_ind)]
+    num = (ctypes.c_int * S)(*[len(x) for x in starts])
+    ptrs = (ctypes.c_void_p * S)(*[x.ptr for x in dev])
+    length = (ctypes.c_longlong * S)(*[int(np.sum(x)) for x in sizes])
+    score = ctypes.c_double()
+    ps._hip_call(nat.hip().ps_pre_row_locality_score(
+        S, num, ptrs, d[0].ptr, length, d[1].ptr, d[2].ptr, window, 16, ctypes.byref(score), None))
+    say(f"{cfg} window={window}: {score.value} (copy {want})")
+    assert score.value == want
