@@ -309,7 +309,7 @@ struct PowerSparseMatrixGPU::Prepared {
       signature_len = sig_len.get();
       clock.Mark(&PreprocessTimings::sigbit_ms);
       sigbit_device.Allocate(sigbit.size());
-      sigbit_device.Upload(sigbit.data(), sigbit.size());
+      StagedUpload(sigbit_device.data(), sigbit.data(), sizeof(int) * sigbit.size());
     }
     return signature_len;
   }

@@ -10,8 +10,8 @@ namespace PowerSparse {
 // Copies `bytes` from host memory `src` (any, e.g. pageable) to device memory
 // `dst` and returns when the copy is complete. Large copies go through two
 // page-locked buffers: while the DMA engine copies chunk k out of one buffer,
-// host threads fill the other with chunk k + 1. Small copies use one plain
-// synchronous copy. Uses the given stream of the current
+// host threads fill the other with chunk k + 1. Copies below 64 KB use one
+// plain synchronous copy. Uses the given stream of the current
 // device (the plain copy: the null stream).
 void StagedUpload(void* dst, const void* src, size_t bytes, ps_stream_t stream = nullptr);
 
