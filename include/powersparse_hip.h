@@ -324,6 +324,15 @@ typedef struct ps_hub_block {
  * in [2^b, 2^(b+1)); the statistics a block is chosen from. */
 int ps_hub_histogram(const int* row_ptr, int rows, const int* col_ind, const int* col_nnz,
                      unsigned long long* hist, ps_stream_t stream);
+/* levels (64 device values): [a] = rows of degree 2^a .. 2^(a+1) - 1, [32 + b] =
+ * columns of count 2^b .. 2^(b+1) - 1. */
+int ps_hub_levels(const int* row_ptr, int rows, const int* col_nnz, int cols,
+                  unsigned long long* levels, ps_stream_t stream);
+/* The ids i < n whose row degree (row_ptr given) or counts[i] lies in [lo, hi),
+ * ascending in list (room for n), index[i] = place there or -1, *selected on
+ * the host. Synchronises the stream. */
+int ps_hub_select(const int* row_ptr, const int* counts, int n, long long lo, long long hi,
+                  int* index, int* list, int* selected, ps_stream_t stream);
 /* Words of the stored bit mask. */
 size_t ps_hub_stored_words(const ps_hub_block* hb);
 /* Columns per dense row: cols rounded up to a multiple of 64 (0 for cols <= 0). */
@@ -365,6 +374,15 @@ int ps_hub_mark_atomic(const ps_hub_block* hb, const int* group_des, int group_n
  * columns are hot; else 0. */
 int ps_hub_tile_flags(const ps_hub_block* hb, const ps_workset* workset, uint8_t* flags,
                       ps_stream_t stream);
+/* 64-nonzero tiles of the block worksets of groups >= 64 nonzeros. */
+size_t ps_hub_tile_total(int workset_count, const ps_workset* worksets);
+/* ps_hub_tile_flags of all of them (flags: ps_hub_tile_total bytes, workset
+ * after workset) and the flagged tiles' list for ps_hub_sddmm_plan (codes: room
+ * for all; *listed on the host). Synchronises the stream. */
+int ps_hub_tiles(const ps_hub_block* hb, int workset_count, const ps_workset* worksets,
+                 uint8_t* flags, uint32_t* codes, uint32_t* listed, ps_stream_t stream);
+/* into[i] |= flags[i], n bytes. */
+int ps_hub_merge_flags(const uint8_t* flags, size_t n, uint8_t* into, ps_stream_t stream);
 /* Device workspace bytes at width N of ps_hub_spmm_launch (op PS_OP_SPMM: one
  * feature slice, up to 128, of B's hot rows in fragment order, and flags) or
  * of ps_hub_sddmm_launch (PS_OP_SDDMM: lhs[hub_rows] and rhs[hot_cols] in

@@ -159,6 +159,16 @@ HIP_API = [
       ctypes.POINTER(c_void_p), c_void_p, ctypes.c_uint32, c_u32_p, c_void_p]),
     ("ps_hub_histogram", ctypes.c_int,
      [c_void_p, ctypes.c_int, c_void_p, c_void_p, c_void_p, c_void_p]),
+    ("ps_hub_levels", ctypes.c_int,
+     [c_void_p, ctypes.c_int, c_void_p, ctypes.c_int, c_void_p, c_void_p]),
+    ("ps_hub_select", ctypes.c_int,
+     [c_void_p, c_void_p, ctypes.c_int, ctypes.c_longlong, ctypes.c_longlong, c_void_p, c_void_p,
+      c_int_p, c_void_p]),
+    ("ps_hub_tile_total", ctypes.c_size_t, [ctypes.c_int, ctypes.POINTER(Workset)]),
+    ("ps_hub_tiles", ctypes.c_int,
+     [ctypes.POINTER(HubBlock), ctypes.c_int, ctypes.POINTER(Workset), c_void_p, c_void_p, c_u32_p,
+      c_void_p]),
+    ("ps_hub_merge_flags", ctypes.c_int, [c_void_p, ctypes.c_size_t, c_void_p, c_void_p]),
     ("ps_hub_stored_words", ctypes.c_size_t, [ctypes.POINTER(HubBlock)]),
     ("ps_hub_dense_build", ctypes.c_int,
      [ctypes.POINTER(HubBlock), c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),

@@ -139,6 +139,63 @@ __global__ __launch_bounds__(kThreads) void hist_kernel(const int* __restrict__ 
     if (h[i]) atomicAdd(&hist[i], (unsigned long long)h[i]);
 }
 
+// The block's selection (levels, hub rows, hot columns) is a few streaming
+// passes over 4 bytes per row or column. As loops of the host with two uploads
+// per tier it held the device idle for 11 ms of a 98 ms build of 1 M rows and
+// 100 M nonzeros, the tile list below (flags downloaded, codes uploaded) for 7.
+//
+// levels[a] = rows of degree with floor(log2) = a, levels[32 + b] = columns of
+// count with floor(log2) = b (rows and columns without nonzeros left out).
+__global__ __launch_bounds__(kThreads) void levels_kernel(const int* __restrict__ row_ptr, int rows,
+                                                           const int* __restrict__ col_nnz, int cols,
+                                                           unsigned long long* __restrict__ levels) {
+  __shared__ unsigned int h[64];
+  if (threadIdx.x < 64) h[threadIdx.x] = 0;
+  __syncthreads();
+  const size_t stride = size_t(gridDim.x) * kThreads;
+  const size_t t = size_t(blockIdx.x) * kThreads + threadIdx.x;
+  for (size_t r = t; r < size_t(rows); r += stride) {
+    const int d = row_ptr[r + 1] - row_ptr[r];
+    if (d > 0) atomicAdd(&h[31 - __builtin_clz(unsigned(d))], 1u);
+  }
+  for (size_t c = t; c < size_t(cols); c += stride) {
+    const int n = col_nnz[c];
+    if (n > 0) atomicAdd(&h[32 + 31 - __builtin_clz(unsigned(n))], 1u);
+  }
+  __syncthreads();
+  if (threadIdx.x < 64 && h[threadIdx.x]) atomicAdd(&levels[threadIdx.x], (unsigned long long)h[threadIdx.x]);
+}
+
+// flag[i] = 1 when row i's degree (row_ptr given) or counts[i] lies in [lo, hi);
+// flag[n] = 0 (the scan's total lands there).
+__global__ __launch_bounds__(kThreads) void select_flags_kernel(const int* __restrict__ row_ptr,
+                                                                 const int* __restrict__ counts,
+                                                                 int n, long long lo, long long hi,
+                                                                 uint32_t* __restrict__ flag) {
+  for (size_t i = size_t(blockIdx.x) * kThreads + threadIdx.x; i <= size_t(n);
+       i += size_t(gridDim.x) * kThreads) {
+    bool in = false;
+    if (i < size_t(n)) {
+      const long long v = row_ptr ? row_ptr[i + 1] - row_ptr[i] : counts[i];
+      in = v >= lo && v < hi;
+    }
+    flag[i] = in ? 1u : 0u;
+  }
+}
+
+// After the scan in place: the selected ids (slot[i + 1] > slot[i]) listed,
+// index[i] = place in the list or -1.
+__global__ __launch_bounds__(kThreads) void select_write_kernel(const uint32_t* __restrict__ slot,
+                                                                 int n, int* __restrict__ index,
+                                                                 int* __restrict__ list) {
+  for (size_t i = size_t(blockIdx.x) * kThreads + threadIdx.x; i < size_t(n);
+       i += size_t(gridDim.x) * kThreads) {
+    const bool in = slot[i + 1] != slot[i];
+    index[i] = in ? int(slot[i]) : -1;
+    if (in) list[slot[i]] = int(i);
+  }
+}
+
 // ------------------------------------------------------------- building
 
 // The dense build, one workgroup per hub row: the row's hot columns are marked
@@ -598,6 +655,38 @@ __global__ __launch_bounds__(kThreads) void fixup_kernel(ps_hub_block hb, const 
 // A listed tile: (workset << kTileBits) | tile index within the workset.
 constexpr int kTileBits = 27;
 constexpr uint32_t kTileMask = (1u << kTileBits) - 1u;
+
+// Flagged tiles of all block worksets, listed in order: flag words for the
+// scan, then code = workset << kTileBits | tile. first[s] = number of tiles
+// before workset s (first[count]: of all). 1.5 M tiles at 100 M nonzeros: the
+// flags stay on the device, the host reads the number of tiles alone.
+struct TileTable {
+  uint32_t first[PS_MAX_WORKSETS + 1];
+  int count;
+};
+__global__ __launch_bounds__(kThreads) void flag_words_kernel(const uint8_t* __restrict__ flags,
+                                                               uint32_t n,
+                                                               uint32_t* __restrict__ words) {
+  for (uint32_t i = blockIdx.x * kThreads + threadIdx.x; i <= n; i += gridDim.x * kThreads)
+    words[i] = i < n ? flags[i] : 0u;
+}
+__global__ __launch_bounds__(kThreads) void tile_codes_kernel(TileTable tt,
+                                                               const uint32_t* __restrict__ slot,
+                                                               uint32_t* __restrict__ codes) {
+  const uint32_t n = tt.first[tt.count];
+  for (uint32_t i = blockIdx.x * kThreads + threadIdx.x; i < n; i += gridDim.x * kThreads) {
+    if (slot[i + 1] == slot[i]) continue;
+    int s = 0;
+    while (i >= tt.first[s + 1]) ++s;
+    codes[slot[i]] = (uint32_t(s) << kTileBits) | (i - tt.first[s]);
+  }
+}
+__global__ __launch_bounds__(kThreads) void merge_flags_kernel(const uint8_t* __restrict__ flags,
+                                                                size_t n, uint8_t* __restrict__ into) {
+  for (size_t i = size_t(blockIdx.x) * kThreads + threadIdx.x; i < n;
+       i += size_t(gridDim.x) * kThreads)
+    into[i] |= flags[i];
+}
 
 struct Worksets {
   ps_workset ws[PS_MAX_WORKSETS];
@@ -1067,6 +1156,46 @@ int ps_hub_histogram(const int* row_ptr, int rows, const int* col_ind, const int
   return PS_OK;
 }
 
+int ps_hub_levels(const int* row_ptr, int rows, const int* col_nnz, int cols,
+                  unsigned long long* levels, ps_stream_t stream) {
+  PS_CHECK_ARG(row_ptr && col_nnz && levels && rows > 0 && cols > 0, "ps_hub_levels: bad arguments");
+  hipStream_t st = ps::to_hip(stream);
+  PS_HIP(hipMemsetAsync(levels, 0, 64 * sizeof(unsigned long long), st));
+  const unsigned grid = ps::grid_for(size_t(rows > cols ? rows : cols), ps::kThreads);
+  ps::levels_kernel<<<grid < 1024 ? grid : 1024, ps::kThreads, 0, st>>>(row_ptr, rows, col_nnz, cols,
+                                                                        levels);
+  PS_LAUNCHED();
+  return PS_OK;
+}
+
+int ps_hub_select(const int* row_ptr, const int* counts, int n, long long lo, long long hi,
+                  int* index, int* list, int* selected, ps_stream_t stream) {
+  PS_CHECK_ARG((row_ptr || counts) && n > 0 && index && list && selected,
+               "ps_hub_select: bad arguments");
+  hipStream_t st = ps::to_hip(stream);
+  const size_t words = ps::round256((size_t(n) + 1) * 4);
+  char* base = nullptr;
+  PS_HIP(ps::dev_malloc(&base, words + ps_scan_workspace_bytes(size_t(n) + 1)));
+  uint32_t* slot = reinterpret_cast<uint32_t*>(base);
+  const unsigned grid = ps::grid_for(size_t(n) + 1, ps::kThreads);
+  ps::select_flags_kernel<<<grid, ps::kThreads, 0, st>>>(row_ptr, counts, n, lo, hi, slot);
+  hipError_t e = hipGetLastError();
+  int rc = PS_OK;
+  if (e == hipSuccess)
+    rc = ps_exclusive_scan_u32(slot, slot, size_t(n) + 1, base + words, stream);
+  if (e == hipSuccess && rc == PS_OK) {
+    ps::select_write_kernel<<<grid, ps::kThreads, 0, st>>>(slot, n, index, list);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess && rc == PS_OK)
+    e = hipMemcpyAsync(selected, slot + n, sizeof(int), hipMemcpyDeviceToHost, st);
+  if (e == hipSuccess) e = hipStreamSynchronize(st);
+  ps::dev_free(base);
+  if (rc != PS_OK) return rc;
+  PS_HIP(e);
+  return PS_OK;
+}
+
 size_t ps_hub_stored_words(const ps_hub_block* hb) {
   return hb ? size_t(hb->rows) * ((size_t(hb->cols) + 31) / 32) : 0;
 }
@@ -1200,6 +1329,68 @@ int ps_hub_tile_flags(const ps_hub_block* hb, const ps_workset* workset, uint8_t
   const size_t tiles = size_t(workset->group_num) * size_t(workset->group_size / 64);
   ps::tile_flags_kernel<<<ps::grid_for(tiles, ps::kThreads / ps::kWave), ps::kThreads, 0, st>>>(
       *hb, *workset, flags);
+  PS_LAUNCHED();
+  return PS_OK;
+}
+
+size_t ps_hub_tile_total(int workset_count, const ps_workset* worksets) {
+  size_t n = 0;
+  for (int s = 1; worksets && s < workset_count; ++s)
+    if (worksets[s].group_num > 0 && worksets[s].group_size >= 64)
+      n += size_t(worksets[s].group_num) * size_t(worksets[s].group_size / 64);
+  return n;
+}
+
+int ps_hub_tiles(const ps_hub_block* hb, int workset_count, const ps_workset* worksets,
+                 uint8_t* flags, uint32_t* codes, uint32_t* listed, ps_stream_t stream) {
+  int rc = ps::check_block(hb);
+  if (rc != PS_OK) return rc;
+  PS_CHECK_ARG(workset_count >= 1 && workset_count <= PS_MAX_WORKSETS && worksets && listed,
+               "ps_hub_tiles: bad arguments");
+  const size_t n = ps_hub_tile_total(workset_count, worksets);
+  *listed = 0;
+  if (n == 0) return PS_OK;
+  PS_CHECK_ARG(flags && codes && n < (size_t(1) << 31), "ps_hub_tiles: bad arguments");
+  ps::TileTable tt{};
+  tt.count = workset_count;
+  for (int s = 0; s < workset_count; ++s) {
+    const size_t own = s > 0 && worksets[s].group_num > 0 && worksets[s].group_size >= 64
+                           ? size_t(worksets[s].group_num) * size_t(worksets[s].group_size / 64)
+                           : 0;
+    PS_CHECK_ARG(own <= size_t(ps::kTileMask), "ps_hub_tiles: too many tiles in a workset");
+    if (own) {
+      rc = ps_hub_tile_flags(hb, &worksets[s], flags + tt.first[s], stream);
+      if (rc != PS_OK) return rc;
+    }
+    tt.first[s + 1] = tt.first[s] + uint32_t(own);
+  }
+  hipStream_t st = ps::to_hip(stream);
+  const size_t words = ps::round256((n + 1) * 4);
+  char* base = nullptr;
+  PS_HIP(ps::dev_malloc(&base, words + ps_scan_workspace_bytes(n + 1)));
+  uint32_t* slot = reinterpret_cast<uint32_t*>(base);
+  const unsigned grid = ps::grid_for(n + 1, ps::kThreads);
+  ps::flag_words_kernel<<<grid, ps::kThreads, 0, st>>>(flags, uint32_t(n), slot);
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess) rc = ps_exclusive_scan_u32(slot, slot, n + 1, base + words, stream);
+  if (e == hipSuccess && rc == PS_OK) {
+    ps::tile_codes_kernel<<<grid, ps::kThreads, 0, st>>>(tt, slot, codes);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess && rc == PS_OK)
+    e = hipMemcpyAsync(listed, slot + n, sizeof(uint32_t), hipMemcpyDeviceToHost, st);
+  if (e == hipSuccess) e = hipStreamSynchronize(st);
+  ps::dev_free(base);
+  if (rc != PS_OK) return rc;
+  PS_HIP(e);
+  return PS_OK;
+}
+
+int ps_hub_merge_flags(const uint8_t* flags, size_t n, uint8_t* into, ps_stream_t stream) {
+  PS_CHECK_ARG(flags && into, "ps_hub_merge_flags: null argument");
+  if (n == 0) return PS_OK;
+  ps::merge_flags_kernel<<<ps::grid_for(n, ps::kThreads), ps::kThreads, 0, ps::to_hip(stream)>>>(
+      flags, n, into);
   PS_LAUNCHED();
   return PS_OK;
 }

@@ -387,7 +387,7 @@ PowerSparseMatrixGPU::PowerSparseMatrixGPU(int row_num, int col_num, int nnz_num
     bool hub = false;
     if (may_tune && _task_order == TaskOrder::kSignature && _want_run_order &&
         policy.hub_block == HubBlock::kAuto)
-      hub = BuildHub(row_ptr, in, policy);
+      hub = BuildHub(in, policy);
     if (!hub && may_tune && _task_order == TaskOrder::kSignature &&
         _group_type_num > kTunedSpmmGroupTypes) {
       PartitionPolicy tuned;
@@ -729,36 +729,14 @@ int PowerSparseMatrixGPU::HubCols(int tier) const {
 }
 
 namespace {
-int FloorLog2(long long v) {
-  int b = -1;
-  while (v > 0) {
-    v >>= 1;
-    ++b;
-  }
-  return b;
-}
 struct TierSpec {
   long long min_degree, max_degree, min_count;  // rows in [min_degree, max_degree)
 };
 }  // namespace
 
-bool PowerSparseMatrixGPU::BuildHub(const int* row_ptr, Prepared& in,
-                                    const PartitionPolicy& policy) {
+bool PowerSparseMatrixGPU::BuildHub(Prepared& in, const PartitionPolicy& policy) {
   const int rows = _matrix_row, cols = _matrix_col, S = _group_type_num;
   if (S < 2) return false;  // fine mode: its store rule differs from a capped partition's
-  const std::vector<int>& cnt = in.col_nnz_host;
-  // rows of degree >= 2^a, columns of count >= 2^b (index 32: none)
-  std::vector<long long> rows_ge(34, 0), cols_ge(34, 0);
-  for (int r = 0; r < rows; ++r) {
-    const int d = row_ptr[r + 1] - row_ptr[r];
-    if (d > 0) ++rows_ge[size_t(FloorLog2(d))];
-  }
-  for (int c = 0; c < cols; ++c)
-    if (cnt[size_t(c)] > 0) ++cols_ge[size_t(FloorLog2(cnt[size_t(c)]))];
-  for (int k = 31; k >= 0; --k) {
-    rows_ge[size_t(k)] += rows_ge[size_t(k) + 1];
-    cols_ge[size_t(k)] += cols_ge[size_t(k) + 1];
-  }
   std::vector<TierSpec> specs;
   const bool forced = policy.hub_min_degree[0] > 0 && policy.hub_min_count[0] > 0;
   if (forced) {
@@ -772,6 +750,19 @@ bool PowerSparseMatrixGPU::BuildHub(const int* row_ptr, Prepared& in,
     }
   } else {
     if (double(_matrix_nnz) < kHubMinGainNonzeros) return false;
+    // rows of degree >= 2^a, columns of count >= 2^b (index 32: none)
+    std::vector<long long> rows_ge(34, 0), cols_ge(34, 0);
+    {
+      DeviceArray<unsigned long long> dev(64);
+      ThrowOnError(ps_hub_levels(in.row_ptr.data(), rows, in.col_nnz.data(), cols, dev.data(),
+                                 nullptr));
+      unsigned long long levels[64];
+      dev.Download(levels, 64);
+      for (int k = 31; k >= 0; --k) {
+        rows_ge[size_t(k)] = rows_ge[size_t(k) + 1] + (long long)levels[k];
+        cols_ge[size_t(k)] = cols_ge[size_t(k) + 1] + (long long)levels[32 + k];
+      }
+    }
     // nonzeros of rows of degree >= 2^a (a >= 8) in columns of count >= 2^b
     DeviceArray<unsigned long long> hist(32 * 32);
     ThrowOnError(ps_hub_histogram(in.row_ptr.data(), rows, in.col_ind.data(), in.col_nnz.data(),
@@ -814,20 +805,17 @@ bool PowerSparseMatrixGPU::BuildHub(const int* row_ptr, Prepared& in,
   auto hub = std::make_unique<HubState>();
   for (const TierSpec& spec : specs) {
     auto t = std::make_unique<HubTier>();
-    std::vector<int> hub_rows, hub_index(size_t(rows), -1), hot_cols, hot_rank(size_t(cols), -1);
-    for (int r = 0; r < rows; ++r) {
-      const long long d = row_ptr[r + 1] - row_ptr[r];
-      if (d >= spec.min_degree && d < spec.max_degree) {
-        hub_index[size_t(r)] = int(hub_rows.size());
-        hub_rows.push_back(r);
-      }
-    }
-    for (int c = 0; c < cols; ++c)
-      if (cnt[size_t(c)] >= spec.min_count) {
-        hot_rank[size_t(c)] = int(hot_cols.size());
-        hot_cols.push_back(c);
-      }
-    const long long R = (long long)hub_rows.size(), H = (long long)hot_cols.size();
+    t->hub_rows.Allocate(size_t(rows));
+    t->hub_index.Allocate(size_t(rows));
+    t->hot_cols.Allocate(size_t(cols));
+    t->hot_rank.Allocate(size_t(cols));
+    int R32 = 0, H32 = 0;
+    ThrowOnError(ps_hub_select(in.row_ptr.data(), nullptr, rows, spec.min_degree, spec.max_degree,
+                               t->hub_index.data(), t->hub_rows.data(), &R32, nullptr));
+    ThrowOnError(ps_hub_select(nullptr, in.col_nnz.data(), cols, spec.min_count,
+                               std::numeric_limits<long long>::max(), t->hot_rank.data(),
+                               t->hot_cols.data(), &H32, nullptr));
+    const long long R = R32, H = H32;
     if (R == 0 || H == 0) continue;
     if (R * H > kHubMaxElements) {
       if (forced)
@@ -835,14 +823,6 @@ bool PowerSparseMatrixGPU::BuildHub(const int* row_ptr, Prepared& in,
                                     std::to_string(kHubMaxElements) + " elements");
       continue;
     }
-    t->hub_rows.Allocate(size_t(R));
-    t->hub_rows.Upload(hub_rows.data(), size_t(R));
-    t->hub_index.Allocate(size_t(rows));
-    t->hub_index.Upload(hub_index.data(), size_t(rows));
-    t->hot_cols.Allocate(size_t(H));
-    t->hot_cols.Upload(hot_cols.data(), size_t(H));
-    t->hot_rank.Allocate(size_t(cols));
-    t->hot_rank.Upload(hot_rank.data(), size_t(cols));
     ps_hub_block& d = t->desc;
     d.matrix_rows = rows;
     d.matrix_cols = cols;
@@ -913,53 +893,30 @@ bool PowerSparseMatrixGPU::BuildHub(const int* row_ptr, Prepared& in,
   // explicit tiers serve both operators.
   std::vector<ps_workset> ws = PublicWorksets();
   const size_t T = hub->tiers.size();
-  std::vector<std::vector<uint32_t>> tiles(T);
-  std::vector<std::vector<std::vector<uint8_t>>> flags(T, std::vector<std::vector<uint8_t>>(size_t(S)));
-  DeviceArray<uint8_t> f_dev;
-  for (int s = 1; s < S; ++s) {
-    const int G = _group_num[s], GS = GROUP_SIZE(s);
-    if (G == 0 || GS < 64) continue;
-    const size_t n = size_t(G) * size_t(GS / 64);  // 64-nonzero stretches
-    f_dev.Allocate(n);
-    for (size_t k = 0; k < T; ++k) {
-      ThrowOnError(ps_hub_tile_flags(&hub->tiers[k]->desc, &ws[size_t(s)], f_dev.data(), nullptr));
-      std::vector<uint8_t>& f = flags[k][size_t(s)];
-      f.resize(n);
-      f_dev.Download(f.data(), f.size());
-      for (size_t t = 0; t < n; ++t)
-        if (f[t]) tiles[k].push_back((uint32_t(s) << 27) | uint32_t(t));
-    }
-  }
-  for (size_t k = 0; k < T && !forced; ++k) {
-    const ps_hub_block& d = hub->tiers[k]->desc;
-    if (double(tiles[k].size()) * 64.0 < kHubSddmmMinFill * double(d.rows) * double(d.cols))
-      tiles[k].clear();
-  }
-  std::vector<DeviceArray<uint8_t>> skip(static_cast<size_t>(S));
+  const size_t tile_total = ps_hub_tile_total(S, ws.data());
+  DeviceArray<uint8_t> flags(tile_total), skip(tile_total);
+  DeviceArray<uint32_t> codes(tile_total);
   std::vector<const uint8_t*> skip_ptr(static_cast<size_t>(S), nullptr);
-  for (int s = 1; s < S; ++s) {
-    std::vector<uint8_t> any;
-    for (size_t k = 0; k < T; ++k) {
-      const std::vector<uint8_t>& f = flags[k][size_t(s)];
-      if (tiles[k].empty() || f.empty()) continue;
-      any.resize(f.size(), 0);
-      for (size_t t = 0; t < f.size(); ++t) any[t] |= f[t];
-    }
-    if (std::find(any.begin(), any.end(), uint8_t(1)) == any.end()) continue;
-    skip[size_t(s)].Allocate(any.size());
-    skip[size_t(s)].Upload(any.data(), any.size());  // tiles inside an SDDMM tier
-    skip_ptr[size_t(s)] = skip[size_t(s)].data();
-  }
+  skip.Zero(nullptr);
   for (size_t k = 0; k < T; ++k) {
-    if (tiles[k].empty()) continue;
     HubTier& t = *hub->tiers[k];
-    const uint32_t n = uint32_t(tiles[k].size());
-    DeviceArray<uint32_t> codes(n);
-    codes.Upload(tiles[k].data(), n);
+    uint32_t n = 0;
+    ThrowOnError(ps_hub_tiles(&t.desc, S, ws.data(), flags.data(), codes.data(), &n, nullptr));
+    if (n == 0 || (!forced && double(n) * 64.0 < kHubSddmmMinFill * double(t.desc.rows) *
+                                                     double(t.desc.cols)))
+      continue;
+    ThrowOnError(ps_hub_merge_flags(flags.data(), tile_total, skip.data(), nullptr));
     t.plan.Allocate(ps_hub_sddmm_plan_bytes(&t.desc, n));
     ThrowOnError(ps_hub_sddmm_plan(&t.desc, S, ws.data(), codes.data(), n, t.plan.data(),
                                    t.plan.size(), nullptr));
     t.plan_tiles = n;
+  }
+  // the tiles inside an SDDMM tier leave the run order
+  size_t first = 0;
+  for (int s = 1; s < S; ++s) {
+    if (_group_num[s] == 0 || GROUP_SIZE(s) < 64) continue;
+    skip_ptr[size_t(s)] = skip.data() + first;
+    first += size_t(_group_num[s]) * size_t(GROUP_SIZE(s) / 64);
   }
   const int k = RunOrderSlot(PS_OP_SDDMM, 32);
   uint32_t count = 0, kept_tasks = 0;

@@ -273,7 +273,7 @@ class PowerSparseMatrixGPU {
   void BuildRunOrders();
   // Chooses and builds the dense hub block and the tuned SpMM partition of
   // the rest; false (nothing built) when no block qualifies.
-  bool BuildHub(const int* row_ptr, Prepared& in, const PartitionPolicy& policy);
+  bool BuildHub(Prepared& in, const PartitionPolicy& policy);
   std::vector<ps_workset> PublicWorksets() const;
 
   int _matrix_row, _matrix_col, _matrix_nnz;
