@@ -114,8 +114,6 @@ int ps_fill_random_async(float* dst, size_t count, uint64_t seed, float lo, floa
 /* ------------------------------------------------------- streams, events */
 /* Replaces: cudaStreamCreate / cudaStreamDestroy (benchmark_utils.h:48-66). */
 int ps_stream_create(ps_stream_t* stream);
-/* A stream that does not order itself against the null stream. */
-int ps_stream_create_nonblocking(ps_stream_t* stream);
 int ps_stream_destroy(ps_stream_t stream);
 int ps_stream_synchronize(ps_stream_t stream);
 /* *idle = 1 when everything enqueued on the stream so far has run, else 0. */

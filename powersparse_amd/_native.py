@@ -120,7 +120,6 @@ HIP_API = [
      [c_void_p, ctypes.c_size_t, ctypes.c_uint64, ctypes.c_float, ctypes.c_float, ctypes.c_int,
       c_void_p]),
     ("ps_stream_create", ctypes.c_int, [ctypes.POINTER(c_void_p)]),
-    ("ps_stream_create_nonblocking", ctypes.c_int, [ctypes.POINTER(c_void_p)]),
     ("ps_stream_destroy", ctypes.c_int, [c_void_p]),
     ("ps_stream_idle", ctypes.c_int, [c_void_p, c_int_p]),
     ("ps_stream_synchronize", ctypes.c_int, [c_void_p]),

@@ -459,14 +459,6 @@ int ps_stream_create(ps_stream_t* stream) {
   return PS_OK;
 }
 
-int ps_stream_create_nonblocking(ps_stream_t* stream) {
-  PS_CHECK_ARG(stream, "ps_stream_create_nonblocking: null output");
-  hipStream_t s = nullptr;
-  PS_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));  // default priority
-  *stream = reinterpret_cast<ps_stream_t>(s);
-  return PS_OK;
-}
-
 int ps_stream_destroy(ps_stream_t stream) {
   if (stream) PS_HIP(hipStreamDestroy(ps::to_hip(stream)));
   return PS_OK;

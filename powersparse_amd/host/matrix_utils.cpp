@@ -2,12 +2,12 @@
 //
 // Follows ParCIS/PowerSparse utils/matrix_utils.cu:470-663 step by step, with
 // every per-nonzero and per-row loop moved to HIP kernels behind the C ABI:
-//   validation (host, as :475-488) -> CSR upload -> worksets S (:31-63, device
-//   degree sums) -> column histogram (:508-514, device) -> each row's nonzeros
-//   ranked by column count descending, ties in CSR order (:518-524, stable
-//   radix sort) -> group counts, scans and metadata (:132-208, device) ->
-//   column signature bits (:65-128, host std::sort as in the reference) ->
-//   signatures and the stable per-word group sort (:261-327, :562-594) ->
+//   validation (:475-488; entries of large matrices on the device) -> CSR
+//   upload (the values after the ranking) -> worksets S (:31-63, device degree
+//   sums) -> column histogram (:508-514, device) -> each row's nonzeros ranked
+//   by column count descending, ties in CSR order (:518-524) -> group counts,
+//   scans and metadata (:132-208, device) -> column signature bits (:65-128,
+//   host std::sort as in the reference) -> signatures and the stable group sort (:261-327, :562-594) ->
 //   final worksets (:596-656).
 // The host signature-bit step overlaps the device rank sort.
 #include "matrix_utils.h"
@@ -192,30 +192,20 @@ class StageClock {
 
 }  // namespace
 
-// Nonzeros from which the columns and values are checked on the device and the
-// values uploaded beside the preprocessing that does not read them: below, the
-// host's checks and one plain copy are quicker than a thread and a stream.
-constexpr int kOverlapNonzeros = 1 << 24;
+// Nonzeros from which the columns and values are checked on the device as they
+// arrive there: below, the host's loop takes no longer than a launch and its wait.
+constexpr int kDeviceCheckNonzeros = 1 << 24;
 
 const char* const kBadEntry = "Invalid CSR column index or sparse value";
 
-// A non-blocking stream: work on it overlaps the null stream's.
-struct SideStream {
-  ps_stream_t s = nullptr;
-  SideStream() { ThrowOnError(ps_stream_create_nonblocking(&s)); }
-  ~SideStream() { (void)ps_stream_destroy(s); }
-  SideStream(const SideStream&) = delete;
-  SideStream& operator=(const SideStream&) = delete;
-};
-
 // The partition-independent stages of the preprocessing. Members are declared
-// so that the helper threads (values, sig_len) are joined before what they
-// write is destroyed.
+// so that the helper thread (sig_len) is joined before what it writes is
+// destroyed.
 struct PowerSparseMatrixGPU::Prepared {
   StageClock clock;
   DeviceArray<int> row_ptr, col_ind;
   DeviceArray<float> sp_data;
-  DeviceArray<uint32_t> flags;  // scratch of the two checks
+  DeviceArray<uint32_t> flag;  // scratch of the checks
   unsigned long long degree_sums[32] = {};
   DeviceArray<int> col_nnz;  // device column counts
   std::vector<int> col_nnz_host, sigbit;
@@ -225,44 +215,24 @@ struct PowerSparseMatrixGPU::Prepared {
   DeviceArray<int> sigbit_device;
   int signature_len = 0;
   std::future<int> sig_len;
-  std::future<bool> values;  // the values' upload; true: one is not finite
 
   Prepared(int rows, int cols, int nnz, const int* host_row_ptr, const int* host_col_ind,
            const float* host_sp_data, PreprocessTimings* timings)
       : clock(timings), row_ptr(size_t(rows) + 1), col_ind(size_t(nnz)), sp_data(size_t(nnz)) {
     StagedUpload(row_ptr.data(), host_row_ptr, sizeof(int) * (size_t(rows) + 1));
     StagedUpload(col_ind.data(), host_col_ind, sizeof(int) * size_t(nnz));
-    if (nnz < kOverlapNonzeros) {
-      StagedUpload(sp_data.data(), host_sp_data, sizeof(float) * size_t(nnz));
-    } else {
-      flags.Allocate(2);
-      int bad = 0, device = 0;
-      ThrowOnError(ps_pre_check_csr(col_ind.data(), nullptr, nnz, cols, flags.data(), &bad, nullptr));
-      if (bad) throw std::invalid_argument(kBadEntry);
-      // The values are first read by the gather: their upload runs beside the
-      // column counts, the ranking and the signatures (C3: 20 of 40 ms).
-      ThrowOnError(ps_get_device(&device));
-      values = std::async(std::launch::async, [this, device, nnz, cols, host_sp_data] {
-        ThrowOnError(ps_set_device(device));
-        SideStream side;
-        StagedUpload(sp_data.data(), host_sp_data, sizeof(float) * size_t(nnz), side.s);
-        int infinite = 0;
-        ThrowOnError(ps_pre_check_csr(nullptr, sp_data.data(), nnz, cols, flags.data() + 1,
-                                      &infinite, side.s));
-        return infinite != 0;
-      });
+    if (nnz >= kDeviceCheckNonzeros) {
+      flag.Allocate(1);
+      Check(col_ind.data(), nullptr, nnz, cols);
     }
     clock.Mark(&PreprocessTimings::upload_ms);
-    Analyze(rows, cols, nnz);
+    Analyze(rows, cols, nnz, host_sp_data);
   }
 
-  // The uploaded, checked values.
-  const float* Values() {
-    if (values.valid()) {
-      if (values.get()) throw std::invalid_argument(kBadEntry);
-      clock.Mark(&PreprocessTimings::upload_ms);
-    }
-    return sp_data.data();
+  void Check(const int* columns, const float* data, int nnz, int cols) {
+    int bad = 0;
+    ThrowOnError(ps_pre_check_csr(columns, data, nnz, cols, flag.data(), &bad, nullptr));
+    if (bad) throw std::invalid_argument(kBadEntry);
   }
 
   // From here on only the nonzeros of a shorter ranking (positions in the same
@@ -275,7 +245,7 @@ struct PowerSparseMatrixGPU::Prepared {
     std::copy(std::begin(sums), std::end(sums), degree_sums);
   }
 
-  void Analyze(int rows, int cols, int nnz) {
+  void Analyze(int rows, int cols, int nnz, const float* host_sp_data) {
     ps_stream_t st = nullptr;
     // Degree sums (AnalyzeMatrix) and the column histogram.
     ThrowOnError(ps_pre_degree_sums(row_ptr.data(), rows, degree_sums, st));
@@ -300,6 +270,12 @@ struct PowerSparseMatrixGPU::Prepared {
     ThrowOnError(ps_pre_rank_sort(row_ptr.data(), rows, col_ind.data(), nnz, col_nnz.data(),
                                   max_count, count_bits, nullptr, vals.data(), st));
     clock.Mark(&PreprocessTimings::rank_ms);
+
+    // The values are first read by the gather: uploaded here, while the other
+    // thread still sorts the columns.
+    StagedUpload(sp_data.data(), host_sp_data, sizeof(float) * size_t(nnz));
+    if (nnz >= kDeviceCheckNonzeros) Check(nullptr, sp_data.data(), nnz, cols);
+    clock.Mark(&PreprocessTimings::upload_ms);
   }
 
   // Joins the signature-bit thread on the first call (sigbit_ms: the time
@@ -363,7 +339,7 @@ PowerSparseMatrixGPU::PowerSparseMatrixGPU(int row_num, int col_num, int nnz_num
 #pragma omp parallel for reduction(| : bad) schedule(static)
   for (int r = 0; r < row_num; ++r) bad |= (row_ptr[r] < 0 || row_ptr[r] > row_ptr[r + 1]);
   if (bad) throw std::invalid_argument("CSR row pointers must be nondecreasing");
-  if (nnz_num < kOverlapNonzeros) {  // else on the device, as they are uploaded
+  if (nnz_num < kDeviceCheckNonzeros) {  // else on the device, as they are uploaded
 #pragma omp parallel for reduction(| : bad) schedule(static)
     for (int p = 0; p < nnz_num; ++p)
       bad |= (col_ind[p] < 0 || col_ind[p] >= col_num || !std::isfinite(sp_data[p]));
@@ -584,7 +560,7 @@ void PowerSparseMatrixGPU::Build(Prepared& in) {
       ThrowOnError(ps_malloc(reinterpret_cast<void**>(&_workset_csr_pos[s]), sizeof(int) * size));
     ThrowOnError(ps_pre_gather_workset_cols(s == 0 ? 0 : GROUP_SIZE(s), _matrix_col, perm[size_t(s)].data(), G,
                                        start[size_t(s)].data(), s == 0 ? _residue_offset : nullptr,
-                                       vals.data(), d_ci.data(), in.Values(), _workset_col_ind[s],
+                                       vals.data(), d_ci.data(), in.sp_data.data(), _workset_col_ind[s],
                                        _workset_sp_data[s],
                                        _keep_csr_pos ? _workset_csr_pos[s] : nullptr, st));
   }
@@ -679,7 +655,7 @@ void PowerSparseMatrixGPU::BuildExecution(Prepared& in, const std::vector<int*>&
       ThrowOnError(ps_malloc(reinterpret_cast<void**>(&_exec_csr_pos[s]), sizeof(int) * size));
     ThrowOnError(ps_pre_gather_workset_cols(
         s == 0 ? 0 : GROUP_SIZE(s), _matrix_col, iota.data(), G, group_start[size_t(s)],
-        s == 0 ? residue_offset : nullptr, in.vals.data(), in.col_ind.data(), in.Values(),
+        s == 0 ? residue_offset : nullptr, in.vals.data(), in.col_ind.data(), in.sp_data.data(),
         _exec_col_ind[s], _exec_sp_data[s], _keep_csr_pos ? _exec_csr_pos[s] : nullptr, nullptr));
   }
 }
@@ -836,7 +812,7 @@ bool PowerSparseMatrixGPU::BuildHub(Prepared& in, const PartitionPolicy& policy)
     t->stored.Allocate(ps_hub_stored_words(&d));
     d.dense = t->dense.data();
     d.stored = t->stored.data();
-    ThrowOnError(ps_hub_dense_build(&d, in.row_ptr.data(), in.col_ind.data(), in.Values(),
+    ThrowOnError(ps_hub_dense_build(&d, in.row_ptr.data(), in.col_ind.data(), in.sp_data.data(),
                                     t->dense.data(), t->stored.data(), nullptr));
     hub->tiers.push_back(std::move(t));
   }

@@ -104,10 +104,10 @@ constexpr int kTunedSpmmGroupTypes = 3;
 // block accumulate into C as the reference's do (they hold more than 32
 // nonzeros); a (row, column) slot stored more than once stays on the sparse
 // SpMM path. Cost: 4 bytes per block element (dense), 12 bytes per planned
-// SDDMM nonzero, the tuned partition's own preprocessing (it no longer
-// shares the public one's), and an operator workspace allocated with the
-// block (SDDMM at N = 512: 2 KiB per hub row and per hot column of the
-// widest tier, padded to whole tiles).
+// SDDMM nonzero, the tuned partition's own grouping, signature sort and
+// gather, and an operator workspace allocated with the block (SDDMM at
+// N = 512: 2 KiB per hub row and per hot column of the widest tier, padded to
+// whole tiles).
 enum class HubBlock { kAuto = 0, kOff = 1 };
 constexpr int kHubMaxTiers = 3;
 constexpr double kHubDenseCost = 0.12, kHubMinGain = 0.05, kHubMinTierGain = 0.02;

@@ -80,7 +80,7 @@ struct Events {
 
 }  // namespace
 
-void StagedUpload(void* dst, const void* src, size_t bytes, ps_stream_t stream) {
+void StagedUpload(void* dst, const void* src, size_t bytes) {
   if (bytes < kMinStaged) {
     ThrowOnError(ps_memcpy_htod(dst, src, bytes));
     return;
@@ -100,6 +100,7 @@ void StagedUpload(void* dst, const void* src, size_t bytes, ps_stream_t stream) 
   }
   Events ev;
   for (ps_event_t& x : ev.e) ThrowOnError(ps_event_create(&x));
+  ps_stream_t const stream = nullptr;
   DrainOnExit drain{stream};
   const char* s = static_cast<const char*>(src);
   char* d = static_cast<char*>(dst);

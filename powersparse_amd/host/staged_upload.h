@@ -11,8 +11,7 @@ namespace PowerSparse {
 // `dst` and returns when the copy is complete. Large copies go through two
 // page-locked buffers: while the DMA engine copies chunk k out of one buffer,
 // host threads fill the other with chunk k + 1. Copies below 64 KB use one
-// plain synchronous copy. Uses the given stream of the current
-// device (the plain copy: the null stream).
-void StagedUpload(void* dst, const void* src, size_t bytes, ps_stream_t stream = nullptr);
+// plain synchronous copy. Uses the null stream of the current device.
+void StagedUpload(void* dst, const void* src, size_t bytes);
 
 }  // namespace PowerSparse
