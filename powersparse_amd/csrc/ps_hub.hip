@@ -143,7 +143,7 @@ __global__ __launch_bounds__(kThreads) void hist_kernel(const int* __restrict__ 
 // passes over 4 bytes per row or column. As loops of the host with two uploads
 // per tier it held the device idle for 11 ms of a 98 ms build of 1.6 M rows
 // and 264 M nonzeros, the tile list below (flags downloaded, codes uploaded)
-// for 7: 81 ms now.
+// for 7 (98 -> 81 ms together).
 //
 // levels[a] = rows of degree with floor(log2) = a, levels[32 + b] = columns of
 // count with floor(log2) = b (rows and columns without nonzeros left out).

@@ -7,7 +7,8 @@
 //   sums) -> column histogram (:508-514, device) -> each row's nonzeros ranked
 //   by column count descending, ties in CSR order (:518-524) -> group counts,
 //   scans and metadata (:132-208, device) -> column signature bits (:65-128,
-//   host std::sort as in the reference) -> signatures and the stable group sort (:261-327, :562-594) ->
+//   host std::sort as in the reference) -> signatures and the stable group sort
+//   (:261-327, :562-594) ->
 //   final worksets (:596-656).
 // The host signature-bit step overlaps the device rank sort.
 #include "matrix_utils.h"
