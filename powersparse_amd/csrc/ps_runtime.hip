@@ -4,12 +4,12 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
-#include <map>
 #include <mutex>
 #include <string>
 #include <unordered_map>
 #include <vector>
 
+#include "ps_block_pool.hpp"
 #include "ps_common.hpp"
 
 namespace ps {
@@ -75,142 +75,30 @@ size_t check_guards(size_t guard, void* user, const Guarded& a) {
   return bad;
 }
 
-// Freed device blocks of 2 MB and more, kept for the next allocation.
-//
-// Building a matrix allocates and frees several times its size, and the driver
-// clears the pages it hands out: a program that builds matrix after matrix is
-// served from cleared pages for some tens of GB and then waits (32 GB freed in
-// 366 - 958 ms, about 33 GB/s; a 264 M-nonzero build slowed from 0.29 s to 0.6 -
-// 1.3 s, and a 50 M-nonzero matrix took 8 ms to destroy). A kept block needs
-// neither the clearing nor the unmapping.
-//
-// A block is synchronised with its whole device before it is kept (as hipFree
-// does), so any stream or thread may get it next. What is kept is bounded by a
-// sixteenth of the device's memory, oldest given back first, and is given back
-// when a block has lain unused for kKeepSeconds at a later call, when an
-// allocation fails, when the free memory is asked for, and by ps_mem_trim.
-constexpr size_t kPoolMin = size_t(2) << 20;
-constexpr int kKeepSeconds = 10;
-using Clock = std::chrono::steady_clock;
-
-struct Pool {
-  struct Live {
-    size_t bytes;
-    int device;
-  };
-  struct Kept {
-    void* ptr;
-    Clock::time_point since;
-  };
-  std::mutex mu;
-  std::unordered_map<void*, Live> live;
-  std::map<int, std::multimap<size_t, Kept>> kept;  // per device, by size
-  std::map<int, size_t> kept_bytes, limit;
+// The device blocks' driver (BlockPool's policy).
+struct HipDriver {
+  using Error = hipError_t;
+  static constexpr Error kOk = hipSuccess, kOutOfMemory = hipErrorOutOfMemory,
+                         kInvalid = hipErrorInvalidValue;
+  static int64_t NowNs() {
+    return std::chrono::duration_cast<std::chrono::nanoseconds>(
+               std::chrono::steady_clock::now().time_since_epoch())
+        .count();
+  }
+  static Error Device(int* device) { return hipGetDevice(device); }
+  static Error SetDevice(int device) { return hipSetDevice(device); }
+  static Error Malloc(void** ptr, size_t bytes) { return hipMalloc(ptr, bytes); }
+  static Error Free(void* ptr) { return hipFree(ptr); }
+  static Error Synchronize() { return hipDeviceSynchronize(); }
+  static Error TotalBytes(size_t* total) {
+    size_t free_bytes = 0;
+    return hipMemGetInfo(&free_bytes, total);
+  }
+  static void ClearError() { (void)hipGetLastError(); }
 };
-Pool& pool() {
-  static Pool* p = new Pool;  // never destroyed: frees may come from any exit path
+BlockPool<HipDriver>& pool() {
+  static auto* p = new BlockPool<HipDriver>;  // never destroyed: frees may come from any exit path
   return *p;
-}
-
-// Gives back the current device's kept blocks: those beyond its limit (oldest
-// first) or unused too long, or with `all` every one.
-int pool_trim(int device, bool all) {
-  Pool& p = pool();
-  std::vector<void*> out;
-  {
-    std::lock_guard<std::mutex> lock(p.mu);
-    auto& kept = p.kept[device];
-    const auto old = Clock::now() - std::chrono::seconds(kKeepSeconds);
-    for (auto it = kept.begin(); it != kept.end();) {
-      if (all || it->second.since < old) {
-        out.push_back(it->second.ptr);
-        p.kept_bytes[device] -= it->first;
-        it = kept.erase(it);
-      } else {
-        ++it;
-      }
-    }
-    while (p.kept_bytes[device] > p.limit[device]) {
-      auto oldest = kept.begin();
-      for (auto it = kept.begin(); it != kept.end(); ++it)
-        if (it->second.since < oldest->second.since) oldest = it;
-      out.push_back(oldest->second.ptr);
-      p.kept_bytes[device] -= oldest->first;
-      kept.erase(oldest);
-    }
-  }
-  for (void* ptr : out) PS_HIP(hipFree(ptr));
-  return PS_OK;
-}
-
-int pool_malloc(void** ptr, size_t bytes) {
-  Pool& p = pool();
-  int device = 0;
-  PS_HIP(hipGetDevice(&device));
-  bytes = (bytes + kPoolMin - 1) / kPoolMin * kPoolMin;
-  {
-    std::lock_guard<std::mutex> lock(p.mu);
-    auto& kept = p.kept[device];
-    const auto it = kept.lower_bound(bytes);
-    if (it != kept.end() && it->first <= bytes + bytes / 4) {
-      *ptr = it->second.ptr;
-      p.live[*ptr] = Pool::Live{it->first, device};
-      p.kept_bytes[device] -= it->first;
-      kept.erase(it);
-      return PS_OK;
-    }
-    if (p.limit[device] == 0) {
-      size_t free_bytes = 0, total = 0;
-      PS_HIP(hipMemGetInfo(&free_bytes, &total));
-      p.limit[device] = total / 16;
-    }
-  }
-  hipError_t e = hipMalloc(ptr, bytes);
-  if (e == hipErrorOutOfMemory) {
-    (void)hipGetLastError();  // the kept blocks may be what is missing
-    const int rc = pool_trim(device, true);
-    if (rc != PS_OK) return rc;
-    e = hipMalloc(ptr, bytes);
-  }
-  PS_HIP(e);
-  std::lock_guard<std::mutex> lock(p.mu);
-  p.live[*ptr] = Pool::Live{bytes, device};
-  return PS_OK;
-}
-
-int pool_free(void* ptr) {
-  Pool& p = pool();
-  Pool::Live block{};
-  {
-    std::lock_guard<std::mutex> lock(p.mu);
-    const auto it = p.live.find(ptr);
-    if (it != p.live.end()) {
-      block = it->second;
-      p.live.erase(it);
-    }
-  }
-  if (block.bytes == 0) {  // a small block
-    PS_HIP(hipFree(ptr));
-    return PS_OK;
-  }
-  int current = 0;
-  PS_HIP(hipGetDevice(&current));
-  if (current != block.device) PS_HIP(hipSetDevice(block.device));
-  hipError_t e = hipDeviceSynchronize();
-  if (e != hipSuccess) (void)hipFree(ptr);
-  if (e == hipSuccess) {
-    {
-      std::lock_guard<std::mutex> lock(p.mu);
-      p.kept[block.device].insert({block.bytes, Pool::Kept{ptr, Clock::now()}});
-      p.kept_bytes[block.device] += block.bytes;
-    }
-    const int rc = pool_trim(block.device, false);
-    if (current != block.device) PS_HIP(hipSetDevice(current));
-    return rc;
-  }
-  if (current != block.device) (void)hipSetDevice(current);
-  PS_HIP(e);
-  return PS_OK;
 }
 }  // namespace
 
@@ -318,15 +206,7 @@ int ps_malloc(void** ptr, size_t bytes) {
   if (bytes == 0) return PS_OK;
   ps::GuardState& g = ps::guards();
   if (g.guard == 0) {
-    if (bytes >= ps::kPoolMin) return ps::pool_malloc(ptr, bytes);
-    hipError_t e = hipMalloc(ptr, bytes);
-    if (e == hipErrorOutOfMemory) {
-      (void)hipGetLastError();
-      const int rc = ps_mem_trim();
-      if (rc != PS_OK) return rc;
-      e = hipMalloc(ptr, bytes);
-    }
-    PS_HIP(e);
+    PS_HIP(ps::pool().Malloc(ptr, bytes));
     return PS_OK;
   }
   char* base = nullptr;
@@ -362,13 +242,15 @@ int ps_free(void* ptr) {
       return PS_OK;
     }
   }
-  return ps::pool_free(ptr);
+  PS_HIP(ps::pool().Free(ptr));
+  return PS_OK;
 }
 
 int ps_mem_trim(void) {
   int device = 0;
   PS_HIP(hipGetDevice(&device));
-  return ps::pool_trim(device, true);
+  PS_HIP(ps::pool().Trim(device, true));
+  return PS_OK;
 }
 
 long long ps_guard_violations(void) {
