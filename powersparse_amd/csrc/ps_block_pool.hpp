@@ -40,7 +40,8 @@ class BlockPool {
   static constexpr int64_t kKeepNs = int64_t(10) * 1000000000;
 
   Error Malloc(void** ptr, size_t bytes) {
-    if (bytes < kMin) return DriverMalloc(ptr, bytes);
+    // (what cannot be rounded up is the driver's to refuse)
+    if (bytes < kMin || bytes > SIZE_MAX - kMin) return DriverMalloc(ptr, bytes);
     int device = 0;
     Error e = Driver::Device(&device);
     if (e != Driver::kOk) return e;

@@ -210,6 +210,7 @@ int ps_malloc(void** ptr, size_t bytes) {
     return PS_OK;
   }
   char* base = nullptr;
+  if (bytes > SIZE_MAX - 2 * g.guard) PS_HIP(hipErrorOutOfMemory);
   PS_HIP(hipMalloc(reinterpret_cast<void**>(&base), bytes + 2 * g.guard));
   hipError_t e = hipMemset(base, ps::kGuardByte, g.guard);
   if (e == hipSuccess) e = hipMemset(base + g.guard + bytes, ps::kGuardByte, g.guard);

@@ -1,0 +1,101 @@
+// Checks of the kept-block pool (powersparse_amd/csrc/ps_block_pool.hpp) on a
+// stand-in driver: memory of 1 GB per device that is counted, not used, a clock
+// that the checks set, and errors for a free of what is not allocated.
+#include <atomic>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+#include "ps_block_pool.hpp"
+
+namespace {
+
+constexpr size_t MB = size_t(1) << 20;
+
+enum Status { kFine = 0, kNoMemory = 2, kBadValue = 1 };
+
+struct Fake {
+  using Error = Status;
+  static constexpr Error kOk = kFine, kOutOfMemory = kNoMemory, kInvalid = kBadValue;
+
+  static inline std::mutex mu;
+  static inline std::map<void*, size_t> allocated;
+  static inline size_t in_use = 0, mallocs = 0;
+  static inline uintptr_t next = uintptr_t(1) << 40;
+  static inline std::atomic<int64_t> now{0};
+  static inline bool refuse_free = false;
+
+  static int64_t NowNs() { return now; }
+  static Error Device(int* device) {
+    *device = 0;
+    return kOk;
+  }
+  static Error SetDevice(int) { return kOk; }
+  static Error Malloc(void** ptr, size_t bytes) {
+    std::lock_guard<std::mutex> lock(mu);
+    *ptr = nullptr;
+    if (bytes == 0) return kOk;
+    if (bytes > 1024 * MB - in_use) return kOutOfMemory;
+    *ptr = reinterpret_cast<void*>(next);
+    next += (bytes + 4095) / 4096 * 4096;
+    allocated[*ptr] = bytes;
+    in_use += bytes;
+    ++mallocs;
+    return kOk;
+  }
+  static Error Free(void* ptr) {
+    std::lock_guard<std::mutex> lock(mu);
+    if (refuse_free) return kBadValue;
+    const auto it = allocated.find(ptr);
+    if (it == allocated.end()) return kBadValue;
+    in_use -= it->second;
+    allocated.erase(it);
+    return kOk;
+  }
+  static Error Synchronize() { return kOk; }
+  static Error TotalBytes(size_t* total) {
+    *total = 1024 * MB;
+    return kOk;
+  }
+  static void ClearError() {}
+};
+
+using Pool = ps::BlockPool<Fake>;
+
+#define CHECK(cond)                                                   \
+  do {                                                                \
+    if (!(cond)) {                                                    \
+      std::printf("%s:%d: %s\n", __FILE__, __LINE__, #cond);          \
+      return 1;                                                       \
+    }                                                                 \
+  } while (0)
+
+// Sizes whose rounding up to 2 MB does not fit size_t are out of memory.
+int huge() {
+  Pool pool;
+  for (size_t bytes : {size_t(-1), size_t(-1) - 2 * MB + 2, size_t(-1) - 2 * MB, size_t(1) << 63}) {
+    void* p = &pool;
+    CHECK(pool.Malloc(&p, bytes) == kNoMemory);
+    CHECK(p == nullptr);
+  }
+  CHECK(Fake::in_use == 0);
+  return 0;
+}
+
+struct Check {
+  const char* name;
+  int (*run)();
+};
+const Check kChecks[] = {{"huge", huge}};
+
+}  // namespace
+
+int main(int argc, char** argv) {
+  for (const Check& c : kChecks)
+    if (argc == 2 && std::strcmp(argv[1], c.name) == 0) return c.run();
+  return 2;
+}

@@ -1,5 +1,6 @@
 """Device blocks kept between ps_free and ps_malloc: reuse, the size rule, and
 giving them back."""
+import ctypes
 from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
@@ -85,3 +86,13 @@ def test_threads_never_share_a_block():
 
     with ThreadPoolExecutor(8) as ex:
         assert all(ex.map(work, range(8)))
+
+
+@pytest.mark.parametrize("nbytes", [-1, -(2 * MB) + 1, -(2 * MB)])
+def test_sizes_beyond_the_address_range(nbytes):
+    # (size_t)-1 and its neighbours: rounding them up to 2 MB must not wrap
+    setup()
+    p = ctypes.c_void_p(1)
+    rc = _native.hip().ps_malloc(ctypes.byref(p), ctypes.c_size_t(nbytes))
+    assert rc == _native.PS_ERR_RUNTIME and not p.value
+    assert "out of memory" in _native.hip().ps_last_error().decode()
