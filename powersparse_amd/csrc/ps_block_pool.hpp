@@ -52,7 +52,7 @@ class BlockPool {
       const auto it = s.kept.lower_bound(bytes);
       if (it != s.kept.end() && it->first <= bytes + bytes / 4) {
         *ptr = it->second.ptr;
-        live_[*ptr] = Live{it->first, device};
+        blocks_[*ptr].state = kLive;
         s.bytes -= it->first;
         s.kept.erase(it);
         return Driver::kOk;
@@ -67,33 +67,40 @@ class BlockPool {
     e = DriverMalloc(ptr, bytes);
     if (e != Driver::kOk) return e;
     std::lock_guard<std::mutex> lock(mu_);
-    live_[*ptr] = Live{bytes, device};
+    blocks_[*ptr] = Block{bytes, device, kLive};
     return Driver::kOk;
   }
 
+  // kInvalid for a block that is kept already (or being kept by another
+  // thread): the driver, which still counts it as allocated, would free it
+  // under the pool.
   Error Free(void* ptr) {
-    Live block{};
+    Block block{};
     {
       std::lock_guard<std::mutex> lock(mu_);
-      const auto it = live_.find(ptr);
-      if (it != live_.end()) {
+      const auto it = blocks_.find(ptr);
+      if (it != blocks_.end()) {
+        if (it->second.state != kLive) return Driver::kInvalid;
+        it->second.state = kReturning;
         block = it->second;
-        live_.erase(it);
       }
     }
     if (block.bytes == 0) return Driver::Free(ptr);  // a small block
-    int current = 0;
+    int current = block.device;
     Error e = Driver::Device(&current);
-    if (e != Driver::kOk) return e;
-    if (current != block.device) e = Driver::SetDevice(block.device);
-    if (e != Driver::kOk) return e;
-    e = Driver::Synchronize();
+    if (e == Driver::kOk && current != block.device) e = Driver::SetDevice(block.device);
+    if (e == Driver::kOk) e = Driver::Synchronize();
     if (e != Driver::kOk) {
+      {
+        std::lock_guard<std::mutex> lock(mu_);
+        blocks_.erase(ptr);
+      }
       (void)Driver::Free(ptr);
     } else {
       {
         std::lock_guard<std::mutex> lock(mu_);
         Shelf& s = shelves_[block.device];
+        blocks_[ptr].state = kKept;
         s.kept.insert({block.bytes, Kept{ptr, Driver::NowNs()}});
         s.bytes += block.bytes;
       }
@@ -117,8 +124,7 @@ class BlockPool {
       for (auto it = s.kept.begin(); it != s.kept.end();) {
         if (all || it->second.since < old) {
           out.push_back(it->second.ptr);
-          s.bytes -= it->first;
-          it = s.kept.erase(it);
+          it = Unlist(s, it);
         } else {
           ++it;
         }
@@ -128,8 +134,7 @@ class BlockPool {
         for (auto it = s.kept.begin(); it != s.kept.end(); ++it)
           if (it->second.since < oldest->second.since) oldest = it;
         out.push_back(oldest->second.ptr);
-        s.bytes -= oldest->first;
-        s.kept.erase(oldest);
+        Unlist(s, oldest);
       }
     }
     for (void* ptr : out) {
@@ -146,9 +151,12 @@ class BlockPool {
   }
 
  private:
-  struct Live {
+  // kReturning: in Free, not yet kept.
+  enum State { kLive, kReturning, kKept };
+  struct Block {
     size_t bytes;
     int device;
+    State state;
   };
   struct Kept {
     void* ptr;
@@ -158,20 +166,43 @@ class BlockPool {
     std::multimap<size_t, Kept> kept;  // by size
     size_t bytes = 0, limit = 0;
   };
+  using KeptAt = typename std::multimap<size_t, Kept>::iterator;
 
-  // The driver's allocation; the kept blocks may be what is missing.
+  // (under the lock)
+  KeptAt Unlist(Shelf& s, KeptAt it) {
+    blocks_.erase(it->second.ptr);
+    s.bytes -= it->first;
+    return s.kept.erase(it);
+  }
+
+  // The driver's allocation; the kept blocks may be what is missing. An address
+  // that the pool still lists was freed behind its back, and is dropped.
   Error DriverMalloc(void** ptr, size_t bytes) {
     Error e = Driver::Malloc(ptr, bytes);
-    if (e != Driver::kOutOfMemory) return e;
-    Driver::ClearError();
-    int device = 0;
-    e = Driver::Device(&device);
-    if (e == Driver::kOk) e = Trim(device, true);
-    return e == Driver::kOk ? Driver::Malloc(ptr, bytes) : e;
+    if (e == Driver::kOutOfMemory) {
+      Driver::ClearError();
+      int device = 0;
+      e = Driver::Device(&device);
+      if (e == Driver::kOk) e = Trim(device, true);
+      if (e == Driver::kOk) e = Driver::Malloc(ptr, bytes);
+    }
+    if (e != Driver::kOk) return e;
+    std::lock_guard<std::mutex> lock(mu_);
+    const auto it = blocks_.find(*ptr);
+    if (it == blocks_.end()) return e;
+    Shelf& s = shelves_[it->second.device];
+    const auto same = s.kept.equal_range(it->second.bytes);
+    for (auto k = same.first; k != same.second; ++k)
+      if (k->second.ptr == *ptr) {
+        Unlist(s, k);
+        return e;
+      }
+    blocks_.erase(it);
+    return e;
   }
 
   std::mutex mu_;
-  std::unordered_map<void*, Live> live_;
+  std::unordered_map<void*, Block> blocks_;
   std::map<int, Shelf> shelves_;  // per device
 };
 

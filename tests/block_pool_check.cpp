@@ -28,6 +28,7 @@ struct Fake {
   static inline uintptr_t next = uintptr_t(1) << 40;
   static inline std::atomic<int64_t> now{0};
   static inline bool refuse_free = false;
+  static inline uintptr_t again = 0;  // the next allocation's address, if set
 
   static int64_t NowNs() { return now; }
   static Error Device(int* device) {
@@ -40,8 +41,9 @@ struct Fake {
     *ptr = nullptr;
     if (bytes == 0) return kOk;
     if (bytes > 1024 * MB - in_use) return kOutOfMemory;
-    *ptr = reinterpret_cast<void*>(next);
-    next += (bytes + 4095) / 4096 * 4096;
+    *ptr = reinterpret_cast<void*>(again ? again : next);
+    if (!again) next += (bytes + 4095) / 4096 * 4096;
+    again = 0;
     allocated[*ptr] = bytes;
     in_use += bytes;
     ++mallocs;
@@ -86,11 +88,51 @@ int huge() {
   return 0;
 }
 
+// A second free of a kept block is refused, and the block handed out once.
+int double_free() {
+  Pool pool;
+  void *p = nullptr, *a = nullptr, *b = nullptr;
+  CHECK(pool.Malloc(&p, 8 * MB) == kFine && pool.Free(p) == kFine);
+  CHECK(pool.Free(p) == kBadValue);
+  CHECK(Fake::allocated.count(p) == 1);
+  CHECK(pool.KeptBytes(0) == 8 * MB);
+  CHECK(pool.Malloc(&a, 8 * MB) == kFine && a == p);
+  CHECK(pool.Malloc(&b, 8 * MB) == kFine && b != p);
+  CHECK(Fake::allocated.count(a) == 1);
+  CHECK(pool.Free(a) == kFine && pool.Free(b) == kFine);
+  CHECK(pool.Trim(0, true) == kFine && Fake::in_use == 0);
+  CHECK(pool.Free(a) == kBadValue);  // given back: the driver's answer
+  return 0;
+}
+
+// A block freed behind the pool's back: when the driver hands its address out
+// again, the pool knows the new block, not the old one's size.
+int freed_elsewhere() {
+  Pool pool;
+  void *p = nullptr, *q = nullptr;
+  CHECK(pool.Malloc(&p, 8 * MB) == kFine);
+  CHECK(Fake::Free(p) == kFine);
+  Fake::again = reinterpret_cast<uintptr_t>(p);
+  CHECK(pool.Malloc(&q, 4096) == kFine && q == p);
+  CHECK(pool.Free(q) == kFine);
+  CHECK(pool.KeptBytes(0) == 0 && Fake::in_use == 0);
+  // the same for a kept one
+  CHECK(pool.Malloc(&p, 8 * MB) == kFine && pool.Free(p) == kFine);
+  CHECK(Fake::Free(p) == kFine);
+  Fake::again = reinterpret_cast<uintptr_t>(p);
+  CHECK(pool.Malloc(&q, 4 * MB) == kFine && q == p);
+  CHECK(pool.KeptBytes(0) == 0);
+  CHECK(pool.Free(q) == kFine && pool.KeptBytes(0) == 4 * MB);
+  CHECK(pool.Trim(0, true) == kFine && Fake::in_use == 0);
+  return 0;
+}
+
 struct Check {
   const char* name;
   int (*run)();
 };
-const Check kChecks[] = {{"huge", huge}};
+const Check kChecks[] = {{"huge", huge}, {"double_free", double_free},
+                         {"freed_elsewhere", freed_elsewhere}};
 
 }  // namespace
 

@@ -20,7 +20,7 @@ def program(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("check", ["huge"])
+@pytest.mark.parametrize("check", ["huge", "double_free", "freed_elsewhere"])
 def test_pool(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr

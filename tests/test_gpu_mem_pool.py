@@ -96,3 +96,22 @@ def test_sizes_beyond_the_address_range(nbytes):
     rc = _native.hip().ps_malloc(ctypes.byref(p), ctypes.c_size_t(nbytes))
     assert rc == _native.PS_ERR_RUNTIME and not p.value
     assert "out of memory" in _native.hip().ps_last_error().decode()
+
+
+def test_second_free_is_refused():
+    setup()
+    hip = _native.hip()
+    hip.ps_mem_trim()
+    a = ps.DeviceBuffer(8 * MB)
+    ptr = a.ptr
+    assert hip.ps_free(ptr) == _native.PS_OK
+    assert hip.ps_free(ptr) == _native.PS_ERR_RUNTIME
+    a.ptr = None
+    b, c = ps.DeviceBuffer(8 * MB), ps.DeviceBuffer(8 * MB)
+    say(f"freed {ptr:#x}, then {b.ptr:#x} and {c.ptr:#x}")
+    assert b.ptr == ptr and c.ptr != ptr
+    for k, d in enumerate((b, c)):
+        d.upload(np.full(2 * MB, k, np.uint32))
+    for k, d in enumerate((b, c)):
+        assert (d.download(np.uint32, 2 * MB) == k).all()
+        d.free()
