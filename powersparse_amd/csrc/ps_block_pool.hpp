@@ -186,7 +186,10 @@ class BlockPool {
       if (e == Driver::kOk) e = Trim(device, true);
       if (e == Driver::kOk) e = Driver::Malloc(ptr, bytes);
     }
-    if (e != Driver::kOk) return e;
+    if (e != Driver::kOk) {
+      Driver::ClearError();  // the caller has it; the next launch's check is not for it
+      return e;
+    }
     std::lock_guard<std::mutex> lock(mu_);
     const auto it = blocks_.find(*ptr);
     if (it == blocks_.end()) return e;

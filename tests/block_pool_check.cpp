@@ -28,6 +28,7 @@ struct Fake {
   static inline uintptr_t next = uintptr_t(1) << 40;
   static inline std::atomic<int64_t> now{0};
   static inline bool refuse_free = false;
+  static inline bool left = false;  // an error that the next check would report
   static inline uintptr_t again = 0;  // the next allocation's address, if set
 
   static int64_t NowNs() { return now; }
@@ -40,7 +41,10 @@ struct Fake {
     std::lock_guard<std::mutex> lock(mu);
     *ptr = nullptr;
     if (bytes == 0) return kOk;
-    if (bytes > 1024 * MB - in_use) return kOutOfMemory;
+    if (bytes > 1024 * MB - in_use) {
+      left = true;
+      return kOutOfMemory;
+    }
     *ptr = reinterpret_cast<void*>(again ? again : next);
     if (!again) next += (bytes + 4095) / 4096 * 4096;
     again = 0;
@@ -63,7 +67,7 @@ struct Fake {
     *total = 1024 * MB;
     return kOk;
   }
-  static void ClearError() {}
+  static void ClearError() { left = false; }
 };
 
 using Pool = ps::BlockPool<Fake>;
@@ -83,6 +87,7 @@ int huge() {
     void* p = &pool;
     CHECK(pool.Malloc(&p, bytes) == kNoMemory);
     CHECK(p == nullptr);
+    CHECK(!Fake::left);
   }
   CHECK(Fake::in_use == 0);
   return 0;

@@ -96,6 +96,10 @@ def test_sizes_beyond_the_address_range(nbytes):
     rc = _native.hip().ps_malloc(ctypes.byref(p), ctypes.c_size_t(nbytes))
     assert rc == _native.PS_ERR_RUNTIME and not p.value
     assert "out of memory" in _native.hip().ps_last_error().decode()
+    # the failure is reported once, not by the next launch's check too
+    x = ps.DeviceBuffer(4096)
+    assert _native.hip().ps_fill_random_async(x.ptr, 1024, 1, 0.0, 1.0, 0, None) == _native.PS_OK
+    ps.synchronize()
 
 
 def test_second_free_is_refused():
