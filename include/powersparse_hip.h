@@ -70,11 +70,19 @@ int ps_device_synchronize(void);
 int ps_malloc(void** ptr, size_t bytes);
 int ps_free(void* ptr);
 /* ps_free keeps blocks of 2 MB and more for later ps_malloc calls, up to a
- * sixteenth of the device's memory: they are given back to the driver after
- * ten seconds unused (at a later ps_free), when an allocation fails, by
- * ps_mem_get_info, and by this call (the current device's). No reference
- * counterpart. */
+ * sixteenth of the device's memory. They are given back to the driver when an
+ * allocation fails, by ps_mem_get_info, by the two calls below, when a matrix has
+ * been built (down to what was kept before it, or 256 MB), and once a block has lain unused for ten seconds, at the next
+ * ps_malloc, ps_free or ps_device_synchronize. A program that frees much and
+ * then makes none of these calls calls ps_mem_trim to hand the memory on.
+ * Block sizes are multiples of 2 MB, and a kept block serves requests from four
+ * fifths of its size up: an allocation may hold a quarter more than it asked
+ * for. No reference counterpart. */
 int ps_mem_trim(void);
+/* The same down to `bytes` kept on the current device (the oldest go first),
+ * and the bytes kept now. */
+int ps_mem_trim_to(size_t bytes);
+int ps_mem_kept(size_t* bytes);
 /* Debugging aid, no reference counterpart. With the environment variable
  * PS_DEVICE_GUARD set to a byte count when the library is first used, every
  * device block the library allocates (ps_malloc, and the temporaries of the

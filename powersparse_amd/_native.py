@@ -106,6 +106,8 @@ HIP_API = [
     ("ps_device_synchronize", ctypes.c_int, []),
     ("ps_malloc", ctypes.c_int, [ctypes.POINTER(c_void_p), ctypes.c_size_t]),
     ("ps_mem_trim", ctypes.c_int, []),
+    ("ps_mem_trim_to", ctypes.c_int, [ctypes.c_size_t]),
+    ("ps_mem_kept", ctypes.c_int, [ctypes.POINTER(ctypes.c_size_t)]),
     ("ps_mem_get_info", ctypes.c_int,
      [ctypes.POINTER(ctypes.c_size_t), ctypes.POINTER(ctypes.c_size_t)]),
     ("ps_free", ctypes.c_int, [c_void_p]),

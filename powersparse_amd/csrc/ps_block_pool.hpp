@@ -12,8 +12,13 @@
 // a kept block serves requests from four fifths of its size up, so an array
 // may hold up to a quarter more than was asked for.
 //
-// What is kept is bounded by a sixteenth of the device's memory, oldest given
-// back first.
+// What is kept is given back to the driver, oldest first, beyond a sixteenth of
+// the device's memory; all of it when an allocation fails; and every block that
+// has lain unused for kKeepNs, at the next Malloc or Free of any size or
+// GiveBackIdle, which the device-wide synchronisation calls. No thread or timer of
+// its own does it (hipFree waits for the device, and is refused while a stream
+// is captured), so a program that makes none of these calls keeps its blocks:
+// the builder of a matrix trims what the build left (Trim).
 //
 // The driver's calls come in as a policy, so that the pool compiles without a
 // GPU runtime (and is tested there):
@@ -23,6 +28,7 @@
 #pragma once
 
 #include <algorithm>
+#include <atomic>
 #include <cstddef>
 #include <cstdint>
 #include <map>
@@ -40,6 +46,95 @@ class BlockPool {
   static constexpr int64_t kKeepNs = int64_t(10) * 1000000000;
 
   Error Malloc(void** ptr, size_t bytes) {
+    const Error e = Take(ptr, bytes);  // (an idle block may be what fits)
+    GiveBackIdle();
+    return e;
+  }
+
+  // kInvalid for a block that is kept already (or being kept by another
+  // thread): the driver, which still counts it as allocated, would free it
+  // under the pool.
+  Error Free(void* ptr) {
+    const Error e = Return(ptr);
+    GiveBackIdle();
+    return e;
+  }
+
+  // Gives back the device's kept blocks, oldest first, until at most `keep`
+  // bytes are left. A block that the driver will not free stays kept.
+  Error Trim(int device, size_t keep) {
+    std::vector<Out> out;
+    {
+      std::lock_guard<std::mutex> lock(mu_);
+      Shelf& s = shelves_[device];
+      while (s.bytes > keep) {
+        auto oldest = s.kept.begin();
+        for (auto it = s.kept.begin(); it != s.kept.end(); ++it)
+          if (it->second.since < oldest->second.since) oldest = it;
+        TakeOut(s, oldest, device, &out);
+      }
+    }
+    return GiveBack(out);
+  }
+
+  // Gives back the blocks unused for kKeepNs, on every device. What the driver
+  // refuses now is tried again when it has lain as long once more.
+  void GiveBackIdle() {
+    if (due_.load(std::memory_order_relaxed) == kNever) return;
+    const int64_t now = Driver::NowNs();
+    if (now < due_.load(std::memory_order_relaxed)) return;
+    std::vector<Out> out;
+    {
+      std::lock_guard<std::mutex> lock(mu_);
+      int64_t due = kNever;
+      for (auto& shelf : shelves_) {
+        Shelf& s = shelf.second;
+        for (auto it = s.kept.begin(); it != s.kept.end();) {
+          const int64_t at = it->second.since + kKeepNs;
+          if (at <= now) {
+            it = TakeOut(s, it, shelf.first, &out);
+          } else {
+            due = std::min(due, at);
+            ++it;
+          }
+        }
+      }
+      due_ = due;
+    }
+    if (GiveBack(out) != Driver::kOk) Driver::ClearError();
+  }
+
+  // Bytes kept on the device.
+  size_t KeptBytes(int device) {
+    std::lock_guard<std::mutex> lock(mu_);
+    return shelves_[device].bytes;
+  }
+
+ private:
+  static constexpr int64_t kNever = INT64_MAX;
+  // kReturning: in Free, not yet kept.
+  enum State { kLive, kReturning, kKept };
+  struct Block {
+    size_t bytes;
+    int device;
+    State state;
+  };
+  struct Kept {
+    void* ptr;
+    int64_t since;
+  };
+  struct Shelf {
+    std::multimap<size_t, Kept> kept;  // by size
+    size_t bytes = 0, limit = 0;
+  };
+  using KeptAt = typename std::multimap<size_t, Kept>::iterator;
+  struct Out {
+    void* ptr;
+    size_t bytes;
+    int device;
+  };
+
+  Error Take(void** ptr, size_t bytes) {
     // (what cannot be rounded up is the driver's to refuse)
     if (bytes < kMin || bytes > SIZE_MAX - kMin) return DriverMalloc(ptr, bytes);
     int device = 0;
@@ -71,10 +166,7 @@ class BlockPool {
     return Driver::kOk;
   }
 
-  // kInvalid for a block that is kept already (or being kept by another
-  // thread): the driver, which still counts it as allocated, would free it
-  // under the pool.
-  Error Free(void* ptr) {
+  Error Return(void* ptr) {
     Block block{};
     {
       std::lock_guard<std::mutex> lock(mu_);
@@ -97,14 +189,13 @@ class BlockPool {
       }
       (void)Driver::Free(ptr);
     } else {
+      size_t limit = 0;
       {
         std::lock_guard<std::mutex> lock(mu_);
-        Shelf& s = shelves_[block.device];
-        blocks_[ptr].state = kKept;
-        s.kept.insert({block.bytes, Kept{ptr, Driver::NowNs()}});
-        s.bytes += block.bytes;
+        Keep(Out{ptr, block.bytes, block.device});
+        limit = shelves_[block.device].limit;
       }
-      e = Trim(block.device, false);
+      e = Trim(block.device, limit);
     }
     if (current != block.device) {
       const Error back = Driver::SetDevice(current);
@@ -113,66 +204,35 @@ class BlockPool {
     return e;
   }
 
-  // Gives back the device's kept blocks: those beyond its limit (oldest first)
-  // or unused too long, or with `all` every one.
-  Error Trim(int device, bool all) {
-    std::vector<void*> out;
-    {
-      std::lock_guard<std::mutex> lock(mu_);
-      Shelf& s = shelves_[device];
-      const int64_t old = Driver::NowNs() - kKeepNs;
-      for (auto it = s.kept.begin(); it != s.kept.end();) {
-        if (all || it->second.since < old) {
-          out.push_back(it->second.ptr);
-          it = Unlist(s, it);
-        } else {
-          ++it;
-        }
-      }
-      while (s.bytes > s.limit) {
-        auto oldest = s.kept.begin();
-        for (auto it = s.kept.begin(); it != s.kept.end(); ++it)
-          if (it->second.since < oldest->second.since) oldest = it;
-        out.push_back(oldest->second.ptr);
-        Unlist(s, oldest);
-      }
-    }
-    for (void* ptr : out) {
-      const Error e = Driver::Free(ptr);
-      if (e != Driver::kOk) return e;
-    }
-    return Driver::kOk;
-  }
-
-  // Bytes kept on the device.
-  size_t KeptBytes(int device) {
-    std::lock_guard<std::mutex> lock(mu_);
-    return shelves_[device].bytes;
-  }
-
- private:
-  // kReturning: in Free, not yet kept.
-  enum State { kLive, kReturning, kKept };
-  struct Block {
-    size_t bytes;
-    int device;
-    State state;
-  };
-  struct Kept {
-    void* ptr;
-    int64_t since;
-  };
-  struct Shelf {
-    std::multimap<size_t, Kept> kept;  // by size
-    size_t bytes = 0, limit = 0;
-  };
-  using KeptAt = typename std::multimap<size_t, Kept>::iterator;
-
   // (under the lock)
+  void Keep(const Out& o) {
+    Shelf& s = shelves_[o.device];
+    const int64_t now = Driver::NowNs();
+    blocks_[o.ptr] = Block{o.bytes, o.device, kKept};
+    s.kept.insert({o.bytes, Kept{o.ptr, now}});
+    s.bytes += o.bytes;
+    due_ = std::min(due_.load(), now + kKeepNs);
+  }
   KeptAt Unlist(Shelf& s, KeptAt it) {
     blocks_.erase(it->second.ptr);
     s.bytes -= it->first;
     return s.kept.erase(it);
+  }
+  KeptAt TakeOut(Shelf& s, KeptAt it, int device, std::vector<Out>* out) {
+    out->push_back(Out{it->second.ptr, it->first, device});
+    return Unlist(s, it);
+  }
+
+  Error GiveBack(const std::vector<Out>& out) {
+    Error first = Driver::kOk;
+    for (const Out& o : out) {
+      const Error e = Driver::Free(o.ptr);
+      if (e == Driver::kOk) continue;
+      if (first == Driver::kOk) first = e;
+      std::lock_guard<std::mutex> lock(mu_);
+      Keep(o);
+    }
+    return first;
   }
 
   // The driver's allocation; the kept blocks may be what is missing. An address
@@ -183,7 +243,7 @@ class BlockPool {
       Driver::ClearError();
       int device = 0;
       e = Driver::Device(&device);
-      if (e == Driver::kOk) e = Trim(device, true);
+      if (e == Driver::kOk) e = Trim(device, 0);
       if (e == Driver::kOk) e = Driver::Malloc(ptr, bytes);
     }
     if (e != Driver::kOk) {
@@ -207,6 +267,7 @@ class BlockPool {
   std::mutex mu_;
   std::unordered_map<void*, Block> blocks_;
   std::map<int, Shelf> shelves_;  // per device
+  std::atomic<int64_t> due_{kNever};  // when the first kept block has lain too long
 };
 
 }  // namespace ps

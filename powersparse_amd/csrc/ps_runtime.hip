@@ -197,6 +197,7 @@ int ps_driver_version(int* version) {
 
 int ps_device_synchronize(void) {
   PS_HIP(hipDeviceSynchronize());
+  ps::pool().GiveBackIdle();
   return PS_OK;
 }
 
@@ -247,10 +248,20 @@ int ps_free(void* ptr) {
   return PS_OK;
 }
 
-int ps_mem_trim(void) {
+int ps_mem_trim(void) { return ps_mem_trim_to(0); }
+
+int ps_mem_trim_to(size_t bytes) {
   int device = 0;
   PS_HIP(hipGetDevice(&device));
-  PS_HIP(ps::pool().Trim(device, true));
+  PS_HIP(ps::pool().Trim(device, bytes));
+  return PS_OK;
+}
+
+int ps_mem_kept(size_t* bytes) {
+  PS_CHECK_ARG(bytes, "ps_mem_kept: null output");
+  int device = 0;
+  PS_HIP(hipGetDevice(&device));
+  *bytes = ps::pool().KeptBytes(device);
   return PS_OK;
 }
 

@@ -199,6 +199,26 @@ constexpr int kDeviceCheckNonzeros = 1 << 24;
 
 const char* const kBadEntry = "Invalid CSR column index or sparse value";
 
+// What a build leaves behind in kept device blocks goes back to the driver as it
+// ends, down to what was kept when it began: a program that builds a matrix
+// and then runs operators holds no more than the matrix. Programs that build
+// and destroy one matrix after another begin with the last one's blocks kept,
+// so theirs stay. kBuildKept is kept in any case (the temporaries of some 10 M
+// nonzeros).
+constexpr size_t kBuildKept = size_t(256) << 20;
+struct KeptMark {
+  size_t bytes = 0;
+  KeptMark() {
+    if (ps_mem_kept(&bytes) != PS_OK || bytes < kBuildKept) bytes = kBuildKept;
+  }
+  ~KeptMark() {
+    size_t now = 0;
+    if (ps_mem_kept(&now) == PS_OK && now > bytes) (void)ps_mem_trim_to(bytes);
+  }
+  KeptMark(const KeptMark&) = delete;
+  KeptMark& operator=(const KeptMark&) = delete;
+};
+
 // The partition-independent stages of the preprocessing. Members are declared
 // so that the helper thread (sig_len) is joined before what it writes is
 // destroyed.
@@ -354,6 +374,7 @@ PowerSparseMatrixGPU::PowerSparseMatrixGPU(int row_num, int col_num, int nnz_num
     ThrowOnError(ps_get_device_props(dev, &props));
     _cu_count = props.cu_count;
   }
+  const KeptMark mark;
   try {
     Prepared in(row_num, col_num, nnz_num, row_ptr, col_ind, sp_data, timings);
     // A tuned SpMM partition may follow only in signature order (kAuto

@@ -105,7 +105,7 @@ int double_free() {
   CHECK(pool.Malloc(&b, 8 * MB) == kFine && b != p);
   CHECK(Fake::allocated.count(a) == 1);
   CHECK(pool.Free(a) == kFine && pool.Free(b) == kFine);
-  CHECK(pool.Trim(0, true) == kFine && Fake::in_use == 0);
+  CHECK(pool.Trim(0, 0) == kFine && Fake::in_use == 0);
   CHECK(pool.Free(a) == kBadValue);  // given back: the driver's answer
   return 0;
 }
@@ -128,7 +128,125 @@ int freed_elsewhere() {
   CHECK(pool.Malloc(&q, 4 * MB) == kFine && q == p);
   CHECK(pool.KeptBytes(0) == 0);
   CHECK(pool.Free(q) == kFine && pool.KeptBytes(0) == 4 * MB);
-  CHECK(pool.Trim(0, true) == kFine && Fake::in_use == 0);
+  CHECK(pool.Trim(0, 0) == kFine && Fake::in_use == 0);
+  return 0;
+}
+
+// Blocks unused for ten seconds go back at the next call of any kind.
+int idle() {
+  for (int call = 0; call < 4; ++call) {
+    Pool pool;
+    void *small = nullptr, *live = nullptr, *a = nullptr, *b = nullptr, *p = nullptr;
+    CHECK(pool.Malloc(&small, 4096) == kFine && pool.Malloc(&live, 64 * MB) == kFine);
+    CHECK(pool.Malloc(&a, 8 * MB) == kFine && pool.Malloc(&b, 16 * MB) == kFine);
+    CHECK(pool.Free(a) == kFine);
+    Fake::now += Pool::kKeepNs / 2;
+    CHECK(pool.Free(b) == kFine && pool.KeptBytes(0) == 24 * MB);
+    Fake::now += Pool::kKeepNs / 2;  // the first is due, the second is not
+    const size_t in_use = Fake::in_use;
+    if (call == 0) pool.GiveBackIdle();
+    if (call == 1) CHECK(pool.Malloc(&p, 64) == kFine);
+    if (call == 2) CHECK(pool.Free(small) == kFine);
+    if (call == 3) CHECK(pool.Free(live) == kFine && pool.Trim(0, 16 * MB) == kFine);
+    CHECK(Fake::allocated.count(a) == 0);
+    if (call == 3) continue;  // (the freed 64 MB are the newest)
+    CHECK(pool.KeptBytes(0) == 16 * MB && Fake::in_use <= in_use - 8 * MB + 64);
+    Fake::now += Pool::kKeepNs;
+    pool.GiveBackIdle();
+    CHECK(pool.KeptBytes(0) == 0);
+  }
+  return 0;
+}
+
+// A kept block that fits is used, however long it has lain.
+int idle_reuse() {
+  Pool pool;
+  void *a = nullptr, *p = nullptr;
+  CHECK(pool.Malloc(&a, 8 * MB) == kFine && pool.Free(a) == kFine);
+  Fake::now += 3 * Pool::kKeepNs;
+  CHECK(pool.Malloc(&p, 8 * MB) == kFine && p == a && Fake::mallocs == 1);
+  return 0;
+}
+
+// What the driver refuses to free stays kept, and goes later.
+int refused() {
+  Pool pool;
+  void *a = nullptr, *b = nullptr, *p = nullptr;
+  CHECK(pool.Malloc(&a, 8 * MB) == kFine && pool.Malloc(&b, 8 * MB) == kFine);
+  CHECK(pool.Free(a) == kFine && pool.Free(b) == kFine);
+  Fake::refuse_free = true;
+  Fake::now += 2 * Pool::kKeepNs;
+  pool.GiveBackIdle();
+  CHECK(pool.KeptBytes(0) == 16 * MB);
+  CHECK(pool.Trim(0, 0) == kBadValue && pool.KeptBytes(0) == 16 * MB);
+  Fake::refuse_free = false;
+  CHECK(pool.Malloc(&p, 8 * MB) == kFine && (p == a || p == b));
+  Fake::now += 2 * Pool::kKeepNs;
+  pool.GiveBackIdle();
+  CHECK(pool.KeptBytes(0) == 0 && Fake::in_use == 8 * MB);
+  return 0;
+}
+
+// Trimming to a size: the oldest go first. The bound of a sixteenth likewise.
+int trim_to() {
+  Pool pool;
+  void* p[40];
+  for (void*& q : p) CHECK(pool.Malloc(&q, 2 * MB) == kFine);
+  for (void* q : p) {
+    ++Fake::now;
+    CHECK(pool.Free(q) == kFine);
+  }
+  CHECK(pool.KeptBytes(0) == 64 * MB);
+  for (int k = 0; k < 40; ++k) CHECK(Fake::allocated.count(p[k]) == (k < 8 ? 0u : 1u));
+  CHECK(pool.Trim(0, 11 * MB) == kFine && pool.KeptBytes(0) == 10 * MB);
+  for (int k = 0; k < 40; ++k) CHECK(Fake::allocated.count(p[k]) == (k < 35 ? 0u : 1u));
+  CHECK(pool.Trim(0, 11 * MB) == kFine && pool.KeptBytes(0) == 10 * MB);
+  return 0;
+}
+
+// Threads that allocate, hold and free while another trims: a block belongs to
+// one thread at a time, and nothing is lost.
+int threads() {
+  Pool pool;
+  std::mutex mu;
+  std::map<void*, int> owner;
+  std::atomic<bool> wrong{false};
+  auto work = [&](int t) {
+    unsigned x = unsigned(t) * 2654435761u + 1u;
+    std::vector<void*> mine;
+    for (int k = 0; k < 3000; ++k) {
+      x = x * 1664525u + 1013904223u;
+      if (mine.size() < 4 && (x >> 16) % 2) {
+        void* p = nullptr;
+        if (pool.Malloc(&p, 4096 + (x >> 8) % (6 * MB)) != kFine) continue;
+        std::lock_guard<std::mutex> lock(mu);
+        if (!owner.emplace(p, t).second) wrong = true;
+        mine.push_back(p);
+      } else if (!mine.empty()) {
+        void* const p = mine.back();
+        mine.pop_back();
+        {
+          std::lock_guard<std::mutex> lock(mu);
+          owner.erase(p);
+        }
+        if (pool.Free(p) != kFine) wrong = true;
+      }
+      if (t == 0 && k % 16 == 0) (void)pool.Trim(0, 8 * MB);
+      if (t == 1) Fake::now += Pool::kKeepNs / 64;
+    }
+    for (void* p : mine) {
+      {
+        std::lock_guard<std::mutex> lock(mu);
+        owner.erase(p);
+      }
+      if (pool.Free(p) != kFine) wrong = true;
+    }
+  };
+  std::vector<std::thread> all;
+  for (int t = 0; t < 6; ++t) all.emplace_back(work, t);
+  for (std::thread& t : all) t.join();
+  CHECK(!wrong);
+  CHECK(pool.Trim(0, 0) == kFine && pool.KeptBytes(0) == 0 && Fake::in_use == 0);
   return 0;
 }
 
@@ -136,8 +254,14 @@ struct Check {
   const char* name;
   int (*run)();
 };
-const Check kChecks[] = {{"huge", huge}, {"double_free", double_free},
-                         {"freed_elsewhere", freed_elsewhere}};
+const Check kChecks[] = {{"huge", huge},
+                         {"double_free", double_free},
+                         {"freed_elsewhere", freed_elsewhere},
+                         {"idle", idle},
+                         {"idle_reuse", idle_reuse},
+                         {"refused", refused},
+                         {"trim_to", trim_to},
+                         {"threads", threads}};
 
 }  // namespace
 

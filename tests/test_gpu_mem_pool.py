@@ -1,6 +1,7 @@
 """Device blocks kept between ps_free and ps_malloc: reuse, the size rule, and
 giving them back."""
 import ctypes
+import time
 from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
@@ -119,3 +120,43 @@ def test_second_free_is_refused():
     for k, d in enumerate((b, c)):
         assert (d.download(np.uint32, 2 * MB) == k).all()
         d.free()
+
+
+def kept_bytes():
+    n = ctypes.c_size_t()
+    assert _native.hip().ps_mem_kept(ctypes.byref(n)) == _native.PS_OK
+    return n.value
+
+
+def test_a_build_leaves_little():
+    # one matrix built: its temporaries go back to the driver as the build ends,
+    # with no later call; matrices built one after another keep theirs
+    setup()
+    _native.hip().ps_mem_trim()
+    csr = ps.synth("C1", seed=3)
+    free0 = raw_free_bytes()
+    m = ps.PowerSparseMatrixGPU.from_csr(csr)
+    say(f"first build: kept {kept_bytes() >> 20} MB, in use {free0 - raw_free_bytes() >> 20} MB")
+    assert kept_bytes() <= 256 * MB
+    m.close()
+    own = kept_bytes()  # the destroyed matrix's blocks
+    seen = []
+    for _ in range(4):
+        m = ps.PowerSparseMatrixGPU.from_csr(csr)
+        seen.append((kept_bytes() >> 20, free0 - raw_free_bytes() >> 20))
+        m.close()
+    say(f"then kept / in use (MB): {seen}")
+    assert own > 256 * MB and seen[-1] == seen[-2]  # nothing allocated, nothing given back
+    _native.hip().ps_mem_trim()
+    assert raw_free_bytes() >= free0 - 96 * MB  # (staging, code and the runtime's own)
+
+
+def test_idle_blocks_go_back():
+    setup()
+    _native.hip().ps_mem_trim()
+    free0 = raw_free_bytes()
+    ps.DeviceBuffer(512 * MB).free()
+    assert raw_free_bytes() <= free0 - 500 * MB
+    time.sleep(10.5)
+    ps.synchronize()
+    assert kept_bytes() == 0 and raw_free_bytes() >= free0 - 4 * MB
