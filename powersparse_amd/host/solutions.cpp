@@ -13,6 +13,7 @@
 
 #include "PowerSparse_SDDMM.h"
 #include "PowerSparse_SpMM.h"
+#include "stream_join.h"
 
 namespace PowerSparse {
 namespace {
@@ -46,51 +47,6 @@ void CheckSddmmArgs(const PowerSparseMatrixGPU& m, int N, const float* lhs, cons
   ValidateDenseShape(m.MatrixRow(), m.MatrixCol(), N);
   if (!lhs || !rhs || !out) throw std::invalid_argument("Invalid SDDMM buffers or stream count");
 }
-
-// The reference runs workset s on streams[s] (spmm_solution.cu:18-26,
-// sddmm_solution.cu:24-26), so work a caller queued on streams[s] before the
-// call runs before that workset. Streams that have run everything queued on
-// them order nothing: when they all have, the fused launch goes to the null
-// stream, behind whatever the caller queued there (the outputs' clearing,
-// usually; ordering a created stream behind the null stream costs about 36 us
-// on MI355X: a 10 k-node SDDMM N = 32 after its clearing 66 -> 26 us a
-// call). Else it goes to streams[0], and every other stream with work left is
-// joined into it by an event, released after the dispatcher's device
-// synchronisation.
-class StreamJoin {
- public:
-  StreamJoin(int count, const ps_stream_t* streams) {
-    std::vector<ps_stream_t> busy;
-    for (int s = 0; s < count; ++s) {
-      int idle = 1;
-      if (streams[s] && (s == 0 || streams[s] != streams[0]))
-        ThrowOnError(ps_stream_idle(streams[s], &idle));
-      if (!idle) busy.push_back(streams[s]);
-    }
-    if (busy.empty()) return;
-    launch_ = streams[0];
-    for (ps_stream_t s : busy) {
-      if (s == launch_) continue;
-      ps_event_t e = nullptr;
-      ThrowOnError(ps_event_create(&e));
-      events_.push_back(e);
-      ThrowOnError(ps_event_record(e, s));
-      ThrowOnError(ps_stream_wait_event(launch_, e));
-    }
-  }
-  ~StreamJoin() {
-    for (ps_event_t e : events_) ps_event_destroy(e);
-  }
-  StreamJoin(const StreamJoin&) = delete;
-  StreamJoin& operator=(const StreamJoin&) = delete;
-
-  // The stream of the fused launch.
-  ps_stream_t Launch() const { return launch_; }
-
- private:
-  std::vector<ps_event_t> events_;
-  ps_stream_t launch_ = nullptr;
-};
 
 }  // namespace
 
