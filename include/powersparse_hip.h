@@ -502,7 +502,8 @@ int ps_pre_rank_keys(const int* row_ptr, int rows, const int* col_ind, int nnz,
  * ps_pre_rank_keys' output by key would (row << count_bits | max_count -
  * col_nnz[col], CSR position), sorting only inside rows (rows arrive in
  * order): one wave per row up to 256 nonzeros, an LDS radix sort per row up to
- * 8192, the same sort tile by tile for longer rows. count_bits <= 32.
+ * 8192, the same sort tile by tile for longer rows, the longest of them by one
+ * device-wide sort. count_bits <= 32.
  * keys may be NULL: only vals is written. Synchronises the stream.
  * Replaces: thrust::sort of NNZPoint (matrix_utils.cu:518-524). */
 int ps_pre_rank_sort(const int* row_ptr, int rows, const int* col_ind, int nnz,

@@ -8,6 +8,7 @@
 // Group membership follows utils/matrix_utils.cu: in a row's ranked order the
 // block groups come first, largest size first, and the residue takes the tail;
 // in fine mode (S == 1) the row is cut into chunks of `fine` nonzeros.
+#include <algorithm>
 #include <vector>
 
 #include "ps_block_sort.hpp"
@@ -221,7 +222,8 @@ __global__ void rank_keys_kernel(const int* __restrict__ row_ptr, int rows,
 // order. Rows of up to 256 nonzeros: one wave per row, each element's rank
 // counted against the others. 257 .. 8192: one workgroup per row, an LDS radix
 // sort (BlockSort; rows up to 2048 in quarter-size tiles). Longer rows: one
-// workgroup per row, the same sort tile by tile.
+// workgroup per row, the same sort tile by tile; the few that would hold the
+// others up (kRankWideMin) together by one radix sort over the device.
 // Output as the stable sort of (row, count key): keys (when asked for) = row <<
 // count_bits | count key, vals = CSR position.
 constexpr int kRankTileSmall = 256 * kSortItems, kRankTileLarge = 1024 * kSortItems;
@@ -334,14 +336,20 @@ __global__ void rank_lists_kernel(int rows, const uint32_t* __restrict__ flag,
   }
 }
 
-// long_start[i] = degree of long row list[i] (scanned into element offsets).
+// long_start[i] = degree of long row list[i] (scanned into element offsets),
+// long_start[n + 1] = the largest (cleared before).
 __global__ void permute_long_degrees_kernel(const uint32_t* __restrict__ list, uint32_t n,
                                             const int* __restrict__ row_ptr,
                                             uint32_t* __restrict__ long_start) {
+  uint32_t most = 0;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     const int r = int(list[i]);
-    long_start[i] = uint32_t(row_ptr[r + 1] - row_ptr[r]);
+    const uint32_t d = uint32_t(row_ptr[r + 1] - row_ptr[r]);
+    long_start[i] = d;
+    most = max(most, d);
   }
+  for (int s = 1; s < kWave; s <<= 1) most = max(most, uint32_t(__shfl_xor(int(most), s, kWave)));
+  if (lane_id() == 0 && most) atomicMax(&long_start[n + 1], most);
 }
 
 // Long rows, one workgroup per row: a stable radix sort over the row's tiles,
@@ -350,6 +358,13 @@ __global__ void permute_long_degrees_kernel(const uint32_t* __restrict__ list, u
 // first. Each tile is put in digit order in LDS, so that its elements leave as
 // runs, one per digit. The row's 8 to 16 bytes per element stay in the caches.
 constexpr int kRankLongThreads = 1024;
+// A row's workgroup takes about 7 ns per element, a device-wide sort 0.3 ms and
+// about 0.06 ns per element: rows longer than a 128th of all long rows' elements,
+// and than kRankWideMin, are sorted over the device (ms for n rows of L
+// elements, one workgroup each against over the device: 1 x 16384 0.25 / 0.31, 1
+// x 65536 0.42 / 0.31, 64 x 65536 0.46 / 0.46, 1 x 1 M 7.2 / 0.37, 64 x 1 M 8.2 / 3.4,
+// 256 x 262144 1.9 / 3.4, 1024 x 65536 2.1 / 4.1, 1 x 16 M 122 / 1.2).
+constexpr uint32_t kRankWideMin = 1 << 16, kRankWideShare = 128;
 __global__ __launch_bounds__(kRankLongThreads, 8) void rank_long_kernel(
     const uint32_t* __restrict__ list, const uint32_t* __restrict__ seg_start,
     const int* __restrict__ row_ptr, const int* __restrict__ col_ind,
@@ -447,6 +462,47 @@ __global__ __launch_bounds__(kRankLongThreads, 8) void rank_long_kernel(
   for (int e = t; e < d; e += kRankLongThreads) {
     if (keys) keys[b + e] = (uint64_t(r) << count_bits) | ks[e];
     vals[b + e] = uint32_t(b) + vs[e];
+  }
+}
+
+// The widest rows: keys (list index << count_bits | count key) and CSR
+// positions of all their elements, for one stable radix sort over the device.
+// start[0 .. n] = where each row's share begins.
+__global__ __launch_bounds__(kThreads) void rank_wide_keys_kernel(
+    const uint32_t* __restrict__ list, const uint32_t* __restrict__ start, uint32_t n,
+    const int* __restrict__ row_ptr, const int* __restrict__ col_ind,
+    const int* __restrict__ col_nnz, int max_count, int count_bits, uint64_t* __restrict__ ck,
+    uint32_t* __restrict__ cv) {
+  const uint32_t total = start[n];
+  for (size_t j = size_t(blockIdx.x) * kThreads + threadIdx.x; j < total;
+       j += size_t(gridDim.x) * kThreads) {
+    uint32_t lo = 0, hi = n;  // start[lo] <= j < start[hi]
+    while (hi - lo > 1) {
+      const uint32_t mid = lo + (hi - lo) / 2;
+      if (start[mid] <= j) lo = mid;
+      else hi = mid;
+    }
+    const int p = row_ptr[list[lo]] + int(uint32_t(j) - start[lo]);
+    ck[j] = (uint64_t(lo) << count_bits) | count_key(col_ind, col_nnz, max_count, p);
+    cv[j] = uint32_t(p);
+  }
+}
+
+// The sorted elements of row i occupy the same share as before the sort.
+__global__ __launch_bounds__(kThreads) void rank_wide_write_kernel(
+    const uint64_t* __restrict__ ck, const uint32_t* __restrict__ cv,
+    const uint32_t* __restrict__ list, const uint32_t* __restrict__ start, uint32_t n,
+    const int* __restrict__ row_ptr, int count_bits, uint64_t* __restrict__ keys,
+    uint32_t* __restrict__ vals) {
+  const uint32_t total = start[n];
+  const uint64_t mask = (uint64_t(1) << count_bits) - 1u;
+  for (size_t j = size_t(blockIdx.x) * kThreads + threadIdx.x; j < total;
+       j += size_t(gridDim.x) * kThreads) {
+    const uint32_t i = uint32_t(ck[j] >> count_bits);
+    const int r = int(list[i]);
+    const int at = row_ptr[r] + int(uint32_t(j) - start[i]);
+    if (keys) keys[at] = (uint64_t(r) << count_bits) | (ck[j] & mask);
+    vals[at] = cv[j];
   }
 }
 
@@ -1749,7 +1805,7 @@ int ps_pre_rank_sort(const int* row_ptr, int rows, const int* col_ind, int nnz,
   hipStream_t st = ps::to_hip(stream);
   const size_t R = size_t(rows);
   using S = ps::Scratch;
-  S ws(S::bytes(3 * R, 4) * 2 + S::bytes(R, 4) * 3 + S::bytes(R + 1, 4) +
+  S ws(S::bytes(3 * R, 4) * 2 + S::bytes(R, 4) * 3 + S::bytes(R + 2, 4) +
        ps_scan_workspace_bytes(R + 1));
   PS_HIP(ws.error());
   uint32_t* flag = ws.take<uint32_t>(3 * R);
@@ -1757,7 +1813,7 @@ int ps_pre_rank_sort(const int* row_ptr, int rows, const int* col_ind, int nnz,
   uint32_t* list1 = ws.take<uint32_t>(R);
   uint32_t* list2 = ws.take<uint32_t>(R);
   uint32_t* list3 = ws.take<uint32_t>(R);
-  uint32_t* long_start = ws.take<uint32_t>(R + 1);
+  uint32_t* long_start = ws.take<uint32_t>(R + 2);
   void* scan_ws = ws.take<char>(ps_scan_workspace_bytes(R + 1));
   // rows of up to 64 nonzeros
   {
@@ -1798,26 +1854,79 @@ int ps_pre_rank_sort(const int* row_ptr, int rows, const int* col_ind, int nnz,
   }
   if (n3 > 0) {
     // element offsets of the long rows, in list order
-    PS_HIP(hipMemsetAsync(long_start, 0, (R + 1) * 4, st));
+    PS_HIP(hipMemsetAsync(long_start, 0, (R + 2) * 4, st));
     ps::permute_long_degrees_kernel<<<ps::grid_for(n3), ps::kThreads, 0, st>>>(
         list3, n3, row_ptr, long_start);
     PS_LAUNCHED();
     rc = ps_exclusive_scan_u32(long_start, long_start, size_t(n3) + 1, scan_ws, stream);
     if (rc != PS_OK) return rc;
-    uint32_t total = 0;
-    PS_HIP(hipMemcpyAsync(&total, long_start + n3, 4, hipMemcpyDeviceToHost, st));
+    uint32_t tail[2] = {0, 0};  // elements, longest row
+    PS_HIP(hipMemcpyAsync(tail, long_start + n3, 8, hipMemcpyDeviceToHost, st));
     PS_HIP(hipStreamSynchronize(st));
-    S lw(4 * S::bytes(total, 4));
-    PS_HIP(lw.error());
-    uint32_t* key_a = lw.take<uint32_t>(total);
-    uint32_t* key_b = lw.take<uint32_t>(total);
-    uint32_t* val_a = lw.take<uint32_t>(total);
-    uint32_t* val_b = lw.take<uint32_t>(total);
-    ps::rank_long_kernel<<<n3, ps::kRankLongThreads, 0, st>>>(
-        list3, long_start, row_ptr, col_ind, col_nnz, max_count, count_bits, key_a, key_b, val_a,
-        val_b, keys, vals);
-    PS_LAUNCHED();
-    PS_HIP(hipStreamSynchronize(st));
+    uint32_t rows_here = n3, here = tail[0], wide = 0;
+    const uint32_t most = std::max(ps::kRankWideMin, here / ps::kRankWideShare);
+    if (tail[1] > most) {
+      // the widest rows go to the end of the list, with starts of their own
+      std::vector<uint32_t> list(n3), start(size_t(n3) + 1), rest, rest_start;
+      PS_HIP(hipMemcpyAsync(list.data(), list3, size_t(n3) * 4, hipMemcpyDeviceToHost, st));
+      PS_HIP(hipMemcpyAsync(start.data(), long_start, start.size() * 4, hipMemcpyDeviceToHost, st));
+      PS_HIP(hipStreamSynchronize(st));
+      rows_here = here = 0;
+      std::vector<uint32_t> lists, starts;
+      for (uint32_t i = 0; i < n3; ++i) {
+        const uint32_t d = start[i + 1] - start[i];
+        const bool w = d > most;
+        (w ? rest : lists).push_back(list[i]);
+        (w ? rest_start : starts).push_back(w ? wide : here);
+        (w ? wide : here) += d;
+      }
+      rows_here = uint32_t(lists.size());
+      starts.push_back(here);
+      rest_start.push_back(wide);
+      lists.insert(lists.end(), rest.begin(), rest.end());
+      starts.insert(starts.end(), rest_start.begin(), rest_start.end());
+      PS_HIP(hipMemcpyAsync(list3, lists.data(), lists.size() * 4, hipMemcpyHostToDevice, st));
+      PS_HIP(hipMemcpyAsync(long_start, starts.data(), starts.size() * 4, hipMemcpyHostToDevice, st));
+      PS_HIP(hipStreamSynchronize(st));
+    }
+    if (rows_here > 0) {
+      S lw(4 * S::bytes(here, 4));
+      PS_HIP(lw.error());
+      uint32_t* key_a = lw.take<uint32_t>(here);
+      uint32_t* key_b = lw.take<uint32_t>(here);
+      uint32_t* val_a = lw.take<uint32_t>(here);
+      uint32_t* val_b = lw.take<uint32_t>(here);
+      ps::rank_long_kernel<<<rows_here, ps::kRankLongThreads, 0, st>>>(
+          list3, long_start, row_ptr, col_ind, col_nnz, max_count, count_bits, key_a, key_b, val_a,
+          val_b, keys, vals);
+      PS_LAUNCHED();
+      PS_HIP(hipStreamSynchronize(st));
+    }
+    if (wide > 0) {
+      const uint32_t n = n3 - rows_here;
+      const uint32_t* const list = list3 + rows_here;
+      const uint32_t* const start = long_start + rows_here + 1;
+      S lw(2 * S::bytes(wide, 8) + 2 * S::bytes(wide, 4) + ps_radix_workspace_bytes(wide));
+      PS_HIP(lw.error());
+      uint64_t* ck = lw.take<uint64_t>(wide);
+      uint64_t* ck_alt = lw.take<uint64_t>(wide);
+      uint32_t* cv = lw.take<uint32_t>(wide);
+      uint32_t* cv_alt = lw.take<uint32_t>(wide);
+      void* radix_ws = lw.take<char>(ps_radix_workspace_bytes(wide));
+      const unsigned grid = ps::grid_for(wide);
+      ps::rank_wide_keys_kernel<<<grid, ps::kThreads, 0, st>>>(
+          list, start, n, row_ptr, col_ind, col_nnz, max_count, count_bits, ck, cv);
+      PS_LAUNCHED();
+      int alt = 0;  // (fewer than kRankWideShare rows)
+      rc = ps_radix_sort_pairs_u64(ck, ck_alt, cv, cv_alt, wide, 0,
+                                   count_bits + ps::bits_for(uint64_t(n - 1)), radix_ws, &alt,
+                                   stream);
+      if (rc != PS_OK) return rc;
+      ps::rank_wide_write_kernel<<<grid, ps::kThreads, 0, st>>>(
+          alt ? ck_alt : ck, alt ? cv_alt : cv, list, start, n, row_ptr, count_bits, keys, vals);
+      PS_LAUNCHED();
+      PS_HIP(hipStreamSynchronize(st));
+    }
   }
   PS_HIP(hipStreamSynchronize(st));
   return PS_OK;

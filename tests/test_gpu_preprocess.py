@@ -233,6 +233,53 @@ def test_rank_sort_row_classes():
     np.testing.assert_array_equal(keys.download(np.uint64), exp_keys)
 
 
+def _wide_degrees(kind):
+    if kind == "edges":  # few long elements: rows beyond 65536 are wide
+        return [50, 65535, 8193, 65536, 65537, 0, 200000, 9000, 300]
+    if kind == "alone":  # no long row left for the workgroups
+        return [300000]
+    # many: a 128th of the long elements is the line, above 65536
+    base = [66000] * 140
+    x = 66000
+    for _ in range(20):
+        x = (sum(base) + 2 * x + 1) // 128
+    assert x == (sum(base) + 2 * x + 1) // 128 and x > 66000
+    return base[:60] + [x + 1] + base[60:] + [x, 40]
+
+
+@pytest.mark.parametrize("kind", ["edges", "alone", "share"])
+@pytest.mark.parametrize("with_keys", [True, False])
+def test_rank_sort_wide_rows(kind, with_keys):
+    # rows on both sides of the line from which they are sorted over the device,
+    # against numpy's stable sort; few distinct column counts, so most keys tie
+    from powersparse_amd import _native
+    setup()
+    rng = np.random.default_rng(29)
+    degrees = _wide_degrees(kind)
+    cols = 1 << 18
+    rp = np.concatenate([[0], np.cumsum(degrees)]).astype(np.int32)
+    rows, nnz = len(degrees), int(rp[-1])
+    ci = rng.integers(0, cols, nnz).astype(np.int32)
+    cn = np.where(rng.random(cols) < 0.01, rng.integers(0, 70000, cols),
+                  rng.integers(1, 6, cols)).astype(np.int32)
+    max_count = int(cn.max())
+    cb = max_count.bit_length()
+    say(f"wide rows {kind}: {nnz} nonzeros, longest {max(degrees)}")
+    ckey = (max_count - cn[ci]).astype(np.uint64)
+    order = np.concatenate([b + np.argsort(ckey[b:e], kind="stable")
+                            for b, e in zip(rp[:-1], rp[1:])])
+    row_of = np.repeat(np.arange(rows), np.diff(rp)).astype(np.uint64)
+    d_rp, d_ci, d_cn = (ps.DeviceBuffer(host=a) for a in (rp, ci, cn))
+    vals = ps.DeviceBuffer(host=np.full(nnz, 0xFFFFFFFF, np.uint32))
+    keys = ps.DeviceBuffer(nnz * 8) if with_keys else None
+    ps._hip_call(_native.hip().ps_pre_rank_sort(d_rp.ptr, rows, d_ci.ptr, nnz, d_cn.ptr, max_count,
+                                                cb, keys.ptr if keys else None, vals.ptr, None))
+    np.testing.assert_array_equal(vals.download(np.uint32), order.astype(np.uint32))
+    if keys:
+        np.testing.assert_array_equal(keys.download(np.uint64),
+                                      (row_of << np.uint64(cb)) | ckey[order])
+
+
 def _snapshot(m):
     """Every public array of a matrix, on the host."""
     ws = [m.download_workset(s) if m.GroupNum()[s] else None for s in range(m.GroupTypeNum())]
