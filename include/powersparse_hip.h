@@ -291,6 +291,18 @@ int ps_sddmm_scatter_launch(int workset_count, const ps_workset* worksets,
                             const int* residue_offset, const int* const* out_base, int rows,
                             int cols, int N, const float* lhs, const float* rhs,
                             float* const* out, int task_chunk, ps_stream_t stream);
+/* Any of the three (out_base NULL: the public positions; task_order NULL: the
+ * stored order), with a bound on the values' magnitude, 0 when none is known.
+ * Beyond N = 128 large launches run in feature slices; with values of at most 1
+ * the residue results are then added slice by slice, else each is computed
+ * whole, since a value times one slice's sum could overflow where the value
+ * times the dot does not (C1, N = 256 / 512: 4.47 / 9.00 against 4.63 / 9.53
+ * ms). No reference counterpart. */
+int ps_sddmm_launch_values(int workset_count, const ps_workset* worksets,
+                           const int* residue_offset, const int* const* out_base, int rows,
+                           int cols, int N, const float* lhs, const float* rhs,
+                           float* const* out, int task_chunk, const uint32_t* task_order,
+                           uint32_t task_count, float max_value, ps_stream_t stream);
 
 /* out_csr[csr_pos[s][p]] = in[s][p] for p < lengths[s]: moves per-nonzero values
  * from workset order (e.g. the outputs of ps_sddmm_launch) to CSR order.
@@ -479,7 +491,8 @@ int ps_pre_degree_sums(const int* row_ptr, int rows, unsigned long long* sums_ho
 
 /* *bad = 1 when a column id lies outside [0, cols) (col_ind given) or a value
  * is not finite (values given; n of either), else 0. `flag`: 4 bytes of
- * scratch. Synchronises the stream.
+ * scratch; afterwards its bit 1 says whether a value's magnitude is above 1.
+ * Synchronises the stream.
  * Replaces: the host loop over the nonzeros (matrix_utils.cu:484-488). */
 int ps_pre_check_csr(const int* col_ind, const float* values, int n, int cols, uint32_t* flag,
                      int* bad, ps_stream_t stream);

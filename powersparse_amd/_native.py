@@ -209,6 +209,10 @@ HIP_API = [
      [ctypes.c_int, ctypes.POINTER(Workset), c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int,
       c_void_p, c_void_p, ctypes.POINTER(c_void_p), ctypes.c_int, c_void_p, ctypes.c_uint32,
       c_void_p]),
+    ("ps_sddmm_launch_values", ctypes.c_int,
+     [ctypes.c_int, ctypes.POINTER(Workset), c_void_p, ctypes.POINTER(c_void_p), ctypes.c_int,
+      ctypes.c_int, ctypes.c_int, c_void_p, c_void_p, ctypes.POINTER(c_void_p), ctypes.c_int,
+      c_void_p, ctypes.c_uint32, ctypes.c_float, c_void_p]),
     ("ps_sddmm_csr_launch_ordered", ctypes.c_int,
      [ctypes.c_int, ctypes.POINTER(Workset), c_void_p, ctypes.POINTER(c_void_p), ctypes.c_int,
       ctypes.c_int, ctypes.c_int, c_void_p, c_void_p, c_void_p, ctypes.c_int, c_void_p,

@@ -39,19 +39,24 @@ __global__ void degree_sums_kernel(const int* __restrict__ row_ptr, int rows,
 }
 
 // *flag |= 1 for a column outside [0, cols) or a value with all exponent bits
-// set. Bound by reading the arrays: 1.06 GB each on C3, 0.25 ms; the host's loop
+// set, |= 2 for a value of magnitude above 1. Bound by reading the arrays: 1.06 GB each on C3, 0.25 ms; the host's loop
 // over both took 8 to 10 ms there.
 __global__ __launch_bounds__(kThreads) void check_csr_kernel(const int* __restrict__ col_ind,
                                                              const float* __restrict__ values,
                                                              size_t n, int cols,
                                                              uint32_t* __restrict__ flag) {
-  bool bad = false;
+  bool bad = false, large = false;
   for (size_t i = size_t(blockIdx.x) * kThreads + threadIdx.x; i < n;
        i += size_t(gridDim.x) * kThreads) {
     if (col_ind) bad |= uint32_t(col_ind[i]) >= uint32_t(cols);
-    if (values) bad |= (__float_as_uint(values[i]) & 0x7F800000u) == 0x7F800000u;
+    if (values) {
+      const uint32_t mag = __float_as_uint(values[i]) & 0x7FFFFFFFu;
+      bad |= mag >= 0x7F800000u;
+      large |= mag > 0x3F800000u;
+    }
   }
-  if (__any(bad) && lane_id() == 0) atomicOr(flag, 1u);
+  const uint32_t found = (__any(bad) ? 1u : 0u) | (__any(large) ? 2u : 0u);
+  if (found && lane_id() == 0) atomicOr(flag, found);
 }
 
 // Column histogram, up to kSplitCols columns. Counting by global atomics costs
@@ -1735,7 +1740,7 @@ int ps_pre_check_csr(const int* col_ind, const float* values, int n, int cols, u
   PS_LAUNCHED();
   PS_HIP(hipMemcpyAsync(&found, flag, sizeof(found), hipMemcpyDeviceToHost, st));
   PS_HIP(hipStreamSynchronize(st));
-  *bad = found != 0;
+  *bad = int(found & 1u);
   return PS_OK;
 }
 

@@ -28,8 +28,16 @@
 // signature-ordered worksets. A task's work, and so every output, is the same
 // in any order; residue tasks keep their 8 consecutive groups.
 //
-// Wide features run as slices, one launch after another: the first stores
-// a_p * <its features>, the others add theirs (kSliceWide / kSliceNarrow).
+// Wide features run as slices, one launch after another (kSliceWide /
+// kSliceNarrow): all but the last leave the dot's sum so far in the output, the
+// last multiplies by a_p, as one launch does (a product per slice could overflow
+// where a_p times the whole dot does not). An output that results are added to
+// (the residue's, in workset order) has no room for a sum so far: where all
+// values are known to be at most 1, each slice adds its product, which is then no
+// larger than its sum; else the last slice computes the residue's dots whole (C1
+// N = 256 / 512 4472 / 9002 -> 4628 / 9532 us; in a launch of its own measured
+// 4807 / 9733; a sum per slice decided value by value in one kernel 4544 / 9150,
+// its registers costing the values at most 1 too).
 //
 // Store modes (kMode): 0 = at the nonzero's own position (as above); 1 = per
 // nonzero map, out[s][map[s][p]]: CSR order (every out[s] is the one
@@ -76,7 +84,12 @@ struct SddmmArgs {
   uint32_t task_begin[PS_MAX_WORKSETS + 1];
   int32_t count;
   uint32_t row_bytes;     // bytes from one X / Y row to the next
-  int32_t accumulate;     // add to the outputs stored by an earlier feature slice
+  int32_t earlier;        // the output holds the sum over earlier feature slices
+  int32_t later;          // more slices follow: leave the sum there
+  int32_t N;              // of all slices, which the added-to residue is computed over
+  const float* lhs_all;   // the operands' first features
+  const float* rhs_all;
+  uint64_t lhs_all_bytes, rhs_all_bytes;
   uint32_t total_tasks;   // tasks of the worksets
   uint32_t launch_tasks;  // waves with work: total_tasks, or the task map's length
   const int* residue_offset;
@@ -98,9 +111,11 @@ struct SddmmArgs {
 // instead of 8 and no row offsets (the same sums, bit for bit; with one pair
 // per batch the K = 128 kernel took 69 VGPRs instead of 79 and ran C3 SDDMM
 // N=128 in 6.26 instead of 6.29 ms).
-template <int KQ, bool kBuf, typename ColOf>
+// kSkip: without the first `skip` of the KQ pieces (uniform; x holds 0 there).
+template <int KQ, bool kBuf, bool kSkip = false, typename ColOf>
 __device__ __forceinline__ float slot_dot(const Rows<kBuf>& Y, uint32_t row_bytes, uint32_t piece,
-                                          const float4 (&x)[KQ], int sub, ColOf col_of) {
+                                          const float4 (&x)[KQ], int sub, ColOf col_of,
+                                          int skip = 0) {
   using Off = typename Rows<kBuf>::Off;
   // pairs per batch: 8 KQ loads in flight up to K = 64, 16 at K = 128
   // (C3 SDDMM N=128 6.234 -> 6.195 ms, C1 2.250 -> 2.230 ms against 8
@@ -119,6 +134,10 @@ __device__ __forceinline__ float slot_dot(const Rows<kBuf>& Y, uint32_t row_byte
       const Off o1 = Off(uint32_t(col_of(i0 + u + 4))) * row_bytes + piece;
 #pragma unroll
       for (int k = 0; k < KQ; ++k) {
+        if (kSkip && k < skip) {
+          y[u][0][k] = y[u][1][k] = float4{0.f, 0.f, 0.f, 0.f};
+          continue;
+        }
         y[u][0][k] = Y.load(o0 + 128u * uint32_t(k));
         y[u][1][k] = Y.load(o1 + 128u * uint32_t(k));
       }
@@ -156,11 +175,13 @@ __device__ __forceinline__ float slot_dot(const Rows<kBuf>& Y, uint32_t row_byte
   return keep + xor_shfl<1>(send);
 }
 
-// kSliced: one of several feature slices (rows further apart than the slice is
-// wide; all but the first add to the outputs).
-template <int KQ, bool kBuf, int kMode, bool kSliced>
+// kSlices: 0 = one launch over all features; 1 = one of several feature slices
+// (rows further apart than the slice is wide); 2 = the same with the added-to
+// residue computed whole in the last one.
+template <int KQ, bool kBuf, int kMode, int kSlices>
 __global__ __launch_bounds__(kWave* kWavesPerBlock) void sddmm_kernel(SddmmArgs args) {
   constexpr int K = 32 * KQ;
+  constexpr bool kSliced = kSlices > 0, kWhole = kSlices == 2;
   __shared__ __attribute__((aligned(16))) int stage[kWavesPerBlock][8 * kStage];
   __shared__ float task_out[kWavesPerBlock][kTaskOut];  // residue results of a task
   // residue values staged with their columns (no dependent value load after
@@ -176,6 +197,9 @@ __global__ __launch_bounds__(kWave* kWavesPerBlock) void sddmm_kernel(SddmmArgs 
   int i = 0;
   while (i + 1 < args.count && task >= args.task_begin[i + 1]) ++i;
   const ps_workset ws = args.ws[i];
+  if constexpr (kWhole) {
+    if (ws.group_size == 0 && args.later) return;
+  }
   float* __restrict__ out = args.out[i];
   const int* __restrict__ out_pos = args.out_pos[i];
   const int local = int(task - args.task_begin[i]);
@@ -185,7 +209,7 @@ __global__ __launch_bounds__(kWave* kWavesPerBlock) void sddmm_kernel(SddmmArgs 
   const Rows<kBuf> X(args.lhs, args.lhs_bytes), Y(args.rhs, args.rhs_bytes);
   using Off = typename Rows<kBuf>::Off;
   const uint32_t row_bytes = kSliced ? args.row_bytes : uint32_t(K) * 4u;
-  const bool accumulate = kSliced && args.accumulate;
+  const bool earlier = kSliced && args.earlier, later = kSliced && args.later;
   const uint32_t piece = uint32_t(sub) * 16u;
   float4 x[KQ];
   int* const wave_stage = stage[threadIdx.x / kWave];
@@ -213,7 +237,7 @@ __global__ __launch_bounds__(kWave* kWavesPerBlock) void sddmm_kernel(SddmmArgs 
       const int gl = pos >> gs_shift;
       if (valid) dst = out_pos[gl] + (pos - gl * ws.group_size);
     }
-    const float before = valid && accumulate ? __builtin_nontemporal_load(out + dst) : 0.f;
+    const float before = valid && earlier ? __builtin_nontemporal_load(out + dst) : 0.f;
 #pragma unroll
     for (int q = 0; q < KQ; ++q) x[q] = X.load(Off(uint32_t(row)) * row_bytes + piece + 128u * q);
     wave_lds_sync();
@@ -224,8 +248,8 @@ __global__ __launch_bounds__(kWave* kWavesPerBlock) void sddmm_kernel(SddmmArgs 
       // every output is written once and not read back by the launch:
       // non-temporal stores keep them from displacing Y rows in the L2 (C3
       // SDDMM N=128 6.374 -> 6.348 ms)
-      __builtin_nontemporal_store(accumulate ? fmaf(dot, a_val, before) : dot * a_val,
-                                  out + dst);
+      const float sum = earlier ? before + dot : dot;
+      __builtin_nontemporal_store(later ? sum : sum * a_val, out + dst);
     }
   } else {
     // One slot per group (the run order's entry local * 8 + slot: order[]
@@ -258,48 +282,90 @@ __global__ __launch_bounds__(kWave* kWavesPerBlock) void sddmm_kernel(SddmmArgs 
     // order (the row's block tiles run long before): non-temporal (C3 SDDMM
     // N=128 6.271 -> 6.254 ms, C4 N=64 1.358 -> 1.348 ms; the block tiles' X
     // rows, shared by a hub row's tiles, measured 2% slower so)
+    if constexpr (!kWhole) {
 #pragma unroll
-    for (int qq = 0; qq < KQ; ++qq)
-      x[qq] = X.load_nt(Off(uint32_t(row)) * row_bytes + piece + 128u * qq);
+      for (int qq = 0; qq < KQ; ++qq)
+        x[qq] = X.load_nt(Off(uint32_t(row)) * row_bytes + piece + 128u * qq);
+    }
     // The group's columns and values pass through the slot's LDS area in
     // chunks of kStage (one chunk for every group the preprocessing builds),
     // positions past the group's end holding its last column (those
     // nonzeros' dots are dropped); the chunk boundaries are the same for the
     // whole wave (c0 is uniform).
+    // (outputs that are stored, not added to)
+    const auto put = [&](float* at, float dot, float a_val) {
+      const float sum = earlier ? *at + dot : dot;
+      *at = later ? sum : sum * a_val;
+    };
     int* const cols_lds = stage[threadIdx.x / kWave] + slot * kStage;
     float* const vals_lds = stage_val[threadIdx.x / kWave] + slot * kStage;
-#pragma unroll 1
-    for (int c0 = 0; __any(c0 < len); c0 += 8) {
-      const int cs = c0 % kStage;  // place of nonzero c0 in the staged chunk
-      if (cs == 0) {
-        if (c0 > 0) wave_lds_sync();  // the previous chunk's reads come first
-#pragma unroll
-        for (int j = sub; j < kStage; j += 8) {
-          const int k = c0 + j;
-          const int at = beg + (k < len ? k : len - 1);
-          cols_lds[j] = len > 0 ? ws.col_ind[at] : 0;
-          vals_lds[j] = len > 0 ? ws.sp_data[at] : 0.f;
-        }
-        wave_lds_sync();
+    const auto emit = [&](int k, float dot, float a_val) {
+      const float v = dot * a_val;
+      if constexpr (kMode == 2) {
+        if (group_collect) res_lds[slot * kStage + k] = v;
+        else if (args.residue_add) unsafeAtomicAdd(out + out_pos[g] + k, v);
+        else put(out + out_pos[g] + k, dot, a_val);
+      } else if constexpr (kMode == 1) {
+        const int at = out_pos[beg + k];
+        if (args.residue_add) unsafeAtomicAdd(out + at, v);
+        else put(out + at, dot, a_val);
+      } else if (collect) {
+        res_lds[beg + k - out0] = v;
+      } else {
+        unsafeAtomicAdd(out + beg + k, v);
       }
-      const float dot = slot_dot<KQ, kBuf>(Y, row_bytes, piece, x, sub,
-                                           [&](int j) { return cols_lds[cs + j]; });
-      const int k = c0 + sub;
-      if (k < len) {
-        const float v = dot * vals_lds[cs + sub];
-        if constexpr (kMode == 2) {
-          if (group_collect) res_lds[slot * kStage + k] = v;
-          else if (args.residue_add) unsafeAtomicAdd(out + out_pos[g] + k, v);
-          else out[out_pos[g] + k] = accumulate ? out[out_pos[g] + k] + v : v;
-        } else if constexpr (kMode == 1) {
-          const int at = out_pos[beg + k];
-          if (args.residue_add) unsafeAtomicAdd(out + at, v);
-          else out[at] = accumulate ? out[at] + v : v;
-        } else if (collect) {
-          res_lds[beg + k - out0] = v;
-        } else {
-          unsafeAtomicAdd(out + beg + k, v);
+    };
+    const auto stage_chunk = [&](int c0) {
+      if (c0 > 0) wave_lds_sync();  // the previous chunk's reads come first
+#pragma unroll
+      for (int j = sub; j < kStage; j += 8) {
+        const int k = c0 + j;
+        const int at = beg + (k < len ? k : len - 1);
+        cols_lds[j] = len > 0 ? ws.col_ind[at] : 0;
+        vals_lds[j] = len > 0 ? ws.sp_data[at] : 0.f;
+      }
+      wave_lds_sync();
+    };
+    if constexpr (kWhole) {
+      const Rows<kBuf> Xall(args.lhs_all, args.lhs_all_bytes);
+      const Rows<kBuf> Yall(args.rhs_all, args.rhs_all_bytes);
+      // the whole dots, window by window of the slice's width (the last one
+      // without what it shares with the one before); a staged chunk's sums stay
+      // in registers
+#pragma unroll 1
+      for (int c0 = 0; __any(c0 < len); c0 += kStage) {
+        stage_chunk(c0);
+        float sum[kStage / 8] = {};
+#pragma unroll 1
+        for (int f0 = 0; f0 < args.N; f0 += K) {
+          const int skip = f0 + K <= args.N ? 0 : (f0 + K - args.N) / 32;
+          const uint32_t at = piece + uint32_t(f0 - 32 * skip) * 4u;
+#pragma unroll
+          for (int qq = 0; qq < KQ; ++qq) {
+            x[qq] = float4{0.f, 0.f, 0.f, 0.f};
+            if (qq >= skip) x[qq] = Xall.load_nt(Off(uint32_t(row)) * row_bytes + at + 128u * qq);
+          }
+#pragma unroll
+          for (int t = 0; t < kStage / 8; ++t)
+            if (__any(c0 + 8 * t < len))
+              sum[t] += slot_dot<KQ, kBuf, true>(Yall, row_bytes, at, x, sub,
+                                                 [&](int j) { return cols_lds[8 * t + j]; }, skip);
         }
+#pragma unroll
+        for (int t = 0; t < kStage / 8; ++t) {
+          const int k = c0 + 8 * t + sub;
+          if (k < len) emit(k, sum[t], vals_lds[8 * t + sub]);
+        }
+      }
+    } else {
+#pragma unroll 1
+      for (int c0 = 0; __any(c0 < len); c0 += 8) {
+        const int cs = c0 % kStage;  // place of nonzero c0 in the staged chunk
+        if (cs == 0) stage_chunk(c0);
+        const float dot = slot_dot<KQ, kBuf>(Y, row_bytes, piece, x, sub,
+                                             [&](int j) { return cols_lds[cs + j]; });
+        const int k = c0 + sub;
+        if (k < len) emit(k, dot, vals_lds[cs + sub]);
       }
     }
     if constexpr (kMode == 2) {
@@ -335,42 +401,48 @@ __global__ void to_csr_kernel(const float* __restrict__ in, const int* __restric
     out[pos[e]] = in[e];
 }
 
-template <int KQ, bool kSliced>
+template <int KQ, int kSlices>
 void launch_mode(const SddmmArgs& a, bool buf, int mode, unsigned grid, hipStream_t stream) {
   constexpr unsigned kBlock = kWave * kWavesPerBlock;
-  if (mode == 1) {
-    if (buf) sddmm_kernel<KQ, true, 1, kSliced><<<grid, kBlock, 0, stream>>>(a);
-    else sddmm_kernel<KQ, false, 1, kSliced><<<grid, kBlock, 0, stream>>>(a);
+  if (mode == 1) {  // (every output stored)
+    constexpr int kStored = kSlices > 0 ? 1 : 0;
+    if (buf) sddmm_kernel<KQ, true, 1, kStored><<<grid, kBlock, 0, stream>>>(a);
+    else sddmm_kernel<KQ, false, 1, kStored><<<grid, kBlock, 0, stream>>>(a);
   } else if (mode == 2) {
-    if (buf) sddmm_kernel<KQ, true, 2, kSliced><<<grid, kBlock, 0, stream>>>(a);
-    else sddmm_kernel<KQ, false, 2, kSliced><<<grid, kBlock, 0, stream>>>(a);
+    if (buf) sddmm_kernel<KQ, true, 2, kSlices><<<grid, kBlock, 0, stream>>>(a);
+    else sddmm_kernel<KQ, false, 2, kSlices><<<grid, kBlock, 0, stream>>>(a);
   } else {
-    if (buf) sddmm_kernel<KQ, true, 0, kSliced><<<grid, kBlock, 0, stream>>>(a);
-    else sddmm_kernel<KQ, false, 0, kSliced><<<grid, kBlock, 0, stream>>>(a);
+    if (buf) sddmm_kernel<KQ, true, 0, kSlices><<<grid, kBlock, 0, stream>>>(a);
+    else sddmm_kernel<KQ, false, 0, kSlices><<<grid, kBlock, 0, stream>>>(a);
   }
 }
 
 template <int KQ>
-void launch_kq(const SddmmArgs& a, bool sliced, bool buf, int mode, unsigned grid,
+void launch_kq(const SddmmArgs& a, int slices, bool buf, int mode, unsigned grid,
                hipStream_t stream) {
   // slices are 96 features wide at least (N > 128 in nearly equal parts), the
   // last one perhaps less, and kSliceCsr at most
   if constexpr (KQ <= kSliceCsr / 32) {
-    if (sliced) {
-      launch_mode<KQ, true>(a, buf, mode, grid, stream);
+    if (slices == 2) {
+      launch_mode<KQ, 2>(a, buf, mode, grid, stream);
+      return;
+    }
+    if (slices == 1) {
+      launch_mode<KQ, 1>(a, buf, mode, grid, stream);
       return;
     }
   }
-  launch_mode<KQ, false>(a, buf, mode, grid, stream);
+  launch_mode<KQ, 0>(a, buf, mode, grid, stream);
 }
 
 // Workset q writes outs[q] at its own positions (mode 0), through the
 // per-nonzero map out_pos[q] (mode 1) or after the per-group bases out_pos[q]
-// (mode 2); residue results are added when residue_add (modes 1-2).
+// (mode 2); residue results are added when residue_add (modes 1-2). max_value:
+// largest magnitude of the values, 0 when unknown.
 int launch(int count, const int* order, const ps_workset* worksets, float* const* outs,
            int mode, const int* const* out_pos, int residue_add, const int* residue_offset,
            int rows, int cols, int N, const float* lhs, const float* rhs, int task_chunk,
-           const uint32_t* task_map, uint32_t task_map_len, hipStream_t stream) {
+           const uint32_t* task_map, uint32_t task_map_len, float max_value, hipStream_t stream) {
   PS_CHECK_ARG(N > 0 && N % 32 == 0 && N <= 512,
                "SDDMM requires N to be a multiple of 32 between 32 and 512");
   PS_CHECK_ARG(int64_t(rows) * N <= INT32_MAX && int64_t(cols) * N <= INT32_MAX,
@@ -447,29 +519,36 @@ int launch(int count, const int* order, const ps_workset* worksets, float* const
                                                : kSliceWide;
   const int slices = (N + most - 1) / most;
   const int width = (N / 32 + slices - 1) / slices * 32;
+  const int sliced = slices == 1 ? 0 : max_value > 0.f && max_value <= 1.f ? 1 : 2;
+  a.N = N;
+  a.lhs_all = lhs;
+  a.rhs_all = rhs;
+  a.lhs_all_bytes = lhs_bytes;
+  a.rhs_all_bytes = rhs_bytes;
   for (int f0 = 0; f0 < N; f0 += width) {
     a.lhs = lhs + f0;
     a.rhs = rhs + f0;
     a.lhs_bytes = lhs_bytes - uint64_t(f0) * 4u;
     a.rhs_bytes = rhs_bytes - uint64_t(f0) * 4u;
-    a.accumulate = f0 > 0;
+    a.earlier = f0 > 0;
+    a.later = f0 + width < N;
     switch ((N - f0 < width ? N - f0 : width) / 32) {
-      case 1: launch_kq<1>(a, slices > 1, buf, mode, grid, stream); break;
-      case 2: launch_kq<2>(a, slices > 1, buf, mode, grid, stream); break;
-      case 3: launch_kq<3>(a, slices > 1, buf, mode, grid, stream); break;
-      case 4: launch_kq<4>(a, slices > 1, buf, mode, grid, stream); break;
-      case 5: launch_kq<5>(a, slices > 1, buf, mode, grid, stream); break;
-      case 6: launch_kq<6>(a, slices > 1, buf, mode, grid, stream); break;
-      case 7: launch_kq<7>(a, slices > 1, buf, mode, grid, stream); break;
-      case 8: launch_kq<8>(a, slices > 1, buf, mode, grid, stream); break;
-      case 9: launch_kq<9>(a, slices > 1, buf, mode, grid, stream); break;
-      case 10: launch_kq<10>(a, slices > 1, buf, mode, grid, stream); break;
-      case 11: launch_kq<11>(a, slices > 1, buf, mode, grid, stream); break;
-      case 12: launch_kq<12>(a, slices > 1, buf, mode, grid, stream); break;
-      case 13: launch_kq<13>(a, slices > 1, buf, mode, grid, stream); break;
-      case 14: launch_kq<14>(a, slices > 1, buf, mode, grid, stream); break;
-      case 15: launch_kq<15>(a, slices > 1, buf, mode, grid, stream); break;
-      default: launch_kq<16>(a, slices > 1, buf, mode, grid, stream); break;
+      case 1: launch_kq<1>(a, sliced, buf, mode, grid, stream); break;
+      case 2: launch_kq<2>(a, sliced, buf, mode, grid, stream); break;
+      case 3: launch_kq<3>(a, sliced, buf, mode, grid, stream); break;
+      case 4: launch_kq<4>(a, sliced, buf, mode, grid, stream); break;
+      case 5: launch_kq<5>(a, sliced, buf, mode, grid, stream); break;
+      case 6: launch_kq<6>(a, sliced, buf, mode, grid, stream); break;
+      case 7: launch_kq<7>(a, sliced, buf, mode, grid, stream); break;
+      case 8: launch_kq<8>(a, sliced, buf, mode, grid, stream); break;
+      case 9: launch_kq<9>(a, sliced, buf, mode, grid, stream); break;
+      case 10: launch_kq<10>(a, sliced, buf, mode, grid, stream); break;
+      case 11: launch_kq<11>(a, sliced, buf, mode, grid, stream); break;
+      case 12: launch_kq<12>(a, sliced, buf, mode, grid, stream); break;
+      case 13: launch_kq<13>(a, sliced, buf, mode, grid, stream); break;
+      case 14: launch_kq<14>(a, sliced, buf, mode, grid, stream); break;
+      case 15: launch_kq<15>(a, sliced, buf, mode, grid, stream); break;
+      default: launch_kq<16>(a, sliced, buf, mode, grid, stream); break;
     }
     PS_LAUNCHED();
   }
@@ -484,58 +563,47 @@ extern "C" {
 int ps_sddmm_launch(int workset_count, const ps_workset* worksets, const int* residue_offset,
                     int rows, int cols, int N, const float* lhs, const float* rhs,
                     float* const* out, int task_chunk, ps_stream_t stream) {
-  PS_CHECK_ARG(workset_count >= 1 && workset_count <= PS_MAX_WORKSETS && worksets && out,
-               "Invalid SDDMM workset count");
-  int order[PS_MAX_WORKSETS];
-  ps_workset ordered[PS_MAX_WORKSETS];
-  float* outs[PS_MAX_WORKSETS];
-  for (int q = 0; q < workset_count; ++q) {
-    order[q] = workset_count - 1 - q;
-    ordered[q] = worksets[workset_count - 1 - q];
-    outs[q] = out[workset_count - 1 - q];
-  }
-  return ps::launch(workset_count, order, ordered, outs, 0, nullptr, 0, residue_offset, rows,
-                    cols, N, lhs, rhs, task_chunk, nullptr, 0, ps::to_hip(stream));
+  return ps_sddmm_launch_values(workset_count, worksets, residue_offset, nullptr, rows, cols, N,
+                                lhs, rhs, out, task_chunk, nullptr, 0, 0.f, stream);
 }
 
 int ps_sddmm_launch_ordered(int workset_count, const ps_workset* worksets,
                             const int* residue_offset, int rows, int cols, int N,
                             const float* lhs, const float* rhs, float* const* out, int task_chunk,
                             const uint32_t* task_order, uint32_t task_count, ps_stream_t stream) {
-  PS_CHECK_ARG(workset_count >= 1 && workset_count <= PS_MAX_WORKSETS && worksets && out,
-               "Invalid SDDMM workset count");
-  int order[PS_MAX_WORKSETS];
-  ps_workset ordered[PS_MAX_WORKSETS];
-  float* outs[PS_MAX_WORKSETS];
-  for (int q = 0; q < workset_count; ++q) {
-    order[q] = workset_count - 1 - q;
-    ordered[q] = worksets[workset_count - 1 - q];
-    outs[q] = out[workset_count - 1 - q];
-  }
-  return ps::launch(workset_count, order, ordered, outs, 0, nullptr, 0, residue_offset, rows,
-                    cols, N, lhs, rhs, task_chunk, task_order, task_count,
-                    ps::to_hip(stream));
+  return ps_sddmm_launch_values(workset_count, worksets, residue_offset, nullptr, rows, cols, N,
+                                lhs, rhs, out, task_chunk, task_order, task_count, 0.f, stream);
 }
 
 int ps_sddmm_scatter_launch(int workset_count, const ps_workset* worksets,
                             const int* residue_offset, const int* const* out_base, int rows,
                             int cols, int N, const float* lhs, const float* rhs,
                             float* const* out, int task_chunk, ps_stream_t stream) {
-  PS_CHECK_ARG(workset_count >= 1 && workset_count <= PS_MAX_WORKSETS && worksets && out_base &&
-                   out,
+  PS_CHECK_ARG(out_base, "Invalid SDDMM workset count");
+  return ps_sddmm_launch_values(workset_count, worksets, residue_offset, out_base, rows, cols, N,
+                                lhs, rhs, out, task_chunk, nullptr, 0, 0.f, stream);
+}
+
+int ps_sddmm_launch_values(int workset_count, const ps_workset* worksets,
+                           const int* residue_offset, const int* const* out_base, int rows,
+                           int cols, int N, const float* lhs, const float* rhs,
+                           float* const* out, int task_chunk, const uint32_t* task_order,
+                           uint32_t task_count, float max_value, ps_stream_t stream) {
+  PS_CHECK_ARG(workset_count >= 1 && workset_count <= PS_MAX_WORKSETS && worksets && out,
                "Invalid SDDMM workset count");
   int order[PS_MAX_WORKSETS];
   ps_workset ordered[PS_MAX_WORKSETS];
-  const int* pos[PS_MAX_WORKSETS];
+  const int* pos[PS_MAX_WORKSETS] = {};
   float* outs[PS_MAX_WORKSETS];
   for (int q = 0; q < workset_count; ++q) {
     order[q] = workset_count - 1 - q;
     ordered[q] = worksets[workset_count - 1 - q];
-    pos[q] = out_base[workset_count - 1 - q];
+    if (out_base) pos[q] = out_base[workset_count - 1 - q];
     outs[q] = out[workset_count - 1 - q];
   }
-  return ps::launch(workset_count, order, ordered, outs, 2, pos, 1, residue_offset, rows, cols,
-                    N, lhs, rhs, task_chunk, nullptr, 0, ps::to_hip(stream));
+  return ps::launch(workset_count, order, ordered, outs, out_base ? 2 : 0, out_base ? pos : nullptr,
+                    out_base ? 1 : 0, residue_offset, rows, cols, N, lhs, rhs, task_chunk,
+                    task_order, task_count, max_value, ps::to_hip(stream));
 }
 
 static int sddmm_csr(int workset_count, const ps_workset* worksets, const int* residue_offset,
@@ -556,7 +624,8 @@ static int sddmm_csr(int workset_count, const ps_workset* worksets, const int* r
     outs[q] = out_csr;
   }
   return ps::launch(workset_count, order, ordered, outs, 1, pos, 0, residue_offset, rows, cols,
-                    N, lhs, rhs, task_chunk, task_order, task_count, ps::to_hip(stream));
+                    N, lhs, rhs, task_chunk, task_order, task_count, 0.f,
+                    ps::to_hip(stream));
 }
 
 int ps_sddmm_csr_launch(int workset_count, const ps_workset* worksets, const int* residue_offset,
@@ -599,7 +668,7 @@ int ps_sddmm_workset_launch(int s, const ps_workset* workset, const int* residue
                             float* out, ps_stream_t stream) {
   PS_CHECK_ARG(s >= 0 && s < PS_MAX_WORKSETS && workset, "Invalid SDDMM workset");
   return ps::launch(1, &s, workset, &out, 0, nullptr, 0, residue_offset, rows, cols, N, lhs,
-                    rhs, 1, nullptr, 0, ps::to_hip(stream));
+                    rhs, 1, nullptr, 0, 0.f, ps::to_hip(stream));
 }
 
 }  // extern "C"

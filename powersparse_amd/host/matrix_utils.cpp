@@ -229,6 +229,7 @@ struct PowerSparseMatrixGPU::Prepared {
   DeviceArray<uint32_t> flag;  // scratch of the checks
   unsigned long long degree_sums[32] = {};
   DeviceArray<int> col_nnz;  // device column counts
+  bool large_values = false;  // (the device's check) a value's magnitude is above 1
   std::vector<int> col_nnz_host, sigbit;
   int max_count = 0, count_bits = 0;
   // Each row's nonzeros ranked by column count (descending, ties in CSR order).
@@ -295,7 +296,12 @@ struct PowerSparseMatrixGPU::Prepared {
     // The values are first read by the gather: uploaded here, while the other
     // thread still sorts the columns.
     StagedUpload(sp_data.data(), host_sp_data, sizeof(float) * size_t(nnz));
-    if (nnz >= kDeviceCheckNonzeros) Check(nullptr, sp_data.data(), nnz, cols);
+    if (nnz >= kDeviceCheckNonzeros) {
+      Check(nullptr, sp_data.data(), nnz, cols);
+      uint32_t found = 0;
+      flag.Download(&found, 1);
+      large_values = (found & 2u) != 0;
+    }
     clock.Mark(&PreprocessTimings::upload_ms);
   }
 
@@ -360,10 +366,13 @@ PowerSparseMatrixGPU::PowerSparseMatrixGPU(int row_num, int col_num, int nnz_num
 #pragma omp parallel for reduction(| : bad) schedule(static)
   for (int r = 0; r < row_num; ++r) bad |= (row_ptr[r] < 0 || row_ptr[r] > row_ptr[r + 1]);
   if (bad) throw std::invalid_argument("CSR row pointers must be nondecreasing");
+  int large = 0;
   if (nnz_num < kDeviceCheckNonzeros) {  // else on the device, as they are uploaded
-#pragma omp parallel for reduction(| : bad) schedule(static)
-    for (int p = 0; p < nnz_num; ++p)
+#pragma omp parallel for reduction(| : bad, large) schedule(static)
+    for (int p = 0; p < nnz_num; ++p) {
       bad |= (col_ind[p] < 0 || col_ind[p] >= col_num || !std::isfinite(sp_data[p]));
+      large |= std::fabs(sp_data[p]) > 1.f;
+    }
     if (bad) throw std::invalid_argument(kBadEntry);
   }
   Configure(policy);
@@ -377,6 +386,7 @@ PowerSparseMatrixGPU::PowerSparseMatrixGPU(int row_num, int col_num, int nnz_num
   const KeptMark mark;
   try {
     Prepared in(row_num, col_num, nnz_num, row_ptr, col_ind, sp_data, timings);
+    _unit_values = !large && !in.large_values;
     // A tuned SpMM partition may follow only in signature order (kAuto
     // decides the order at the end of the build).
     const bool may_tune =

@@ -232,6 +232,8 @@ class PowerSparseMatrixGPU {
     return order == TaskOrder::kRow ? _locality[1] : _locality[0];
   }
   // Whether the operators run in the locality run order (see PartitionPolicy).
+  // Whether no value's magnitude is above 1.
+  bool UnitValues() const { return _unit_values; }
   bool RunOrderUsed() const { return _run_order[0] != nullptr || _run_order[2] != nullptr; }
   // The partition SpMM runs on: the tuned one (SpmmPartition::kTuned), or
   // this matrix itself when none was built. With a dense hub block it holds
@@ -301,6 +303,7 @@ class PowerSparseMatrixGPU {
   bool* _residue_atomic = nullptr;
   // locality run orders, by RunOrderSlot()
   bool _want_run_order = true;
+  bool _unit_values = false;
   uint32_t* _run_order[3] = {nullptr, nullptr, nullptr};
   uint32_t _run_order_tasks[3] = {0, 0, 0};
   int _max_group_types = 0;

@@ -92,19 +92,12 @@ void SDDMMAsync(const PowerSparseMatrixGPU& m, int N, const float* lhs, const fl
     if (m.GroupNum()[s] != 0 && !out[s]) throw std::invalid_argument("Missing SDDMM output workset");
   const ExecutionLayout e = m.Execution();
   const auto ws = Worksets(m, e);
-  if (e.out_base)  // row-ordered copy: results written to the public layout
-    ThrowOnError(ps_sddmm_scatter_launch(m.GroupTypeNum(), ws.data(), e.residue_offset,
-                                         e.out_base, m.MatrixRow(), m.MatrixCol(), N, lhs, rhs,
-                                         out, e.task_chunk, stream));
-  else if (e.run_order[RunOrderSlot(PS_OP_SDDMM, N)])
-    ThrowOnError(ps_sddmm_launch_ordered(m.GroupTypeNum(), ws.data(), e.residue_offset,
-                                         m.MatrixRow(), m.MatrixCol(), N, lhs, rhs, out,
-                                         e.task_chunk, e.run_order[RunOrderSlot(PS_OP_SDDMM, N)],
-                                         e.run_order_tasks[RunOrderSlot(PS_OP_SDDMM, N)],
-                                         stream));
-  else
-    ThrowOnError(ps_sddmm_launch(m.GroupTypeNum(), ws.data(), e.residue_offset, m.MatrixRow(),
-                                 m.MatrixCol(), N, lhs, rhs, out, e.task_chunk, stream));
+  // the row-ordered copy's results are written to the public layout
+  const int k = RunOrderSlot(PS_OP_SDDMM, N);
+  ThrowOnError(ps_sddmm_launch_values(m.GroupTypeNum(), ws.data(), e.residue_offset, e.out_base,
+                                      m.MatrixRow(), m.MatrixCol(), N, lhs, rhs, out, e.task_chunk,
+                                      e.run_order[k], e.run_order_tasks[k],
+                                      m.UnitValues() ? 1.f : 0.f, stream));
   // the groups inside the dense hub block (left out of the run order)
   if (m.HubBlockUsed()) m.HubSddmm(N, lhs, rhs, out, nullptr, stream);
 }
