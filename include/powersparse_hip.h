@@ -362,20 +362,12 @@ size_t ps_hub_dense_floats(int rows, int cols);
  * more than once left out; the same block on every build. */
 int ps_hub_dense_build(const ps_hub_block* hb, const int* row_ptr, const int* col_ind,
                        const float* sp_data, float* dense, uint32_t* stored, ps_stream_t stream);
-/* counts[r] = stored entries of row r outside the block's stored slots
- * (matrix_rows values; run after ps_hub_dense_build). */
-int ps_hub_kept_counts(const ps_hub_block* hb, const int* row_ptr, const int* col_ind,
-                       uint32_t* counts, ps_stream_t stream);
-/* The CSR without the entries of the block's stored slots (order within rows
- * kept); new_row_ptr is the exclusive scan of ps_hub_kept_counts. */
-int ps_hub_compact(const ps_hub_block* hb, const int* row_ptr, const int* col_ind,
-                   const float* sp_data, const uint32_t* new_row_ptr, int* new_col,
-                   float* new_val, ps_stream_t stream);
-/* The same over several tiers of disjoint rows, for a matrix whose rows are
- * already ranked (ps_pre_rank_sort): counts[r] = entries of row r outside every
+/* The matrix without the block, over several tiers of disjoint rows, its rows
+ * ranked already (ps_pre_rank_sort): counts[r] = entries of row r outside every
  * tier's stored slots, and new_ranked[new_row_ptr[r] ..] = row r's ranked
  * positions of those entries, in order; new_row_ptr is the exclusive scan of
- * the counts. hubs: up to PS_HUB_MAX_TIERS descriptors (host array). */
+ * the counts. hubs: up to PS_HUB_MAX_TIERS descriptors (host array), after
+ * ps_hub_dense_build. */
 #define PS_HUB_MAX_TIERS 4
 int ps_hub_rest_counts(int tiers, const ps_hub_block* hubs, const int* row_ptr, uint32_t* counts,
                        ps_stream_t stream);

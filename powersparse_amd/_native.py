@@ -173,11 +173,6 @@ HIP_API = [
     ("ps_hub_stored_words", ctypes.c_size_t, [ctypes.POINTER(HubBlock)]),
     ("ps_hub_dense_build", ctypes.c_int,
      [ctypes.POINTER(HubBlock), c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
-    ("ps_hub_kept_counts", ctypes.c_int,
-     [ctypes.POINTER(HubBlock), c_void_p, c_void_p, c_void_p, c_void_p]),
-    ("ps_hub_compact", ctypes.c_int,
-     [ctypes.POINTER(HubBlock), c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
-      c_void_p]),
     ("ps_hub_rest_counts", ctypes.c_int,
      [ctypes.c_int, ctypes.POINTER(HubBlock), c_void_p, c_void_p, c_void_p]),
     ("ps_hub_rest_ranked", ctypes.c_int,

@@ -143,7 +143,7 @@ __global__ __launch_bounds__(kThreads) void hist_kernel(const int* __restrict__ 
 // passes over 4 bytes per row or column. As loops of the host with two uploads
 // per tier it held the device idle for 11 ms of a 98 ms build of 1.6 M rows
 // and 264 M nonzeros, the tile list below (flags downloaded, codes uploaded)
-// for 7 (98 -> 81 ms together).
+// for 7.
 //
 // levels[a] = rows of degree with floor(log2) = a, levels[32 + b] = columns of
 // count with floor(log2) = b (rows and columns without nonzeros left out).
@@ -253,56 +253,6 @@ __device__ __forceinline__ bool in_block(const ps_hub_block& hb, int i, int h) {
   if (i < 0 || h < 0) return false;
   const size_t words = (size_t(hb.cols) + 31) / 32;
   return (hb.stored[size_t(i) * words + h / 32] >> (h % 32)) & 1u;
-}
-
-// counts[r] = stored entries of row r outside the SpMM block. One wave per row.
-__global__ __launch_bounds__(kThreads) void kept_kernel(ps_hub_block hb,
-                                                         const int* __restrict__ row_ptr,
-                                                         const int* __restrict__ col_ind,
-                                                         uint32_t* __restrict__ counts) {
-  const int waves = kThreads / kWave;
-  for (int r = blockIdx.x * waves + threadIdx.x / kWave; r < hb.matrix_rows;
-       r += gridDim.x * waves) {
-    const int b = row_ptr[r], e = row_ptr[r + 1];
-    uint32_t n = uint32_t(e - b);
-    const int i = hb.hub_index[r];
-    if (i >= 0) {
-      uint32_t inside = 0;
-      for (int p = b + lane_id(); p < e; p += kWave) inside += in_block(hb, i, hb.hot_rank[col_ind[p]]);
-      for (int o = 32; o > 0; o >>= 1) inside += __shfl_xor(inside, o);
-      n -= inside;
-    }
-    if (lane_id() == 0) counts[r] = n;
-  }
-}
-
-// The CSR without the SpMM block's entries, in the original order within rows.
-__global__ __launch_bounds__(kThreads) void compact_kernel(ps_hub_block hb,
-                                                            const int* __restrict__ row_ptr,
-                                                            const int* __restrict__ col_ind,
-                                                            const float* __restrict__ sp_data,
-                                                            const uint32_t* __restrict__ new_row_ptr,
-                                                            int* __restrict__ new_col,
-                                                            float* __restrict__ new_val) {
-  const int waves = kThreads / kWave;
-  for (int r = blockIdx.x * waves + threadIdx.x / kWave; r < hb.matrix_rows;
-       r += gridDim.x * waves) {
-    const int b = row_ptr[r], e = row_ptr[r + 1];
-    const int i = hb.hub_index[r];
-    uint32_t out = new_row_ptr[r];
-    for (int p0 = b; p0 < e; p0 += kWave) {
-      const int p = p0 + lane_id();
-      const int c = p < e ? col_ind[p] : 0;
-      const bool keep = p < e && !(i >= 0 && in_block(hb, i, hb.hot_rank[c]));
-      const uint64_t m = __ballot(keep);
-      if (keep) {
-        const uint32_t at = out + uint32_t(__popcll(m & ((1ull << lane_id()) - 1ull)));
-        new_col[at] = c;
-        new_val[at] = sp_data[p];
-      }
-      out += uint32_t(__popcll(m));
-    }
-  }
 }
 
 // ---- the matrix without the block, as a shorter ranking ----
@@ -1219,35 +1169,6 @@ int ps_hub_dense_build(const ps_hub_block* hb, const int* row_ptr, const int* co
   const size_t lds = 2 * sizeof(uint32_t) * (words < ps::kMarkWords ? words : ps::kMarkWords);
   ps::dense_build_kernel<<<ps::grid_for(size_t(hb->rows), 1), ps::kMarkThreads, lds, st>>>(
       *hb, row_ptr, col_ind, sp_data, dense, stored);
-  PS_LAUNCHED();
-  return PS_OK;
-}
-
-int ps_hub_kept_counts(const ps_hub_block* hb, const int* row_ptr, const int* col_ind,
-                       uint32_t* counts, ps_stream_t stream) {
-  const int rc = ps::check_block(hb);
-  if (rc != PS_OK) return rc;
-  PS_CHECK_ARG(hb->stored, "ps_hub_kept_counts: missing stored bits");
-  PS_CHECK_ARG(row_ptr && col_ind && counts, "ps_hub_kept_counts: null argument");
-  hipStream_t st = ps::to_hip(stream);
-  ps::kept_kernel<<<ps::grid_for(size_t(hb->matrix_rows), ps::kThreads / ps::kWave), ps::kThreads,
-                    0, st>>>(*hb, row_ptr, col_ind, counts);
-  PS_LAUNCHED();
-  return PS_OK;
-}
-
-int ps_hub_compact(const ps_hub_block* hb, const int* row_ptr, const int* col_ind,
-                   const float* sp_data, const uint32_t* new_row_ptr, int* new_col, float* new_val,
-                   ps_stream_t stream) {
-  const int rc = ps::check_block(hb);
-  if (rc != PS_OK) return rc;
-  PS_CHECK_ARG(hb->stored, "ps_hub_compact: missing stored bits");
-  PS_CHECK_ARG(row_ptr && col_ind && sp_data && new_row_ptr && new_col && new_val,
-               "ps_hub_compact: null argument");
-  hipStream_t st = ps::to_hip(stream);
-  ps::compact_kernel<<<ps::grid_for(size_t(hb->matrix_rows), ps::kThreads / ps::kWave),
-                       ps::kThreads, 0, st>>>(*hb, row_ptr, col_ind, sp_data, new_row_ptr, new_col,
-                                              new_val);
   PS_LAUNCHED();
   return PS_OK;
 }

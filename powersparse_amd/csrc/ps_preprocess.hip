@@ -1629,8 +1629,8 @@ __global__ __launch_bounds__(kWindowThreads) void row_window_kernel(
 constexpr int kGatherTileMax = 1024 * kSortItems;
 
 // As many groups per tile as fit both the tile and the bits that the columns
-// leave free in a 32-bit key (128 groups of 64 in a tile: columns below 2^27
-// lose nothing).
+// leave free in a 32-bit key (32 groups of 64 in a tile of 2048: columns below
+// 2^27 lose nothing).
 template <int NT>
 int gather_tile(int group_size, int cols, const uint32_t* perm, int groups, const int* group_start,
                 const uint32_t* ranked_vals, const int* col_ind, const float* sp_data,
