@@ -716,6 +716,11 @@ struct PowerSparseMatrixGPU::HubState {
   DeviceArray<char> ws;
   ps_event_t done = nullptr;
   bool recorded = false;
+  // SDDMM uses the block from this width on, with the run order that leaves
+  // its tiles out
+  int sddmm_from = 0;
+  DeviceArray<uint32_t> sddmm_order;
+  uint32_t sddmm_tasks = 0;
   ~HubState() {
     if (done) ps_event_destroy(done);
   }
@@ -728,6 +733,12 @@ struct PowerSparseMatrixGPU::HubState {
   }
 };
 
+bool PowerSparseMatrixGPU::HubSddmmUsed(int N, const uint32_t** order, uint32_t* tasks) const {
+  if (!_hub || N < _hub->sddmm_from) return false;
+  *order = _hub->sddmm_order.data();
+  *tasks = _hub->sddmm_tasks;
+  return true;
+}
 int PowerSparseMatrixGPU::HubTiers() const { return _hub ? int(_hub->tiers.size()) : 0; }
 int PowerSparseMatrixGPU::HubRows(int tier) const {
   return tier >= 0 && tier < HubTiers() ? _hub->tiers[size_t(tier)]->desc.rows : 0;
@@ -746,6 +757,7 @@ bool PowerSparseMatrixGPU::BuildHub(Prepared& in, const PartitionPolicy& policy)
   const int rows = _matrix_row, cols = _matrix_col, S = _group_type_num;
   if (S < 2) return false;  // fine mode: its store rule differs from a capped partition's
   std::vector<TierSpec> specs;
+  bool small = false;  // a block kept for the share of the matrix it holds
   const bool forced = policy.hub_min_degree[0] > 0 && policy.hub_min_count[0] > 0;
   if (forced) {
     for (int k = 0; k < kHubMaxTiers; ++k) {
@@ -800,9 +812,11 @@ bool PowerSparseMatrixGPU::BuildHub(Prepared& in, const PartitionPolicy& policy)
             bb = b;
           }
         }
-      if (ba < 0 || best < (k == 0 ? kHubMinGain : kHubMinTierGain) * double(_matrix_nnz) ||
-          (k == 0 && best < kHubMinGainNonzeros))
-        break;
+      if (ba < 0 || best < (k == 0 ? kHubMinGain : kHubMinTierGain) * double(_matrix_nnz)) break;
+      if (k == 0 && best < kHubMinGainNonzeros) {
+        if (best < kHubMinGainSmall || best < kHubMinGainShare * double(_matrix_nnz)) break;
+        small = true;
+      }
       specs.push_back({1LL << ba, top < 32 ? (1LL << top) : std::numeric_limits<long long>::max(),
                        1LL << bb});
       top = ba;
@@ -926,26 +940,25 @@ bool PowerSparseMatrixGPU::BuildHub(Prepared& in, const PartitionPolicy& policy)
     skip_ptr[size_t(s)] = skip.data() + first;
     first += size_t(_group_num[s]) * size_t(GROUP_SIZE(s) / 64);
   }
-  const int k = RunOrderSlot(PS_OP_SDDMM, 32);
-  uint32_t count = 0, kept_tasks = 0;
+  hub->sddmm_from = small ? kHubSmallSddmmFrom : 0;
+  uint32_t count = 0;
   ThrowOnError(ps_task_count(PS_OP_SDDMM, 32, S, ws.data(), &count));
-  uint32_t* order = nullptr;
   if (count > 0) {
-    ThrowOnError(ps_malloc(reinterpret_cast<void**>(&order), sizeof(uint32_t) * count));
-    const int rc = ps_task_order_build_subset(PS_OP_SDDMM, 32, S, ws.data(), skip_ptr.data(),
-                                              order, count, &kept_tasks, nullptr);
-    if (rc != PS_OK) {
-      ps_free(order);
-      ThrowOnError(rc);
-    }
+    hub->sddmm_order.Allocate(count);
+    ThrowOnError(ps_task_order_build_subset(PS_OP_SDDMM, 32, S, ws.data(), skip_ptr.data(),
+                                            hub->sddmm_order.data(), count, &hub->sddmm_tasks,
+                                            nullptr));
   }
   // the workspace for every width: SpMM runs feature slices of at most 128,
   // SDDMM widths go up to 512
   hub->ws.Allocate(std::max(hub->Workspace(PS_OP_SPMM, 128), hub->Workspace(PS_OP_SDDMM, 512)));
   ThrowOnError(ps_event_create(&hub->done));
-  ps_free(_run_order[k]);
-  _run_order[k] = order;
-  _run_order_tasks[k] = kept_tasks;
+  if (!small) {  // no width runs the whole order
+    const int k = RunOrderSlot(PS_OP_SDDMM, 32);
+    ps_free(_run_order[k]);
+    _run_order[k] = nullptr;
+    _run_order_tasks[k] = 0;
+  }
   _spmm_tuned = part.release();
   _hub = hub.release();
   return true;

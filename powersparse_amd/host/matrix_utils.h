@@ -93,7 +93,16 @@ constexpr int kTunedSpmmGroupTypes = 3;
 // 22.8 M (128 M nonzeros) 0.94 / 0.86, 1.01 / 1.00; 12.7 M (66 M) 1.01 / 0.87,
 // 1.05 / 0.94; 7.9 M (100 M) 1.05 / 0.97, 1.00 / 1.00; 6.3 M (32 M) 1.16 / 0.94,
 // 1.14 / 0.94; 3.6 M (16.5 M) 1.38 / 0.98, 1.08 / 0.93; 0.9 M (4 M) 2.34 /
-// 1.57, 1.74 / 1.17. The next tier takes the rows below 2^a the same way, kept from kHubMinTierGain
+// 1.57, 1.74 / 1.17. A smaller block that holds most of its matrix
+// (kHubMinGainShare of the nonzeros gained, kHubMinGainSmall at least) pays for
+// SpMM at every width and for SDDMM from kHubSmallSddmmFrom features, where it
+// is used (the same ratios, SDDMM N = 32 / 64 / 128): 2000 x 20 k, 12 M nonzeros,
+// gain 7.2 M, 0.84 / 0.49, 1.75 / 1.10 / 0.70; 2000 rows of 8 k over 30 k columns
+// beside 1 M of 8, 24 M, gain 9.2 M, 0.92 / 0.80, 1.43 / 1.08 / 0.91; 1000 of 8 k
+// over 20 k beside 200 k of 20, 12 M, gain 5.8 M, 0.99 / 0.83, 1.56 / 1.13 / 0.91,
+// beside 500 k, 18 M, 0.99 / 0.92, 1.29 / 1.07 / 0.95; 2000 x 100 k, 33 M, gain 8.8
+// M, 0.91 / 0.60 (too thin for SDDMM). The next tier takes the rows below 2^a the
+// same way, kept from kHubMinTierGain
 // (kHubDenseCost: the dense element's cost relative to the sparse nonzero it
 // replaces, measured on MI355X). SDDMM computes a tier's dense dots whole and
 // takes from it only the tiles lying inside it, so it uses a tier when those
@@ -111,7 +120,8 @@ constexpr int kTunedSpmmGroupTypes = 3;
 enum class HubBlock { kAuto = 0, kOff = 1 };
 constexpr int kHubMaxTiers = 3;
 constexpr double kHubDenseCost = 0.12, kHubMinGain = 0.05, kHubMinTierGain = 0.02;
-constexpr double kHubMinGainNonzeros = 10e6;
+constexpr double kHubMinGainNonzeros = 10e6, kHubMinGainSmall = 5e6, kHubMinGainShare = 0.25;
+constexpr int kHubSmallSddmmFrom = 128;
 constexpr double kHubSddmmMinFill = 0.25;
 constexpr int kHubMinRows = 256, kHubMinCols = 1024;
 constexpr long long kHubMaxElements = 1LL << 29;
@@ -244,6 +254,9 @@ class PowerSparseMatrixGPU {
   // The dense hub block in use (HubBlock): its tiers, each rows x columns
   // (0 x 0 beyond the last).
   bool HubBlockUsed() const { return _hub != nullptr; }
+  // Whether SDDMM at width N uses it; if so, *order and *tasks become the run
+  // order without its tiles.
+  bool HubSddmmUsed(int N, const uint32_t** order, uint32_t* tasks) const;
   int HubTiers() const;
   int HubRows(int tier = 0) const;
   int HubCols(int tier = 0) const;

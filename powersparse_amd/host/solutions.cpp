@@ -93,13 +93,14 @@ void SDDMMAsync(const PowerSparseMatrixGPU& m, int N, const float* lhs, const fl
   const ExecutionLayout e = m.Execution();
   const auto ws = Worksets(m, e);
   // the row-ordered copy's results are written to the public layout
-  const int k = RunOrderSlot(PS_OP_SDDMM, N);
+  const uint32_t* order = e.run_order[RunOrderSlot(PS_OP_SDDMM, N)];
+  uint32_t tasks = e.run_order_tasks[RunOrderSlot(PS_OP_SDDMM, N)];
+  const bool hub = m.HubSddmmUsed(N, &order, &tasks);
   ThrowOnError(ps_sddmm_launch_values(m.GroupTypeNum(), ws.data(), e.residue_offset, e.out_base,
                                       m.MatrixRow(), m.MatrixCol(), N, lhs, rhs, out, e.task_chunk,
-                                      e.run_order[k], e.run_order_tasks[k],
-                                      m.UnitValues() ? 1.f : 0.f, stream));
+                                      order, tasks, m.UnitValues() ? 1.f : 0.f, stream));
   // the groups inside the dense hub block (left out of the run order)
-  if (m.HubBlockUsed()) m.HubSddmm(N, lhs, rhs, out, nullptr, stream);
+  if (hub) m.HubSddmm(N, lhs, rhs, out, nullptr, stream);
 }
 
 void SDDMMToCSR(const PowerSparseMatrixGPU& m, int N, const float* lhs, const float* rhs,
@@ -110,17 +111,18 @@ void SDDMMToCSR(const PowerSparseMatrixGPU& m, int N, const float* lhs, const fl
         "SDDMMToCSR needs a matrix built with PartitionPolicy::csr_positions");
   const ExecutionLayout e = m.Execution();
   const auto ws = Worksets(m, e);
-  const int k = RunOrderSlot(PS_OP_SDDMM, N);
-  if (e.run_order[k])
+  const uint32_t* order = e.run_order[RunOrderSlot(PS_OP_SDDMM, N)];
+  uint32_t tasks = e.run_order_tasks[RunOrderSlot(PS_OP_SDDMM, N)];
+  const bool hub = m.HubSddmmUsed(N, &order, &tasks);
+  if (order)
     ThrowOnError(ps_sddmm_csr_launch_ordered(m.GroupTypeNum(), ws.data(), e.residue_offset,
                                              e.csr_pos, m.MatrixRow(), m.MatrixCol(), N, lhs,
-                                             rhs, out_csr, e.task_chunk, e.run_order[k],
-                                             e.run_order_tasks[k], stream));
+                                             rhs, out_csr, e.task_chunk, order, tasks, stream));
   else
     ThrowOnError(ps_sddmm_csr_launch(m.GroupTypeNum(), ws.data(), e.residue_offset, e.csr_pos,
                                      m.MatrixRow(), m.MatrixCol(), N, lhs, rhs, out_csr,
                                      e.task_chunk, stream));
-  if (m.HubBlockUsed()) m.HubSddmm(N, lhs, rhs, nullptr, out_csr, stream);
+  if (hub) m.HubSddmm(N, lhs, rhs, nullptr, out_csr, stream);
 }
 
 void WorksetToCSR(const PowerSparseMatrixGPU& m, const float* const* values, float* out_csr,

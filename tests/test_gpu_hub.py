@@ -620,3 +620,69 @@ def test_hub_auto_rule_on_c3():
     assert (r1, h1) == (20713, 3578) and g1 >= 0.02 * csr.nnz
     for lo, c in [(512, 8192), (2048, 8192), (1024, 4096), (1024, 16384)]:
         assert gain(lo, 16384, c)[0] <= g1, (lo, c)
+
+
+def test_hub_auto_rule_on_a_dense_share():
+    """A block that gains less than 10 M nonzeros is kept when that is a quarter of
+    the matrix: SpMM uses it at every width, SDDMM from 128 features on, in
+    workset and in CSR order; below, SDDMM is the sparse path's, bit for bit. The
+    same rows beside a million others (a fifth of the matrix) get no block."""
+    setup()
+    rng = np.random.default_rng(71)
+    hub, hot, d = 1000, 20000, 8192
+
+    def graph(rows, deg):
+        step = hot / d
+        a = (np.arange(d)[None, :] * step + rng.random((hub, d)) * step).astype(np.int64)
+        b = rng.integers(0, rows, rows * deg)
+        ci = np.concatenate([a.clip(0, hot - 1).reshape(-1), b]).astype(np.int32)
+        degrees = np.concatenate([np.full(hub, d), np.full(rows, deg)])
+        rp = np.concatenate([[0], np.cumsum(degrees)]).astype(np.int32)
+        return ps.HostCsr(hub + rows, rows, rp, ci,
+                          rng.uniform(-1, 1, ci.size).astype(np.float32))
+
+    m = ps.PowerSparseMatrixGPU.from_csr(graph(1000000, 20))
+    say(f"a fifth: {m.hub_block}")
+    assert m.hub_block == []
+    m.close()
+    csr = graph(200000, 20)
+    on = ps.PowerSparseMatrixGPU.from_csr(csr, csr_positions=True)
+    off = ps.PowerSparseMatrixGPU.from_csr(csr, csr_positions=True, hub_block="off")
+    say(f"a share of {csr.nnz} nonzeros: {on.hub_block}")
+    assert on.hub_block == [(hub, hot)] and off.hub_block == []
+    sizes = on.sddmm_output_sizes()
+    row = np.repeat(np.arange(csr.rows), np.diff(csr.row_ptr))
+    for N in (32, 96, 128, 160):
+        X = rng.uniform(-1, 1, (csr.rows, N)).astype(np.float32)
+        Y = rng.uniform(-1, 1, (csr.cols, N)).astype(np.float32)
+        dX, dY = ps.DeviceBuffer(host=X), ps.DeviceBuffer(host=Y)
+        got = []
+        for m in (on, off):
+            outs = [ps.DeviceBuffer.zeros(max(n, 1) * 4) for n in sizes]
+            flat = ps.DeviceBuffer(host=np.full(csr.nnz, np.nan, np.float32))
+            C = ps.DeviceBuffer.zeros(csr.rows * N * 4)
+            ps.SDDMMAsync(m, N, dX, dY, outs)
+            ps.SDDMMToCSR(m, N, dX, dY, flat)
+            ps.SpMMAsync(m, N, dY, C)
+            ps.synchronize()
+            by_csr = ps.DeviceBuffer.zeros(csr.nnz * 4)
+            ps.WorksetToCSR(m, outs, by_csr)
+            ps.synchronize()
+            got.append([b.download(np.float32, n) for b, n in
+                        ((by_csr, csr.nnz), (flat, csr.nnz), (C, csr.rows * N))])
+        differ = [int((a != b).sum()) for a, b in zip(*got)]
+        say(f"  N={N}: outputs that differ from the sparse path's {differ}")
+        assert (differ[0] > 0) == (differ[1] > 0) == (N >= 128) and differ[2] > 0
+        E, M = oracle.spmm(csr.row_ptr, csr.col_ind, csr.values, N, Y, with_mag=True)
+        tolerance.check(got[0][2].reshape(csr.rows, N), E, M, f"SpMM N={N}")
+        if N == 128:
+            E, M = np.empty(csr.nnz), np.empty(csr.nnz)
+            for b in range(0, csr.nnz, 1 << 20):
+                e = b + (1 << 20)
+                x, y = X[row[b:e]].astype(np.float64), Y[csr.col_ind[b:e]].astype(np.float64)
+                E[b:e] = (x * y).sum(1) * csr.values[b:e]
+                M[b:e] = np.abs(x * y).sum(1) * np.abs(csr.values[b:e])
+            tolerance.check(got[0][0], E, M, "SDDMM N=128")
+            tolerance.check(got[0][1], E, M, "SDDMM N=128 in CSR order")
+    on.close()
+    off.close()
