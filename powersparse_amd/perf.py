@@ -104,9 +104,10 @@ def short_name(name):
 
 def kernel_op(name):
     """(op, lanes-template) of an operator kernel name, else None."""
-    # spmm_kernel<lanes, buf>, sddmm_kernel<KQ, buf, store mode>; the hub
-    # block's kernels (hub_spmm_kernel<..>, hub_sddmm_kernel<..>) are not
-    m = re.search(r"(?:^|::)(spmm|sddmm)_kernel<(\d+), (true|false)(, \d+)?>", short_name(name))
+    # spmm_kernel<lanes, buf>, sddmm_kernel<KQ, buf, store mode, slices>; the
+    # hub block's kernels (hub_spmm_kernel<..>, hub_sddmm_kernel<..>) are not
+    m = re.search(r"(?:^|::)(spmm|sddmm)_kernel<(\d+), (?:true|false)(?:, \d+)*>",
+                  short_name(name))
     return (m.group(1), int(m.group(2))) if m else None
 
 

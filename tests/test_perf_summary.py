@@ -4,6 +4,7 @@ like rocprofv3's, the counters bench.py reads back from it, and bench.py's
 refusal of more than one GPU."""
 import json
 import os
+import re
 import sqlite3
 import subprocess
 import sys
@@ -18,8 +19,8 @@ from powersparse_amd import perf  # noqa: E402
 KIB = 1024.0
 SPMM32 = "void ps::spmm_kernel<8, true>(ps::(anonymous namespace)::SpmmArgs)"
 SPMM128 = "void ps::spmm_kernel<8, true>(ps::(anonymous namespace)::SpmmArgs)"
-SDDMM128 = "void ps::(anonymous namespace)::sddmm_kernel<4, true, 0>(ps::SddmmArgs)"
-SDDMM32 = "void ps::(anonymous namespace)::sddmm_kernel<1, true, 0>(ps::SddmmArgs)"
+SDDMM128 = "void ps::(anonymous namespace)::sddmm_kernel<4, true, 0, 0>(ps::SddmmArgs)"
+SDDMM32 = "void ps::(anonymous namespace)::sddmm_kernel<1, true, 0, 0>(ps::SddmmArgs)"
 COPY = "void ps::copy_f32_kernel(float*, float const*, unsigned long)"
 PRE = "void ps::rank_small_kernel(int const*, int, int const*)"
 FILL = "void ps::(anonymous namespace)::fill_random_kernel(float*, unsigned long)"
@@ -151,6 +152,22 @@ def test_bench_one_gpu_only():
     r = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), "--gpus", "2"],
                        capture_output=True, text=True, timeout=120)
     assert r.returncode == 2 and "one GPU only" in r.stderr
+
+
+def test_operator_kernels_of_the_library_are_recognised():
+    """The names the summary looks for are those of the kernels as built."""
+    lib = os.path.join(ROOT, "powersparse_amd", "lib", "libpowersparse_hip.so")
+    symbols = subprocess.run(["nm", "-C", lib], check=True, capture_output=True, text=True).stdout
+    names = {line.split(" ", 2)[2] for line in symbols.splitlines()
+             if re.search(r"::(hub_)?(spmm|sddmm)_kernel<", line)}
+    for op in ("spmm", "sddmm"):
+        mine = [n for n in names if f"::{op}_kernel<" in n]
+        assert mine
+        for n in mine:
+            first = int(re.search(r"_kernel<(\d+)", n).group(1))
+            assert perf.kernel_op(n) == (op, first), n
+    hub = [n for n in names if "::hub_" in n]
+    assert hub and all(perf.kernel_op(n) is None for n in hub)
 
 
 def test_operator_calls_take_the_hub_kernels_that_follow():
