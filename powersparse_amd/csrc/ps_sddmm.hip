@@ -72,8 +72,22 @@ constexpr int kAutoChunkMax = 256;
 //   20 k nodes in CSR order, N = 288       98 -> 103 (256)
 // Launches that gather less than kSliceMinGather (an upper bound: every task
 // full) are not cut: another launch costs about 3.5 us (61 k nonzeros, N = 448:
-// 25.9 us in one launch, 29.3 in two).
+// 25.9 us in one launch, 29.3 in two). Nor, with a residue that results are
+// added to, are those of which two hold:
+//   fewer than kSliceFew features;
+//   values not known to be at most 1 (the residue's dots whole, see above);
+//   fewer than kSliceMinBlocks block nonzeros per residue group (nearly all of
+//   the matrix in the residue, whose rows' X each slice loads again).
+// Time of slices against one launch (600 k x 1 M of degree 24, no blocks; 512 k
+// community graph, 9 block nonzeros per residue group; 1 M power law of mean
+// 20), at N = 160, 192, 256, 320, 512:
+//   values at most 1: 1.00 1.08 1.01 1.00 0.98; 1.00 0.96 0.94 0.88 0.85;
+//                     1.01 0.97 0.96 0.91 0.89
+//   larger:           1.07 1.14 1.11 1.09 1.03; 1.01 1.04 1.02 0.93 0.96;
+//                     1.04 1.02 0.99 0.94 0.93
 constexpr int kSliceNarrow = 128, kSliceWide = 256, kSliceCsr = 320;
+constexpr int kSliceFew = 256;
+constexpr uint64_t kSliceMinBlocks = 4;
 constexpr uint64_t kWideRhsBytes = uint64_t(48) << 20;
 constexpr uint64_t kSliceMinGather = uint64_t(512) << 20;
 static_assert(kTaskOut >= 8 * kStage, "a task's slots each collect up to kStage results");
@@ -458,7 +472,7 @@ int launch(int count, const int* order, const ps_workset* worksets, float* const
   const uint64_t rhs_bytes = uint64_t(cols) * uint64_t(N) * 4u;
   const bool buf = lhs_bytes <= 0xFFFFFFFFull && rhs_bytes <= 0xFFFFFFFFull;
   a.residue_offset = residue_offset;
-  uint64_t tasks = 0;
+  uint64_t tasks = 0, block_nnz = 0, residue_groups = 0;
   int n = 0;
   // Validate every workset before submitting any work (sddmm_solution.cu:16-22).
   for (int q = 0; q < count; ++q) {
@@ -480,8 +494,10 @@ int launch(int count, const int* order, const ps_workset* worksets, float* const
                    "Block workset exceeds the 32-bit kernel indexing range");
       const uint64_t T = uint64_t(sddmm_task_shape().tile_nnz);
       t = (uint64_t(w.group_num) * w.group_size + T - 1) / T;
+      block_nnz += uint64_t(w.group_num) * uint64_t(w.group_size);
     } else {
       PS_CHECK_ARG(residue_offset, "Missing residue offsets");
+      residue_groups += uint64_t(w.group_num);
       const uint64_t R = uint64_t(sddmm_task_shape().residue_groups);  // one slot per group
       t = (uint64_t(w.group_num) + R - 1) / R;
     }
@@ -513,13 +529,17 @@ int launch(int count, const int* order, const ps_workset* worksets, float* const
   a.chunk_log2 = uint32_t(task_chunk_log2(task_chunk, grid, kAutoChunkMax));
   // slices of nearly equal width, multiples of 32 features
   const uint64_t gathered = uint64_t(a.launch_tasks) * 64 * uint64_t(N) * 4u;
-  const int most = gathered < kSliceMinGather ? 512
+  const bool added = mode != 1 && residue_groups > 0;
+  const bool whole = added && !(max_value > 0.f && max_value <= 1.f);
+  const bool against = added && (N < kSliceFew) + whole +
+                                        (block_nnz < kSliceMinBlocks * residue_groups) >= 2;
+  const int most = gathered < kSliceMinGather || against ? 512
                    : mode == 1 ? (rhs_bytes > kWideRhsBytes ? kSliceWide : kSliceCsr)
                    : rhs_bytes > kWideRhsBytes ? kSliceNarrow
                                                : kSliceWide;
   const int slices = (N + most - 1) / most;
   const int width = (N / 32 + slices - 1) / slices * 32;
-  const int sliced = slices == 1 ? 0 : max_value > 0.f && max_value <= 1.f ? 1 : 2;
+  const int sliced = slices == 1 ? 0 : whole ? 2 : 1;
   a.N = N;
   a.lhs_all = lhs;
   a.rhs_all = rhs;

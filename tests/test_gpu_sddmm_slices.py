@@ -147,3 +147,43 @@ def test_values_near_the_limit(N, wide, order):
         assert (outs[s].download(np.float32, n) == np.float32(2.0**125)).all(), s
     assert (flat.download(np.float32, csr.nnz) == np.float32(2.0**125)).all()
     m.close()
+
+
+@pytest.mark.parametrize("degree,rows", [(6, 90000), (40, 20000)])
+@pytest.mark.parametrize("scale", [1, 5])
+@pytest.mark.parametrize("N", [192, 256])
+def test_one_launch_where_slices_cost_more(N, scale, degree, rows):
+    # two of: fewer than 256 features, values above 1, nearly all nonzeros in
+    # the residue. CSR order is one launch up to 256 features, so workset order
+    # gives its dots bit for bit exactly when it is one launch too
+    setup()
+    one = (N < 256) + (scale > 1) + (degree < 32) >= 2
+    rng = np.random.default_rng(N + degree + scale)
+    cols = 70000
+    ci = (rng.integers(0, cols, (rows, 1)) + np.arange(degree) * 1313) % cols
+    rp = np.arange(rows + 1, dtype=np.int32) * degree
+    values = (rng.uniform(0.5, 1, rows * degree) * scale).astype(np.float32)
+    csr = ps.HostCsr(rows, cols, rp, np.sort(ci, 1).reshape(-1).astype(np.int32), values)
+    m = ps.PowerSparseMatrixGPU.from_csr(csr, cu_count=1, csr_positions=True, hub_block="off")
+    say(f"SDDMM N={N} values up to {scale} degree {degree}: groups={m.GroupNum()}")
+    assert (sum(m.GroupNum()[1:]) > 0) == (degree > 32)
+    X = rng.uniform(-1, 1, (rows, N)).astype(np.float32)
+    Y = rng.uniform(-1, 1, (cols, N)).astype(np.float32)
+    dX, dY = ps.DeviceBuffer(host=X), ps.DeviceBuffer(host=Y)
+    outs = [ps.DeviceBuffer.zeros(max(n, 1) * 4) for n in m.sddmm_output_sizes()]
+    ps.SDDMMAsync(m, N, dX, dY, outs)
+    flat, csr_order = ps.DeviceBuffer.zeros(csr.nnz * 4), ps.DeviceBuffer.zeros(csr.nnz * 4)
+    ps.WorksetToCSR(m, outs, flat)
+    ps.SDDMMToCSR(m, N, dX, dY, csr_order)
+    ps.synchronize()
+    got, want = flat.download(np.float32, csr.nnz), csr_order.download(np.float32, csr.nnz)
+    assert np.array_equal(got, want) == one
+    row = np.repeat(np.arange(rows), degree)
+    E, M = np.empty(csr.nnz), np.empty(csr.nnz)
+    for b in range(0, csr.nnz, 1 << 16):
+        s = slice(b, b + (1 << 16))
+        xy = X[row[s]].astype(np.float64) * Y[csr.col_ind[s]]
+        E[s], M[s] = xy.sum(1) * values[s], np.abs(xy).sum(1) * np.abs(values[s])
+    tolerance.check(got, E, M, "workset order")
+    tolerance.check(want, E, M, "CSR order")
+    m.close()
