@@ -71,10 +71,11 @@ int ps_malloc(void** ptr, size_t bytes);
 int ps_free(void* ptr);
 /* ps_free keeps blocks of 2 MB and more for later ps_malloc calls, up to a
  * sixteenth of the device's memory. They are given back to the driver when an
- * allocation fails, by ps_mem_get_info, by the two calls below, when a matrix has
- * been built (down to what was kept before it, or 256 MB), and once a block has lain unused for ten seconds, at the next
- * ps_malloc, ps_free or ps_device_synchronize. A program that frees much and
- * then makes none of these calls calls ps_mem_trim to hand the memory on.
+ * allocation fails, by ps_mem_get_info, by the two calls below, when a matrix
+ * has been built (down to what was kept before it, or 256 MB), and, once a
+ * block has lain unused for ten seconds, at the next ps_malloc, ps_free or
+ * ps_device_synchronize. A program that frees much and then makes none of
+ * these calls calls ps_mem_trim to hand the memory on.
  * Block sizes are multiples of 2 MB, and a kept block serves requests from four
  * fifths of its size up: an allocation may hold a quarter more than it asked
  * for. No reference counterpart. */

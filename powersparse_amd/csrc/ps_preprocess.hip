@@ -39,8 +39,8 @@ __global__ void degree_sums_kernel(const int* __restrict__ row_ptr, int rows,
 }
 
 // *flag |= 1 for a column outside [0, cols) or a value with all exponent bits
-// set, |= 2 for a value of magnitude above 1. Bound by reading the arrays: 1.06 GB each on C3, 0.25 ms; the host's loop
-// over both took 8 to 10 ms there.
+// set, |= 2 for a value of magnitude above 1. Bound by reading the arrays: 1.06
+// GB each on C3, 0.32 ms; the host's loop over both took 8 to 10 ms there.
 __global__ __launch_bounds__(kThreads) void check_csr_kernel(const int* __restrict__ col_ind,
                                                              const float* __restrict__ values,
                                                              size_t n, int cols,

@@ -82,8 +82,7 @@ constexpr int kTunedSpmmGroupTypes = 3;
 // block, SDDMM on the public worksets with the block's tiles (64 consecutive
 // nonzeros of a block group) left out of the run order and their outputs
 // written from dense tiles of the product computed in registers. The block
-// comes in up to
-// kHubMaxTiers tiers of disjoint row ranges, each with its own columns: the
+// comes in up to kHubMaxTiers tiers of disjoint row ranges, each with its own columns: the
 // first tier is the pair of power-of-two thresholds (row degree >= 2^a,
 // column count >= 2^b) that maximises block nonzeros - kHubDenseCost * rows
 // * columns, kept when that gain is at least kHubMinGain of the nonzeros and
@@ -108,9 +107,9 @@ constexpr int kTunedSpmmGroupTypes = 3;
 // takes from it only the tiles lying inside it, so it uses a tier when those
 // hold at least kHubSddmmMinFill nonzeros per dense element (C3: both tiers,
 // 2526 x 72840 and rows of degree 1024..16383 x 3578 columns). It is used
-// with the tuned SpMM partition and the locality run order only. Results match the sparse path within FP32 summation order;
-// Inf / NaN in B reach exactly the rows that store their column; rows of the
-// block accumulate into C as the reference's do (they hold more than 32
+// with the tuned SpMM partition and the locality run order only. Results match
+// the sparse path within FP32 summation order; Inf / NaN in B reach exactly the
+// rows that store their column; rows of the block accumulate into C as the reference's do (they hold more than 32
 // nonzeros); a (row, column) slot stored more than once stays on the sparse
 // SpMM path. Cost: 4 bytes per block element (dense), 12 bytes per planned
 // SDDMM nonzero, the tuned partition's own grouping, signature sort and
