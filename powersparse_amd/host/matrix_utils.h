@@ -82,8 +82,8 @@ constexpr int kTunedSpmmGroupTypes = 3;
 // block, SDDMM on the public worksets with the block's tiles (64 consecutive
 // nonzeros of a block group) left out of the run order and their outputs
 // written from dense tiles of the product computed in registers. The block
-// comes in up to kHubMaxTiers tiers of disjoint row ranges, each with its own columns: the
-// first tier is the pair of power-of-two thresholds (row degree >= 2^a,
+// comes in up to kHubMaxTiers tiers of disjoint row ranges, each with its own
+// columns: the first tier is the pair of power-of-two thresholds (row degree >= 2^a,
 // column count >= 2^b) that maximises block nonzeros - kHubDenseCost * rows
 // * columns, kept when that gain is at least kHubMinGain of the nonzeros and
 // kHubMinGainNonzeros: below it the block's extra launches and the cheaper
